@@ -400,7 +400,7 @@ int rtt_prepare_external_a(const rtt_smatrix *host, const int *row_new_to_old,
     }
     auto t_tiles = rtt::Clock::now();
     RTT_TRY(rtt::build_tiles(*tiled, nullptr, a->active_rows, a->active_inner, host->m, host->n,
-                             false, dense_threshold, false, &a->tiles, &a->build));
+                             false, dense_threshold, &a->tiles, &a->build));
     RTT_TRY(rtt::fill_tile_row_of(&a->tiles));
     RTT_TRY(rtt::build_colmajor_values(&a->tiles));
     RTT_HIP(hipStreamSynchronize(rtt::ctx().stream));
@@ -487,11 +487,13 @@ int rtt_rebuild_b(const rtt_prepared_a *a_const, int aat, rtt_dynamic_b **inout,
         // B = A with rows gathered through the inner permutation, columns kept.
         st.path = 0;
         RTT_TRY(rtt::build_tiles(a->csr, inner_map, a->active_inner, a->cols, a->cols, a->cols,
-                                 true, a->dense_threshold, false, &b->tiles, &b->build));
+                                 true, a->dense_threshold, &b->tiles, &b->build, &a->tiles));
     } else if (a->row_identity) {
         // B = A^T straight from A's tiles.
         st.path = 1;
         RTT_TRY(rtt::transpose_tiles(a->tiles, a->rows, &b->tiles, &b->build));
+        RTT_TRY(rtt::build_pair_extents(a->tiles, &b->tiles));
+        RTT_HIP(hipStreamSynchronize(rtt::ctx().stream));
     } else {
         st.path = 2;
         auto tp = rtt::Clock::now();
@@ -499,12 +501,8 @@ int rtt_rebuild_b(const rtt_prepared_a *a_const, int aat, rtt_dynamic_b **inout,
         RTT_HIP(hipStreamSynchronize(rtt::ctx().stream));
         st.csr_row_permute_ms = rtt::ms_since(tp);
         RTT_TRY(rtt::build_tiles(a->csr_t, inner_map, a->active_inner, a->rows, a->cols, a->rows,
-                                 true, a->dense_threshold, false, &b->tiles, &b->build));
+                                 true, a->dense_threshold, &b->tiles, &b->build, &a->tiles));
     }
-    if (!b->tiles.transpose_of)   // the transpose writes its records itself
-        RTT_TRY(rtt::order_by_class(&b->tiles, &b->build));
-    RTT_TRY(rtt::build_pair_extents(a->tiles, &b->tiles));
-    RTT_HIP(hipStreamSynchronize(rtt::ctx().stream));
     b->a_id = a->id;
     ++b->gen;
     st.total_ms = rtt::ms_since(t0);
@@ -577,11 +575,8 @@ int rtt_rebuild_b_general(const rtt_prepared_a *a_const, const rtt_device_csr *s
     // B's rows through A's inner permutation, all of B's columns, and the
     // source-to-payload map for later values-only updates.
     RTT_TRY(rtt::build_tiles(src->csr, inner_map, a_const->active_inner, src->csr.cols,
-                             a_const->cols, src->csr.cols, true, a_const->dense_threshold, false,
-                             &b->tiles, &b->build, true));
-    RTT_TRY(rtt::order_by_class(&b->tiles, &b->build));
-    RTT_TRY(rtt::build_pair_extents(a_const->tiles, &b->tiles));
-    RTT_HIP(hipStreamSynchronize(rtt::ctx().stream));
+                             a_const->cols, src->csr.cols, true, a_const->dense_threshold,
+                             &b->tiles, &b->build, &a_const->tiles, true));
     b->a_id = a_const->id;
     ++b->gen;
     st.total_ms = rtt::ms_since(t0);

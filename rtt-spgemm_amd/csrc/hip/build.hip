@@ -1,13 +1,6 @@
-// CSR upload/validation and the CSR -> hybrid tile builders.
-//
-// Tiles are formed without a global sort: rows are kept column-sorted (they
-// are sorted once at upload when they arrive unsorted), so the tiles of one
-// tile row are the ordered merge of its TR row streams.  A group of TR lanes
-// owns one tile row; each lane walks one scalar row.  The group repeatedly
-// takes the minimum tile column among its lanes' heads, ORs the lanes' bits
-// into the tile mask and writes the tile.  This replaces the reference's
-// 64-bit key radix sort + reduce_by_key (src/gpu_dmma_tiles.h:1117-1395) and
-// its 4-lane ordered-warp B path (src/gpu_dmma_tiles.h:313-560).
+// CSR upload/validation, B = A^T from A's tiles, and what the SpGEMM core
+// reads beside the tiles (records, pair extents, tile columns).  The CSR ->
+// tile builder is in tilebuild.hip.
 #include <atomic>
 #include <hipcub/hipcub.hpp>
 
@@ -59,22 +52,11 @@ __global__ void gather_f64_kernel(int64_t n, const int *__restrict__ idx,
         out[i] = in[idx[i]];
 }
 
-// Position of physical slot `phys` in the tile's values_cm order: stride-4
-// group k = phys & 3 first, then by phys >> 2 within the group.
-__device__ __forceinline__ int kmajor_slot(uint32_t mask, int phys)
-{
-    const int k = phys & 3;
-    const uint32_t lower_groups = k == 0 ? 0u : (k == 1 ? 0x11111111u
-                                                : (k == 2 ? 0x33333333u : 0x77777777u));
-    const uint32_t group = mask & (0x11111111u << k);
-    return __popc(mask & lower_groups) + __popc(group & ((1u << phys) - 1u));
-}
-
 // flags: 1 row_ptr not monotone / wrong ends, 2 column out of range,
 //        4 some row not column-sorted (duplicates allowed).
 __global__ void validate_csr_kernel(int rows, int cols, int64_t nnz,
                                     const int *__restrict__ rp,
-                                    const int *__restrict__ ci, int *flags)
+                                    const int *__restrict__ ci, int *flags, int *max_row)
 {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i == 0 && (rp[0] != 0 || rp[rows] != nnz))
@@ -85,6 +67,8 @@ __global__ void validate_csr_kernel(int rows, int cols, int64_t nnz,
         if (b < 0 || e < b || static_cast<int64_t>(e) > nnz) {
             atomicOr(flags, 1);
         } else {
+            if (e - b > __hip_atomic_load(max_row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(max_row, e - b);
             for (int x = b + 1; x < e; ++x)
                 if (ci[x] < ci[x - 1]) {
                     atomicOr(flags, 4);
@@ -97,223 +81,6 @@ __global__ void validate_csr_kernel(int rows, int cols, int64_t nnz,
         if (c < 0 || c >= cols)
             atomicOr(flags, 2);
     }
-}
-
-// Columns of its 64 rows a wave stages in LDS before the walk (when the rows
-// are contiguous in the CSR and fit), so that the lanes' entry-by-entry walk
-// reads LDS instead of issuing one dependent global load per entry.  The
-// stage is sized per launch (dynamic LDS, at most kBuildStage columns per
-// wave) from the operand's average row length: a fixed 3072-column stage
-// held the kernel to 3 waves per SIMD on every operand.
-constexpr int kBuildStage = 3072;
-
-int build_stage_cap(const DevCsr &src, bool row_map)
-{
-    if (row_map || src.rows <= 0)
-        return 0;   // a row map disables the staging
-    const double per_wave = 1.5 * kWave * static_cast<double>(src.nnz) / src.rows;
-    const int cap = (static_cast<int>(per_wave) + 255) / 256 * 256;
-    return std::min(kBuildStage, std::max(256, cap));
-}
-
-// One group of TR lanes per tile row.  COUNT pass: per tile row the number of
-// tiles, payload slots and dense tiles.  FILL pass: tile columns, masks,
-// value offsets and payload.  Duplicates (adjacent equal columns in a sorted
-// row) are summed in row order.
-template <int TR, int TC, bool COL_MAJOR, bool FILL>
-__global__ __launch_bounds__(kThreads) void tile_build_kernel(
-    int tile_row_count, int active_rows, int active_cols,
-    const int *__restrict__ rp, const int *__restrict__ ci,
-    const double *__restrict__ val, const int *__restrict__ row_map,
-    int dense_threshold, int64_t *__restrict__ row_tiles,
-    int64_t *__restrict__ row_payload, int64_t *__restrict__ row_dense,
-    const int64_t *__restrict__ tile_off, const int64_t *__restrict__ payload_off,
-    int *__restrict__ tile_col_idx, uint32_t *__restrict__ masks,
-    int *__restrict__ value_offsets, double *__restrict__ values, int4 *__restrict__ meta,
-    int2 *__restrict__ src_slot, int *__restrict__ dup_flag, int stage_cap)
-{
-    static_assert(TR * TC == 32, "tiles hold 32 elements");
-    static_assert(kWave % TR == 0, "a wave holds whole tile rows");
-    extern __shared__ int s_build_stage[];   // stage_cap columns per wave
-    const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    // Row gid (= tile row gid / TR, row gid % TR of it).  The wave's rows are
-    // 64 consecutive rows; without a row map their entries are one stretch
-    // of the CSR, whose first stage_cap columns are staged in LDS (all of
-    // them when they fit).
-    const int64_t wave_row0 = gid - lane_id();
-    const int64_t lim = min<int64_t>(static_cast<int64_t>(tile_row_count) * TR, active_rows);
-    int e0 = 0, ns = 0;
-    if (!row_map && wave_row0 < lim) {
-        e0 = rp[wave_row0];
-        ns = min(rp[min<int64_t>(wave_row0 + kWave, lim)] - e0, stage_cap);
-    }
-    int *stage = s_build_stage + (threadIdx.x / kWave) * stage_cap;
-    for (int x = lane_id(); x < ns; x += kWave)
-        stage[x] = ci[e0 + x];
-    wave_sync();
-    auto col = [&](int x) { return x - e0 < ns ? stage[x - e0] : ci[x]; };
-    const int64_t tr = gid / TR;
-    const int r = static_cast<int>(gid % TR);
-    if (tr >= tile_row_count)
-        return;   // whole groups leave together
-    const int64_t row = tr * TR + r;
-    int p = 0, end = 0;
-    if (row < active_rows) {
-        const int src = row_map ? row_map[row] : static_cast<int>(row);
-        p = rp[src];
-        end = rp[src + 1];
-    }
-    // Columns at or beyond active_cols are outside the tiled extent.
-    while (end > p && col(end - 1) >= active_cols)
-        --end;
-
-    int64_t ntiles = 0, payload = 0, ndense = 0;
-    int64_t t_out = FILL ? tile_off[tr] : 0;
-    int64_t p_out = FILL ? payload_off[tr] : 0;
-    for (;;) {
-        int head = p < end ? col(p) / TC : INT_MAX;
-#pragma unroll
-        for (int o = TR / 2; o > 0; o >>= 1)
-            head = min(head, __shfl_xor(head, o, TR));
-        if (head == INT_MAX)
-            break;
-        uint32_t bits = 0;
-        int q = p;
-        if (p + TC - e0 <= ns) {
-            // The first TC columns from p, staged in LDS, are read together;
-            // without duplicates a row has at most TC entries in a tile.
-            // (Unstaged, the extra reads would be global loads of columns
-            // past a sparse tile's few entries.)
-            int cb[TC];
-#pragma unroll
-            for (int u = 0; u < TC; ++u)
-                cb[u] = p + u < end ? col(p + u) : -1;
-            bool in_tile = true;
-#pragma unroll
-            for (int u = 0; u < TC; ++u) {
-                in_tile = in_tile && cb[u] >= 0 && cb[u] / TC == head;
-                if (in_tile) {
-                    const int lc = cb[u] % TC;
-                    bits |= 1u << (COL_MAJOR ? lc * TR + r : r * TC + lc);
-                    ++q;
-                }
-            }
-        }
-        while (q < end) {   // the rest (all of it when unstaged)
-            const int c = col(q);
-            if (c / TC != head)
-                break;
-            const int lc = c % TC;
-            bits |= 1u << (COL_MAJOR ? lc * TR + r : r * TC + lc);
-            ++q;
-        }
-        uint32_t mask = bits;
-#pragma unroll
-        for (int o = TR / 2; o > 0; o >>= 1)
-            mask |= __shfl_xor(mask, o, TR);
-        const int cnt = __popc(mask);
-        const bool dense = cnt >= dense_threshold;
-        if constexpr (FILL) {
-            if (r == 0) {
-                tile_col_idx[t_out] = head;
-                masks[t_out] = mask;
-                value_offsets[t_out] = static_cast<int>(p_out);
-                uint32_t bytes = 0;
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    bytes |= stride4_bits(mask, k) << (8 * k);
-                meta[t_out] = make_int4(head, static_cast<int>(mask), static_cast<int>(bytes),
-                                        static_cast<int>(p_out) | (dense ? INT_MIN : 0));
-            }
-            if (dense) {
-                // Absent slots of this lane's row are explicit zeros.
-#pragma unroll
-                for (int lc = 0; lc < TC; ++lc) {
-                    const int phys = COL_MAJOR ? lc * TR + r : r * TC + lc;
-                    if (!(bits & (1u << phys)))
-                        values[p_out + phys] = 0.0;
-                }
-            }
-            // Sum of source entries x0 .. x-1 (duplicates of column c, in
-            // entry order) into its payload slot.
-            auto store = [&](int c, double s, int x0, int x) {
-                const int lc = c % TC;
-                const int phys = COL_MAJOR ? lc * TR + r : r * TC + lc;
-                const int slot = static_cast<int>(p_out) + payload_slot(mask, dense ? 32 : cnt, phys);
-                values[slot] = s;
-                if (src_slot) {
-                    const int2 sl = make_int2(slot, static_cast<int>(p_out) + kmajor_slot(mask, phys));
-                    for (int y = x0; y < x; ++y)
-                        src_slot[y] = sl;
-                    if (x - x0 > 1)
-                        *dup_flag = 1;
-                }
-            };
-            if (q - p == 1) {
-                store(col(p), val[p], p, q);   // the common case of sparse operands
-            } else if (!row_map && q - p <= TC) {
-                // At most TC entries (always, without duplicates): their
-                // values are loaded together, not one dependent load each.
-                // (Measured slower for rows gathered through a row map.)
-                double vb[TC];
-#pragma unroll
-                for (int u = 0; u < TC; ++u)
-                    vb[u] = p + u < q ? val[p + u] : 0.0;
-                int cprev = -1, x0 = p;
-                double s = 0.0;
-#pragma unroll
-                for (int u = 0; u < TC; ++u) {
-                    if (p + u < q) {
-                        const int c = col(p + u);
-                        if (c != cprev) {
-                            if (cprev >= 0)
-                                store(cprev, s, x0, p + u);
-                            cprev = c;
-                            x0 = p + u;
-                            s = vb[u];
-                        } else {
-                            s += vb[u];
-                        }
-                    }
-                }
-                if (cprev >= 0)
-                    store(cprev, s, x0, q);
-            } else {
-                int x = p;
-                while (x < q) {
-                    const int c = col(x);
-                    const int x0 = x;
-                    double s = val[x];
-                    ++x;
-                    while (x < q && col(x) == c) {
-                        s += val[x];
-                        ++x;
-                    }
-                    store(c, s, x0, x);
-                }
-            }
-            ++t_out;
-            p_out += dense ? 32 : cnt;
-        }
-        ++ntiles;
-        payload += dense ? 32 : cnt;
-        ndense += dense ? 1 : 0;
-        p = q;
-    }
-    if constexpr (!FILL) {
-        if (r == 0) {
-            row_tiles[tr] = ntiles;
-            row_payload[tr] = payload;
-            row_dense[tr] = ndense;
-        }
-    }
-}
-
-__global__ void gather3_kernel(const int64_t *a, const int64_t *b, const int64_t *c, int64_t *out)
-{
-    out[0] = *a;
-    out[1] = *b;
-    out[2] = *c;
 }
 
 __global__ void narrow_i64_kernel(const int64_t *in, int *out, int64_t n)
@@ -410,17 +177,76 @@ __global__ void row_ptr_from_sorted_kernel(const int *__restrict__ keys, int64_t
         ptr[k] = static_cast<int>(i);
 }
 
-// Part `part` of a tile's record (meta, then the first kRecVals values of
-// the tile's k-major payload: row k's entries contiguous, columns ascending).
-// Parts of a record that hold something: the meta, then one part per two of
-// the tile's first kRecVals values.  The kernels that read records use a
-// value only when the tile has it, so the parts past these are never used;
-// the writers that hold the meta anyway skip them.
-__device__ __forceinline__ int record_parts_used(const int4 &m)
+// Value planes (1 .. kRecParts-1) of B's records and the k-major copy of what
+// they do not hold, from the payload: one tile per thread.  A record holds
+// its tile's first kRecVals values in k-major order (row k's entries
+// contiguous, columns ascending); the values past them go to the same places
+// of the k-major copy, whose first kRecVals slots per tile nothing reads.
+// All of the record's values are loaded before the first plane is written;
+// consecutive threads write consecutive entries of every plane.  The planes
+// past a tile's values are never read.  Against a re-pack of every value
+// into the copy followed by a pass from the copy to the planes: one read of
+// the payload instead of two, and no copy at all for tiles of up to kRecVals
+// entries (AMG batch of 8: 0.58 ms for the two passes before).
+__global__ void record_values_kernel(int64_t n, const double *__restrict__ vals,
+                                     int4 *__restrict__ planes, double *__restrict__ kmajor)
 {
-    return 1 + (min(kRecVals, __popc(static_cast<uint32_t>(m.y))) + 1) / 2;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= n)
+        return;
+    const int4 m = planes[t];
+    const uint32_t mask = static_cast<uint32_t>(m.y);
+    const bool dense = m.w < 0;
+    const uint32_t off = static_cast<uint32_t>(m.w) & 0x7FFFFFFFu;
+    const int nv = __popc(mask);
+    uint32_t mz = static_cast<uint32_t>(m.z);   // bit k * 8 + c
+    // Next entry's value: bit c * 4 + k of the payload's order.
+    auto next = [&]() {
+        const int pos = __builtin_ctz(mz);
+        mz &= mz - 1;
+        const int phys = (pos & 7) * 4 + (pos >> 3);
+        return vals[off + (dense ? phys : __popc(mask & ((1u << phys) - 1u)))];
+    };
+    double v[kRecVals];
+#pragma unroll
+    for (int j = 0; j < kRecVals; ++j)
+        v[j] = mz ? next() : 0.0;
+#pragma unroll
+    for (int part = 1; part < kRecParts; ++part)
+        if (2 * (part - 1) < nv)
+            planes[part * n + t] = *reinterpret_cast<const int4 *>(
+                &reinterpret_cast<const double2 *>(v)[part - 1]);
+    for (int j = kRecVals; mz; j += kRecVals) {
+#pragma unroll
+        for (int u = 0; u < kRecVals; ++u)
+            v[u] = mz ? next() : 0.0;
+#pragma unroll
+        for (int u = 0; u < kRecVals; ++u)
+            if (j + u < nv)
+                kmajor[off + j + u] = v[u];
+    }
 }
 
+// Values-only update: the first source entry of each slot's run sums the
+// run in entry order (the order the tile build sums duplicates in).  Runs
+// are adjacent because duplicates of a coordinate are adjacent in a
+// row-sorted CSR.
+__global__ void scatter_runs_kernel(int64_t nnz, const int *__restrict__ slot,
+                                    const double *__restrict__ v, double *__restrict__ values)
+{
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (e >= nnz)
+        return;
+    const int s = slot[e];
+    if (s < 0 || (e > 0 && slot[e - 1] == s))
+        return;
+    double sum = v[e];
+    for (int64_t f = e + 1; f < nnz && slot[f] == s; ++f)
+        sum += v[f];
+    values[s] = sum;
+}
+
+// Part `part` of the record of a tile with meta m and k-major payload.
 __device__ __forceinline__ int4 record_part(int part, const int4 &m, const double *kmajor)
 {
     if (part == 0)
@@ -432,55 +258,6 @@ __device__ __forceinline__ int4 record_part(int part, const int4 &m, const doubl
     v.x = j < nv ? kmajor[off + j] : 0.0;
     v.y = j + 1 < nv ? kmajor[off + j + 1] : 0.0;
     return *reinterpret_cast<const int4 *>(&v);
-}
-
-// Value parts (1 .. kRecParts-1) of B's record planes, one tile per thread;
-// part 0 (meta) is left as it is.  A thread reads its tile's first values
-// once (one contiguous stretch, consecutive tiles' stretches adjacent) and
-// writes each plane's entry (consecutive threads, consecutive entries).
-__global__ void record_values_kernel(int64_t n, const int4 *__restrict__ meta,
-                                     const double *__restrict__ kmajor,
-                                     int4 *__restrict__ planes)
-{
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n)
-        return;
-    const int4 m = meta[t];
-    const int used = record_parts_used(m);
-    // Every value the record holds is loaded before any plane is written.
-    const uint32_t off = static_cast<uint32_t>(m.w) & 0x7FFFFFFFu;
-    const int nv = min(kRecVals, __popc(static_cast<uint32_t>(m.y)));
-    double v[kRecVals];
-#pragma unroll
-    for (int j = 0; j < kRecVals; ++j)
-        v[j] = j < nv ? kmajor[off + j] : 0.0;
-#pragma unroll
-    for (int part = 1; part < kRecParts; ++part)
-        if (part < used)
-            planes[part * n + t] = *reinterpret_cast<const int4 *>(
-                &reinterpret_cast<const double2 *>(v)[part - 1]);
-}
-
-// Values-only update: the first source entry of each slot's run sums the
-// run in entry order (the order the tile build sums duplicates in) and
-// stores the sum into both payload layouts.  Runs are adjacent because
-// duplicates of a coordinate are adjacent in a row-sorted CSR.
-__global__ void scatter_runs_kernel(int64_t nnz, const int2 *__restrict__ slot,
-                                    const double *__restrict__ v, double *__restrict__ values,
-                                    double *__restrict__ kmajor)
-{
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e >= nnz)
-        return;
-    const int2 s = slot[e];
-    if (s.x < 0 || (e > 0 && slot[e - 1].x == s.x))
-        return;
-    double sum = v[e];
-    for (int64_t f = e + 1; f < nnz && slot[f].x == s.x; ++f)
-        sum += v[f];
-    values[s.x] = sum;
-    if (kmajor)
-        kmajor[s.y] = sum;
 }
 
 // Offline, per A tile: the record a B tile built as A^T takes over, its meta
@@ -665,8 +442,12 @@ __global__ void __launch_bounds__(kThreads) column_max_kernel(int cols, int *__r
 // one column k, only the light tiles of row k can meet it.
 __global__ __launch_bounds__(kThreads) void pair_extent_kernel(
     int64_t n, const int4 *__restrict__ a_meta, const int *__restrict__ groups,
-    int4 *__restrict__ out, int2 *__restrict__ light, unsigned long long *__restrict__ pairs)
+    int4 *__restrict__ out, int2 *__restrict__ light, unsigned long long *__restrict__ pairs,
+    const unsigned int *__restrict__ flag, long long *__restrict__ flag_out)
 {
+    // Passes the tile build's duplicate flag on to the host's buffer.
+    if (flag && blockIdx.x == 0 && threadIdx.x == 0)
+        *flag_out = *flag;
     // Grid-stride, so that the pair total takes one atomic per workgroup.
     __shared__ unsigned long long s_sum[kThreads / kWave];
     unsigned long long sum = 0;
@@ -703,147 +484,6 @@ __global__ __launch_bounds__(kThreads) void pair_extent_kernel(
     }
 }
 
-// Stable partition of each B row's tiles by class (tiles arrive in column
-// order): the order a stable sort by (row, class) gives.  Rows of up to
-// kPartRow tiles take one thread, which packs its per-class counts into the
-// bytes of a 64-bit word; longer rows are listed for a wave each.
-constexpr int kPartRow = 64;
-constexpr int kPartBatch = 8;    // metas a thread loads at once
-constexpr int kClassesUsed = 5;   // heavy, light k = 0..3
-
-__device__ __forceinline__ int meta_class(const int4 &m)
-{
-    return b_tile_class(static_cast<uint32_t>(m.y), static_cast<uint32_t>(m.z));
-}
-
-__global__ void class_partition_kernel(int R, const int *__restrict__ trp,
-                                       const int4 *__restrict__ meta, int4 *__restrict__ out,
-                                       int4 *__restrict__ plane0, int *__restrict__ groups,
-                                       int *__restrict__ long_rows, int *__restrict__ n_long)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r > R)
-        return;
-    const int s = trp[r];
-    if (r == R) {
-        groups[static_cast<int64_t>(kClassSlots) * R] = s;
-        return;
-    }
-    const int e = trp[r + 1];
-    if (e - s > kPartRow) {
-        long_rows[atomicAdd(n_long, 1)] = r;
-        return;
-    }
-    // The row's metas come kPartBatch at a time, loads issued together; a
-    // row of at most kPartBatch tiles keeps them for the placing pass.
-    int4 m[kPartBatch];
-#pragma unroll
-    for (int u = 0; u < kPartBatch; ++u)
-        m[u] = make_int4(0, 0, 0, 0);
-    unsigned long long cnt = 0;   // byte c: tiles of class c
-    for (int x0 = s; x0 < e; x0 += kPartBatch) {
-#pragma unroll
-        for (int u = 0; u < kPartBatch; ++u)
-            if (x0 + u < e)
-                m[u] = meta[x0 + u];
-#pragma unroll
-        for (int u = 0; u < kPartBatch; ++u)
-            if (x0 + u < e)
-                cnt += 1ull << (8 * meta_class(m[u]));
-    }
-    // Byte c: tiles of classes below c (at most kPartRow, so no carries).
-    unsigned long long pos = (cnt << 8) * 0x0101010101010101ull;
-    int *g = groups + static_cast<int64_t>(kClassSlots) * r;
-#pragma unroll
-    for (int c = 0; c < kClassSlots; ++c)
-        g[c] = s + static_cast<int>((pos >> (8 * c)) & 0xFFu);
-    const bool held = e - s <= kPartBatch;
-    for (int x0 = s; x0 < e; x0 += kPartBatch) {
-        if (!held) {
-#pragma unroll
-            for (int u = 0; u < kPartBatch; ++u)
-                if (x0 + u < e)
-                    m[u] = meta[x0 + u];
-        }
-#pragma unroll
-        for (int u = 0; u < kPartBatch; ++u) {
-            if (x0 + u < e) {
-                const int c = meta_class(m[u]);
-                const int p = s + static_cast<int>((pos >> (8 * c)) & 0xFFu);
-                pos += 1ull << (8 * c);
-                out[p] = m[u];
-                plane0[p] = m[u];
-            }
-        }
-    }
-}
-
-// The listed long rows, a wave each: class counts by ballot, then every
-// tile placed after the row's tiles of lower classes and the earlier tiles
-// of its own.
-__global__ void __launch_bounds__(kThreads)
-    class_partition_long_kernel(const int *__restrict__ trp, const int4 *__restrict__ meta,
-                                int4 *__restrict__ out, int4 *__restrict__ plane0,
-                                int *__restrict__ groups, const int *__restrict__ long_rows,
-                                const int *__restrict__ n_long)
-{
-    const int lane = lane_id();
-    const int waves = gridDim.x * (blockDim.x / kWave);
-    const int count = *n_long;
-    const uint64_t below = (1ull << lane) - 1ull;
-    for (int i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; i < count; i += waves) {
-        const int r = long_rows[i];
-        const int s = trp[r], e = trp[r + 1];
-        int run[kClassesUsed];
-#pragma unroll
-        for (int c = 0; c < kClassesUsed; ++c)
-            run[c] = 0;
-        for (int x0 = s; x0 < e; x0 += kWave) {
-            const int x = x0 + lane;
-            const int c = x < e ? meta_class(meta[x]) : -1;
-#pragma unroll
-            for (int k = 0; k < kClassesUsed; ++k)
-                run[k] += __popcll(__ballot(c == k));
-        }
-        int start = s;
-#pragma unroll
-        for (int k = 0; k < kClassesUsed; ++k) {
-            const int nk = run[k];
-            run[k] = start;
-            start += nk;
-        }
-        if (lane < kClassSlots) {
-            int v = e;
-#pragma unroll
-            for (int k = 0; k < kClassesUsed; ++k)
-                if (lane == k)
-                    v = run[k];
-            groups[static_cast<int64_t>(kClassSlots) * r + lane] = v;
-        }
-        for (int x0 = s; x0 < e; x0 += kWave) {
-            const int x = x0 + lane;
-            int4 m = make_int4(0, 0, 0, 0);
-            int c = -1;
-            if (x < e) {
-                m = meta[x];
-                c = meta_class(m);
-            }
-            int p = 0;
-#pragma unroll
-            for (int k = 0; k < kClassesUsed; ++k) {
-                const uint64_t b = __ballot(c == k);
-                if (c == k)
-                    p = run[k] + __popcll(b & below);
-                run[k] += __popcll(b);
-            }
-            if (x < e) {
-                out[p] = m;
-                plane0[p] = m;
-            }
-        }
-    }
-}
-
 // Sort key of a B tile: its row times kClassSlots plus its class.
 __global__ void class_keys_kernel(int64_t n, const int *__restrict__ row,
                                   const int4 *__restrict__ meta, int *__restrict__ keys)
@@ -863,20 +503,6 @@ __global__ void group_row_ptr_kernel(int rows, const int *__restrict__ groups,
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r <= rows)
         trp[r] = groups[static_cast<int64_t>(kClassSlots) * r];
-}
-
-// Gathers a B's meta into class order (the record value planes are built
-// afterwards, from the ordered meta, when a kernel needs them).
-__global__ void gather_meta_kernel(int64_t n, const int *__restrict__ perm,
-                                   const int4 *__restrict__ meta_in, int4 *__restrict__ meta_out,
-                                   int4 *__restrict__ plane0)
-{
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n)
-        return;
-    const int4 m = meta_in[perm[t]];
-    meta_out[t] = m;
-    plane0[t] = m;
 }
 
 __global__ void entry_rows_kernel(int rows, const int *__restrict__ rp,
@@ -998,86 +624,6 @@ int build_csc(DevTiles *t, BuildWork *w)
     return RTT_OK;
 }
 
-template <int TR, int TC, bool CM>
-int run_tile_build(const DevCsr &src, const int *row_map, int active_rows,
-                   int active_cols, int dense_threshold, DevTiles *out,
-                   BuildWork *w, int2 *src_slot, int *dup_flag)
-{
-    hipStream_t s = ctx().stream;
-    const int R = out->tile_row_count;
-    RTT_TRY(w->row_tiles.ensure((R + 1) * sizeof(int64_t)));
-    RTT_TRY(w->row_payload.ensure((R + 1) * sizeof(int64_t)));
-    RTT_TRY(w->row_dense.ensure((R + 1) * sizeof(int64_t)));
-    // counters: [0, R] tile prefix, [R+1, 2R+1] payload prefix, then dense sum
-    RTT_TRY(w->counters.ensure((2 * (R + 1) + 1) * sizeof(int64_t)));
-    int64_t *tile_pre = w->counters.as<int64_t>();
-    int64_t *pay_pre = tile_pre + (R + 1);
-    int64_t *dense_pre = w->spans.ensure((R + 1) * sizeof(int64_t)) == RTT_OK
-                             ? w->spans.as<int64_t>()
-                             : nullptr;
-    if (!dense_pre)
-        return RTT_ERR_OOM;
-    hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(1), 0, s, w->row_tiles.as<int64_t>() + R,
-                       int64_t(1), int64_t(0));
-    hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(1), 0, s,
-                       w->row_payload.as<int64_t>() + R, int64_t(1), int64_t(0));
-    hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(1), 0, s, w->row_dense.as<int64_t>() + R,
-                       int64_t(1), int64_t(0));
-    const int64_t threads_total = static_cast<int64_t>(R) * TR;
-    const int stage_cap = build_stage_cap(src, row_map != nullptr);
-    const size_t stage_bytes = static_cast<size_t>(kThreads / kWave) * stage_cap * sizeof(int);
-    if (R > 0)
-        hipLaunchKernelGGL((tile_build_kernel<TR, TC, CM, false>),
-                           dim3(blocks_for(threads_total, kThreads)), dim3(kThreads), stage_bytes,
-                           s, R, active_rows, active_cols, src.row_ptr.as<int>(),
-                           src.col_idx.as<int>(), src.values.as<double>(), row_map,
-                           dense_threshold, w->row_tiles.as<int64_t>(),
-                           w->row_payload.as<int64_t>(), w->row_dense.as<int64_t>(),
-                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                           nullptr, nullptr, stage_cap);
-    RTT_HIP(hipGetLastError());
-    RTT_TRY(exclusive_scan_i64(w->row_tiles.as<int64_t>(), tile_pre, R, &w->scan_tmp, s));
-    RTT_TRY(exclusive_scan_i64(w->row_payload.as<int64_t>(), pay_pre, R, &w->scan_tmp, s));
-    RTT_TRY(exclusive_scan_i64(w->row_dense.as<int64_t>(), dense_pre, R, &w->scan_tmp, s));
-    // The three totals in one readback.
-    int64_t totals[3] = {0, 0, 0};
-    RTT_TRY(w->totals.ensure(3 * sizeof(int64_t)));
-    hipLaunchKernelGGL(gather3_kernel, dim3(1), dim3(1), 0, s, tile_pre + R, pay_pre + R,
-                       dense_pre + R, w->totals.as<int64_t>());
-    RTT_HIP(hipMemcpyAsync(totals, w->totals.ptr, sizeof(totals), hipMemcpyDeviceToHost, s));
-    RTT_HIP(hipStreamSynchronize(s));
-    if (totals[0] > INT_MAX || totals[1] > INT_MAX)
-        return fail(RTT_ERR_OVERFLOW,
-                    "tile count %lld or payload %lld exceeds the int32 tile ABI",
-                    (long long)totals[0], (long long)totals[1]);
-    out->num_tiles = totals[0];
-    out->payload = totals[1];
-    out->dense = totals[2];
-    out->sparse = totals[0] - totals[2];
-    RTT_TRY(out->tile_row_ptr.ensure((R + 1) * sizeof(int)));
-    RTT_TRY(out->tile_col_idx.ensure(out->num_tiles * sizeof(int)));
-    RTT_TRY(out->masks.ensure(out->num_tiles * sizeof(uint32_t)));
-    RTT_TRY(out->value_offsets.ensure((out->num_tiles + 1) * sizeof(int)));
-    RTT_TRY(out->values.ensure(out->payload * sizeof(double)));
-    RTT_TRY(out->meta.ensure(out->num_tiles * sizeof(int4)));
-    hipLaunchKernelGGL(narrow_i64_kernel, dim3(blocks_for(R + 1, kThreads)), dim3(kThreads), 0,
-                       s, tile_pre, out->tile_row_ptr.as<int>(), static_cast<int64_t>(R) + 1);
-    // value_offsets[num_tiles] = payload total.
-    hipLaunchKernelGGL(narrow_i64_kernel, dim3(1), dim3(1), 0, s, pay_pre + R,
-                       out->value_offsets.as<int>() + out->num_tiles, int64_t(1));
-    if (R > 0 && out->num_tiles > 0)
-        hipLaunchKernelGGL((tile_build_kernel<TR, TC, CM, true>),
-                           dim3(blocks_for(threads_total, kThreads)), dim3(kThreads), stage_bytes,
-                           s, R, active_rows, active_cols, src.row_ptr.as<int>(),
-                           src.col_idx.as<int>(), src.values.as<double>(), row_map,
-                           dense_threshold, nullptr, nullptr, nullptr, tile_pre, pay_pre,
-                           out->tile_col_idx.as<int>(), out->masks.as<uint32_t>(),
-                           out->value_offsets.as<int>(), out->values.as<double>(),
-                           out->meta.as<int4>(), src_slot, dup_flag, stage_cap);
-    RTT_HIP(hipGetLastError());
-    return RTT_OK;
-}
-
 } // namespace
 
 void DevTiles::view(rtt_device_tiles *v) const
@@ -1102,70 +648,40 @@ void DevTiles::view(rtt_device_tiles *v) const
     v->csc_tile_ids = has_csc ? csc_tile_ids.as<int>() : nullptr;
 }
 
+static int write_record_values(DevTiles *b)
+{
+    RTT_TRY(b->values_cm.ensure(static_cast<size_t>(b->payload > 0 ? b->payload : 1) *
+                                sizeof(double)));
+    if (b->num_tiles > 0)
+        hipLaunchKernelGGL(record_values_kernel, dim3(blocks_for(b->num_tiles, kThreads)),
+                           dim3(kThreads), 0, ctx().stream, b->num_tiles, b->values.as<double>(),
+                           b->records.as<int4>(), b->values_cm.as<double>());
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
+}
+
 int ensure_record_values(DevTiles *b)
 {
     if (b->transpose_of || b->rec_values_ready)
         return RTT_OK;
-    RTT_TRY(build_colmajor_values(b));
-    RTT_TRY(b->records.ensure(b->num_tiles * sizeof(BRecord)));
-    if (b->num_tiles > 0)
-        hipLaunchKernelGGL(record_values_kernel, dim3(blocks_for(b->num_tiles, kThreads)),
-                           dim3(kThreads), 0, ctx().stream, b->num_tiles, b->meta.as<int4>(),
-                           b->values_cm.as<double>(), b->records.as<int4>());
-    RTT_HIP(hipGetLastError());
+    RTT_TRY(write_record_values(b));
     b->rec_values_ready = true;
     return RTT_OK;
 }
 
-int build_pair_extents(const DevTiles &a, DevTiles *b)
+int build_pair_extents(const DevTiles &a, DevTiles *b, const unsigned int *flag,
+                       long long *flag_out)
 {
     RTT_TRY(b->a_brange.ensure(a.num_tiles * sizeof(int4)));
     RTT_TRY(b->a_blight.ensure(a.num_tiles * sizeof(int2)));
-    RTT_TRY(b->pair_total.ensure(sizeof(unsigned long long)));
     hipStream_t s = ctx().stream;
-    hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(1), 0, s, b->pair_total.as<int64_t>(),
-                       int64_t(1), int64_t(0));
     const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    if (a.num_tiles > 0)
-        hipLaunchKernelGGL(pair_extent_kernel,
-                           dim3(static_cast<unsigned>(std::min<int64_t>(4 * cus, blocks_for(a.num_tiles, kThreads)))),
-                           dim3(kThreads), 0, s, a.num_tiles, a.meta.as<int4>(),
-                           b->row_groups.as<int>(), b->a_brange.as<int4>(),
-                           b->a_blight.as<int2>(), b->pair_total.as<unsigned long long>());
-    RTT_HIP(hipGetLastError());
-    return RTT_OK;
-}
-
-int order_by_class(DevTiles *b, BuildWork *w)
-{
-    hipStream_t s = ctx().stream;
-    const int64_t n = b->num_tiles;
-    const int R = b->tile_row_count;
-    const int64_t slots = static_cast<int64_t>(kClassSlots) * R;
-    RTT_TRY(b->row_groups.ensure((slots + 1) * sizeof(int)));
-    RTT_TRY(w->keys_in.ensure((static_cast<size_t>(R) + 1) * sizeof(int)));   // long rows
-    RTT_TRY(w->keys_out.ensure(sizeof(int)));                                 // their count
-    RTT_TRY(w->meta2.ensure((n > 0 ? n : 1) * sizeof(int4)));
-    RTT_TRY(b->records.ensure((n > 0 ? n : 1) * sizeof(BRecord)));
-    int *n_long = w->keys_out.as<int>();
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(1), 0, s, n_long, int64_t(1), 0);
-    // Meta in class order, also as record plane 0; the value planes follow
-    // from it in ensure_record_values.
-    hipLaunchKernelGGL(class_partition_kernel, dim3(blocks_for(static_cast<int64_t>(R) + 1, kThreads)),
-                       dim3(kThreads), 0, s, R, b->tile_row_ptr.as<int>(), b->meta.as<int4>(),
-                       w->meta2.as<int4>(), b->records.as<int4>(), b->row_groups.as<int>(),
-                       w->keys_in.as<int>(), n_long);
-    if (n > kPartRow) {
-        const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-        hipLaunchKernelGGL(class_partition_long_kernel, dim3(static_cast<unsigned>(2 * cus)),
-                           dim3(kThreads), 0, s, b->tile_row_ptr.as<int>(), b->meta.as<int4>(),
-                           w->meta2.as<int4>(), b->records.as<int4>(), b->row_groups.as<int>(),
-                           w->keys_in.as<int>(), n_long);
-    }
-    if (n > 0)
-        RTT_HIP(hipMemcpyAsync(b->meta.ptr, w->meta2.ptr, n * sizeof(int4),
-                               hipMemcpyDeviceToDevice, s));
-    b->rec_values_ready = false;
+    const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(
+        4 * cus, std::max<int64_t>(1, blocks_for(a.num_tiles, kThreads))));
+    hipLaunchKernelGGL(pair_extent_kernel, dim3(blocks), dim3(kThreads), 0, s, a.num_tiles,
+                       a.meta.as<int4>(), b->row_groups.as<int>(), b->a_brange.as<int4>(),
+                       b->a_blight.as<int2>(), b->pair_total.as<unsigned long long>(), flag,
+                       flag_out);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
@@ -1209,14 +725,14 @@ int build_b_columns(DevTiles *b, BuildWork *w)
         RTT_TRY(w->ids_in.ensure(n * sizeof(int)));
         RTT_TRY(w->ids_out.ensure(n * sizeof(int)));
         hipLaunchKernelGGL(column_keys_kernel, dim3(blocks_for(n, kThreads)), dim3(kThreads), 0, s,
-                           n, b->meta.as<int4>(), w->keys_in.as<int>());
+                           n, b->records.as<int4>(), w->keys_in.as<int>());
         hipLaunchKernelGGL(iota_kernel, dim3(blocks_for(n, kThreads)), dim3(kThreads), 0, s,
                            w->ids_in.as<int>(), n);
         RTT_TRY(sort_pairs(w->keys_in.as<int>(), w->keys_out.as<int>(), w->ids_in.as<int>(),
                            w->ids_out.as<int>(), n, bits_for(BC), &w->scan_tmp, s));
         hipLaunchKernelGGL(column_entries_kernel, dim3(blocks_for(n, kThreads)), dim3(kThreads), 0,
                            s, n, w->ids_out.as<int>(), b->tile_row_of.as<int>(),
-                           b->meta.as<int4>(), b->col_ent.as<int4>());
+                           b->records.as<int4>(), b->col_ent.as<int4>());
     }
     hipLaunchKernelGGL(row_ptr_from_sorted_kernel, dim3(blocks_for(n + 1, kThreads)),
                        dim3(kThreads), 0, s, w->keys_out.as<int>(), n, BC, b->col_ptr.as<int>());
@@ -1225,7 +741,7 @@ int build_b_columns(DevTiles *b, BuildWork *w)
     return RTT_OK;
 }
 
-// An 8x4 tile's payload re-packed column-major: entry (r, k) goes to off +
+// An 8x4 A tile's payload re-packed column-major: entry (r, k) goes to off +
 // (rows of columns < k) + (rows < r in column k).  LANES = 8: lane r takes
 // tile row r (physical slots r * 4 .. r * 4 + 3), so the lanes of a
 // well-filled tile read its payload as one stretch.  LANES = 1: one lane
@@ -1390,16 +906,18 @@ int upload_csr(const rtt_smatrix &host, DevCsr *out, BuildWork *w, double *h2d_m
 
     t0 = Clock::now();
     RTT_TRY(w->counters.ensure(sizeof(int64_t)));
-    int *flags = w->counters.as<int>();
-    RTT_HIP(hipMemsetAsync(flags, 0, sizeof(int), s));
+    int *flags = w->counters.as<int>();   // the flags, then the longest row
+    RTT_HIP(hipMemsetAsync(flags, 0, 2 * sizeof(int), s));
     const int64_t work = std::max<int64_t>(host.m, host.nnz) + 1;
     hipLaunchKernelGGL(validate_csr_kernel, dim3(blocks_for(work, kThreads)), dim3(kThreads), 0,
                        s, host.m, host.n, static_cast<int64_t>(host.nnz),
-                       out->row_ptr.as<int>(), out->col_idx.as<int>(), flags);
+                       out->row_ptr.as<int>(), out->col_idx.as<int>(), flags, flags + 1);
     RTT_HIP(hipGetLastError());
-    int hflags = 0;
-    RTT_HIP(hipMemcpyAsync(&hflags, flags, sizeof(int), hipMemcpyDeviceToHost, s));
+    int got[2] = {0, 0};
+    RTT_HIP(hipMemcpyAsync(got, flags, sizeof(got), hipMemcpyDeviceToHost, s));
     RTT_HIP(hipStreamSynchronize(s));
+    const int hflags = got[0];
+    out->max_row = got[1];
     *validate_ms = ms_since(t0);
     if (hflags & 3)
         return fail(RTT_ERR_INVALID, "CSR validation failed (flags %d)", hflags);
@@ -1445,63 +963,6 @@ int upload_csr(const rtt_smatrix &host, DevCsr *out, BuildWork *w, double *h2d_m
     return RTT_OK;
 }
 
-int build_tiles(const DevCsr &src, const int *row_map, int active_rows, int active_cols,
-                int logical_rows, int logical_cols, bool col_major, int dense_threshold,
-                bool want_csc, DevTiles *out, BuildWork *w, bool want_source_map)
-{
-    RTT_TRY(require_ctx());
-    const int TR = col_major ? kTileK : kTileM;
-    const int TC = col_major ? kTileN : kTileK;
-    out->rows = logical_rows;
-    out->cols = logical_cols;
-    out->tile_rows = TR;
-    out->tile_cols = TC;
-    out->tile_row_count = (active_rows + TR - 1) / TR;
-    out->tile_col_count = (active_cols + TC - 1) / TC;
-    out->has_csc = false;
-    out->arrays_ready = true;
-    out->cols_ready = false;
-    out->transpose_of = nullptr;
-    hipStream_t s = ctx().stream;
-    int2 *src_slot = nullptr;
-    int *dup_flag = nullptr;
-    out->map_source_id = 0;
-    out->map_nnz = 0;
-    out->map_dups = false;
-    if (want_source_map) {
-        RTT_TRY(out->src_slot.ensure(static_cast<size_t>(src.nnz > 0 ? src.nnz : 1) *
-                                     sizeof(int2)));
-        RTT_TRY(w->flag.ensure(sizeof(int)));
-        src_slot = out->src_slot.as<int2>();
-        dup_flag = w->flag.as<int>();
-        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(1), 0, s, dup_flag, int64_t(1), 0);
-        if (src.nnz > 0)
-            hipLaunchKernelGGL(fill_int_kernel, dim3(blocks_for(2 * src.nnz, kThreads)),
-                               dim3(kThreads), 0, s, reinterpret_cast<int *>(src_slot),
-                               2 * src.nnz, -1);
-        RTT_HIP(hipGetLastError());
-    }
-    if (col_major)
-        RTT_TRY((run_tile_build<kTileK, kTileN, true>(src, row_map, active_rows, active_cols,
-                                                      dense_threshold, out, w, src_slot,
-                                                      dup_flag)));
-    else
-        RTT_TRY((run_tile_build<kTileM, kTileK, false>(src, row_map, active_rows, active_cols,
-                                                       dense_threshold, out, w, src_slot,
-                                                       dup_flag)));
-    if (want_source_map) {
-        int dups = 0;
-        RTT_HIP(hipMemcpyAsync(&dups, dup_flag, sizeof(int), hipMemcpyDeviceToHost, s));
-        RTT_HIP(hipStreamSynchronize(s));
-        out->map_source_id = src.structure_id;
-        out->map_nnz = src.nnz;
-        out->map_dups = dups != 0;
-    }
-    if (want_csc)
-        RTT_TRY(build_csc(out, w));
-    return RTT_OK;
-}
-
 int transpose_tiles(const DevTiles &a, int b_cols, DevTiles *b, BuildWork *w)
 {
     RTT_TRY(require_ctx());
@@ -1529,6 +990,9 @@ int transpose_tiles(const DevTiles &a, int b_cols, DevTiles *b, BuildWork *w)
     RTT_TRY(w->ids_in.ensure(n * sizeof(int)));
     RTT_TRY(w->keys_in.ensure(n * sizeof(int)));
     RTT_TRY(w->keys_out.ensure(n * sizeof(int)));
+    RTT_TRY(b->pair_total.ensure(sizeof(unsigned long long)));
+    hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(1), 0, s, b->pair_total.as<int64_t>(),
+                       int64_t(1), int64_t(0));
     if (n > 0 && a.max_col_tiles >= 0 && a.max_col_tiles <= kShortCol &&
         n < (int64_t(1) << kOrderIdBits)) {
         // The same order by counting: B's rows are short.
@@ -1664,6 +1128,7 @@ int transpose_csr(const DevCsr &src, DevCsr *out, BuildWork *w)
     out->rows = src.cols;
     out->cols = src.rows;
     out->nnz = nnz;
+    out->max_row = -1;
     RTT_TRY(out->row_ptr.ensure((static_cast<size_t>(src.cols) + 1) * sizeof(int)));
     RTT_TRY(out->col_idx.ensure(nnz * sizeof(int)));
     RTT_TRY(out->values.ensure(nnz * sizeof(double)));
@@ -1762,27 +1227,18 @@ int update_b_values(const DevCsr &src, bool clear, DevTiles *b)
     if (b->map_source_id == 0 || b->map_source_id != src.structure_id ||
         b->map_nnz != src.nnz || b->transpose_of)
         return fail(RTT_ERR_INVALID, "B has no source map for this CSR");
-    // The k-major copy and the record value planes are kept current only
-    // once a kernel has asked for them (ensure_record_values); otherwise they
-    // are rebuilt from the payload when next needed.
-    const bool kmajor = b->rec_values_ready;
-    if (clear && b->payload > 0) {
+    if (clear && b->payload > 0)
         hipLaunchKernelGGL(fill_f64_kernel, dim3(blocks_for(b->payload, kThreads)),
                            dim3(kThreads), 0, s, b->values.as<double>(), b->payload, 0.0);
-        if (kmajor)
-            hipLaunchKernelGGL(fill_f64_kernel, dim3(blocks_for(b->payload, kThreads)),
-                               dim3(kThreads), 0, s, b->values_cm.as<double>(), b->payload, 0.0);
-    }
     if (src.nnz > 0)
         hipLaunchKernelGGL(scatter_runs_kernel, dim3(blocks_for(src.nnz, kThreads)),
-                           dim3(kThreads), 0, s, src.nnz, b->src_slot.as<int2>(),
-                           src.values.as<double>(), b->values.as<double>(),
-                           kmajor ? b->values_cm.as<double>() : nullptr);
-    if (kmajor && b->num_tiles > 0)
-        hipLaunchKernelGGL(record_values_kernel, dim3(blocks_for(b->num_tiles, kThreads)),
-                           dim3(kThreads), 0, s, b->num_tiles, b->meta.as<int4>(),
-                           b->values_cm.as<double>(), b->records.as<int4>());
+                           dim3(kThreads), 0, s, src.nnz, b->src_slot.as<int>(),
+                           src.values.as<double>(), b->values.as<double>());
     RTT_HIP(hipGetLastError());
+    // The records are kept current only once a kernel has asked for them
+    // (ensure_record_values); otherwise they are written when next needed.
+    if (b->rec_values_ready)
+        RTT_TRY(write_record_values(b));
     return RTT_OK;
 }
 

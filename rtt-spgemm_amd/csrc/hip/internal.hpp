@@ -86,6 +86,7 @@ struct PinnedBuf {
 struct DevCsr {
     int rows = 0, cols = 0;
     int64_t nnz = 0;
+    int max_row = -1;   // entries of the longest row (-1: not counted)
     DevBuf row_ptr, col_idx, values;
     // When the upload sorted rows: input_of[x] = input position of sorted entry x.
     bool reordered = false;
@@ -108,8 +109,9 @@ struct DevTiles {
     DevBuf tile_row_ptr, tile_col_idx, value_offsets, masks, values;
     DevBuf tile_col_ptr, tile_row_idx, csc_tile_ids;
     DevBuf tile_row_of;   // tile -> tile row (A: used by the B transpose)
-    DevBuf meta;          // int4 per tile
-    DevBuf records;       // B only: kRecParts planes of int4, num_tiles entries each
+    DevBuf meta;          // A only: int4 per tile
+    DevBuf records;       // B only: kRecParts planes of int4, num_tiles entries each; plane
+                          // 0 is the tiles' meta, every row in class order
     DevBuf a_brange;      // B only: per A tile, {first B tile, heavy, count} of B row K
     DevBuf a_blight;      // B only: per A tile, {first, count} of the light tiles it can meet
     DevBuf pair_total;    // B only: u64, sum over A tiles of their B row's tile count
@@ -119,7 +121,8 @@ struct DevTiles {
                           // {tile row K, mask, per-k byte sets, offset | dense bit}
     DevBuf values_cm;     // each tile's values with the stride-4 bit groups in order:
                           // A (8x4): column-major; B (4x8): k-major (row k's entries
-                          // contiguous).  Packed from the tile's offset.  For B built as
+                          // contiguous), only the values past the first kRecVals of a
+                          // tile.  Packed from the tile's offset.  For B built as
                           // A^T this is A's array (payload_kmajor()).
 
     DevBuf transpose_src; // A only: per tile, the BRecord of the B = A^T tile it becomes
@@ -129,9 +132,9 @@ struct DevTiles {
     // sorted_ids[b] is the A tile behind B tile b.
     const DevTiles *transpose_of = nullptr;
     DevBuf sorted_ids;
-    // B built from a CSR with a source map: src_slot[x] = {values slot,
-    // values_cm slot} of source entry x, {-1, -1} outside the tiled extent.
-    // Duplicate entries share a slot and are adjacent.
+    // B built from a CSR with a source map: src_slot[x] = values slot of
+    // source entry x, -1 outside the tiled extent.  Duplicate entries share a
+    // slot and are adjacent.
     DevBuf src_slot;
     uint64_t map_source_id = 0;  // DevCsr::structure_id the map belongs to (0: none)
     int64_t map_nnz = 0;
@@ -180,13 +183,11 @@ struct SpgemmWork {
 
 // Scratch of the tile builders, reused across calls.
 struct BuildWork {
-    DevBuf row_tiles, row_payload, row_dense, scan_tmp, counters;
+    DevBuf row_tiles, row_payload, scan_tmp, counters;
     DevBuf keys_in, keys_out, ids_in, ids_out, spans;
-    DevBuf meta2, records2;                     // heavy-first reordering
-    DevBuf tcsr_row_ptr, tcsr_col, tcsr_val;   // transposed CSR (reordered AAT)
-    DevBuf flag;                                // one int (duplicate detection)
     DevBuf staging;                             // uploaded values before the gather
-    DevBuf totals;                              // tile build: tiles, payload, dense
+    DevBuf long_rows, long_of;                  // tile build: long tile rows and their sizes
+    PinnedBuf host_totals;                      // tile build: sizes, written by the kernels
 };
 
 struct Events {
@@ -210,15 +211,19 @@ int require_ctx();
 int upload_csr(const rtt_smatrix &host, DevCsr *out, BuildWork *work,
                double *h2d_ms, double *validate_ms, double *sort_ms,
                int *rows_were_sorted);
-// Builds hybrid tiles from a row-sorted CSR.  row_map (device, may be null)
-// maps tiled row -> source row for rows < active_rows.
+// Builds hybrid tiles from a row-sorted CSR: A's (8x4 row-major) or, with
+// b_layout, B's (4x8 column-major, every row's meta in class order as record
+// plane 0; the value planes are left to ensure_record_values).  row_map
+// (device, may be null) maps tiled row -> source row for rows < active_rows.
+// With pairs_of (A's tiles), the pair extents of B are built too.  Waits for
+// the sizes once (twice when the arrays had to grow).
 int build_tiles(const DevCsr &src, const int *row_map, int active_rows,
                 int active_cols, int logical_rows, int logical_cols,
-                bool col_major, int dense_threshold, bool build_csc,
-                DevTiles *out, BuildWork *work, bool want_source_map = false);
+                bool b_layout, int dense_threshold, DevTiles *out, BuildWork *work,
+                const DevTiles *pairs_of = nullptr, bool want_source_map = false);
 // Values-only update of a B built with a source map from `src`: optional
-// clear, in-order sums of each slot's source entries into values and
-// values_cm, then the value parts of the records.
+// clear, in-order sums of each slot's source entries into values, then the
+// value parts of the records.
 int update_b_values(const DevCsr &src, bool clear, DevTiles *b);
 // Uploaded values in the caller's entry order -> src->values (sorted order).
 int set_csr_values(DevCsr *csr, const double *host_values, BuildWork *work);
@@ -239,17 +244,15 @@ int build_colmajor_values(DevTiles *t);
 // t->row_payload_off.
 int build_transpose_source(DevTiles *t, BuildWork *w);
 // b->a_brange[t] = {B.tile_row_ptr[K], heavy tiles, count} and b->a_blight[t]
-// for every A tile t in column K.
-int build_pair_extents(const DevTiles &a, DevTiles *b);
+// for every A tile t in column K; adds into b->pair_total, which the B build
+// has zeroed.  With flag, its value also goes to *flag_out (host memory).
+int build_pair_extents(const DevTiles &a, DevTiles *b, const unsigned int *flag = nullptr,
+                       long long *flag_out = nullptr);
 // Builds b->col_ptr / b->col_ent (tile columns, tile rows ascending) of a B
 // built from a CSR; no-op for B = A^T at tile level, whose columns are A's
 // tile rows (b_columns below).
 int build_b_columns(DevTiles *b, BuildWork *w);
-// Reorders b->meta of a B built from CSR into class order within every row
-// (stable), writes it as record plane 0 and fills b->row_groups.  The record
-// value planes and the k-major payload are left to ensure_record_values.
-int order_by_class(DevTiles *b, BuildWork *w);
-// Builds values_cm and the record value planes of a B built from a CSR when
+// Builds the record value planes (and values_cm) of a B built from a CSR when
 // they are missing (the LDS-accumulator numeric kernels read them; the
 // symbolic and tile-pair kernels do not).
 int ensure_record_values(DevTiles *b);
