@@ -38,6 +38,7 @@ struct rtt_prepared_a {
     rtt::DevBuf d_inner_new_to_old;
     rtt::BuildWork build;
     rtt::SpgemmWork core;
+    rtt::RowRouting routing;  // rows of the tile-pair kernel at the last threshold asked for
     rtt::Events events;
     rtt::DevC last_c;
     bool has_c = false;
@@ -750,7 +751,9 @@ int rtt_tilespgemm(const rtt_prepared_a *a_const, const rtt_dynamic_b *b, rtt_sm
     float fill = path == RTT_NUMERIC_TILE ? 0.f : static_cast<float>(sc.tile_fill_threshold);
     int64_t tile_rows = 0, nonempty = 0;
     if (path == RTT_NUMERIC_AUTO) {
-        RTT_TRY(rtt::count_tile_rows(a->tiles, fill, &a->core.tile_rows, &tile_rows, &nonempty));
+        RTT_TRY(rtt::count_tile_rows(a->tiles, fill, &a->build.counters, &a->routing));
+        tile_rows = a->routing.tile_rows;
+        nonempty = a->routing.nonempty;
         if (tile_rows == 0)
             path = RTT_NUMERIC_VECTOR;
         else if (tile_rows == nonempty)

@@ -123,4 +123,51 @@ __device__ __forceinline__ int upper_index(const int *pre, int n, int p)
     return lo;
 }
 
+// Decoupled look-back over workgroups, two sums (below 2^62) each: the words
+// of workgroup b are look[2 b] and look[2 b + 1], state in the top two bits (0
+// nothing yet, 1 the workgroup's own sums, 2 sums up to and with it).  All
+// words start at zero.
+constexpr unsigned long long kOwn = 1ull << 62, kUpTo = 2ull << 62, kSums = kOwn - 1ull;
+
+__device__ __forceinline__ void publish(unsigned long long *look, int64_t b,
+                                        unsigned long long state, unsigned long long x,
+                                        unsigned long long y)
+{
+    __hip_atomic_store(look + 2 * b, state | x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(look + 2 * b + 1, state | y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sums of the workgroups before b, by one wave, 64 of them at a time.
+// Workgroups take their numbers from a ticket, so every workgroup before b
+// has started and publishes its own sums without waiting for anything: the
+// wait ends.
+__device__ __forceinline__ void look_back(const unsigned long long *look, int64_t b,
+                                          unsigned long long *x, unsigned long long *y)
+{
+    unsigned long long sx = 0, sy = 0;
+    for (int64_t hi = b; hi > 0; hi -= kWave) {
+        const int64_t i = hi - 1 - lane_id();
+        unsigned long long wx = kUpTo, wy = kUpTo;
+        if (i >= 0) {
+            for (;;) {
+                wx = __hip_atomic_load(look + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                wy = __hip_atomic_load(look + 2 * i + 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                if ((wx >> 62) != 0 && (wx >> 62) == (wy >> 62))
+                    break;
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        const unsigned long long done = __ballot((wx >> 62) == 2);
+        const int last = done ? __builtin_ctzll(done) : kWave - 1;
+        const bool take = lane_id() <= last;
+        sx += wave_sum(take ? wx & kSums : 0ull);
+        sy += wave_sum(take ? wy & kSums : 0ull);
+        if (done)
+            break;
+    }
+    *x = sx;
+    *y = sy;
+}
+
 } // namespace rtt

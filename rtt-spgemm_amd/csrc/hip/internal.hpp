@@ -161,7 +161,9 @@ struct DevC {
 // Scratch of the SpGEMM core, reused across calls.
 struct SpgemmWork {
     DevBuf row_tiles, row_nnz, row_level;   // per A tile row
-    DevBuf scan_tmp, counters, l3_rows, num_rows, lds_rows, tiny_rows, mid_rows, slab;
+    DevBuf scan_tmp, counters, slab;
+    DevBuf l3_rows, sym_slab_rows;          // rows past the wave and the workgroup table
+    DevBuf class_rows[5];                   // rows of each numeric kernel (spgemm.hip RowClass)
     PinnedBuf host_counters;
     DevBuf stage_j, stage_m;                // staged sorted tile lists
     DevBuf c_row_nnz_off;                   // per tile row, int64
@@ -175,7 +177,7 @@ struct SpgemmWork {
     uint64_t slab_stage_cap = 0, slab_stage_need = 0;
     DevBuf tile_queue;                      // row-queue heads of the tile-pair kernels
     DevBuf tile_pairs;                      // u64: pairs the tile-pair kernel multiplied
-    DevBuf tile_rows;                       // u64 x 2: rows counted for routing
+    PinnedBuf host_tile_stats;              // u64: pairs, tail reason, records, chunks
     // Tail queue of the tile-pair path: records, state, chunk prefix, heavy
     // tile bitset and the chunks' partial tiles.
     DevBuf tail_records, tail_state, tail_chunk_base, tail_heavy, tail_workspace;
@@ -281,16 +283,17 @@ int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const 
 // only: no allocation, no host synchronisation; no tail split.
 int tile_values_noalloc(const DevTiles &a, const TileColumns &bc, const DevC &c, int precision,
                         void *scratch, size_t scratch_bytes, double *c_values, hipStream_t s);
-// Gate decision, admitted records and chunks of the last tail admission.
-int tail_stats(SpgemmWork *w, int *reason, unsigned long long *records,
-               unsigned long long *chunks);
 // The admitted records (slot order): tile, merge scans and matches, chunks.
 int tail_records(SpgemmWork *w, int max_records, long long *task, int *scans, int *matches,
                  int *chunks, int *count);
 // Tile rows of A the tile-pair kernel would take at `fill`, and the tile
-// rows holding any tile (one readback).
-int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, int64_t *tile_rows,
-                    int64_t *nonempty_rows);
+// rows holding any tile.  A's tiles never change after its preparation, so a
+// prepared A counts once per fill threshold it is asked for.
+struct RowRouting {
+    float fill = -1.f;   // threshold counted for (negative: none)
+    int64_t tile_rows = 0, nonempty = 0;
+};
+int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, RowRouting *out);
 // Per-row numeric routing of one call: rows whose A tiles hold at least
 // `fill` stored values on average take the tile-pair kernel in `precision`.
 // With `tail`, C tiles whose K-merge costs more than `threshold` (FP32

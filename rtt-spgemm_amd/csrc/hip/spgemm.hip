@@ -472,7 +472,8 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
     Operands g, int stage_limit, Stage st, const int *__restrict__ rows,
-    int64_t *__restrict__ row_tiles, int64_t *__restrict__ row_nnz, int *__restrict__ row_level)
+    int64_t *__restrict__ row_tiles, int64_t *__restrict__ row_nnz, int *__restrict__ row_level,
+    int *__restrict__ slab_rows, unsigned long long *__restrict__ n_slab)
 {
     __shared__ __align__(16) int s_key[kSymSlots];
     __shared__ unsigned long long s_msk[kSymSlots];
@@ -592,6 +593,7 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
             row_level[row] = kLevelSlab;
             row_tiles[row] = 0;
             row_nnz[row] = 0;
+            slab_rows[atomicAdd(n_slab, 1ull)] = row;
         }
         return;
     }
@@ -1813,87 +1815,173 @@ __global__ __launch_bounds__(kThreads) void numeric_slab_kernel(
     }
 }
 
-// Appends v to out (count holds the length) for the threads where pred
-// holds: one atomic per workgroup of NW waves (an atomic per wave on one
-// counter serialised at the L2 on millions of rows), positions in thread
-// order within the workgroup.  s holds NW + 1 ints; every thread calls it.
-template <int NW>
-__device__ __forceinline__ void block_append(bool pred, int v, int *__restrict__ out,
-                                             int *__restrict__ count, int *s)
-{
-    const unsigned long long m = __ballot(pred);
-    const int w = threadIdx.x / kWave;
-    if (lane_id() == 0)
-        s[w] = __popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int total = 0;
-#pragma unroll
-        for (int i = 0; i < NW; ++i)
-            total += s[i];
-        s[NW] = total ? atomicAdd(count, total) : 0;
-    }
-    __syncthreads();
-    int base = s[NW];
-#pragma unroll
-    for (int i = 0; i < NW; ++i)
-        base += i < w ? s[i] : 0;
-    if (pred)
-        out[base + __popcll(m & ((1ull << lane_id()) - 1ull))] = v;
-    __syncthreads();   // s is reused by the next call
-}
+// The numeric kernel that takes a row of the LDS level, by its sizes: the
+// smallest instance that holds it, the slab kernel when none does.
+enum RowClass : int { kRowTiny, kRowSmall, kRowMid, kRowLarge, kRowSlab, kRowClasses };
 
-// Lists rows for the other passes.  mode 0: symbolic slab rows; mode 2:
-// rows for the workgroup symbolic table; mode 1: numeric rows off
-// SmallRow, into the LargeRow list (out_lds), the slab list (out_slab),
-// the TinyRow list (out_tiny) and the MediumRow list (out_mid).
-__global__ __launch_bounds__(kThreads) void collect_rows_kernel(int n, int mode, const int *__restrict__ level,
-                                    const int64_t *__restrict__ tile_ptr,
-                                    const int64_t *__restrict__ nnz_off,
-                                    const int *__restrict__ a_trp, const int *__restrict__ a_off,
-                                    int *__restrict__ out_slab, int *__restrict__ n_slab,
-                                    int *__restrict__ out_lds, int *__restrict__ n_lds,
-                                    float tile_fill = INFINITY, int *__restrict__ out_tiny = nullptr,
-                                    int *__restrict__ n_tiny = nullptr,
-                                    int *__restrict__ out_mid = nullptr,
-                                    int *__restrict__ n_mid = nullptr)
+// Counters the host reads back after the symbolic pass, and the state of the
+// kernels that fill them (zeroed with them).
+enum Counter : int {
+    kCtrPairs,       // (A tile, B tile) pairs
+    kCtrTiles,       // C tiles
+    kCtrNnz,         // nnz(C)
+    kCtrOutgrown,    // rows that outgrew the wave table
+    kCtrSymSlab,     // rows that outgrew the workgroup table too
+    kCtrSlabTiles,   // slab tiles the staging cursor handed out
+    kCtrRows,        // rows of each RowClass, kRowClasses of them
+    kCtrTicket = kCtrRows + kRowClasses,
+    kCtrDone,
+    kCounters
+};
+
+struct RowLists {
+    int *__restrict__ rows[kRowClasses];
+    int *__restrict__ outgrown;
+};
+
+// Sizes of C and the numeric routing from the rows' counts, in one launch:
+// every workgroup sums its rows, takes the rows' offsets by a decoupled
+// look-back, lists its rows for the numeric kernels, and the last one to
+// finish writes the counters to the host's buffer.  Rows that still wait
+// for another symbolic pass (outgrown, or slab rows before theirs) count as
+// empty; the host then runs that pass and this kernel again.  It replaces
+// two row-listing passes, two scans, a gather and a copy: eight launches of
+// 2 to 10 us each, most of what a product of a few thousand rows spent
+// between its symbolic and its numeric pass.
+__global__ __launch_bounds__(kThreads) void row_sizes_kernel(
+    int n, const int *__restrict__ level, bool slab_done, const int64_t *__restrict__ tiles,
+    const int64_t *__restrict__ nnz, const int *__restrict__ a_trp,
+    const int *__restrict__ a_row_off, float tile_fill, bool list, int64_t *__restrict__ tile_ptr,
+    int64_t *__restrict__ nnz_off, int64_t *__restrict__ tile_nnz, int64_t tile_nnz_len,
+    RowLists out, unsigned long long *__restrict__ ctr, unsigned long long *__restrict__ look,
+    unsigned long long *__restrict__ host)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool to_slab = false, to_lds = false, to_tiny = false, to_mid = false;
+    __shared__ unsigned int s_block;
+    __shared__ unsigned long long s_x[kWavesPerBlock + 1], s_y[kWavesPerBlock + 1];
+    __shared__ int s_count[kRowClasses + 1][kWavesPerBlock];
+    __shared__ int s_base[kRowClasses + 1];
+    const int tid = threadIdx.x, w = tid / kWave;
+    if (tid == 0)
+        s_block = static_cast<unsigned int>(atomicAdd(&ctr[kCtrTicket], 1ull));
+    __syncthreads();
+    const int64_t b = s_block;
+    const int64_t i = b * kThreads + tid;
+    unsigned long long nt = 0, nz = 0;
+    int cls = -1;   // list the row goes to, kRowClasses for an outgrown row
     if (i < n) {
         const int lv = level[i];
-        if (mode == 0 || mode == 2) {
-            to_slab = lv == (mode == 0 ? kLevelSlab : kLevelLarge);
-        } else if (tile_routed(tile_fill, a_trp[i + 1] - a_trp[i],
-                               a_off[a_trp[i + 1]] - a_off[a_trp[i]])) {
-            // numeric on the tile-pair kernel
-        } else if (lv == kLevelSlab) {
-            to_slab = true;
-        } else if (lv == kLevelLds) {
-            const int64_t nt = tile_ptr[i + 1] - tile_ptr[i];
-            const int64_t nz = nnz_off[i + 1] - nnz_off[i];
-            const int64_t alen = a_off[a_trp[i + 1]] - a_off[a_trp[i]];
-            if (nt > LargeRow::kTiles || nz > LargeRow::kAcc || alen > LargeRow::kAStage)
-                to_slab = true;
-            else if (fits_row<SmallRow>(nt, nz, alen))
-                to_tiny = fits_row<TinyRow>(nt, nz, alen);
-            else if (fits_row<MediumRow>(nt, nz, alen))
-                to_mid = true;
-            else
-                to_lds = true;
+        const bool sized = lv == kLevelLds || (lv == kLevelSlab && slab_done);
+        if (sized) {
+            nt = static_cast<unsigned long long>(tiles[i]);
+            nz = static_cast<unsigned long long>(nnz[i]);
+        }
+        const int a_tiles = a_trp[i + 1] - a_trp[i];
+        const int64_t alen = a_row_off[i + 1] - a_row_off[i];
+        if (lv == kLevelLarge) {
+            cls = kRowClasses;
+        } else if (sized && list && !tile_routed(tile_fill, a_tiles, static_cast<int>(alen))) {
+            const int64_t t = static_cast<int64_t>(nt), z = static_cast<int64_t>(nz);
+            cls = lv == kLevelSlab                ? kRowSlab
+                  : fits_row<TinyRow>(t, z, alen)   ? kRowTiny
+                  : fits_row<SmallRow>(t, z, alen)  ? kRowSmall
+                  : fits_row<MediumRow>(t, z, alen) ? kRowMid
+                  : fits_row<LargeRow>(t, z, alen)  ? kRowLarge
+                                                    : kRowSlab;
         }
     }
-    __shared__ int s_app[kWavesPerBlock + 1];
-    block_append<kWavesPerBlock>(to_slab, i, out_slab, n_slab, s_app);
-    if (mode == 1) {
-        block_append<kWavesPerBlock>(to_lds, i, out_lds, n_lds, s_app);
-        block_append<kWavesPerBlock>(to_tiny, i, out_tiny, n_tiny, s_app);
-        block_append<kWavesPerBlock>(to_mid, i, out_mid, n_mid, s_app);
+    const unsigned long long ix = wave_inclusive_scan(nt), iy = wave_inclusive_scan(nz);
+    if (lane_id() == kWave - 1) {
+        s_x[w] = ix;
+        s_y[w] = iy;
+    }
+    int rank = 0;
+#pragma unroll
+    for (int c = 0; c <= kRowClasses; ++c) {
+        const unsigned long long m = __ballot(cls == c);
+        if (cls == c)
+            rank = __popcll(m & ((1ull << lane_id()) - 1ull));
+        if (lane_id() == 0)
+            s_count[c][w] = __popcll(m);
+    }
+    __syncthreads();
+    unsigned long long bx = 0, by = 0, all_x = 0, all_y = 0;
+#pragma unroll
+    for (int k = 0; k < kWavesPerBlock; ++k) {
+        bx += k < w ? s_x[k] : 0ull;
+        by += k < w ? s_y[k] : 0ull;
+        all_x += s_x[k];
+        all_y += s_y[k];
+    }
+    if (tid <= kRowClasses) {
+        // One atomic per list and workgroup that has rows for it.
+        int sum = 0;
+#pragma unroll
+        for (int k = 0; k < kWavesPerBlock; ++k)
+            sum += s_count[tid][k];
+        unsigned long long *at = tid == kRowClasses ? &ctr[kCtrOutgrown] : &ctr[kCtrRows + tid];
+        s_base[tid] = sum ? static_cast<int>(atomicAdd(at, static_cast<unsigned long long>(sum))) : 0;
+    }
+    if (w == 0) {
+        if (lane_id() == 0)
+            publish(look, b, b == 0 ? kUpTo : kOwn, all_x, all_y);
+        unsigned long long px = 0, py = 0;
+        if (b > 0) {
+            look_back(look, b, &px, &py);
+            if (lane_id() == 0)
+                publish(look, b, kUpTo, px + all_x, py + all_y);
+        }
+        if (lane_id() == 0) {
+            s_x[kWavesPerBlock] = px;
+            s_y[kWavesPerBlock] = py;
+        }
+    }
+    __syncthreads();
+    const unsigned long long px = s_x[kWavesPerBlock], py = s_y[kWavesPerBlock];
+    if (i < n) {
+        tile_ptr[i] = static_cast<int64_t>(px + bx + ix - nt);
+        nnz_off[i] = static_cast<int64_t>(py + by + iy - nz);
+        if (cls >= 0) {
+            int at = s_base[cls] + rank;
+#pragma unroll
+            for (int k = 0; k < kWavesPerBlock; ++k)
+                at += k < w ? s_count[cls][k] : 0;
+            (cls == kRowClasses ? out.outgrown : out.rows[cls])[at] = static_cast<int>(i);
+        }
+    }
+    if ((b + 1) * kThreads >= n && tid == 0) {   // the workgroup of the last row
+        const int64_t t = static_cast<int64_t>(px + all_x), z = static_cast<int64_t>(py + all_y);
+        tile_ptr[n] = t;
+        nnz_off[n] = z;
+        if (t < tile_nnz_len)
+            tile_nnz[t] = z;
+        __hip_atomic_store(&ctr[kCtrTiles], px + all_x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctr[kCtrNnz], py + all_y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (tid == 0) {
+        __threadfence();
+        if (atomicAdd(&ctr[kCtrDone], 1ull) + 1 == gridDim.x) {
+            __threadfence();
+            for (int c = 0; c < kCtrTicket; ++c)
+                host[c] = __hip_atomic_load(&ctr[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
-// Number of (A tile, B tile) pairs: the sum of the per-A-tile extents, one
-// atomic per workgroup.
+// Zeroes the look-back words and the counters from `first` on; with a pair
+// total, also sets that counter and the queue heads.
+__global__ void sizes_init_kernel(unsigned long long *ctr, int first, unsigned long long *look,
+                                  int64_t words, const unsigned long long *pair_total, int *queue,
+                                  int n_queue)
+{
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < words)
+        look[i] = 0ull;
+    if (i < kCounters && i >= first)
+        ctr[i] = i == kCtrPairs && pair_total ? *pair_total : 0ull;
+    if (pair_total && i < n_queue)
+        queue[i] = 0;
+}
+
 __global__ void fill_i32_kernel(int *p, int64_t n, int v)
 {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1909,30 +1997,6 @@ __global__ void fill_u64_kernel(unsigned long long *p, int64_t n)
 }
 
 __global__ void set_last_kernel(int64_t *p, const int64_t *v) { *p = *v; }
-
-__global__ void set_last2_kernel(int64_t *p, const int64_t *v, int64_t *q, const int64_t *u)
-{
-    *p = *v;
-    *q = *u;
-}
-
-// Zeroes the host-read counters except [0], which takes the pair total, the
-// trailing entries of the per-row size arrays and the queue heads.
-__global__ void symbolic_init_kernel(unsigned long long *ctr, int n_ctr,
-                                     const unsigned long long *pair_total,
-                                     unsigned long long *row_tiles_end,
-                                     unsigned long long *row_nnz_end, int *queue, int n_queue)
-{
-    const int i = threadIdx.x;
-    if (i < n_ctr)
-        ctr[i] = i == 0 ? *pair_total : 0ull;
-    if (i < n_queue)
-        queue[i] = 0;
-    if (i == 0) {
-        *row_tiles_end = 0ull;
-        *row_nnz_end = 0ull;
-    }
-}
 
 double event_ms(hipEvent_t a, hipEvent_t b)
 {
@@ -2078,34 +2142,31 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     g.tile_fill = tile ? tile->fill : INFINITY;
 
     const int num_cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    // Counters read back by the host: [0] pairs, [1] symbolic slab rows,
-    // [2] numeric slab rows, [3] numeric large-LDS rows, [4] C tiles,
-    // [5] nnz(C), [6] rows for the workgroup symbolic table, [7] slab tiles
-    // the staging cursor handed out, [8] numeric one-wave (TinyRow) rows,
-    // [9] numeric MediumRow rows.
-    constexpr int kCounters = 10;
-    RTT_TRY(w->counters.ensure(kCounters * sizeof(unsigned long long)));
+    // The counters and the look-back words of the sizes pass; the host's copy
+    // of the counters is written by the pass itself.
+    const int64_t size_blocks = std::max<int64_t>(1, blocks_for(R, kThreads));
+    const int64_t words = 2 * size_blocks;
+    RTT_TRY(w->counters.ensure(static_cast<size_t>(kCounters + words) * sizeof(unsigned long long)));
     RTT_TRY(w->host_counters.ensure(kCounters * sizeof(unsigned long long)));
     unsigned long long *ctr = w->counters.as<unsigned long long>();
-    unsigned long long *hctr = w->host_counters.as<unsigned long long>();
-    int *slab_count = reinterpret_cast<int *>(ctr + 1);
-    int *num_slab_count = reinterpret_cast<int *>(ctr + 2);
-    int *num_lds_count = reinterpret_cast<int *>(ctr + 3);
-    int *large_count = reinterpret_cast<int *>(ctr + 6);
-    int *num_tiny_count = reinterpret_cast<int *>(ctr + 8);
-    int *num_mid_count = reinterpret_cast<int *>(ctr + 9);
+    unsigned long long *look = ctr + kCounters;
+    const unsigned long long *hctr = w->host_counters.as<unsigned long long>();
 
     auto t_sym = Clock::now();
     // ---- symbolic: per-row tile sets, staged ------------------------------
     const int stage_limit = 3 * kSymSlots / 4;
+    const size_t row_ints = (static_cast<size_t>(R) + 1) * sizeof(int);
     RTT_TRY(w->row_tiles.ensure((R + 1) * sizeof(int64_t)));
     RTT_TRY(w->row_nnz.ensure((R + 1) * sizeof(int64_t)));
-    RTT_TRY(w->row_level.ensure((R + 1) * sizeof(int)));
-    RTT_TRY(w->l3_rows.ensure((R + 1) * sizeof(int)));
-    RTT_TRY(w->num_rows.ensure((R + 1) * sizeof(int)));
-    RTT_TRY(w->lds_rows.ensure((R + 1) * sizeof(int)));
-    RTT_TRY(w->tiny_rows.ensure((R + 1) * sizeof(int)));
-    RTT_TRY(w->mid_rows.ensure((R + 1) * sizeof(int)));
+    RTT_TRY(w->row_level.ensure(row_ints));
+    RTT_TRY(w->l3_rows.ensure(row_ints));
+    RTT_TRY(w->sym_slab_rows.ensure(row_ints));
+    RowLists lists;
+    for (int c = 0; c < kRowClasses; ++c) {
+        RTT_TRY(w->class_rows[c].ensure(row_ints));
+        lists.rows[c] = w->class_rows[c].as<int>();
+    }
+    lists.outgrown = w->l3_rows.as<int>();
     RTT_TRY(w->stage_j.ensure(static_cast<size_t>(R) * stage_limit * sizeof(int)));
     RTT_TRY(w->stage_m.ensure(static_cast<size_t>(R) * stage_limit * sizeof(uint64_t)));
     RTT_TRY(c->tile_ptr.ensure((R + 1) * sizeof(int64_t)));
@@ -2114,12 +2175,11 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     // Queue heads: [0] symbolic slab count, [1] symbolic slab fill, [2] numeric slab.
     RTT_TRY(w->queue.ensure(4 * sizeof(int)));
     int *queue = w->queue.as<int>();
-    // Counter [0] is the pair total, summed by the B update's pair-extent pass.
-    hipLaunchKernelGGL(symbolic_init_kernel, dim3(1), dim3(kCounters), 0, s, ctr, kCounters,
-                       b.pair_total.as<unsigned long long>(),
-                       reinterpret_cast<unsigned long long *>(w->row_tiles.as<int64_t>() + R),
-                       reinterpret_cast<unsigned long long *>(w->row_nnz.as<int64_t>() + R),
-                       queue, 4);
+    // The pair total was summed by the B update's pair-extent pass.
+    hipLaunchKernelGGL(sizes_init_kernel,
+                       dim3(blocks_for(std::max<int64_t>(words, kCounters), kThreads)),
+                       dim3(kThreads), 0, s, ctr, 0, look, words,
+                       b.pair_total.as<unsigned long long>(), queue, 4);
     // One wave per row first; rows that outgrow its table go to the
     // workgroup table, and rows that outgrow that to the slab.
     RTT_HIP(hipEventRecord(ev->ev[0], s));
@@ -2128,64 +2188,43 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
                            w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(),
                            w->row_level.as<int>());
     RTT_HIP(hipGetLastError());
+    RTT_HIP(hipEventRecord(ev->ev[1], s));
     int n_slab = 0;
     COut none{};
-    // Sizes of C from the per-row counts: row offsets, the numeric routing
-    // lists, and every counter read back with one copy.  Rows of the
-    // tile-pair kernel are not listed.
-    auto finish_sizes = [&]() -> int {
-        RTT_TRY(exclusive_scan_i64(w->row_tiles.as<int64_t>(), c->tile_ptr.as<int64_t>(), R,
-                                   &w->scan_tmp, s));
-        RTT_TRY(exclusive_scan_i64(w->row_nnz.as<int64_t>(), w->c_row_nnz_off.as<int64_t>(), R,
-                                   &w->scan_tmp, s));
-        if (R > 0 && any_vector)
-            hipLaunchKernelGGL(collect_rows_kernel, dim3(blocks_for(R, kThreads)),
-                               dim3(kThreads), 0, s, R, 1, w->row_level.as<int>(),
-                               c->tile_ptr.as<int64_t>(), w->c_row_nnz_off.as<int64_t>(),
-                               g.a_trp, g.a_off, w->num_rows.as<int>(), num_slab_count,
-                               w->lds_rows.as<int>(), num_lds_count, g.tile_fill,
-                               w->tiny_rows.as<int>(), num_tiny_count, w->mid_rows.as<int>(),
-                               num_mid_count);
-        hipLaunchKernelGGL(set_last2_kernel, dim3(1), dim3(1), 0, s,
-                           reinterpret_cast<int64_t *>(ctr + 4), c->tile_ptr.as<int64_t>() + R,
-                           reinterpret_cast<int64_t *>(ctr + 5),
-                           w->c_row_nnz_off.as<int64_t>() + R);
-        RTT_HIP(hipMemcpyAsync(hctr, ctr, kCounters * sizeof(unsigned long long),
-                               hipMemcpyDeviceToHost, s));
+    // Sizes of C from the per-row counts, the numeric routing lists and
+    // every counter, in one launch and one wait.  Rows of the tile-pair
+    // kernel are not listed.
+    auto finish_sizes = [&](bool slab_done) -> int {
+        hipLaunchKernelGGL(row_sizes_kernel, dim3(static_cast<unsigned>(size_blocks)),
+                           dim3(kThreads), 0, s, R, w->row_level.as<int>(), slab_done,
+                           w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(), g.a_trp,
+                           g.a_row_off, g.tile_fill, any_vector, c->tile_ptr.as<int64_t>(),
+                           w->c_row_nnz_off.as<int64_t>(), c->tile_nnz.as<int64_t>(),
+                           static_cast<int64_t>(c->tile_nnz.bytes / sizeof(int64_t)), lists, ctr,
+                           look, w->host_counters.as<unsigned long long>());
+        RTT_HIP(hipGetLastError());
         RTT_HIP(hipStreamSynchronize(s));
         return RTT_OK;
     };
-    bool sized = false;
-    if (R > 0) {
-        hipLaunchKernelGGL(collect_rows_kernel, dim3(blocks_for(R, kThreads)), dim3(kThreads), 0,
-                           s, R, 2, w->row_level.as<int>(), nullptr, nullptr, nullptr, nullptr,
-                           w->l3_rows.as<int>(), large_count, nullptr, nullptr);
+    auto clear_sizes = [&]() {
+        hipLaunchKernelGGL(sizes_init_kernel, dim3(blocks_for(words, kThreads)), dim3(kThreads), 0,
+                           s, ctr, static_cast<int>(kCtrRows), look, words, nullptr, nullptr, 0);
+    };
+    static_assert(kCounters <= kThreads, "one workgroup clears the counters");
+    // Sized at once, as if every row fit the wave table: one wait when none
+    // outgrew it (the usual case), redone when some did.
+    RTT_TRY(finish_sizes(false));
+    const int n_large = static_cast<int>(hctr[kCtrOutgrown]);
+    if (n_large > 0) {
+        clear_sizes();
+        hipLaunchKernelGGL(symbolic_count_kernel, dim3(n_large), dim3(kThreads), 0, s, g,
+                           stage_limit, st, w->l3_rows.as<int>(), w->row_tiles.as<int64_t>(),
+                           w->row_nnz.as<int64_t>(), w->row_level.as<int>(),
+                           w->sym_slab_rows.as<int>(), ctr + kCtrSymSlab);
+        RTT_HIP(hipGetLastError());
         RTT_HIP(hipEventRecord(ev->ev[1], s));
-        // Sized at once, as if every row fit the wave table: one readback
-        // when none outgrew it (the usual case), redone below when some did.
-        RTT_TRY(finish_sizes());
-        sized = true;
-        const int n_large = static_cast<int>(hctr[6] & 0xffffffffu);
-        if (n_large > 0) {
-            sized = false;
-            hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(2), 0, s, ctr + 2, int64_t(2));
-            hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(2), 0, s, ctr + 8, int64_t(2));
-            hipLaunchKernelGGL(symbolic_count_kernel, dim3(n_large), dim3(kThreads), 0, s, g,
-                               stage_limit, st, w->l3_rows.as<int>(),
-                               w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(),
-                               w->row_level.as<int>());
-            RTT_HIP(hipGetLastError());
-            hipLaunchKernelGGL(collect_rows_kernel, dim3(blocks_for(R, kThreads)), dim3(kThreads),
-                               0, s, R, 0, w->row_level.as<int>(), nullptr, nullptr, nullptr,
-                               nullptr, w->l3_rows.as<int>(), slab_count, nullptr, nullptr);
-            RTT_HIP(hipMemcpyAsync(hctr, ctr, 2 * sizeof(unsigned long long),
-                                   hipMemcpyDeviceToHost, s));
-            RTT_HIP(hipStreamSynchronize(s));
-            n_slab = static_cast<int>(hctr[1] & 0xffffffffu);
-            RTT_HIP(hipEventRecord(ev->ev[1], s));
-        }
-    } else {
-        RTT_HIP(hipEventRecord(ev->ev[1], s));
+        RTT_TRY(finish_sizes(false));
+        n_slab = static_cast<int>(hctr[kCtrSymSlab]);
     }
     int slab_blocks = 0;
     const int *slab_rows = nullptr;
@@ -2209,16 +2248,16 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
         }
         RTT_TRY(w->slab_row_off.ensure(static_cast<size_t>(R) * sizeof(int64_t)));
         ss.row_off = w->slab_row_off.as<int64_t>();
-        ss.cursor = ctr + 7;
+        ss.cursor = ctr + kCtrSlabTiles;
         if (w->slab_stage_cap > 0) {
             ss.j = w->slab_stage_j.as<int>();
             ss.m = w->slab_stage_m.as<unsigned long long>();
             ss.capacity = w->slab_stage_cap;
         }
         slab_blocks = slab_grid(n_slab, num_cus, BC, sizeof(uint64_t), w->slab);
-        slab_rows = w->l3_rows.as<int>();
+        slab_rows = w->sym_slab_rows.as<int>();
         if (lb_mode == RTT_LB_ADAPTIVE_TAIL)
-            RTT_TRY(order_rows_by_cost(w->l3_rows.as<int>(), n_slab, g, w, s, &slab_rows));
+            RTT_TRY(order_rows_by_cost(slab_rows, n_slab, g, w, s, &slab_rows));
         RTT_TRY(w->slab.ensure(static_cast<size_t>(slab_blocks) * BC * sizeof(uint64_t)));
         hipLaunchKernelGGL(fill_u64_kernel,
                            dim3(blocks_for(static_cast<int64_t>(slab_blocks) * BC, kThreads)),
@@ -2229,17 +2268,17 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
                            w->slab.as<unsigned long long>(), w->row_tiles.as<int64_t>(),
                            w->row_nnz.as<int64_t>(), ss, none);
         RTT_HIP(hipGetLastError());
+        clear_sizes();
+        RTT_TRY(finish_sizes(true));
     }
-    if (!sized)
-        RTT_TRY(finish_sizes());
-    w->slab_stage_need = std::max<uint64_t>(w->slab_stage_need, hctr[7]);
-    const unsigned long long pairs = hctr[0];
-    const int n_num_slab = static_cast<int>(hctr[2] & 0xffffffffu);
-    const int n_num_lds = static_cast<int>(hctr[3] & 0xffffffffu);
-    const int n_num_tiny = static_cast<int>(hctr[8] & 0xffffffffu);
-    const int n_num_mid = static_cast<int>(hctr[9] & 0xffffffffu);
-    const int64_t total_tiles = static_cast<int64_t>(hctr[4]);
-    const int64_t total_nnz = static_cast<int64_t>(hctr[5]);
+    w->slab_stage_need = std::max<uint64_t>(w->slab_stage_need, hctr[kCtrSlabTiles]);
+    const unsigned long long pairs = hctr[kCtrPairs];
+    int n_rows[kRowClasses];
+    for (int k = 0; k < kRowClasses; ++k)
+        n_rows[k] = static_cast<int>(hctr[kCtrRows + k]);
+    const int n_num_slab = n_rows[kRowSlab];
+    const int64_t total_tiles = static_cast<int64_t>(hctr[kCtrTiles]);
+    const int64_t total_nnz = static_cast<int64_t>(hctr[kCtrNnz]);
     const double sym_count_ms = ms_since(t_sym);
 
     // ---- allocate C -----------------------------------------------------
@@ -2248,6 +2287,8 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     c->nnz = total_nnz;
     RTT_TRY(c->tile_col.ensure(c->num_tiles * sizeof(int)));
     RTT_TRY(c->tile_mask.ensure(c->num_tiles * sizeof(uint64_t)));
+    // The sizes pass wrote the last offset where the array was long enough.
+    const bool ended = (c->num_tiles + 1) * sizeof(int64_t) <= c->tile_nnz.bytes;
     RTT_TRY(c->tile_nnz.ensure((c->num_tiles + 1) * sizeof(int64_t)));
     RTT_TRY(c->tile_csr_ptr.ensure(c->num_tiles * 8));
     RTT_TRY(c->tile_csr_col.ensure(c->nnz));
@@ -2276,7 +2317,7 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
                            g.tile_fill, g.a_trp, g.a_row_off);
     if (n_num_slab > 0 && c->num_tiles > 0)
         hipLaunchKernelGGL(symbolic_write_kernel, dim3(blocks_for(n_num_slab, kWavesPerBlock)),
-                           dim3(kThreads), 0, s, w->num_rows.as<int>(), n_num_slab, st,
+                           dim3(kThreads), 0, s, lists.rows[kRowSlab], n_num_slab, st,
                            w->row_level.as<int>(), co, 0.f, nullptr, nullptr);
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[3], s));
@@ -2284,9 +2325,10 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
         hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(slab_blocks), dim3(kThreads), 0, s,
                            g, slab_rows, n_slab, queue + 1, static_rows,
                            w->slab.as<unsigned long long>(), nullptr, nullptr, ss, co);
-    hipLaunchKernelGGL(set_last_kernel, dim3(1), dim3(1), 0, s,
-                       c->tile_nnz.as<int64_t>() + c->num_tiles,
-                       w->c_row_nnz_off.as<int64_t>() + R);
+    if (!ended)
+        hipLaunchKernelGGL(set_last_kernel, dim3(1), dim3(1), 0, s,
+                           c->tile_nnz.as<int64_t>() + c->num_tiles,
+                           w->c_row_nnz_off.as<int64_t>() + R);
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[6], s));
     // ---- numeric ----------------------------------------------------------
@@ -2322,31 +2364,30 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
         RTT_TRY(tile_numeric(a, tile->bc, *c, *tile, w, s));
         RTT_HIP(hipEventRecord(ev->ev[5], s));
     }
-    if (any_vector && R > 0 && c->nnz > 0) {
-        if (trace_slots)
-            hipLaunchKernelGGL((numeric_row_kernel<SmallRow, true>), dim3(R), dim3(kThreads), 0,
-                               s, g, b.records.as<int4>(), b.num_tiles, nullptr,
-                               w->row_level.as<int>(), st, co, tl);
-        else
-            hipLaunchKernelGGL((numeric_row_kernel<SmallRow>), dim3(R), dim3(kThreads), 0, s, g,
-                               b.records.as<int4>(), b.num_tiles, nullptr,
-                               w->row_level.as<int>(), st, co, tl);
-    }
+    auto rows_launch = [&](auto kernel, int cls, int threads, bool every) {
+        if (n_rows[cls] > 0)
+            hipLaunchKernelGGL(kernel, dim3(n_rows[cls]), dim3(threads), 0, s, g,
+                               b.records.as<int4>(), b.num_tiles,
+                               every ? nullptr : lists.rows[cls], w->row_level.as<int>(), st, co,
+                               Timeline{});
+    };
+    // SmallRow takes the rows of its list, or every row when all of them are
+    // its own (a list entry is one more dependent load per row).  Launched
+    // over every row whatever its class, as the traced form still is, the
+    // workgroups that leave at once took 0.3 of the AMG batch's 3.0 ms.
+    if (trace_slots && any_vector)
+        hipLaunchKernelGGL((numeric_row_kernel<SmallRow, true>), dim3(R), dim3(kThreads), 0, s, g,
+                           b.records.as<int4>(), b.num_tiles, nullptr, w->row_level.as<int>(), st,
+                           co, tl);
+    else
+        rows_launch(numeric_row_kernel<SmallRow>, kRowSmall, SmallRow::kThreads,
+                    n_rows[kRowSmall] == R);
     RTT_HIP(hipGetLastError());
     if (!any_tile)
         RTT_HIP(hipEventRecord(ev->ev[5], s));
-    if (any_vector && n_num_tiny > 0)
-        hipLaunchKernelGGL((numeric_row_kernel<TinyRow>), dim3(n_num_tiny), dim3(TinyRow::kThreads),
-                           0, s, g, b.records.as<int4>(), b.num_tiles, w->tiny_rows.as<int>(),
-                           w->row_level.as<int>(), st, co, Timeline{});
-    if (any_vector && n_num_mid > 0)
-        hipLaunchKernelGGL((numeric_row_kernel<MediumRow>), dim3(n_num_mid), dim3(kThreads), 0,
-                           s, g, b.records.as<int4>(), b.num_tiles, w->mid_rows.as<int>(),
-                           w->row_level.as<int>(), st, co, Timeline{});
-    if (n_num_lds > 0)
-        hipLaunchKernelGGL((numeric_row_kernel<LargeRow>), dim3(n_num_lds), dim3(kThreads), 0,
-                           s, g, b.records.as<int4>(), b.num_tiles, w->lds_rows.as<int>(),
-                           w->row_level.as<int>(), st, co, Timeline{});
+    rows_launch(numeric_row_kernel<TinyRow>, kRowTiny, TinyRow::kThreads, false);
+    rows_launch(numeric_row_kernel<MediumRow>, kRowMid, MediumRow::kThreads, false);
+    rows_launch(numeric_row_kernel<LargeRow>, kRowLarge, LargeRow::kThreads, false);
     if (n_num_slab > 0) {
         DevBuf &tab = w->slab;   // reused: the symbolic slab pass has been queued before
         const int blocks = slab_grid(n_num_slab, num_cus, BC, sizeof(int4), tab);
@@ -2355,22 +2396,22 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
         hipLaunchKernelGGL(fill_i32_kernel, dim3(blocks_for(4 * ents, kThreads)), dim3(kThreads), 0,
                            s, tab.as<int>(), 4 * ents, -1);
         // The symbolic fill pass above is queued before this sort reuses rows_sorted.
-        const int *num_rows = w->num_rows.as<int>();
+        const int *num_rows = lists.rows[kRowSlab];
         if (lb_mode == RTT_LB_ADAPTIVE_TAIL)
-            RTT_TRY(order_rows_by_cost(w->num_rows.as<int>(), n_num_slab, g, w, s, &num_rows));
+            RTT_TRY(order_rows_by_cost(num_rows, n_num_slab, g, w, s, &num_rows));
         hipLaunchKernelGGL(numeric_slab_kernel, dim3(blocks), dim3(kThreads), 0, s, g,
                            b.records.as<int4>(), b.num_tiles, num_rows, n_num_slab, queue + 2,
                            static_rows, tab.as<int4>(), co);
         RTT_HIP(hipGetLastError());
     }
-    RTT_HIP(hipEventRecord(ev->ev[7], s));
     RTT_HIP(hipStreamSynchronize(s));
     if (any_tile && c->num_tiles > 0) {
-        RTT_HIP(hipMemcpy(&times->mfma_pairs, w->tile_pairs.ptr, sizeof(unsigned long long),
-                          hipMemcpyDeviceToHost));
-        if (tile->tail)
-            RTT_TRY(tail_stats(w, &times->tail_reason, &times->tail_records,
-                               &times->tail_chunks));
+        // Written by the last of the tile-pair path's kernels.
+        const unsigned long long *st = w->host_tile_stats.as<unsigned long long>();
+        times->mfma_pairs = st[0];
+        times->tail_reason = static_cast<int>(st[1]);
+        times->tail_records = st[2];
+        times->tail_chunks = st[3];
     }
     if (trace_slots)
         RTT_TRY(write_timeline(trace_path, tl, trace_slots, static_cast<uint64_t>(R),
@@ -2385,7 +2426,7 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     times->sym_fill_kernel_ms = event_ms(ev->ev[2], ev->ev[3]);
     times->numeric_kernel_ms = event_ms(ev->ev[4], ev->ev[5]);
     times->pairs = pairs;
-    times->heavy_rows = static_cast<unsigned long long>(n_num_slab + n_num_lds + n_num_mid);
+    times->heavy_rows = static_cast<unsigned long long>(n_num_slab + n_rows[kRowLarge] + n_rows[kRowMid]);
     return RTT_OK;
 }
 

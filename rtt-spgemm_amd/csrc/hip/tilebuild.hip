@@ -139,53 +139,9 @@ __device__ __forceinline__ int4 tile_meta(int col, uint32_t mask, int64_t off, b
                      static_cast<int>(off) | (dense ? INT_MIN : 0));
 }
 
-// Look-back words of workgroup b: state in the top two bits (0 nothing yet,
-// 1 the workgroup's own sums, 2 sums up to and with it); word 0 holds tiles
-// (31 bits) over dense tiles (31 bits), word 1 payload slots.  Both fields
-// of word 0 stay below 2^31: there are at most nnz <= INT_MAX tiles.
-constexpr unsigned long long kOwn = 1ull << 62, kUpTo = 2ull << 62, kSums = kOwn - 1ull;
-
-__device__ __forceinline__ void publish(unsigned long long *look, int64_t b,
-                                        unsigned long long state, unsigned long long x,
-                                        unsigned long long y)
-{
-    __hip_atomic_store(look + 2 * b, state | x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(look + 2 * b + 1, state | y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Sums of the workgroups before b, by one wave, 64 of them at a time.
-// Workgroups take their numbers from a ticket, so every workgroup before b
-// has started and publishes its own sums without waiting for anything: the
-// wait ends.
-__device__ __forceinline__ void look_back(const unsigned long long *look, int64_t b,
-                                          unsigned long long *x, unsigned long long *y)
-{
-    unsigned long long sx = 0, sy = 0;
-    for (int64_t hi = b; hi > 0; hi -= kWave) {
-        const int64_t i = hi - 1 - lane_id();
-        unsigned long long wx = kUpTo, wy = kUpTo;
-        if (i >= 0) {
-            for (;;) {
-                wx = __hip_atomic_load(look + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                wy = __hip_atomic_load(look + 2 * i + 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                if ((wx >> 62) != 0 && (wx >> 62) == (wy >> 62))
-                    break;
-                __builtin_amdgcn_s_sleep(1);
-            }
-        }
-        const unsigned long long done = __ballot((wx >> 62) == 2);
-        const int last = done ? __builtin_ctzll(done) : kWave - 1;
-        const bool take = lane_id() <= last;
-        sx += wave_sum(take ? wx & kSums : 0ull);
-        sy += wave_sum(take ? wy & kSums : 0ull);
-        if (done)
-            break;
-    }
-    *x = sx;
-    *y = sy;
-}
-
+// Look-back words of the build: word 0 holds tiles (31 bits) over dense tiles
+// (31 bits), word 1 payload slots.  Both fields of word 0 stay below 2^31:
+// there are at most nnz <= INT_MAX tiles.
 __global__ void build_init_kernel(unsigned long long *p, int64_t n, unsigned long long *q)
 {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;

@@ -45,7 +45,7 @@ constexpr int kBatch = 4;       // pairs whose operand loads are issued together
                                 // block-FEM product 5 % faster than 8: fewer registers, no
                                 // spills, and the next batch's loads are issued sooner)
 constexpr int kEnumRounds = 4;  // rounds of 64 B column entries whose K are loaded together
-constexpr int kRowGrab = 8;     // tile rows a wave takes from a row queue at once (one atomic:
+constexpr int kRowGrab = 8;     // most tile rows a wave takes from a row queue at once (one atomic:
                                 // per-row atomics on 8 heads serialise at the L2); with the
                                 // queues interleaved, 8 ran 6 % faster than 16 and 4 or 32
 static_assert(kPairCap % kBatch == 0 && kPairCap >= 2 * kWave, "pair buffer");
@@ -66,6 +66,7 @@ struct TileTask {
     const int *__restrict__ a_row_off;   // A payload offset of each tile row
     float fill;                          // rows taken: A tiles' mean stored values >= fill
     int *__restrict__ queue;             // kXcds row-queue heads, zero at launch
+    int grab;                            // rows per queue chunk
     unsigned long long *__restrict__ mfma_pairs;   // pairs multiplied (one MFMA each)
     // Heavy C tiles split into chunks (bit t of heavy: C tile t), used when
     // tail->enabled; null when no admission ran.
@@ -725,7 +726,7 @@ void tile_numeric_kernel(TileTask g)
     const int home = blockIdx.x % kXcds;
     for (int probe = 0; probe < kXcds; ++probe) {
         const int x = (home + probe) % kXcds;
-        // Queue x hands out chunks x, x + 8, x + 16, ... of kRowGrab rows, so
+        // Queue x hands out chunks x, x + 8, x + 16, ... of g.grab rows, so
         // that the XCDs work through one window of consecutive rows
         // together (faster than a contiguous eighth of the rows each).
         for (;;) {
@@ -733,11 +734,11 @@ void tile_numeric_kernel(TileTask g)
             if (lane == 0)
                 r = atomicAdd(&g.queue[x], 1);
             const int64_t base64 =
-                (static_cast<int64_t>(read_lane(r, 0)) * kXcds + x) * kRowGrab;
+                (static_cast<int64_t>(read_lane(r, 0)) * kXcds + x) * g.grab;
             if (base64 >= g.rows)
                 break;
             const int base = static_cast<int>(base64);
-            const int rend = min(base + kRowGrab, g.rows);
+            const int rend = min(base + g.grab, g.rows);
             for (int row = base; row < rend; ++row) {
                 const int64_t c0 = g.c_ptr[row], c1 = g.c_ptr[row + 1];
                 if (c0 == c1)
@@ -1092,6 +1093,25 @@ __global__ void zero_queue_kernel(int *q, int n, unsigned long long *pairs)
         *pairs = 0ull;
 }
 
+// The call's tile statistics to the host's buffer: pairs, tail gate reason,
+// admitted records, chunks of the split tiles.
+__global__ void tile_stats_kernel(const unsigned long long *pairs, const TailState *st,
+                                  unsigned long long *host)
+{
+    host[0] = *pairs;
+    host[1] = st ? static_cast<unsigned long long>(st->reason) : 0ull;
+    host[2] = st ? st->count : 0ull;
+    host[3] = st && st->enabled ? st->chunks : 0ull;
+}
+
+// Rows a wave takes from a row queue at once: kRowGrab for the fewest queue
+// atomics, fewer when that would leave waves without rows (a wave of a
+// 2000-row product held 8 rows while seven eighths of the chip idled).
+int row_grab(int64_t rows, int64_t waves)
+{
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kRowGrab, rows / (2 * waves))));
+}
+
 } // namespace
 
 TileColumns b_columns(const DevTiles &b)
@@ -1125,14 +1145,13 @@ __global__ __launch_bounds__(kCountThreads) void count_tile_rows_kernel(
     unsigned int m = 0, n = 0;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
         const int t = trp[r + 1] - trp[r];
-        const bool any = t > 0;
-        const bool take =
-            any && static_cast<float>(row_off[r + 1] - row_off[r]) >= fill * static_cast<float>(t);
-        m += __popcll(__ballot(take));
-        n += __popcll(__ballot(any));
+        n += t > 0 ? 1u : 0u;
+        m += t > 0 && static_cast<float>(row_off[r + 1] - row_off[r]) >= fill * static_cast<float>(t)
+                 ? 1u
+                 : 0u;
     }
-    // Lane 0 holds the wave's smallest row, so it takes part in every ballot
-    // of its wave and its sums are the wave's totals.
+    m = wave_sum(m);
+    n = wave_sum(n);
     if (lane_id() == 0) {
         s_m[threadIdx.x / kWave] = m;
         s_n[threadIdx.x / kWave] = n;
@@ -1152,9 +1171,10 @@ __global__ __launch_bounds__(kCountThreads) void count_tile_rows_kernel(
     }
 }
 
-int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, int64_t *tile_rows,
-                    int64_t *nonempty_rows)
+int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, RowRouting *out)
 {
+    if (out->fill == fill)
+        return RTT_OK;
     hipStream_t s = ctx().stream;
     RTT_TRY(scratch->ensure(2 * sizeof(unsigned long long)));
     unsigned long long *d = scratch->as<unsigned long long>();
@@ -1170,8 +1190,9 @@ int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, int64_t *til
     unsigned long long h[2] = {0, 0};
     RTT_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
     RTT_HIP(hipStreamSynchronize(s));
-    *tile_rows = static_cast<int64_t>(h[0]);
-    *nonempty_rows = static_cast<int64_t>(h[1]);
+    out->tile_rows = static_cast<int64_t>(h[0]);
+    out->nonempty = static_cast<int64_t>(h[1]);
+    out->fill = fill;
     return RTT_OK;
 }
 
@@ -1185,6 +1206,7 @@ int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const 
         return fail(RTT_ERR_INVALID, "unknown tile numeric precision %d", precision);
     RTT_TRY(w->tile_queue.ensure(kXcds * sizeof(int)));
     RTT_TRY(w->tile_pairs.ensure(sizeof(unsigned long long)));
+    RTT_TRY(w->host_tile_stats.ensure(4 * sizeof(unsigned long long)));
     TileTask g;
     g.rows = static_cast<int>(c.tilem);
     g.a_trp = a.tile_row_ptr.as<int>();
@@ -1254,6 +1276,7 @@ int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const 
     // Persistent: enough workgroups to fill every CU several times over.
     const int blocks = static_cast<int>(std::min<int64_t>(
         static_cast<int64_t>(cus) * 8, (static_cast<int64_t>(g.rows) + kTWaves - 1) / kTWaves));
+    g.grab = row_grab(g.rows, static_cast<int64_t>(blocks) * kTWaves);
     if (precision == 0)
         hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(std::max(blocks, 1)),
                            dim3(kTThreads), 0, s, g);
@@ -1271,6 +1294,9 @@ int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const 
         hipLaunchKernelGGL(tail_reduce_kernel, dim3(cus * 2), dim3(kTThreads), 0, s, g, t);
         RTT_HIP(hipGetLastError());
     }
+    hipLaunchKernelGGL(tile_stats_kernel, dim3(1), dim3(1), 0, s, g.mfma_pairs, g.tail,
+                       w->host_tile_stats.as<unsigned long long>());
+    RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
 
@@ -1315,6 +1341,7 @@ int tile_values_noalloc(const DevTiles &a, const TileColumns &bc, const DevC &c,
     const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
     const int blocks = static_cast<int>(std::min<int64_t>(
         static_cast<int64_t>(cus) * 8, (static_cast<int64_t>(g.rows) + kTWaves - 1) / kTWaves));
+    g.grab = row_grab(g.rows, static_cast<int64_t>(blocks) * kTWaves);
     if (precision == 0)
         hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(std::max(blocks, 1)),
                            dim3(kTThreads), 0, s, g);
@@ -1322,17 +1349,6 @@ int tile_values_noalloc(const DevTiles &a, const TileColumns &bc, const DevC &c,
         hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(std::max(blocks, 1)),
                            dim3(kTThreads), 0, s, g);
     RTT_HIP(hipGetLastError());
-    return RTT_OK;
-}
-
-int tail_stats(SpgemmWork *w, int *reason, unsigned long long *records,
-               unsigned long long *chunks)
-{
-    TailState st{};
-    RTT_HIP(hipMemcpy(&st, w->tail_state.ptr, sizeof(st), hipMemcpyDeviceToHost));
-    *reason = st.reason;
-    *records = st.count;
-    *chunks = st.enabled ? st.chunks : 0ull;
     return RTT_OK;
 }
 
