@@ -411,7 +411,8 @@ typedef struct rtt_stats {       /* DmmaSpGemmStats subset */
                                           C tiles were cut into (0 when not split) */
     int output_materialized;
     int numeric_path;                  /* VECTOR, TILE, or AUTO when rows took both */
-    double b_columns_ms;               /* TILE: B's tile columns built for the call */
+    double b_columns_ms;               /* TILE: B's tile columns built for the call (only
+                                          when a C tile can reach the tail queue) */
     unsigned long long mfma_pairs;     /* TILE: tile pairs multiplied: one FP64 MFMA
                                           (4 blocks x 4x4x4, 512 flops) each, or for
                                           SPLIT_BF16 eight BF16 16x16x32 MFMAs */
@@ -440,12 +441,10 @@ int rtt_tilespgemm(const rtt_prepared_a *a, const rtt_dynamic_b *b,
  * (by rtt_tilespgemm with B = b, every row on the TILE path, b not rebuilt
  * since; a values-only rtt_update_b_values in between is what it is for)
  * into c_values, nnz(C) doubles of device memory the caller owns, in C's
- * value order, with `precision` (enum rtt_precision).  Allocates nothing:
- * its scratch (8 row-queue heads and a pair counter, 40 bytes) lives in a
- * fixed 256-byte device array per GPU, cleared by a kernel on every call.
- * Calls that overlap on one GPU race on that array.  Heavy tiles run whole
- * (no tail split).  Queues the kernels on the library stream and returns;
- * rtt_sync() waits for them. */
+ * value order, with `precision` (enum rtt_precision).  Allocates nothing and
+ * needs no scratch.  Heavy tiles run whole (no tail split).  Queues one kernel
+ * on the library stream and returns;
+ * rtt_sync() waits for it. */
 int rtt_tile_values_noalloc(const rtt_prepared_a *a, const rtt_dynamic_b *b, int precision,
                             double *c_values);
 

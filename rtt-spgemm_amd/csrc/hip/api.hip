@@ -13,17 +13,6 @@
 
 #include "internal.hpp"
 
-// Scratch of rtt_tile_values_noalloc: a fixed device array instead of an
-// allocation (each GPU holds its own copy until the process ends).  Host code
-// uses only the per-device address hipGetSymbolAddress returned for it.
-constexpr size_t kNoAllocScratchBytes = 256;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
-
-namespace {
-constexpr int kMaxDevices = 64;
-void *g_scratch_dev[kMaxDevices] = {};   // address of `scratch` on each device
-} // namespace
-
 struct rtt_prepared_a {
     rtt::DevCsr csr;          // input CSR, rows column-sorted (B source)
     rtt::DevCsr csr_tiled;    // reordered copy when a permutation is given
@@ -233,11 +222,6 @@ int rtt_init(int device)
         return fail(RTT_ERR_INVALID, "rtt_init: device %d not present (%d devices)", device,
                     count);
     RTT_HIP(hipSetDevice(device));
-    if (device < kMaxDevices && !g_scratch_dev[device]) {
-        void *p = nullptr;
-        RTT_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-        g_scratch_dev[device] = p;
-    }
     RTT_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
     RTT_HIP(hipDeviceGetAttribute(&c.num_cus, hipDeviceAttributeMultiprocessorCount, device));
     c.device = device;
@@ -773,16 +757,16 @@ int rtt_tilespgemm(const rtt_prepared_a *a_const, const rtt_dynamic_b *b, rtt_sm
     topt.record_capacity = sc.tail_record_capacity;
     if (path != RTT_NUMERIC_TILE)
         RTT_TRY(rtt::ensure_record_values(&const_cast<rtt_dynamic_b *>(b)->tiles));
-    if (path != RTT_NUMERIC_VECTOR) {
-        rtt_dynamic_b *bm = const_cast<rtt_dynamic_b *>(b);
-        auto tc = rtt::Clock::now();
-        RTT_TRY(rtt::build_b_columns(&bm->tiles, &bm->build));
-        RTT_HIP(hipStreamSynchronize(rtt::ctx().stream));
-        stats->b_columns_ms = rtt::ms_since(tc);
-        topt.bc = rtt::b_columns(b->tiles);
+    topt.b = &const_cast<rtt_dynamic_b *>(b)->tiles;
+    topt.b_work = &const_cast<rtt_dynamic_b *>(b)->build;
+    if (path != RTT_NUMERIC_VECTOR && topt.tail) {
+        if (a->routing.fill < 0.f)
+            RTT_TRY(rtt::count_tile_rows(a->tiles, fill, &a->build.counters, &a->routing));
+        topt.longest_a = a->routing.longest;
     }
     RTT_TRY(rtt::spgemm_core(a->tiles, b->tiles, &a->last_c, &a->core, &a->events, &times,
                             sc.lb_mode, path == RTT_NUMERIC_VECTOR ? nullptr : &topt));
+    stats->b_columns_ms = times.b_columns_ms;
     stats->numeric_path = path;
     stats->precision = path == RTT_NUMERIC_VECTOR ? RTT_PRECISION_FP64 : sc.precision;
     a->last_b = b;
@@ -996,14 +980,7 @@ int rtt_tile_values_noalloc(const rtt_prepared_a *a, const rtt_dynamic_b *b, int
         return fail(RTT_ERR_INVALID,
                     "rtt_tile_values_noalloc: needs C's structure from an rtt_tilespgemm on this "
                     "(A, B) whose rows all took the TILE path, with B not rebuilt since");
-    if (!b->tiles.transpose_of && !b->tiles.cols_ready)
-        return fail(RTT_ERR_INVALID, "rtt_tile_values_noalloc: B's tile columns are not built");
-    const int dev = rtt::ctx().device;
-    if (dev < 0 || dev >= kMaxDevices || !g_scratch_dev[dev])
-        return fail(RTT_ERR_INVALID, "rtt_tile_values_noalloc: no scratch address for device %d",
-                    dev);
-    return rtt::tile_values_noalloc(a->tiles, rtt::b_columns(b->tiles), a->last_c, precision,
-                                    g_scratch_dev[dev], kNoAllocScratchBytes, c_values,
+    return rtt::tile_values_noalloc(a->tiles, b->tiles, a->last_c, precision, c_values,
                                     rtt::ctx().stream);
 }
 

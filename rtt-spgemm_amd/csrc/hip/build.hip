@@ -416,8 +416,9 @@ __global__ void column_count_kernel(int64_t n, const int *__restrict__ col, int 
         atomicAdd(&counts[col[t]], 1);
 }
 
-// One atomic per workgroup: an atomic per wave on the one address
-// serialises (0.1 ms on 2^19 columns).
+// At most one atomic per workgroup, and none once the largest count so far
+// is as large: an atomic per wave on the one address serialises (0.1 ms on
+// 2^19 columns).
 __global__ void __launch_bounds__(kThreads) column_max_kernel(int cols, int *__restrict__ counts)
 {
     __shared__ int s_max[kThreads / kWave];
@@ -432,7 +433,7 @@ __global__ void __launch_bounds__(kThreads) column_max_kernel(int cols, int *__r
     if (threadIdx.x == 0) {
         for (int w = 1; w < kThreads / kWave; ++w)
             m = max(m, s_max[w]);
-        if (m > 0)
+        if (m > __hip_atomic_load(&counts[cols], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             atomicMax(&counts[cols], m);
     }
 }
@@ -707,6 +708,30 @@ __global__ void column_entries_kernel(int64_t n, const int *__restrict__ ids,
     const int t = ids[p];
     const int4 m = meta[t];
     out[p] = make_int4(row_of[t], m.y, m.z, m.w);
+}
+
+__global__ void column_longest_kernel(const int *counts, int cols, unsigned long long *host)
+{
+    *host = static_cast<unsigned long long>(counts[cols]);
+}
+
+int longest_b_column(const DevTiles &b, DevBuf *scratch, unsigned long long *host)
+{
+    hipStream_t s = ctx().stream;
+    const int C = b.tile_col_count;
+    RTT_TRY(scratch->ensure((static_cast<size_t>(C) + 1) * sizeof(int)));
+    int *counts = scratch->as<int>();
+    hipLaunchKernelGGL(fill_int_kernel, dim3(blocks_for(C + 1, kThreads)), dim3(kThreads), 0, s,
+                       counts, static_cast<int64_t>(C) + 1, 0);
+    if (b.num_tiles > 0) {
+        hipLaunchKernelGGL(column_count_kernel, dim3(blocks_for(b.num_tiles, kThreads)),
+                           dim3(kThreads), 0, s, b.num_tiles, b.tile_col_idx.as<int>(), counts);
+        hipLaunchKernelGGL(column_max_kernel, dim3(blocks_for(C, kThreads)), dim3(kThreads), 0, s,
+                           C, counts);
+    }
+    hipLaunchKernelGGL(column_longest_kernel, dim3(1), dim3(1), 0, s, counts, C, host);
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
 }
 
 int build_b_columns(DevTiles *b, BuildWork *w)

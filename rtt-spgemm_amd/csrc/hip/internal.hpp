@@ -106,7 +106,8 @@ struct DevTiles {
     bool cols_ready = false;    // col_ptr / col_ent valid (B built from a CSR)
     bool rec_values_ready = true;   // B from a CSR: values_cm and record planes 1.. valid
     bool arrays_ready = true;   // tile_col_idx / masks / value_offsets / values valid
-    DevBuf tile_row_ptr, tile_col_idx, value_offsets, masks, values;
+    DevBuf tile_row_ptr, tile_col_idx, value_offsets, masks;
+    DevBuf values;        // payload, then (tiles built from a CSR) one zero
     DevBuf tile_col_ptr, tile_row_idx, csc_tile_ids;
     DevBuf tile_row_of;   // tile -> tile row (A: used by the B transpose)
     DevBuf meta;          // A only: int4 per tile
@@ -116,8 +117,8 @@ struct DevTiles {
     DevBuf a_blight;      // B only: per A tile, {first, count} of the light tiles it can meet
     DevBuf pair_total;    // B only: u64, sum over A tiles of their B row's tile count
     DevBuf row_groups;    // B only: start of each (row, class) run, kClassSlots per row
-    DevBuf col_ptr;       // B only: tile-column pointer of col_ent (tile_col_count + 1)
-    DevBuf col_ent;       // B only: per tile column, its tiles in tile-row order as
+    DevBuf col_ptr;       // B, tail queue only: tile-column pointer of col_ent (tile_col_count + 1)
+    DevBuf col_ent;       // B, tail queue only: per tile column, its tiles in tile-row order as
                           // {tile row K, mask, per-k byte sets, offset | dense bit}
     DevBuf values_cm;     // each tile's values with the stride-4 bit groups in order:
                           // A (8x4): column-major; B (4x8): k-major (row k's entries
@@ -175,12 +176,12 @@ struct SpgemmWork {
     // call's start, never while a fill pass may still read the buffer).
     DevBuf slab_stage_j, slab_stage_m, slab_row_off;
     uint64_t slab_stage_cap = 0, slab_stage_need = 0;
-    DevBuf tile_queue;                      // row-queue heads of the tile-pair kernels
-    DevBuf tile_pairs;                      // u64: pairs the tile-pair kernel multiplied
+    DevBuf tile_pairs;                      // u64: pairs the tile-pair kernel multiplied, sharded
     PinnedBuf host_tile_stats;              // u64: pairs, tail reason, records, chunks
     // Tail queue of the tile-pair path: records, state, chunk prefix, heavy
     // tile bitset and the chunks' partial tiles.
     DevBuf tail_records, tail_state, tail_chunk_base, tail_heavy, tail_workspace;
+    bool tail_ran = false;   // the last tile-pair call ran the admission
 };
 
 // Scratch of the tile builders, reused across calls.
@@ -254,35 +255,39 @@ int build_pair_extents(const DevTiles &a, DevTiles *b, const unsigned int *flag 
 // built from a CSR; no-op for B = A^T at tile level, whose columns are A's
 // tile rows (b_columns below).
 int build_b_columns(DevTiles *b, BuildWork *w);
+// Queues the count of the tiles in B's longest tile column (B built from a
+// CSR) into *host.
+int longest_b_column(const DevTiles &b, DevBuf *scratch, unsigned long long *host);
 // Builds the record value planes (and values_cm) of a B built from a CSR when
 // they are missing (the LDS-accumulator numeric kernels read them; the
 // symbolic and tile-pair kernels do not).
 int ensure_record_values(DevTiles *b);
 
 // ---- tile-pair numeric path (tiletask.hip) ---------------------------------
-// B's tile columns as the tile-pair kernels read them: ptr[J]..ptr[J+1] index
+// B's tile columns as the tail queue reads them: ptr[J]..ptr[J+1] index
 // ent, entries {tile row K, mask, per-k bytes, payload offset | dense bit} in
-// increasing K, payload `vals` (each tile column-major).
+// increasing K.
 struct TileColumns {
     const int *ptr = nullptr;
     const int4 *ent = nullptr;
-    const double *vals = nullptr;
 };
 TileColumns b_columns(const DevTiles &b);
-// Values of the C tiles of every tile row whose A tiles hold at least `fill`
-// stored values on average (0: every row), from C's finished structure:
-// precision 0 on FP64 matrix cores, 1 by BF16 slices (Ozaki scheme) with
-// FP64 recombination.  Deterministic: each tile sums its pairs in
-// increasing K.
+// Whether some C tile can clear the tail queue's admission threshold when an
+// A tile row holds at most a_tiles tiles and a B tile column b_tiles.
+bool tail_possible(int a_tiles, int64_t b_tiles, float threshold);
+// Values of the C tiles of every tile row whose A tiles hold at least
+// opt.fill stored values on average (0: every row), from C's finished
+// structure: precision 0 on FP64 matrix cores, 1 by BF16 slices (Ozaki
+// scheme) with FP64 recombination.  Deterministic: each tile sums its pairs
+// in increasing K.  The tail queue runs when its columns are given.
 struct TileOpts;
-int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const TileOpts &opt,
-                 SpgemmWork *w, hipStream_t s);
+int tile_numeric(const DevTiles &a, const DevTiles &b, const DevC &c, const TileOpts &opt,
+                 const TileColumns *tail_columns, SpgemmWork *w, hipStream_t s);
 // C's values for C's existing structure, every row on the tile-pair kernel,
-// written to c_values; the row-queue heads and pair counter live in the
-// caller's `scratch` (device memory of scratch_bytes).  Launches kernels
-// only: no allocation, no host synchronisation; no tail split.
-int tile_values_noalloc(const DevTiles &a, const TileColumns &bc, const DevC &c, int precision,
-                        void *scratch, size_t scratch_bytes, double *c_values, hipStream_t s);
+// written to c_values.  One kernel: no scratch, no allocation, no host
+// synchronisation; no tail split.
+int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, int precision,
+                        double *c_values, hipStream_t s);
 // The admitted records (slot order): tile, merge scans and matches, chunks.
 int tail_records(SpgemmWork *w, int max_records, long long *task, int *scans, int *matches,
                  int *chunks, int *count);
@@ -292,6 +297,7 @@ int tail_records(SpgemmWork *w, int max_records, long long *task, int *scans, in
 struct RowRouting {
     float fill = -1.f;   // threshold counted for (negative: none)
     int64_t tile_rows = 0, nonempty = 0;
+    int longest = 0;     // most A tiles in a tile row
 };
 int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, RowRouting *out);
 // Per-row numeric routing of one call: rows whose A tiles hold at least
@@ -301,7 +307,10 @@ int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, RowRouting *
 struct TileOpts {
     float fill = 0.f;
     int precision = 0;
-    TileColumns bc;
+    int longest_a = 0;   // most A tiles in a tile row
+    // B's columns for the tail queue, built by the call that needs them.
+    DevTiles *b = nullptr;
+    BuildWork *b_work = nullptr;
     bool tail = false;
     float threshold = 16384.f, target = 8192.f;
     int max_chunks = 8;
@@ -315,6 +324,7 @@ struct CoreTimes {
     double symbolic_ms = 0, allocation_ms = 0, numeric_ms = 0;
     double sym_count_kernel_ms = 0, sym_fill_kernel_ms = 0, numeric_kernel_ms = 0;
     unsigned long long pairs = 0, heavy_rows = 0;
+    double b_columns_ms = 0;             // tail queue: B's tile columns built
     unsigned long long mfma_pairs = 0;   // tile path: (A tile, B tile) products on MFMA
     int tail_reason = 0;                 // tile path: tail gate (0: no admission ran)
     unsigned long long tail_records = 0, tail_chunks = 0;
@@ -328,7 +338,7 @@ struct CoreTimes {
 // values computed by the tile-pair kernel, the others as before.
 int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *work,
                 Events *events, CoreTimes *times, int lb_mode = RTT_LB_ADAPTIVE_TAIL,
-                const TileOpts *tile = nullptr);
+                TileOpts *tile = nullptr);
 
 // ---- scans (scan.hip) -------------------------------------------------------
 // Exclusive sum of n int64 values into out[0..n] (out[n] = total).

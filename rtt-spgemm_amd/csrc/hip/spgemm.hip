@@ -2107,7 +2107,7 @@ static int slab_grid(int rows, int num_cus, int64_t cols, size_t entry, const De
 }
 
 int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Events *ev,
-                CoreTimes *times, int lb_mode, const TileOpts *tile)
+                CoreTimes *times, int lb_mode, TileOpts *tile)
 {
     // tile: rows routed to the tile-pair kernel (all when fill is 0);
     // vector: rows left to the LDS-accumulator kernels.
@@ -2147,7 +2147,7 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     const int64_t size_blocks = std::max<int64_t>(1, blocks_for(R, kThreads));
     const int64_t words = 2 * size_blocks;
     RTT_TRY(w->counters.ensure(static_cast<size_t>(kCounters + words) * sizeof(unsigned long long)));
-    RTT_TRY(w->host_counters.ensure(kCounters * sizeof(unsigned long long)));
+    RTT_TRY(w->host_counters.ensure((kCounters + 1) * sizeof(unsigned long long)));
     unsigned long long *ctr = w->counters.as<unsigned long long>();
     unsigned long long *look = ctr + kCounters;
     const unsigned long long *hctr = w->host_counters.as<unsigned long long>();
@@ -2180,6 +2180,17 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
                        dim3(blocks_for(std::max<int64_t>(words, kCounters), kThreads)),
                        dim3(kThreads), 0, s, ctr, 0, look, words,
                        b.pair_total.as<unsigned long long>(), queue, 4);
+    // The tail queue needs B's tile columns only if some C tile can clear its
+    // threshold: told from B's tile rows where that is enough, else from its
+    // longest tile column (for B = A^T at tile level A's longest tile row),
+    // read with the sizes.
+    bool tail = any_tile && tile->tail && tail_possible(tile->longest_a, b.tile_row_count, tile->threshold);
+    const bool count_columns = tail && !b.transpose_of;
+    if (tail && b.transpose_of)
+        tail = tail_possible(tile->longest_a, tile->longest_a, tile->threshold);
+    if (count_columns)
+        RTT_TRY(longest_b_column(b, &tile->b_work->keys_in,
+                                 w->host_counters.as<unsigned long long>() + kCounters));
     // One wave per row first; rows that outgrow its table go to the
     // workgroup table, and rows that outgrow that to the slab.
     RTT_HIP(hipEventRecord(ev->ev[0], s));
@@ -2332,6 +2343,17 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[6], s));
     // ---- numeric ----------------------------------------------------------
+    if (count_columns)
+        tail = tail_possible(tile->longest_a, static_cast<int64_t>(hctr[kCounters]),
+                             tile->threshold);
+    TileColumns columns;
+    if (tail) {
+        auto tc = Clock::now();
+        RTT_TRY(build_b_columns(tile->b, tile->b_work));
+        RTT_HIP(hipStreamSynchronize(s));
+        times->b_columns_ms = ms_since(tc);
+        columns = b_columns(*tile->b);
+    }
     Timeline tl;
     size_t trace_slots = 0;
     const char *trace_path = std::getenv("DMMA_TRACE_FILE");
@@ -2361,7 +2383,7 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     }
     RTT_HIP(hipEventRecord(ev->ev[4], s));
     if (any_tile) {
-        RTT_TRY(tile_numeric(a, tile->bc, *c, *tile, w, s));
+        RTT_TRY(tile_numeric(a, b, *c, *tile, tail ? &columns : nullptr, w, s));
         RTT_HIP(hipEventRecord(ev->ev[5], s));
     }
     auto rows_launch = [&](auto kernel, int cls, int threads, bool every) {

@@ -364,8 +364,10 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
         g.tile_row_ptr[g.R] = static_cast<int>(end_tiles);
         if constexpr (B)
             g.groups[static_cast<int64_t>(kClassSlots) * g.R] = static_cast<int>(end_tiles);
-        if (fits)
+        if (fits) {
             g.value_offsets[end_tiles] = static_cast<int>(end_pay);
+            g.values[end_pay] = 0.0;   // the zero that absent entries read
+        }
         g.head->fits = fits ? 1u : 0u;
         g.totals[0] = end_tiles;
         g.totals[1] = end_pay;
@@ -784,7 +786,8 @@ int run_build(const DevCsr &src, const int *row_map, int active_rows, int active
                       meta.bytes / meta_size}));
         g.cap_tiles = std::min<long long>(
             g.cap_tiles, static_cast<long long>(out->value_offsets.bytes / sizeof(int)) - 1);
-        g.cap_payload = static_cast<long long>(out->values.bytes / sizeof(double));
+        // One slot more than the payload: a zero (see DevTiles::values).
+        g.cap_payload = static_cast<long long>(out->values.bytes / sizeof(double)) - 1;
         g.tile_col_idx = out->tile_col_idx.as<int>();
         g.masks = out->masks.as<uint32_t>();
         g.value_offsets = out->value_offsets.as<int>();
@@ -822,7 +825,7 @@ int run_build(const DevCsr &src, const int *row_map, int active_rows, int active
         RTT_TRY(out->tile_col_idx.ensure(n * sizeof(int)));
         RTT_TRY(out->masks.ensure(n * sizeof(uint32_t)));
         RTT_TRY(out->value_offsets.ensure((n + 1) * sizeof(int)));
-        RTT_TRY(out->values.ensure(static_cast<size_t>(totals[1]) * sizeof(double)));
+        RTT_TRY(out->values.ensure((static_cast<size_t>(totals[1]) + 1) * sizeof(double)));
         RTT_TRY(meta.ensure(std::max<size_t>(n, 1) * meta_size));
     }
     out->num_tiles = totals[0];

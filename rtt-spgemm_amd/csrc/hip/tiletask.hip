@@ -12,16 +12,24 @@
 // increasing K, so C's values do not depend on scheduling: two calls give the
 // same bits.
 //
-// Work unit: one wave per C tile row, taken from per-XCD row queues (queue x
-// hands out chunks x, x + 8, x + 16, ... of 8 consecutive rows, so the XCDs
-// work through one window of the rows together; a wave whose XCD queue is
-// drained takes rows from the next XCD's).  The wave stages A row I's tile
-// columns in LDS, then, for up to 64 C tiles at a time, enumerates the B
-// column entries of all of them (one lane per entry), finds each entry's K
-// among A's columns by binary search and compacts the matches, in (C tile,
-// K) order, into an LDS pair list.  The pair loop then issues the operand
-// loads of four pairs at once and runs their products into the running sum,
-// storing each C tile's entries when its pairs end.
+// Work unit: one wave per C tile row, or per part of its C tiles when there
+// are too few rows for the chip, in the launch's own order (chunks of
+// consecutive rows dealt to the XCDs, so that they work through one window of
+// the rows together).  Persistent waves that took rows from eight queue heads
+// in one cache line spent 10 ns an atomic on them, 40000 in a launch of any
+// size: 0.2 ms of a 2000-row product's 0.23 ms.
+//
+// Pairs are found from A's side, up to 64 A tiles at a time: every tile (K,
+// J) of the B rows those A tiles select is one lane's, which finds J among
+// up to 64 C tiles of the row and sets the A tile's bit in that C tile's
+// 64-bit word.  The words give every pair its place: C tiles in order, within
+// one the number of lower bits (its smaller K).  The pairs are written there
+// into an LDS list and run by P::run, which keeps a batch of operand loads in
+// flight behind the products and stores each C tile when its pairs end.
+// Every B tile enumerated belongs to a pair (or to no C tile at all), and B
+// needs no column structure; the search of A's keys for every entry of every
+// B column that this replaces, with the radix sort that made the columns,
+// took the block-FEM 500k step 1.5 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -38,26 +46,33 @@ namespace {
 
 constexpr int kTThreads = 128;
 constexpr int kTWaves = kTThreads / kWave;
-constexpr int kAKeys = 128;     // A tiles of a row staged in LDS (keys, masks, offsets)
-constexpr int kAVals = 512;     // A payload values of a row staged in LDS (0: read from HBM)
-constexpr int kPairCap = 128;   // pairs a wave buffers before running them
-constexpr int kBatch = 4;       // pairs whose operand loads are issued together (4 ran the
-                                // block-FEM product 5 % faster than 8: fewer registers, no
-                                // spills, and the next batch's loads are issued sooner)
-constexpr int kEnumRounds = 4;  // rounds of 64 B column entries whose K are loaded together
-constexpr int kRowGrab = 8;     // most tile rows a wave takes from a row queue at once (one atomic:
-                                // per-row atomics on 8 heads serialise at the L2); with the
-                                // queues interleaved, 8 ran 6 % faster than 16 and 4 or 32
-static_assert(kPairCap % kBatch == 0 && kPairCap >= 2 * kWave, "pair buffer");
+constexpr int kAVals = 512;     // A payload values of a row staged in LDS
+constexpr int kPairCap = 192;   // pairs a wave buffers before running them: 9.3 KB of LDS per
+                                // wave lets the 16 waves run that the registers allow
+constexpr int kBatch = 8;       // pairs whose operand loads are issued together
+constexpr int kEnumRounds = 4;  // rounds of 64 B tiles whose metas are loaded together (and
+                                // kept, when they are all there is)
+constexpr int kXcdChunk = 4;    // workgroups of consecutive units dealt to an XCD at a time
+constexpr int kPairShards = 256;   // counters of the pairs multiplied, a 128-byte line each (one
+constexpr int kShardStride = 16;   // counter would take an atomic from every wave)
+constexpr int kMaxParts = 4;    // most units a tile row is cut into
+constexpr int kPairWords = kPairCap / 64;
+constexpr int kPad = 2 * kBatch;   // pairs of zeros past a list: the batch that its last pairs
+                                   // share, and the batch loaded ahead of that one
+static_assert(kPairCap % 64 == 0 && kPairWords == 3, "words of the end bits");
+static_assert(kPairCap >= kWave, "a C tile has at most 64 pairs per group of A tiles");
 
 struct TileTask {
     int rows;                            // tile rows of A and C
     const int *__restrict__ a_trp;       // A tile row pointer
     const int4 *__restrict__ a_meta;     // {K, mask, per-k bytes, offset | dense}
     const double *__restrict__ a_vals;   // A payload, each tile row-major
-    const int *__restrict__ b_cptr;      // B tile column pointer
-    const int4 *__restrict__ b_cent;     // {K, mask, per-k bytes, offset | dense}
+    const int4 *__restrict__ a_brange;   // per A tile: {first B tile of row K, -, tiles}
+    const int4 *__restrict__ b_meta;     // B tiles row by row: {J, mask, bytes, offset | dense}
     const double *__restrict__ b_vals;   // B payload, each tile column-major
+    uint32_t a_zero, b_zero;             // slots past the payloads that hold 0.0
+    const int *__restrict__ b_cptr;      // tail only: B tile column pointer
+    const int4 *__restrict__ b_cent;     // tail only: {K, mask, per-k bytes, offset | dense}
     const int64_t *__restrict__ c_ptr;   // C tile row pointer
     const int *__restrict__ c_col;
     const unsigned long long *__restrict__ c_mask;
@@ -65,9 +80,9 @@ struct TileTask {
     double *__restrict__ c_val;
     const int *__restrict__ a_row_off;   // A payload offset of each tile row
     float fill;                          // rows taken: A tiles' mean stored values >= fill
-    int *__restrict__ queue;             // kXcds row-queue heads, zero at launch
-    int grab;                            // rows per queue chunk
-    unsigned long long *__restrict__ mfma_pairs;   // pairs multiplied (one MFMA each)
+    int parts;                           // units per tile row
+    unsigned long long *__restrict__ mfma_pairs;   // pairs multiplied (one MFMA each), kPairShards
+                                                   // counters; null: not counted
     // Heavy C tiles split into chunks (bit t of heavy: C tile t), used when
     // tail->enabled; null when no admission ran.
     const uint32_t *__restrict__ heavy;
@@ -97,57 +112,36 @@ struct TailState {
 };
 
 constexpr uint32_t kDense = 0x80000000u;
+constexpr int kTailNone = 4;   // gate reason: no heavy tile
 
-// Entry `phys` (bit position) of a hybrid tile: dense tiles hold all 32 slots
-// (absent entries are zeros), sparse tiles their entries in mask-bit order.
-__device__ __forceinline__ double tile_entry(const double *__restrict__ vals, uint32_t mask,
-                                             uint32_t offw, int phys)
+// A tile in the pair list is {mask, offset} with a full mask for a dense tile
+// (which holds all 32 slots, absent entries as zeros): entry `phys` then lies
+// at offset + popc(mask & below), below = (1 << phys) - 1, whatever the kind.
+__device__ __forceinline__ uint32_t list_mask(int mask, int offw)
 {
-    const uint32_t off = offw & ~kDense;
-    if (offw & kDense)
-        return vals[off + phys];
-    if (!((mask >> phys) & 1u))
-        return 0.0;
-    return vals[off + __popc(mask & ((1u << phys) - 1u))];
+    return offw < 0 ? 0xFFFFFFFFu : static_cast<uint32_t>(mask);
+}
+
+// Slot of an entry, `zero` (a slot that holds 0.0) when the mask lacks it, so
+// that the load is unconditional and its value needs no select.
+__device__ __forceinline__ uint32_t entry_slot(uint32_t mask, uint32_t off, int phys,
+                                               uint32_t below, uint32_t zero)
+{
+    const uint32_t at = off + __popc(mask & below);
+    return (mask >> phys) & 1u ? at : zero;
 }
 
 __device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 
-// Entry `phys` of a tile that is the same in every lane, split so that the
-// load is unconditional: its mask and offset move to scalar registers, the
-// load reads a slot inside the tile (the tile's first slot when the entry is
-// absent), and *has says whether the value counts.  The caller applies `has`
-// where it uses the value, so that the wait for the load lands there and not
-// right after the load.
-__device__ __forceinline__ double tile_entry_raw(const double *vals, uint32_t mask, uint32_t offw,
-                                                 int phys, uint32_t below, bool *has)
+// Value of lane ^ 8 (a rotation by 8 within rows of 16 lanes).
+__device__ __forceinline__ double from_lane_xor8(double v)
 {
-    mask = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(mask)));
-    offw = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(offw)));
-    const uint32_t off = offw & ~kDense;
-    const bool dense = (offw & kDense) != 0;
-    const bool bit = ((mask >> phys) & 1u) != 0;
-    *has = dense || bit;
-    const uint32_t idx = dense ? static_cast<uint32_t>(phys) : (bit ? __popc(mask & below) : 0u);
-    return vals[off + idx];
-}
-
-// tile_entry for a tile that is the same in every lane (the pair loops'
-// operands): its mask and offset move to scalar registers, so the dense test
-// is a scalar branch and a lane's own work is its mask bit and the popcount
-// below it (`below` = (1 << phys) - 1, fixed per lane).
-__device__ __forceinline__ double tile_entry_uniform(const double *__restrict__ vals,
-                                                     uint32_t mask, uint32_t offw, int phys,
-                                                     uint32_t below)
-{
-    mask = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(mask)));
-    offw = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(offw)));
-    const uint32_t off = offw & ~kDense;
-    if (offw & kDense)
-        return vals[off + phys];
-    if (!((mask >> phys) & 1u))
-        return 0.0;
-    return vals[off + __popc(mask & below)];
+    const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0x128, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), 0x128, 0xf, 0xf, false);
+    return __longlong_as_double(static_cast<long long>(
+        (static_cast<unsigned long long>(static_cast<uint32_t>(hi)) << 32) |
+        static_cast<uint32_t>(lo)));
 }
 
 // Lane roles of v_mfma_f64_4x4x4f64 (four independent 4x4x4 blocks; block b,
@@ -159,10 +153,12 @@ struct LaneRoles {
     int a_phys;   // A tile bit r*4+k this lane supplies
     int b_phys;   // B tile bit c*4+k
     int c_bit;    // C tile bit r*8+c this lane accumulates
+    bool lower;   // rows 4..7 of the A tile (h = 1)
     uint32_t a_below, b_below;   // (1 << phys) - 1
     __device__ LaneRoles(int lane)
     {
         const int blk = (lane >> 2) & 3, lo = lane & 3, hi = lane >> 4;
+        lower = (blk >> 1) != 0;
         a_phys = ((blk >> 1) * 4 + lo) * 4 + hi;
         b_phys = ((blk & 1) * 4 + lo) * 4 + hi;
         c_bit = ((blk >> 1) * 4 + hi) * 8 + (blk & 1) * 4 + lo;
@@ -193,9 +189,13 @@ struct Fp64Product {
         double v = 0.0;
     };
     static constexpr unsigned long long kMfmaPerPair = 1;
-    // Waves per SIMD the tile kernel is compiled for: the kernel is bound by
-    // memory latency, and 4 waves (at most 128 VGPRs) ran it 20 % faster
-    // than the 3 the compiler picks unconstrained.
+    // Waves per SIMD the tile kernel is compiled for: its waves wait 64 % of
+    // their time for memory and its vector units are busy 53 %, and 4 waves
+    // (at most 128 VGPRs) ran it 20 % faster than the 3 the compiler picks
+    // unconstrained.  Block-FEM 500k: 2.18 ms for 2.16e7 pairs (5.1 TFLOP/s
+    // on the matrix cores), 2.95 ms with the column search, 2.51 ms before
+    // the list took dense masks and zero slots (31 vector instructions a
+    // pair, 46 before).
     static constexpr int kOccupancy = 4;
 
     __device__ static void store(const TileTask &g, const Lane &ln, int c_local,
@@ -204,8 +204,20 @@ struct Fp64Product {
         const unsigned long long m = read_lane64(cm, c_local);
         const long long off = static_cast<long long>(read_lane64(static_cast<unsigned long long>(co), c_local));
         const int bit = ln.roles.c_bit;
-        if ((m >> bit) & 1ull)
+        if (m == ~0ull)   // a full tile, the same in every lane
+            g.c_val[off + bit] = acc.v;
+        else if ((m >> bit) & 1ull)
             g.c_val[off + __popcll(m & ((1ull << bit) - 1ull))] = acc.v;
+    }
+
+    // Lane's entry of a C tile as store() left it.
+    __device__ static double load(const TileTask &g, const Lane &ln, int c_local,
+                                  unsigned long long cm, long long co)
+    {
+        const unsigned long long m = read_lane64(cm, c_local);
+        const long long off = static_cast<long long>(read_lane64(static_cast<unsigned long long>(co), c_local));
+        const int bit = ln.roles.c_bit;
+        return (m >> bit) & 1ull ? g.c_val[off + __popcll(m & ((1ull << bit) - 1ull))] : 0.0;
     }
 
     // Lane's entry of a finished tile into a 64-slot partial (bit order).
@@ -214,72 +226,96 @@ struct Fp64Product {
         slot64[ln.roles.c_bit] = acc.v;
     }
 
-    // B entries of buffered pairs [p0, p0 + kBatch): one unconditional load
-    // each (pairs past n repeat pair n - 1; their values are not used); bit
-    // i of *has: the entry counts.
-    __device__ static void load_b(const TileTask &g, const Lane &ln, const int4 *pm, int p0, int n,
-                                  double (&bv)[kBatch], uint32_t *has)
+    // B entries of listed pairs [p0, p0 + kBatch).  A B entry is needed by two
+    // lanes, l and l ^ 8 (the two halves of the A tile's rows), so of every
+    // two pairs one half's lanes load the first and the other's the second,
+    // and the products take the partner's by a DPP move: half the loads, and
+    // twice the pairs in flight per register.
+    static __device__ __forceinline__ void load_b(const TileTask &g, const Lane &ln, const int4 *pm,
+                                                  int p0, double (&bv)[kBatch / 2])
     {
-        uint32_t h = 0;
+        const int4 *p = pm + p0 + (ln.roles.lower ? 1 : 0);
 #pragma unroll
-        for (int i = 0; i < kBatch; ++i) {
-            const int4 m = pm[min(p0 + i, n - 1)];
-            bool hi;
-            bv[i] = tile_entry_raw(g.b_vals, static_cast<uint32_t>(m.z), static_cast<uint32_t>(m.w),
-                                   ln.roles.b_phys, ln.roles.b_below, &hi);
-            h |= hi ? (1u << i) : 0u;
+        for (int i = 0; i < kBatch / 2; ++i) {
+            const int2 m = reinterpret_cast<const int2 *>(p + 2 * i)[1];
+            bv[i] = g.b_vals[entry_slot(static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y),
+                                        ln.roles.b_phys, ln.roles.b_below, g.b_zero)];
         }
-        *has = h;
     }
 
-    // Runs buffered pairs [0, n) in order; a change of C tile stores the
-    // finished one.  The B loads of the next batch are issued before the
-    // products of the current one, so one batch's loads are always in flight
-    // behind the matrix-core work.
-    __device__ static void run(const TileTask &g, const Lane &ln, const double *a_vals,
-                               const int4 *pm, const unsigned char *pc, int n, int &cur, Acc &acc,
-                               unsigned long long cm, long long co)
+    // Products of listed pairs [0, n), padded to kBatch past the end (see
+    // kPad).  The B loads of the next batch are issued before the products
+    // of the current one.  after(p0, i) runs after the product of pair p0 + i.
+    template <class After>
+    static __device__ __forceinline__ void products(const TileTask &g, const Lane &ln,
+                                                    const double *a_vals, uint32_t a_zero,
+                                                    const int4 *pm, int n, Acc &acc, After &&after)
     {
-        if (n <= 0)
-            return;
-        double bv[kBatch];
-        uint32_t bh = 0;
-        load_b(g, ln, pm, 0, n, bv, &bh);
+        double bv[kBatch / 2];
+        load_b(g, ln, pm, 0, bv);
         for (int p0 = 0; p0 < n; p0 += kBatch) {
-            double bn[kBatch];
-            uint32_t bnh = 0;
-            load_b(g, ln, pm, p0 + kBatch, n, bn, &bnh);
-            const int nbat = min(kBatch, n - p0);
+            double bn[kBatch / 2];
+            load_b(g, ln, pm, p0 + kBatch, bn);
             double av[kBatch];
-            uint32_t ah = 0;
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
-                const int4 m = pm[min(p0 + i, n - 1)];
-                bool hi;
-                av[i] = tile_entry_raw(a_vals, static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y),
-                                       ln.roles.a_phys, ln.roles.a_below, &hi);
-                ah |= hi ? (1u << i) : 0u;
+                const int2 m = reinterpret_cast<const int2 *>(pm + p0 + i)[0];
+                av[i] = a_vals[entry_slot(static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y),
+                                          ln.roles.a_phys, ln.roles.a_below, a_zero)];
             }
 #pragma unroll
-            for (int i = 0; i < kBatch; ++i) {
-                if (i < nbat) {
-                    const int t = __builtin_amdgcn_readfirstlane(pc[p0 + i]);
-                    if (t != cur) {
-                        if (cur >= 0)
-                            store(g, ln, cur, cm, co, acc);
-                        cur = t;
-                        acc.v = 0.0;
-                    }
-                    const double a = ((ah >> i) & 1u) ? av[i] : 0.0;
-                    const double b = ((bh >> i) & 1u) ? bv[i] : 0.0;
-                    acc.v = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, acc.v, 0, 0, 0);
+            for (int i = 0; i < kBatch; i += 2) {
+                const double own = bv[i / 2], other = from_lane_xor8(own);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const double b = ln.roles.lower == (u == 1) ? own : other;
+                    acc.v = __builtin_amdgcn_mfma_f64_4x4x4f64(av[i + u], b, acc.v, 0, 0, 0);
+                    after(p0, i + u);
                 }
             }
 #pragma unroll
-            for (int i = 0; i < kBatch; ++i)
+            for (int i = 0; i < kBatch / 2; ++i)
                 bv[i] = bn[i];
-            bh = bnh;
         }
+    }
+
+    // Runs a list of whole C tiles in order, storing each after its last pair.
+    // cnt: pairs of the lane's C tile; ends: bit p set when a tile ends with
+    // pair p (all of them in scalar registers, off the vector units); live:
+    // the listed tiles.  A C tile in `started` has its sum over earlier A
+    // tiles in C already.  (Products of the padding follow the last store.)
+    static __device__ __forceinline__ void run(const TileTask &g, const Lane &ln, const double *a_vals,
+                               uint32_t a_zero, const int4 *pm, int n, int,
+                               const unsigned long long (&ends)[kPairWords],
+                               unsigned long long live, unsigned long long started,
+                               unsigned long long cm, long long co)
+    {
+        Acc acc;
+        auto begin = [&]() {
+            const int t = __builtin_ctzll(live);
+            acc.v = (started >> t) & 1ull ? load(g, ln, t, cm, co) : 0.0;
+        };
+        if (started)
+            begin();
+        unsigned long long word = 0;
+        products(g, ln, a_vals, a_zero, pm, n, acc, [&](int p0, int i) {
+            if (i == 0)
+                word = (p0 < 64 ? ends[0] : (p0 < 128 ? ends[1] : ends[2])) >> (p0 & 63);
+            if ((word >> i) & 1ull) {
+                store(g, ln, __builtin_ctzll(live), cm, co, acc);
+                live &= live - 1;
+                acc.v = 0.0;
+                if (started && live)
+                    begin();
+            }
+        });
+    }
+
+    // Adds listed pairs [0, n) to acc.
+    static __device__ __forceinline__ void add(const TileTask &g, const Lane &ln, const double *a_vals,
+                               uint32_t a_zero, const int4 *pm, int n, Acc &acc)
+    {
+        products(g, ln, a_vals, a_zero, pm, n, acc, [](int, int) {});
     }
 };
 
@@ -437,9 +473,15 @@ struct SplitProduct {
         return e ? e : 0x7FF;
     }
 
+    __device__ static double entry(const double *vals, int mask, int off, int phys, uint32_t zero)
+    {
+        return vals[entry_slot(static_cast<uint32_t>(mask), static_cast<uint32_t>(off), phys,
+                               (1u << phys) - 1u, zero)];
+    }
+
     // Pairs [p0, p0 + n) of one C tile, n <= kSplitBatch, added into acc.
     __device__ static void batch(const TileTask &g, const Lane &ln, const double *a_vals,
-                                 const int4 *pm, int p0, int n, Acc &acc)
+                                 uint32_t a_zero, const int4 *pm, int p0, int n, Acc &acc)
     {
         double av[kSplitBatch], bv[kSplitBatch];
         int ea = 0, eb = 0, ea_lo = 0x7FF, eb_lo = 0x7FF;
@@ -450,10 +492,8 @@ struct SplitProduct {
             if (i < n) {
                 const int4 m = pm[p0 + i];
                 if (ln.a_live)
-                    av[i] = tile_entry(a_vals, static_cast<uint32_t>(m.x),
-                                       static_cast<uint32_t>(m.y), ln.a_phys);
-                bv[i] = tile_entry(g.b_vals, static_cast<uint32_t>(m.z),
-                                   static_cast<uint32_t>(m.w), ln.b_phys);
+                    av[i] = entry(a_vals, m.x, m.y, ln.a_phys, a_zero);
+                bv[i] = entry(g.b_vals, m.z, m.w, ln.b_phys, g.b_zero);
             }
             ea = max(ea, align_exp(av[i]));
             eb = max(eb, align_exp(bv[i]));
@@ -479,10 +519,8 @@ struct SplitProduct {
                 if (i >= n)
                     break;
                 const int4 m = pm[p0 + i];
-                const double a = tile_entry(a_vals, static_cast<uint32_t>(m.x),
-                                            static_cast<uint32_t>(m.y), ln.f64.a_phys);
-                const double b = tile_entry(g.b_vals, static_cast<uint32_t>(m.z),
-                                            static_cast<uint32_t>(m.w), ln.f64.b_phys);
+                const double a = entry(a_vals, m.x, m.y, ln.f64.a_phys, a_zero);
+                const double b = entry(g.b_vals, m.z, m.w, ln.f64.b_phys, g.b_zero);
                 acc.f64 = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, acc.f64, 0, 0, 0);
             }
             return;
@@ -562,143 +600,193 @@ struct SplitProduct {
         }
     }
 
-    __device__ static void run(const TileTask &g, const Lane &ln, const double *a_vals,
-                               const int4 *pm, const unsigned char *pc, int n, int &cur, Acc &acc,
-                               unsigned long long cm, long long co)
+    // Lane's four outputs of a C tile as store() left them.
+    __device__ static void load(const TileTask &g, const Lane &ln, int c_local,
+                                unsigned long long cm, long long co, Acc &acc)
     {
-        int p = 0;
-        while (p < n) {
-            const int t = pc[p];
-            if (t != cur) {
-                if (cur >= 0)
-                    store(g, ln, cur, cm, co, acc);
-                cur = t;
-                acc = Acc{};
-            }
-            int q = p + 1;
-            while (q < n && q - p < kSplitBatch && pc[q] == t)
-                ++q;
-            batch(g, ln, a_vals, pm, p, q - p, acc);
-            p = q;
+        const unsigned long long m = read_lane64(cm, c_local);
+        const long long off = static_cast<long long>(read_lane64(static_cast<unsigned long long>(co), c_local));
+        if (!ln.out_live)
+            return;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int bit = (ln.out_row0 + v) * 8 + ln.out_col;
+            if ((m >> bit) & 1ull)
+                acc.v[v] = g.c_val[off + __popcll(m & ((1ull << bit) - 1ull))];
         }
+    }
+
+    static __device__ __forceinline__ void run(const TileTask &g, const Lane &ln, const double *a_vals,
+                               uint32_t a_zero, const int4 *pm, int, int cnt,
+                               const unsigned long long (&)[kPairWords], unsigned long long live,
+                               unsigned long long started, unsigned long long cm, long long co)
+    {
+        for (int p = 0; live; live &= live - 1) {
+            const int t = __builtin_ctzll(live);
+            const int end = p + read_lane(cnt, t);
+            Acc acc;
+            if ((started >> t) & 1ull)
+                load(g, ln, t, cm, co, acc);
+            for (; p < end; p += kSplitBatch)
+                batch(g, ln, a_vals, a_zero, pm, p, min(kSplitBatch, end - p), acc);
+            p = end;
+            store(g, ln, t, cm, co, acc);
+        }
+    }
+
+    static __device__ __forceinline__ void add(const TileTask &g, const Lane &ln, const double *a_vals,
+                               uint32_t a_zero, const int4 *pm, int n, Acc &acc)
+    {
+        for (int p = 0; p < n; p += kSplitBatch)
+            batch(g, ln, a_vals, a_zero, pm, p, min(kSplitBatch, n - p), acc);
     }
 };
 
-// The C tiles of tile row `row` ([c0, c1)), up to 64 at a time: their B
-// column entries are matched against A row I's K list and the pairs run.
-// kStaged: A row I's keys, {mask, offset} and payload are in LDS (offsets
-// relative to the row's first value); otherwise they are read from HBM.
-template <class P, bool kStaged>
+// A wave's LDS.
+struct WaveStage {
+    double av[kAVals + 2];            // A row's payload, when it fits; then 0.0
+    int4 pm[kPairCap + kPad];         // {A mask, A offset, B mask, B offset}
+    unsigned long long word[kWave];   // per C tile: its A tiles
+    unsigned long long ends[kPairWords + 1];   // bit p: a C tile ends with pair p
+    int2 am[kWave];                   // per A tile: {mask, offset}
+    int start[kWave];                 // per A tile: its first B tile in the enumeration
+    int b0[kWave];                    // per A tile: first B tile minus start
+    int cj[kWave];                    // columns of the C tiles
+    int base[kWave];                  // per C tile: its first pair
+};
+
+// C tiles [c0, c1) of tile row `row`, up to 64 at a time, over A's tiles, up
+// to 64 at a time.  a_vals and a_sub: A's payload staged in LDS and the row's
+// first value, or A's array and 0.
+template <class P>
 __device__ __forceinline__ unsigned long long tile_row(const TileTask &g,
                                                        const typename P::Lane &ln, int64_t c0,
-                                                       int64_t c1, int a0, int na, const int *keys,
-                                                       const int2 *am, const double *avals,
-                                                       int4 *pm, unsigned char *pc, int *start,
-                                                       int *cbeg, bool heavy_on)
+                                                       int64_t c1, int a0, int na,
+                                                       const double *a_vals, uint32_t a_sub,
+                                                       uint32_t a_zero, WaveStage &s, bool heavy_on)
 {
     const int lane = lane_id();
-    const double *a_vals = (kStaged && kAVals > 0) ? avals : g.a_vals;
     unsigned long long done = 0;
     for (int64_t cc = c0; cc < c1; cc += kWave) {
         const int nc = static_cast<int>(min<int64_t>(kWave, c1 - cc));
-        // Lane c of the chunk holds C tile cc + c: mask, offset, B column run.
+        // Lane c of the chunk holds C tile cc + c: column, mask, offset.
         unsigned long long cm = 0;
         long long co = 0;
-        int nb = 0, cb = 0;
+        int cj = INT_MAX;
+        bool whole = false;   // not a heavy tile (the chunk kernels compute those)
         if (lane < nc) {
-            const int j = g.c_col[cc + lane];
-            cm = g.c_mask[cc + lane];
-            co = g.c_off[cc + lane];
-            cb = g.b_cptr[j];
-            nb = g.b_cptr[j + 1] - cb;
-            // Heavy tiles are computed by the chunk kernels instead.
             const int64_t t = cc + lane;
-            if (heavy_on && ((g.heavy[t >> 5] >> (t & 31)) & 1u))
-                nb = 0;
+            cj = g.c_col[t];
+            cm = g.c_mask[t];
+            co = g.c_off[t];
+            whole = !(heavy_on && ((g.heavy[t >> 5] >> (t & 31)) & 1u));
         }
-        const int incl = wave_inclusive_scan(nb);
-        const int total = __shfl(incl, kWave - 1, kWave);
-        start[lane] = incl - nb;
-        cbeg[lane] = cb;
-        if (lane == 0)
-            start[kWave] = total;
-        wave_sync();
-        int npairs = 0;
-        int cur = -1;
-        typename P::Acc acc;
-        const int rounds = (total + kWave - 1) / kWave;
-        for (int r0 = 0; r0 < rounds; r0 += kEnumRounds) {
-            // The K of kEnumRounds rounds of B column entries, loaded at once.
-            int key[kEnumRounds], bix[kEnumRounds], cl[kEnumRounds];
-#pragma unroll
-            for (int i = 0; i < kEnumRounds; ++i) {
-                const int q = (r0 + i) * kWave + lane;
-                key[i] = -1;
-                bix[i] = 0;
-                cl[i] = 0;
-                if (r0 + i < rounds && q < total) {
-                    const int c = upper_index(start, nc, q);
-                    cl[i] = c;
-                    bix[i] = cbeg[c] + (q - start[c]);
-                    key[i] = g.b_cent[bix[i]].x;
-                }
+        s.cj[lane] = cj;
+        unsigned long long started = 0;
+        for (int ag = 0; ag < na; ag += kWave) {
+            const int n = min(kWave, na - ag);
+            int nb = 0, b0 = 0;
+            if (lane < n) {
+                const int4 m = g.a_meta[a0 + ag + lane];
+                const int4 br = g.a_brange[a0 + ag + lane];
+                s.am[lane] = make_int2(static_cast<int>(list_mask(m.y, m.w)),
+                                       static_cast<int>((static_cast<uint32_t>(m.w) & ~kDense) - a_sub));
+                b0 = br.x;
+                nb = br.z;
             }
+            const int incl = wave_inclusive_scan(nb);
+            const int total = __shfl(incl, kWave - 1, kWave);
+            s.start[lane] = incl - nb;
+            s.b0[lane] = b0 - (incl - nb);
+            s.word[lane] = 0ull;
+            wave_sync();
+            // kEnumRounds rounds of B tiles from e0: each lane's A tile (with
+            // the C tile above it, -1 when there is none), mask and offset.
+            int key[kEnumRounds], bm[kEnumRounds], bo[kEnumRounds];
+            auto enumerate = [&](int e0) {
+                int col[kEnumRounds];
 #pragma unroll
-            for (int i = 0; i < kEnumRounds; ++i) {
-                if (r0 + i >= rounds)
-                    break;
-                int ai = -1;
-                if (key[i] >= 0) {
-                    int l = 0, h = na;
-                    while (l < h) {
-                        const int mid = (l + h) >> 1;
-                        const int k = kStaged ? keys[mid] : g.a_meta[a0 + mid].x;
-                        if (k < key[i])
-                            l = mid + 1;
-                        else
-                            h = mid;
+                for (int i = 0; i < kEnumRounds; ++i) {
+                    const int p = e0 + i * kWave + lane;
+                    key[i] = -1;
+                    if (p < total) {
+                        const int k = upper_index(s.start, n, p);
+                        const int4 m = g.b_meta[s.b0[k] + p];
+                        key[i] = k;
+                        col[i] = m.x;
+                        bm[i] = static_cast<int>(list_mask(m.y, m.w));
+                        bo[i] = static_cast<int>(static_cast<uint32_t>(m.w) & ~kDense);
                     }
-                    if (l < na && (kStaged ? keys[l] : g.a_meta[a0 + l].x) == key[i])
-                        ai = l;
                 }
-                const unsigned long long match = __ballot(ai >= 0);
-                if (ai >= 0) {
-                    int amask, aoff;
-                    if (kStaged) {
-                        const int2 m = am[ai];
-                        amask = m.x;
-                        aoff = m.y;
-                    } else {
-                        const int4 m = g.a_meta[a0 + ai];
-                        amask = m.y;
-                        aoff = m.w;
-                    }
-                    const int slot = npairs + __popcll(match & ((1ull << lane) - 1ull));
-                    pm[slot] = make_int4(amask, aoff, bix[i], 0);
-                    pc[slot] = static_cast<unsigned char>(cl[i]);
+#pragma unroll
+                for (int i = 0; i < kEnumRounds; ++i) {
+                    if (key[i] < 0)
+                        continue;
+                    int at = 0;   // the C tiles with smaller columns
+#pragma unroll
+                    for (int step = kWave / 2; step > 0; step >>= 1)
+                        at += s.cj[at + step - 1] < col[i] ? step : 0;
+                    key[i] = s.cj[at] == col[i] ? key[i] | (at << 8) : -1;
                 }
-                npairs += __popcll(match);
-                // Run the buffered pairs once another round might not fit.
-                const bool last = r0 + i + 1 >= rounds;
-                if (npairs + kWave > kPairCap || last) {
-                    wave_sync();
-                    // The matched B entries' {mask, offset}: one round of
-                    // independent loads for the whole buffer.
-                    for (int p = lane; p < npairs; p += kWave) {
-                        const int4 b = g.b_cent[pm[p].z];
-                        pm[p].z = b.y;
-                        pm[p].w = b.w;
-                    }
-                    wave_sync();
-                    P::run(g, ln, a_vals, pm, pc, npairs, cur, acc, cm, co);
-                    done += static_cast<unsigned long long>(npairs);
-                    npairs = 0;
-                    wave_sync();
-                }
+            };
+            for (int e0 = 0; e0 < total; e0 += kEnumRounds * kWave) {
+                enumerate(e0);
+#pragma unroll
+                for (int i = 0; i < kEnumRounds; ++i)
+                    if (key[i] >= 0)
+                        atomicOr(&s.word[key[i] >> 8], 1ull << (key[i] & 63));
             }
+            wave_sync();
+            const unsigned long long word = whole ? s.word[lane] : 0ull;
+            const int cnt = __popcll(word);
+            const int pi = wave_inclusive_scan(cnt);
+            const int pairs = __shfl(pi, kWave - 1, kWave);
+            s.word[lane] = word;
+            s.base[lane] = pi - cnt;
+            wave_sync();
+            for (int lo = 0; lo < pairs;) {
+                // As many whole C tiles as the buffer holds.
+                const unsigned long long fit = __ballot(pi <= lo + kPairCap);
+                const int hi = __shfl(pi, __popcll(fit) - 1, kWave);
+                const bool listed = cnt > 0 && pi > lo && pi <= hi;
+                const unsigned long long live = __ballot(listed);
+                if (lane < kPairWords)
+                    s.ends[lane] = 0ull;
+                if (lane < kPad)
+                    s.pm[hi - lo + lane] = make_int4(0, 0, 0, 0);
+                wave_sync();
+                if (listed)
+                    atomicOr(&s.ends[(pi - 1 - lo) >> 6], 1ull << ((pi - 1 - lo) & 63));
+                for (int e0 = 0; e0 < total; e0 += kEnumRounds * kWave) {
+                    if (total > kEnumRounds * kWave)
+                        enumerate(e0);   // otherwise as the first pass left it
+#pragma unroll
+                    for (int i = 0; i < kEnumRounds; ++i) {
+                        if (key[i] < 0)
+                            continue;
+                        const int c = key[i] >> 8, k = key[i] & 63;
+                        const unsigned long long w = s.word[c];
+                        const int slot =
+                            s.base[c] + __popcll(w & ((1ull << k) - 1ull)) - lo;
+                        if (((w >> k) & 1ull) && slot >= 0 && slot < hi - lo) {
+                            const int2 m = s.am[k];
+                            s.pm[slot] = make_int4(m.x, m.y, bm[i], bo[i]);
+                        }
+                    }
+                }
+                wave_sync();
+                unsigned long long ends[kPairWords];
+#pragma unroll
+                for (int i = 0; i < kPairWords; ++i)
+                    ends[i] = read_lane64(s.ends[i], 0);
+                P::run(g, ln, a_vals, a_zero, s.pm, hi - lo, cnt, ends, live, started, cm, co);
+                lo = hi;
+                wave_sync();
+            }
+            done += static_cast<unsigned long long>(pairs);
+            started |= __ballot(cnt > 0);
+            wave_sync();
         }
-        if (cur >= 0)
-            P::store(g, ln, cur, cm, co, acc);
         wave_sync();
     }
     return done;
@@ -708,73 +796,41 @@ template <class P>
 __global__ __launch_bounds__(kTThreads) __attribute__((amdgpu_waves_per_eu(P::kOccupancy)))
 void tile_numeric_kernel(TileTask g)
 {
-    __shared__ int s_keys[kTWaves][kAKeys];
-    __shared__ int2 s_am[kTWaves][kAKeys];              // {mask, offset | dense} from the row's first value
-    __shared__ double s_av[kTWaves][kAVals > 0 ? kAVals : 1];   // A row's payload
-    __shared__ int4 s_pm[kTWaves][kPairCap];            // {A mask, A offset, B mask, B offset}
-    __shared__ unsigned char s_pc[kTWaves][kPairCap];   // C tile (chunk-local) of each pair
-    __shared__ int s_start[kTWaves][kWave + 1];
-    __shared__ int s_cb[kTWaves][kWave];
+    __shared__ WaveStage s_wave[kTWaves];
     const int w = threadIdx.x / kWave;
     const int lane = lane_id();
-    int *keys = s_keys[w];
-    int2 *am = s_am[w];
-    double *av = s_av[w];
+    WaveStage &s = s_wave[w];
+    const int64_t u =
+        static_cast<int64_t>(xcd_chunk_row<kXcdChunk>(static_cast<int>(blockIdx.x),
+                                                      static_cast<int>(gridDim.x))) * kTWaves + w;
+    const int row = static_cast<int>(u / g.parts), part = static_cast<int>(u % g.parts);
+    if (row >= g.rows)
+        return;
+    const int64_t r0 = g.c_ptr[row], nt = g.c_ptr[row + 1] - r0;
+    const int64_t c0 = r0 + nt * part / g.parts, c1 = r0 + nt * (part + 1) / g.parts;
+    const int a0 = g.a_trp[row];
+    const int na = g.a_trp[row + 1] - a0;
+    const int v0 = g.a_row_off[row];
+    const int nv = g.a_row_off[row + 1] - v0;
+    // Rows below the fill threshold belong to the LDS-accumulator kernels.
+    if (c0 == c1 || static_cast<float>(nv) < g.fill * static_cast<float>(na))
+        return;
+    const bool heavy_on = g.heavy && g.tail->enabled;
     const typename P::Lane ln(lane);
     unsigned long long done = 0;   // pairs this wave multiplied
-    const bool heavy_on = g.heavy && g.tail->enabled;
-    const int home = blockIdx.x % kXcds;
-    for (int probe = 0; probe < kXcds; ++probe) {
-        const int x = (home + probe) % kXcds;
-        // Queue x hands out chunks x, x + 8, x + 16, ... of g.grab rows, so
-        // that the XCDs work through one window of consecutive rows
-        // together (faster than a contiguous eighth of the rows each).
-        for (;;) {
-            int r = 0;
-            if (lane == 0)
-                r = atomicAdd(&g.queue[x], 1);
-            const int64_t base64 =
-                (static_cast<int64_t>(read_lane(r, 0)) * kXcds + x) * g.grab;
-            if (base64 >= g.rows)
-                break;
-            const int base = static_cast<int>(base64);
-            const int rend = min(base + g.grab, g.rows);
-            for (int row = base; row < rend; ++row) {
-                const int64_t c0 = g.c_ptr[row], c1 = g.c_ptr[row + 1];
-                if (c0 == c1)
-                    continue;
-                const int a0 = g.a_trp[row];
-                const int na = g.a_trp[row + 1] - a0;
-                const int v0 = g.a_row_off[row];
-                const int nv = g.a_row_off[row + 1] - v0;
-                // Rows below the fill threshold belong to the LDS-accumulator kernels.
-                if (static_cast<float>(nv) < g.fill * static_cast<float>(na))
-                    continue;
-                if (na <= kAKeys && (kAVals == 0 || nv <= kAVals)) {
-                    // Offsets relative to the row's first value when the
-                    // payload is staged too.
-                    const uint32_t base = kAVals > 0 ? static_cast<uint32_t>(v0) : 0u;
-                    for (int i = lane; i < na; i += kWave) {
-                        const int4 m = g.a_meta[a0 + i];
-                        keys[i] = m.x;
-                        const uint32_t ow = static_cast<uint32_t>(m.w);
-                        am[i] = make_int2(m.y, static_cast<int>(((ow & ~kDense) - base) | (ow & kDense)));
-                    }
-                    if (kAVals > 0)
-                        for (int i = lane; i < nv; i += kWave)
-                            av[i] = g.a_vals[v0 + i];
-                    wave_sync();
-                    done += tile_row<P, true>(g, ln, c0, c1, a0, na, keys, am, av, s_pm[w], s_pc[w],
-                                              s_start[w], s_cb[w], heavy_on);
-                } else {
-                    done += tile_row<P, false>(g, ln, c0, c1, a0, na, keys, am, av, s_pm[w],
-                                               s_pc[w], s_start[w], s_cb[w], heavy_on);
-                }
-            }
-        }
+    if (nv <= kAVals) {
+        for (int i = lane; i < nv; i += kWave)
+            s.av[i] = g.a_vals[v0 + i];
+        if (lane == 0)
+            s.av[nv] = 0.0;
+        wave_sync();
+        done = tile_row<P>(g, ln, c0, c1, a0, na, s.av, static_cast<uint32_t>(v0),
+                           static_cast<uint32_t>(nv), s, heavy_on);
+    } else {
+        done = tile_row<P>(g, ln, c0, c1, a0, na, g.a_vals, 0u, g.a_zero, s, heavy_on);
     }
-    if (lane == 0 && done)
-        atomicAdd(g.mfma_pairs, done);
+    if (lane == 0 && done && g.mfma_pairs)
+        atomicAdd(&g.mfma_pairs[blockIdx.x % kPairShards * kShardStride], done);
 }
 
 // Chunks of a task whose merge takes `scans` steps with `matches` matched
@@ -915,7 +971,7 @@ __global__ void tail_gate_kernel(TailArgs t)
     if (st->overflow || st->count > t.capacity)
         reason = 5;
     else if (st->count == 0u)
-        reason = 4;
+        reason = kTailNone;
     else if (!t.force && static_cast<double>(st->count) / static_cast<double>(t.tiles) >
                              t.max_heavy_fraction)
         reason = 6;
@@ -983,12 +1039,10 @@ __global__ __launch_bounds__(kTThreads) void tail_chunk_base_kernel(TailArgs t)
 template <class P>
 __global__ __launch_bounds__(kTThreads) void tail_chunk_kernel(TileTask g, TailArgs t)
 {
-    __shared__ int4 s_pm[kTWaves][kPairCap];
-    __shared__ unsigned char s_pc[kTWaves][kPairCap];
+    __shared__ int4 s_pm[kTWaves][kPairCap + kPad];
     const int w = threadIdx.x / kWave;
     const int lane = lane_id();
     int4 *pm = s_pm[w];
-    unsigned char *pc = s_pc[w];
     const typename P::Lane ln(lane);
     const TailState *st = t.state;
     if (!st->enabled)
@@ -1013,7 +1067,7 @@ __global__ __launch_bounds__(kTThreads) void tail_chunk_kernel(TileTask g, TailA
         const int nb = g.b_cptr[jj + 1] - cb;
         const int e0 = cb + static_cast<int>(static_cast<long long>(nb) * j / rec.chunks);
         const int e1 = cb + static_cast<int>(static_cast<long long>(nb) * (j + 1) / rec.chunks);
-        int npairs = 0, cur = -1;
+        int npairs = 0;
         typename P::Acc acc;
         for (int p0 = e0; p0 < e1; p0 += kWave) {
             const int p = p0 + lane;
@@ -1036,13 +1090,17 @@ __global__ __launch_bounds__(kTThreads) void tail_chunk_kernel(TileTask g, TailA
             if (ai >= 0) {
                 const int4 am = g.a_meta[ai];
                 const int slot = npairs + __popcll(match & ((1ull << lane) - 1ull));
-                pm[slot] = make_int4(am.y, am.w, be.y, be.w);
-                pc[slot] = 0;
+                pm[slot] = make_int4(static_cast<int>(list_mask(am.y, am.w)),
+                                     static_cast<int>(static_cast<uint32_t>(am.w) & ~kDense),
+                                     static_cast<int>(list_mask(be.y, be.w)),
+                                     static_cast<int>(static_cast<uint32_t>(be.w) & ~kDense));
             }
             npairs += __popcll(match);
             if (npairs + kWave > kPairCap || p0 + kWave >= e1) {
+                if (lane < kPad)
+                    pm[npairs + lane] = make_int4(0, 0, 0, 0);
                 wave_sync();
-                P::run(g, ln, g.a_vals, pm, pc, npairs, cur, acc, 0ull, 0ll);
+                P::add(g, ln, g.a_vals, g.a_zero, pm, npairs, acc);
                 npairs = 0;
                 wave_sync();
             }
@@ -1095,21 +1153,54 @@ __global__ void zero_queue_kernel(int *q, int n, unsigned long long *pairs)
 
 // The call's tile statistics to the host's buffer: pairs, tail gate reason,
 // admitted records, chunks of the split tiles.
-__global__ void tile_stats_kernel(const unsigned long long *pairs, const TailState *st,
-                                  unsigned long long *host)
+__global__ __launch_bounds__(kPairShards) void tile_stats_kernel(const unsigned long long *pairs,
+                                                                 const TailState *st, int reason,
+                                                                 unsigned long long *host)
 {
-    host[0] = *pairs;
-    host[1] = st ? static_cast<unsigned long long>(st->reason) : 0ull;
+    __shared__ unsigned long long s_sum[kPairShards / kWave];
+    const unsigned long long mine = wave_sum(pairs[threadIdx.x * kShardStride]);
+    if (lane_id() == 0)
+        s_sum[threadIdx.x / kWave] = mine;
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    unsigned long long all = 0;
+    for (int i = 0; i < kPairShards / kWave; ++i)
+        all += s_sum[i];
+    host[0] = all;
+    host[1] = static_cast<unsigned long long>(st ? st->reason : reason);
     host[2] = st ? st->count : 0ull;
     host[3] = st && st->enabled ? st->chunks : 0ull;
 }
 
-// Rows a wave takes from a row queue at once: kRowGrab for the fewest queue
-// atomics, fewer when that would leave waves without rows (a wave of a
-// 2000-row product held 8 rows while seven eighths of the chip idled).
-int row_grab(int64_t rows, int64_t waves)
+// The operands, C's structure, the units of a launch and its workgroups.  A
+// product of fewer rows than the chip holds waves is cut into parts of a row.
+TileTask make_task(const DevTiles &a, const DevTiles &b, const DevC &c, float fill,
+                   double *c_values, unsigned long long *pairs, unsigned *blocks)
 {
-    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kRowGrab, rows / (2 * waves))));
+    TileTask g{};
+    g.rows = static_cast<int>(c.tilem);
+    g.a_trp = a.tile_row_ptr.as<int>();
+    g.a_meta = a.meta.as<int4>();
+    g.a_vals = a.values.as<double>();
+    g.a_brange = b.a_brange.as<int4>();
+    g.b_meta = b.records.as<int4>();
+    g.b_vals = b.payload_values();
+    g.a_zero = static_cast<uint32_t>(a.payload);
+    g.b_zero = static_cast<uint32_t>(b.payload);   // of B = A^T: A's, whose payload it is
+    g.c_ptr = c.tile_ptr.as<int64_t>();
+    g.c_col = c.tile_col.as<int>();
+    g.c_mask = c.tile_mask.as<unsigned long long>();
+    g.c_off = c.tile_nnz.as<int64_t>();
+    g.c_val = c_values;
+    g.a_row_off = a.row_payload_off.as<int>();
+    g.fill = fill;
+    g.mfma_pairs = pairs;
+    const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    const int64_t waves = cus * 16;
+    g.parts = static_cast<int>(std::min<int64_t>(kMaxParts, (waves + g.rows - 1) / g.rows));
+    *blocks = blocks_for(static_cast<int64_t>(g.rows) * g.parts, kTWaves);
+    return g;
 }
 
 } // namespace
@@ -1122,17 +1213,15 @@ TileColumns b_columns(const DevTiles &b)
         // B's column J is A's tile row J.
         v.ptr = b.transpose_of->tile_row_ptr.as<int>();
         v.ent = b.transpose_of->meta.as<int4>();
-        v.vals = b.transpose_of->values.as<double>();
     } else {
         v.ptr = b.col_ptr.as<int>();
         v.ent = b.col_ent.as<int4>();
-        v.vals = b.values.as<double>();
     }
     return v;
 }
 
 // count[0]: tile rows routed to the tile-pair kernel at `fill`; count[1]:
-// tile rows holding any tile.  A grid-stride pass of at most kCountBlocks
+// tile rows holding any tile; count[2]: most tiles in a row.  A grid-stride pass of at most kCountBlocks
 // workgroups with one atomic pair per workgroup: an atomic pair per wave on
 // the same two counters serialised at the L2 (0.3 ms for 2.6 M rows).
 constexpr int kCountThreads = 256;
@@ -1142,9 +1231,12 @@ __global__ __launch_bounds__(kCountThreads) void count_tile_rows_kernel(
     unsigned long long *__restrict__ count)
 {
     __shared__ unsigned int s_m[kCountThreads / kWave], s_n[kCountThreads / kWave];
+    __shared__ int s_l[kCountThreads / kWave];
     unsigned int m = 0, n = 0;
+    int longest = 0;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
         const int t = trp[r + 1] - trp[r];
+        longest = max(longest, t);
         n += t > 0 ? 1u : 0u;
         m += t > 0 && static_cast<float>(row_off[r + 1] - row_off[r]) >= fill * static_cast<float>(t)
                  ? 1u
@@ -1152,7 +1244,11 @@ __global__ __launch_bounds__(kCountThreads) void count_tile_rows_kernel(
     }
     m = wave_sum(m);
     n = wave_sum(n);
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1)
+        longest = max(longest, __shfl_xor(longest, o, kWave));
     if (lane_id() == 0) {
+        s_l[threadIdx.x / kWave] = longest;
         s_m[threadIdx.x / kWave] = m;
         s_n[threadIdx.x / kWave] = n;
     }
@@ -1163,9 +1259,13 @@ __global__ __launch_bounds__(kCountThreads) void count_tile_rows_kernel(
         for (int w = 0; w < kCountThreads / kWave; ++w) {
             bm += s_m[w];
             bn += s_n[w];
+            longest = max(longest, s_l[w]);
         }
         if (bm)
             atomicAdd(count, bm);
+        if (static_cast<unsigned long long>(longest) >
+            __hip_atomic_load(count + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(count + 2, static_cast<unsigned long long>(longest));
         if (bn)
             atomicAdd(count + 1, bn);
     }
@@ -1176,10 +1276,10 @@ int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, RowRouting *
     if (out->fill == fill)
         return RTT_OK;
     hipStream_t s = ctx().stream;
-    RTT_TRY(scratch->ensure(2 * sizeof(unsigned long long)));
+    RTT_TRY(scratch->ensure(3 * sizeof(unsigned long long)));
     unsigned long long *d = scratch->as<unsigned long long>();
     hipLaunchKernelGGL(zero_queue_kernel, dim3(1), dim3(4), 0, s, reinterpret_cast<int *>(d), 4,
-                       d + 1);
+                       d + 2);
     const int R = a.tile_row_count;
     if (R > 0)
         hipLaunchKernelGGL(count_tile_rows_kernel,
@@ -1187,50 +1287,40 @@ int count_tile_rows(const DevTiles &a, float fill, DevBuf *scratch, RowRouting *
                            dim3(kCountThreads), 0, s, R, a.tile_row_ptr.as<int>(),
                            a.row_payload_off.as<int>(), fill, d);
     RTT_HIP(hipGetLastError());
-    unsigned long long h[2] = {0, 0};
+    unsigned long long h[3] = {0, 0, 0};
     RTT_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
     RTT_HIP(hipStreamSynchronize(s));
+    out->longest = static_cast<int>(h[2]);
     out->tile_rows = static_cast<int64_t>(h[0]);
     out->nonempty = static_cast<int64_t>(h[1]);
     out->fill = fill;
     return RTT_OK;
 }
 
-int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const TileOpts &opt,
-                 SpgemmWork *w, hipStream_t s)
+int tile_numeric(const DevTiles &a, const DevTiles &b, const DevC &c, const TileOpts &opt,
+                 const TileColumns *tail_columns, SpgemmWork *w, hipStream_t s)
 {
     if (c.tilem == 0 || c.num_tiles == 0)
         return RTT_OK;
     const int precision = opt.precision;
     if (precision != 0 && precision != 1)
         return fail(RTT_ERR_INVALID, "unknown tile numeric precision %d", precision);
-    RTT_TRY(w->tile_queue.ensure(kXcds * sizeof(int)));
-    RTT_TRY(w->tile_pairs.ensure(sizeof(unsigned long long)));
+    constexpr int kShardWords = kPairShards * kShardStride;
+    RTT_TRY(w->tile_pairs.ensure(kShardWords * sizeof(unsigned long long)));
     RTT_TRY(w->host_tile_stats.ensure(4 * sizeof(unsigned long long)));
-    TileTask g;
-    g.rows = static_cast<int>(c.tilem);
-    g.a_trp = a.tile_row_ptr.as<int>();
-    g.a_meta = a.meta.as<int4>();
-    g.a_vals = a.values.as<double>();
-    g.b_cptr = bc.ptr;
-    g.b_cent = bc.ent;
-    g.b_vals = bc.vals;
-    g.c_ptr = c.tile_ptr.as<int64_t>();
-    g.c_col = c.tile_col.as<int>();
-    g.c_mask = c.tile_mask.as<unsigned long long>();
-    g.c_off = c.tile_nnz.as<int64_t>();
-    g.c_val = c.tile_csr_val.as<double>();
-    g.a_row_off = a.row_payload_off.as<int>();
-    g.fill = opt.fill;
-    g.queue = w->tile_queue.as<int>();
-    g.mfma_pairs = w->tile_pairs.as<unsigned long long>();
-    g.heavy = nullptr;
-    g.tail = nullptr;
-    hipLaunchKernelGGL(zero_queue_kernel, dim3(1), dim3(kXcds), 0, s, g.queue, kXcds,
-                       g.mfma_pairs);
+    unsigned blocks = 0;
+    TileTask g = make_task(a, b, c, opt.fill, c.tile_csr_val.as<double>(),
+                           w->tile_pairs.as<unsigned long long>(), &blocks);
+    w->tail_ran = tail_columns != nullptr;
+    if (tail_columns) {
+        g.b_cptr = tail_columns->ptr;
+        g.b_cent = tail_columns->ent;
+    }
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(blocks_for(2 * kShardWords, 256)), dim3(256), 0, s,
+                       w->tile_pairs.as<uint32_t>(), static_cast<int64_t>(2 * kShardWords));
     const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
     TailArgs t{};
-    if (opt.tail) {
+    if (tail_columns) {
         // Record capacity as the reference sizes it: one past the admissible
         // heavy count (floor(tiles * max_fraction)), or every tile when the
         // split is forced, and never more than tail_record_capacity
@@ -1273,18 +1363,14 @@ int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const 
         g.heavy = t.heavy;
         g.tail = t.state;
     }
-    // Persistent: enough workgroups to fill every CU several times over.
-    const int blocks = static_cast<int>(std::min<int64_t>(
-        static_cast<int64_t>(cus) * 8, (static_cast<int64_t>(g.rows) + kTWaves - 1) / kTWaves));
-    g.grab = row_grab(g.rows, static_cast<int64_t>(blocks) * kTWaves);
     if (precision == 0)
-        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(std::max(blocks, 1)),
+        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(blocks),
                            dim3(kTThreads), 0, s, g);
     else
-        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(std::max(blocks, 1)),
+        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(blocks),
                            dim3(kTThreads), 0, s, g);
     RTT_HIP(hipGetLastError());
-    if (opt.tail) {
+    if (tail_columns) {
         if (precision == 0)
             hipLaunchKernelGGL(tail_chunk_kernel<Fp64Product>, dim3(cus * 4), dim3(kTThreads), 0,
                                s, g, t);
@@ -1294,67 +1380,49 @@ int tile_numeric(const DevTiles &a, const TileColumns &bc, const DevC &c, const 
         hipLaunchKernelGGL(tail_reduce_kernel, dim3(cus * 2), dim3(kTThreads), 0, s, g, t);
         RTT_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(tile_stats_kernel, dim3(1), dim3(1), 0, s, g.mfma_pairs, g.tail,
-                       w->host_tile_stats.as<unsigned long long>());
+    // With the queue on and no tile to admit, the gate's answer is known.
+    hipLaunchKernelGGL(tile_stats_kernel, dim3(1), dim3(kPairShards), 0, s, g.mfma_pairs, g.tail,
+                       opt.tail ? kTailNone : 0, w->host_tile_stats.as<unsigned long long>());
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
 
-int tile_values_noalloc(const DevTiles &a, const TileColumns &bc, const DevC &c, int precision,
-                        void *scratch, size_t scratch_bytes, double *c_values, hipStream_t s)
+int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, int precision,
+                        double *c_values, hipStream_t s)
 {
-    // Scratch: the kXcds row-queue heads, then the pair counter.
-    const size_t need = kXcds * sizeof(int) + sizeof(unsigned long long);
-    if (need > scratch_bytes)
-        return fail(RTT_ERR_INVALID, "tile values need %zu scratch bytes, %zu available", need,
-                    scratch_bytes);
     if (c.tilem > INT_MAX)
-        return fail(RTT_ERR_INVALID, "C has %lld tile rows: beyond the row queues' range",
+        return fail(RTT_ERR_INVALID, "C has %lld tile rows: beyond the kernel's range",
                     (long long)c.tilem);
     if (precision != 0 && precision != 1)
         return fail(RTT_ERR_INVALID, "unknown tile numeric precision %d", precision);
     if (c.tilem == 0 || c.num_tiles == 0)
         return RTT_OK;
-    TileTask g;
-    g.rows = static_cast<int>(c.tilem);
-    g.a_trp = a.tile_row_ptr.as<int>();
-    g.a_meta = a.meta.as<int4>();
-    g.a_vals = a.values.as<double>();
-    g.b_cptr = bc.ptr;
-    g.b_cent = bc.ent;
-    g.b_vals = bc.vals;
-    g.c_ptr = c.tile_ptr.as<int64_t>();
-    g.c_col = c.tile_col.as<int>();
-    g.c_mask = c.tile_mask.as<unsigned long long>();
-    g.c_off = c.tile_nnz.as<int64_t>();
-    g.c_val = c_values;
-    g.a_row_off = a.row_payload_off.as<int>();
-    g.fill = 0.f;
-    g.queue = static_cast<int *>(scratch);
-    g.mfma_pairs = reinterpret_cast<unsigned long long *>(static_cast<char *>(scratch) +
-                                                          kXcds * sizeof(int));
-    g.heavy = nullptr;
-    g.tail = nullptr;
-    // Cleared by a kernel (the scratch keeps the previous call's contents).
-    hipLaunchKernelGGL(zero_queue_kernel, dim3(1), dim3(kXcds), 0, s, g.queue, kXcds,
-                       g.mfma_pairs);
-    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    const int blocks = static_cast<int>(std::min<int64_t>(
-        static_cast<int64_t>(cus) * 8, (static_cast<int64_t>(g.rows) + kTWaves - 1) / kTWaves));
-    g.grab = row_grab(g.rows, static_cast<int64_t>(blocks) * kTWaves);
+    unsigned blocks = 0;
+    const TileTask g = make_task(a, b, c, 0.f, c_values, nullptr, &blocks);
     if (precision == 0)
-        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(std::max(blocks, 1)),
+        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(blocks),
                            dim3(kTThreads), 0, s, g);
     else
-        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(std::max(blocks, 1)),
+        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(blocks),
                            dim3(kTThreads), 0, s, g);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
 
+bool tail_possible(int a_tiles, int64_t b_tiles, float threshold)
+{
+    // The admission kernel's own bound, at the longest lists.
+    const float ub = 1.0f * static_cast<float>(a_tiles + b_tiles) +
+                     8.0f * static_cast<float>(std::min<int64_t>(a_tiles, b_tiles));
+    return ub > threshold;
+}
+
 int tail_records(SpgemmWork *w, int max_records, long long *task, int *scans, int *matches,
                  int *chunks, int *count)
 {
+    *count = 0;
+    if (!w->tail_ran)
+        return RTT_OK;
     TailState st{};
     RTT_HIP(hipMemcpy(&st, w->tail_state.ptr, sizeof(st), hipMemcpyDeviceToHost));
     const int n = static_cast<int>(std::min<unsigned long long>(
