@@ -757,15 +757,14 @@ int rtt_tilespgemm(const rtt_prepared_a *a_const, const rtt_dynamic_b *b, rtt_sm
     topt.record_capacity = sc.tail_record_capacity;
     if (path != RTT_NUMERIC_TILE)
         RTT_TRY(rtt::ensure_record_values(&const_cast<rtt_dynamic_b *>(b)->tiles));
-    topt.b = &const_cast<rtt_dynamic_b *>(b)->tiles;
-    topt.b_work = &const_cast<rtt_dynamic_b *>(b)->build;
     if (path != RTT_NUMERIC_VECTOR && topt.tail) {
         if (a->routing.fill < 0.f)
             RTT_TRY(rtt::count_tile_rows(a->tiles, fill, &a->build.counters, &a->routing));
         topt.longest_a = a->routing.longest;
     }
-    RTT_TRY(rtt::spgemm_core(a->tiles, b->tiles, &a->last_c, &a->core, &a->events, &times,
-                            sc.lb_mode, path == RTT_NUMERIC_VECTOR ? nullptr : &topt));
+    rtt_dynamic_b *bm = const_cast<rtt_dynamic_b *>(b);
+    RTT_TRY(rtt::spgemm_core(a->tiles, bm->tiles, &bm->build, &a->last_c, &a->core, &a->events,
+                             &times, sc.lb_mode, path == RTT_NUMERIC_VECTOR ? nullptr : &topt));
     stats->b_columns_ms = times.b_columns_ms;
     stats->numeric_path = path;
     stats->precision = path == RTT_NUMERIC_VECTOR ? RTT_PRECISION_FP64 : sc.precision;

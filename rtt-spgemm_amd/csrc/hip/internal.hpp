@@ -162,7 +162,7 @@ struct DevC {
 // Scratch of the SpGEMM core, reused across calls.
 struct SpgemmWork {
     DevBuf row_tiles, row_nnz, row_level;   // per A tile row
-    DevBuf scan_tmp, counters, slab;
+    DevBuf scan_tmp, counters;
     DevBuf l3_rows, sym_slab_rows;          // rows past the wave and the workgroup table
     DevBuf class_rows[5];                   // rows of each numeric kernel (spgemm.hip RowClass)
     PinnedBuf host_counters;
@@ -170,11 +170,17 @@ struct SpgemmWork {
     DevBuf c_row_nnz_off;                   // per tile row, int64
     DevBuf queue;                           // work-queue heads of the slab kernels
     DevBuf row_cost, row_cost2, rows_sorted;   // slab rows, heaviest first
+    DevBuf slab_base;                       // their tasks
     DevBuf trace_start, trace_end, trace_cu;   // numeric timeline samples
+    // Slab rows: A's slot codes (once per prepared A), B's entries by scalar
+    // row (every call that has such rows) and the cursors of long rows.
+    DevBuf slot_k, slot_r, b_start, b_col, b_val, slab_cursors;
+    bool slot_codes_ready = false;
+    int64_t slab_cursor_stride = 0;
     // Slab rows' (column, mask) lists between the symbolic passes: entries
     // allocated, and the most the previous calls needed (grown at the next
     // call's start, never while a fill pass may still read the buffer).
-    DevBuf slab_stage_j, slab_stage_m, slab_row_off;
+    DevBuf slab_stage_j, slab_stage_m, slab_task_size;
     uint64_t slab_stage_cap = 0, slab_stage_need = 0;
     DevBuf tile_pairs;                      // u64: pairs the tile-pair kernel multiplied, sharded
     PinnedBuf host_tile_stats;              // u64: pairs, tail reason, records, chunks
@@ -308,9 +314,6 @@ struct TileOpts {
     float fill = 0.f;
     int precision = 0;
     int longest_a = 0;   // most A tiles in a tile row
-    // B's columns for the tail queue, built by the call that needs them.
-    DevTiles *b = nullptr;
-    BuildWork *b_work = nullptr;
     bool tail = false;
     float threshold = 16384.f, target = 8192.f;
     int max_chunks = 8;
@@ -336,9 +339,9 @@ struct CoreTimes {
 // tile == nullptr runs the LDS-accumulator kernels for every row; otherwise
 // the rows tile->fill selects have their structure written first and their
 // values computed by the tile-pair kernel, the others as before.
-int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *work,
+int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, SpgemmWork *work,
                 Events *events, CoreTimes *times, int lb_mode = RTT_LB_ADAPTIVE_TAIL,
-                TileOpts *tile = nullptr);
+                const TileOpts *tile = nullptr);
 
 // ---- scans (scan.hip) -------------------------------------------------------
 // Exclusive sum of n int64 values into out[0..n] (out[n] = total).

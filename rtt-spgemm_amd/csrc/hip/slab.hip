@@ -1,0 +1,881 @@
+// Rows beyond the LDS tables (hub rows of graphs, scattered wide rows): their
+// tiles hold one or two entries each, so they are multiplied entry by entry
+// (row-wise Gustavson on scalars) instead of tile by tile.
+//
+// A row of more work than its share is cut into tasks by columns (the hub row
+// of R-MAT 2^18 held one workgroup for 88 ms).
+//
+// Operands: every slot of A's payload gets its column and its row within the
+// tile (built once per prepared A); B's entries are laid out by scalar row,
+// columns ascending, from its tiles (rebuilt by every call that has such
+// rows).  A workgroup owns one tile row of C, or a part of it, at a time.  A thread owns one
+// slot of the row's A payload, with a cursor into the B row it selects, for
+// chunks of kSlabThreads slots.
+//
+// The row is walked in windows of C columns.  In a window, every thread
+// gallops its cursor to the window's end; the products are numbered by a
+// scan, a bit word per 64 products marks where a thread's products begin, and
+// product p of the window finds its thread with one word and one count.
+// Consecutive lanes so take consecutive entries of a B row.
+//  * symbolic: the window's C tile masks are ORed in LDS, then counted and
+//    appended to the staged lists, or written to C's structure.
+//  * numeric: the window's C tiles (masks and first values) lie in LDS
+//    directly mapped by column, and their values accumulate in LDS in C's
+//    order, to be stored once, whatever the number of A entries.
+//
+// On R-MAT 2^18 (2.9e9 products, a pair of tiles carries 1.3) the count takes
+// 8.0 ms and the numeric pass 23.8 ms, at about 4 TB/s of L2 fetches: short
+// pieces of B rows, of which the L2s reuse little.  Tile by tile, with a binary
+// search over 1280 runs and a 16-byte table entry from HBM per pair, they took
+// 35 and 108 ms, waiting on dependent loads.
+#include <algorithm>
+#include <climits>
+
+#include "core.hpp"
+
+namespace rtt {
+
+namespace {
+
+constexpr int kSlabThreads = 512;
+constexpr int kSlabWaves = kSlabThreads / kWave;
+constexpr int kSubProducts = 16384;            // products numbered by the bit words at once
+constexpr int kSubWords = kSubProducts / 64;
+constexpr int kSymWin = 8192;                  // C tile columns of a symbolic window
+constexpr int kNumCols = 2048;                 // C tile columns of a numeric window
+constexpr int kNumVals = 4096;                 // C values of a numeric window
+constexpr int kNumTiles = kNumCols / kSlabThreads;   // C tiles a thread looks at per window
+constexpr int kUnroll = 4;                     // products a thread loads together
+static_assert(kSubWords <= 4 * kWave, "one wave ranks the bit words");
+static_assert(kNumVals <= 65536 - 64, "16-bit value positions");
+
+// Column (-1: an absent slot of a dense tile) and row of every slot of A's
+// payload; a thread per tile.
+__global__ void slot_codes_kernel(int64_t n, const int4 *__restrict__ meta, int *__restrict__ k,
+                                  uint8_t *__restrict__ r)
+{
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= n)
+        return;
+    const int4 m = meta[t];
+    const uint32_t mask = static_cast<uint32_t>(m.y);
+    const uint32_t off = static_cast<uint32_t>(m.w) & 0x7FFFFFFFu;
+    const bool dense = m.w < 0;
+    for (int phys = 0, j = 0; phys < 32; ++phys) {
+        const bool has = (mask >> phys) & 1u;
+        if (!has && !dense)
+            continue;
+        k[off + j] = has ? 4 * m.x + (phys & 3) : -1;
+        r[off + j] = static_cast<uint8_t>(phys >> 2);
+        ++j;
+    }
+}
+
+// B's entries by scalar row: tile row K's entries lie in its stretch of the
+// payload, row 4K first, columns ascending; row 4K + k is start[5K + k] ..
+// start[5K + k + 1].  T threads per tile row (a wave, or a workgroup).
+template <int T>
+__global__ __launch_bounds__(256) void scalar_rows_kernel(
+    int R, const int *__restrict__ trp, const int *__restrict__ tcol,
+    const uint32_t *__restrict__ masks, const int *__restrict__ offs,
+    const double *__restrict__ vals, int *__restrict__ start, int *__restrict__ col,
+    double *__restrict__ val)
+{
+    constexpr int kRows = 256 / T;   // tile rows per workgroup
+    __shared__ unsigned long long s_sum[256 / kWave];
+    const int lt = threadIdx.x % T;
+    const int K = blockIdx.x * kRows + threadIdx.x / T;
+    const bool live = K < R;
+    const int t0 = live ? trp[K] : 0, t1 = live ? trp[K + 1] : 0;
+    // Entries per k in 16-bit fields (at most 8 per tile and k).
+    auto count = [&](uint32_t m) {
+        unsigned long long c = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            c |= static_cast<unsigned long long>(__popc(m & (0x11111111u << k))) << (16 * k);
+        return c;
+    };
+    // Sum over the row's threads of c, and before[]: the threads below.
+    auto scan = [&](unsigned long long c, unsigned long long *before) {
+        const unsigned long long incl = wave_inclusive_scan(c);
+        unsigned long long all = __shfl(incl, kWave - 1, kWave);
+        *before = incl - c;
+        if constexpr (T > kWave) {
+            const int w = threadIdx.x / kWave;
+            if (lane_id() == 0)
+                s_sum[w] = all;
+            __syncthreads();
+            all = 0;
+            for (int i = 0; i < T / kWave; ++i) {
+                *before += i < w ? s_sum[i] : 0ull;
+                all += s_sum[i];
+            }
+            __syncthreads();
+        }
+        return all;
+    };
+    int total[4] = {0, 0, 0, 0};
+    for (int t = t0; t < t1; t += T) {
+        unsigned long long before;
+        const unsigned long long all =
+            scan(t + lt < t1 ? count(masks[t + lt]) : 0ull, &before);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            total[k] += static_cast<int>(all >> (16 * k) & 0xFFFFull);
+    }
+    if (!live)
+        return;   // a whole wave or workgroup
+    int at[4];
+    int run = offs[t0];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        at[k] = run;
+        run += total[k];
+    }
+    if (lt < 5)
+        start[5 * static_cast<int64_t>(K) + lt] =
+            lt == 0 ? at[0] : (lt == 1 ? at[1] : (lt == 2 ? at[2] : (lt == 3 ? at[3] : run)));
+    for (int t = t0; t < t1; t += T) {
+        const uint32_t m = t + lt < t1 ? masks[t + lt] : 0u;
+        unsigned long long before;
+        const unsigned long long all = scan(count(m), &before);
+        if (m) {
+            const int off = offs[t + lt];
+            const bool dense = offs[t + lt + 1] - off == 32;
+            const int c0 = 8 * tcol[t + lt];
+            int j = 0;
+            for (uint32_t x = m; x; x &= x - 1, ++j) {
+                const int phys = __builtin_ctz(x), k = phys & 3;
+                const int below = __popc(m & (0x11111111u << k) & ((1u << phys) - 1u));
+                const int base = k == 0 ? at[0] : (k == 1 ? at[1] : (k == 2 ? at[2] : at[3]));
+                const int p = base + static_cast<int>(before >> (16 * k) & 0xFFFFull) + below;
+                col[p] = c0 + (phys >> 2);
+                val[p] = vals[off + (dense ? phys : j)];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            at[k] += static_cast<int>(all >> (16 * k) & 0xFFFFull);
+    }
+}
+
+struct SlabOps {
+    const int *__restrict__ a_row_off;   // A payload offset of each tile row
+    const int *__restrict__ a_k;         // per slot: column, -1 absent
+    const uint8_t *__restrict__ a_r;     // per slot: row within the tile
+    const double *__restrict__ a_vals;
+    const int *__restrict__ b_start;     // scalar_rows_kernel's layout
+    const int *__restrict__ b_col;
+    const double *__restrict__ b_val;
+    SlabTasks tasks;
+    int *__restrict__ queue;
+    int static_rows;
+    int2 *__restrict__ cursors;          // per workgroup: a run per slot of a long row
+    int64_t cursor_stride;
+};
+
+// A workgroup's task: part `part` of `parts` of a tile row, cut by columns.
+struct Task {
+    int id, row, part, parts;
+    int64_t lo, hi;   // its columns [lo, hi), multiples of 8
+};
+
+// The next task: round robin, or from the queue.  The cuts of a row in parts
+// are quantiles of the longest B row it selects: hub columns hold most of a
+// power-law row's products, and equal stretches of columns would leave most
+// of them in the first part.
+__device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_task,
+                                          unsigned long long *s_long, Task *t)
+{
+    __syncthreads();   // the previous task's readers of s_task
+    if (threadIdx.x == 0) {
+        const int i = o.static_rows
+                          ? static_cast<int>(blockIdx.x) + step * static_cast<int>(gridDim.x)
+                          : atomicAdd(o.queue, 1);
+        s_task[0] = i;
+        if (i < o.tasks.base[o.tasks.nrows]) {
+            const int r = upper_index(o.tasks.base, o.tasks.nrows, i);
+            s_task[1] = o.tasks.rows[r];
+            s_task[2] = i - o.tasks.base[r];
+            s_task[3] = o.tasks.base[r + 1] - o.tasks.base[r];
+        } else {
+            s_task[1] = -1;
+        }
+        *s_long = 0ull;
+    }
+    __syncthreads();
+    t->id = s_task[0];
+    t->row = s_task[1];
+    if (t->row < 0)
+        return false;
+    t->part = s_task[2];
+    t->parts = s_task[3];
+    t->lo = 0;
+    t->hi = INT64_MAX;
+    if (t->parts > 1) {
+        // {entries, slot from the end}: the longest, the first of equals.
+        unsigned long long best = 0;
+        const int s0 = o.a_row_off[t->row], s1 = o.a_row_off[t->row + 1];
+        for (int x = s0 + static_cast<int>(threadIdx.x); x < s1; x += kSlabThreads) {
+            const int k = o.a_k[x];
+            if (k < 0)
+                continue;
+            const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
+            best = max(best, (static_cast<unsigned long long>(p[1] - p[0]) << 32) |
+                                 static_cast<uint32_t>(s1 - x));
+        }
+#pragma unroll
+        for (int d = kWave / 2; d > 0; d >>= 1)
+            best = max(best, __shfl_xor(best, d, kWave));
+        if (lane_id() == 0)
+            atomicMax(s_long, best);
+        __syncthreads();
+        const int x = s1 - static_cast<int>(*s_long & 0xFFFFFFFFull);
+        if (*s_long != 0) {
+            const int k = o.a_k[x];
+            const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
+            const int64_t len = p[1] - p[0];
+            auto cut = [&](int q) {
+                return static_cast<int64_t>(o.b_col[p[0] + len * q / t->parts]) & ~int64_t(7);
+            };
+            if (len > 0 && t->part > 0)
+                t->lo = cut(t->part);
+            if (len > 0 && t->part + 1 < t->parts)
+                t->hi = cut(t->part + 1);
+        }
+    }
+    return true;
+}
+
+// First entry of [lo, hi) whose column is >= lim.
+__device__ __forceinline__ int first_at(const int *__restrict__ col, int lo, int hi, int64_t lim)
+{
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (col[mid] < lim)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// Entries [*lo, *hi) of the B row that slot s of A selects, within the task.
+__device__ __forceinline__ void slot_run(const SlabOps &o, const Task &t, int s, int *lo, int *hi)
+{
+    const int k = o.a_k[s];
+    *lo = *hi = 0;
+    if (k >= 0) {
+        const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
+        *lo = t.part > 0 ? first_at(o.b_col, p[0], p[1], t.lo) : p[0];
+        *hi = t.part + 1 < t.parts ? first_at(o.b_col, *lo, p[1], t.hi) : p[1];
+    }
+}
+
+// First entry at or after a, below end, whose column is >= lim: doubling
+// steps, then a binary search in the last one.
+__device__ __forceinline__ int gallop(const int *__restrict__ col, int a, int end, int64_t lim)
+{
+    int lo = a;
+    int64_t step = 1;
+    while (lo + step <= end && col[lo + step - 1] < lim) {
+        lo += static_cast<int>(step);
+        step <<= 1;
+    }
+    int hi = static_cast<int>(min<int64_t>(lo + step - 1, end));
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (col[mid] < lim)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// *at = min(*at, v) over the workgroup's threads (one LDS atomic per wave).
+__device__ __forceinline__ void lds_min(int *at, int v)
+{
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1)
+        v = min(v, __shfl_xor(v, d, kWave));
+    if (lane_id() == 0)
+        atomicMin(at, v);
+}
+
+// A window's runs in LDS: run i (one per thread with products) covers the
+// products from s_pre on, entry = pw + product.
+struct Runs {
+    int pw[kSlabThreads];
+    uint8_t r[kSlabThreads];
+    unsigned long long bits[kSubWords];   // bit p: a run begins with product p
+    int rank[kSubWords];                  // runs that begin before the word
+    int scan[2 * kSlabWaves];
+};
+
+// The products of the workgroup's threads, cnt each from entry `first` of B
+// on.  stage(i) stores the thread's operands as those of run i; load(e)
+// fetches what product needs of B's entry e, use(i, x) consumes it.  Every
+// thread calls it; it ends with a barrier.
+template <class X, class StageF, class LoadF, class UseF>
+__device__ __forceinline__ void for_products(Runs &s, int cnt, int first, int r, StageF &&stage,
+                                             LoadF &&load, UseF &&use)
+{
+    const int tid = threadIdx.x;
+    int pre, run, total, nrun;
+    dual_exclusive_scan<kSlabWaves>(cnt, cnt > 0 ? 1 : 0, s.scan, &pre, &run, &total, &nrun);
+    if (cnt > 0) {
+        s.pw[run] = first - pre;
+        s.r[run] = static_cast<uint8_t>(r);
+        stage(run);
+    }
+    for (int q0 = 0; q0 < total; q0 += kSubProducts) {
+        const int begun = q0 ? __syncthreads_count(cnt > 0 && pre < q0) : 0;
+        if (tid < kSubWords)
+            s.bits[tid] = 0ull;
+        __syncthreads();
+        if (cnt > 0 && pre >= q0 && pre < q0 + kSubProducts)
+            atomicOr(&s.bits[(pre - q0) >> 6], 1ull << ((pre - q0) & 63));
+        __syncthreads();
+        if (tid < kWave) {
+            constexpr int kPer = kSubWords / kWave;
+            int c[kPer], sum = 0;
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                c[i] = __popcll(s.bits[tid * kPer + i]);
+                sum += c[i];
+            }
+            int at = begun + wave_inclusive_scan(sum) - sum;
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                s.rank[tid * kPer + i] = at;
+                at += c[i];
+            }
+        }
+        __syncthreads();
+        const int n = min(total - q0, kSubProducts);
+        for (int p0 = tid; p0 < n; p0 += kUnroll * kSlabThreads) {
+            X x[kUnroll];
+            int id[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                const int p = p0 + u * kSlabThreads;
+                id[u] = -1;
+                if (p < n) {
+                    // The run that begins last at or before p.
+                    const unsigned long long upto = ~0ull >> (63 - (p & 63));
+                    id[u] = s.rank[p >> 6] + __popcll(s.bits[p >> 6] & upto) - 1;
+                    x[u] = load(s.pw[id[u]] + q0 + p);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+                if (id[u] >= 0)
+                    use(id[u], x[u]);
+        }
+        __syncthreads();
+    }
+    if (total == 0)
+        __syncthreads();   // the scan's buffer is reused
+}
+
+// Staged tile lists of slab rows: a task's list is a chain of segments, one
+// per window, each a header entry (j: its tiles, m: the next segment's
+// header, ~0 at the end) and its tiles in column order; a chain per task.
+// task[id] holds {first header or -1 when the task did not fit, tiles,
+// entries}.  cursor sums what every task needs, fitted or not, so that the
+// caller learns the capacity.
+struct TaskSize {
+    long long head, tiles, nnz;
+};
+struct SlabStage {
+    int *j = nullptr;
+    unsigned long long *m = nullptr;
+    TaskSize *task = nullptr;
+    unsigned long long *cursor = nullptr;
+    unsigned long long capacity = 0;
+};
+
+template <bool FILL>
+__global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps o,
+                                                                     int64_t *__restrict__ row_tiles,
+                                                                     int64_t *__restrict__ row_nnz,
+                                                                     SlabStage ss, COut c)
+{
+    __shared__ unsigned long long s_wm[kSymWin];
+    __shared__ Runs s;
+    __shared__ int s_min[2];
+    __shared__ long long s_base;
+    __shared__ int s_task[4];
+    __shared__ unsigned long long s_long;
+    const int tid = threadIdx.x;
+    constexpr int kPer = kSymWin / kSlabThreads;
+    for (int i = tid; i < kSymWin; i += kSlabThreads)
+        s_wm[i] = 0ull;
+    for (int step = 0;; ++step) {
+        Task task;
+        if (!next_task(o, step, s_task, &s_long, &task))
+            break;
+        const int row = task.row;
+        int64_t tb = 0, zb = 0;
+        if constexpr (FILL) {
+            tb = c.tile_ptr[row];
+            zb = c.row_nnz_off[row];
+            for (int q = task.id - task.part; q < task.id; ++q) {
+                tb += ss.task[q].tiles;
+                zb += ss.task[q].nnz;
+            }
+            int64_t seg = ss.task[task.id].head;
+            if (seg >= 0) {
+                while (seg >= 0) {
+                    const int n = ss.j[seg];
+                    for (int q0 = 0; q0 < n; q0 += kSlabThreads) {
+                        const int q = q0 + tid;
+                        unsigned long long m = 0;
+                        int j = 0;
+                        if (q < n) {
+                            j = ss.j[seg + 1 + q];
+                            m = ss.m[seg + 1 + q];
+                        }
+                        int npc = 0;
+                        const int zpos = block_exclusive_scan<kSlabWaves>(__popcll(m), s.scan, &npc);
+                        if (q < n)
+                            write_tile_structure(c, tb + q, j, m, zb + zpos);
+                        zb += npc;
+                    }
+                    tb += n;
+                    seg = static_cast<int64_t>(ss.m[seg]);
+                }
+                continue;
+            }
+        }
+        const int s0 = o.a_row_off[row], s1 = o.a_row_off[row + 1];
+        const bool one = s1 - s0 <= kSlabThreads;   // one chunk: cursors in registers
+        int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
+        int cur = 0, end = 0;
+        if (tid == 0)
+            s_min[0] = INT_MAX;
+        __syncthreads();
+        for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+            cur = end = 0;
+            if (c0 + tid < s1)
+                slot_run(o, task, c0 + tid, &cur, &end);
+            lds_min(&s_min[0], cur < end ? o.b_col[cur] : INT_MAX);
+            if (!one && c0 + tid < s1)
+                cursors[c0 - s0 + tid] = make_int2(cur, end);
+        }
+        __syncthreads();
+        int64_t tiles = 0, nz = 0;
+        int64_t head = -1;    // header of the task's last staged segment
+        long long first_seg = -1;   // thread 0: the first segment's
+        bool fits = ss.capacity > 0;
+        for (int w = 0;; w ^= 1) {
+            // The window starts at the lowest column left (none: done).
+            const int first = s_min[w];
+            if (first == INT_MAX)
+                break;
+            if (tid == 0)
+                s_min[w ^ 1] = INT_MAX;
+            __syncthreads();
+            const int wlo = first >> 3;
+            const int64_t lim = (static_cast<int64_t>(wlo) + kSymWin) * 8;
+            for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+                int r = 0;
+                if (!one) {
+                    cur = end = 0;
+                    if (c0 + tid < s1) {
+                        const int2 run = cursors[c0 - s0 + tid];
+                        cur = run.x;
+                        end = run.y;
+                    }
+                }
+                if (c0 + tid < s1)
+                    r = o.a_r[c0 + tid];
+                const int from = cur;
+                if (cur < end)
+                    cur = gallop(o.b_col, cur, end, lim);
+                lds_min(&s_min[w ^ 1], cur < end ? o.b_col[cur] : INT_MAX);
+                if (!one && c0 + tid < s1)
+                    cursors[c0 - s0 + tid].x = cur;
+                for_products<int>(
+                    s, cur - from, from, r, [](int) {}, [&](int e) { return o.b_col[e]; },
+                    [&](int i, int col) {
+                        const int t = (col >> 3) - wlo;
+                        const int rr = s.r[i];
+                        atomicOr(reinterpret_cast<unsigned int *>(&s_wm[t]) + (rr >> 2),
+                                 1u << ((rr & 3) * 8 + (col & 7)));
+                    });
+            }
+            // A wave's stretch of the window's masks, 64 at a time, counted
+            // and cleared.
+            unsigned long long m[kPer];
+            int nt = 0, npc = 0;
+            const int i0 = (tid / kWave) * (kPer * kWave) + lane_id();
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                m[i] = s_wm[i0 + i * kWave];
+                s_wm[i0 + i * kWave] = 0ull;
+                nt += __popcll(__ballot(m[i] != 0));
+                npc += __popcll(m[i]);
+            }
+            npc = wave_sum(npc);
+            if (lane_id() == 0) {
+                s.scan[tid / kWave] = nt;
+                s.scan[kSlabWaves + tid / kWave] = npc;
+            }
+            __syncthreads();
+            int tpos = 0, zpos = 0, all = 0, zall = 0;
+#pragma unroll
+            for (int i = 0; i < kSlabWaves; ++i) {
+                const int x = s.scan[i], y = s.scan[kSlabWaves + i];
+                tpos += i < tid / kWave ? x : 0;
+                zpos += i < tid / kWave ? y : 0;
+                all += x;
+                zall += y;
+            }
+            const unsigned long long below = (1ull << lane_id()) - 1ull;
+            if constexpr (FILL) {
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const unsigned long long has = __ballot(m[i] != 0);
+                    const int pc = __popcll(m[i]);
+                    const int incl = wave_inclusive_scan(pc);
+                    if (m[i])
+                        write_tile_structure(c, tb + tiles + tpos + __popcll(has & below),
+                                             wlo + i0 + i * kWave, m[i], zb + nz + zpos + incl - pc);
+                    tpos += __popcll(has);
+                    zpos += __shfl(incl, kWave - 1, kWave);
+                }
+            } else {
+                if (tid == 0) {
+                    long long b = -1;
+                    if (ss.cursor) {
+                        const unsigned long long need = static_cast<unsigned long long>(all) + 1;
+                        const unsigned long long at = atomicAdd(ss.cursor, need);
+                        if (at + need <= ss.capacity)
+                            b = static_cast<long long>(at);
+                    }
+                    s_base = b;
+                }
+                __syncthreads();
+                const long long b = s_base;
+                fits = fits && b >= 0;
+                if (fits) {
+                    if (tid == 0) {
+                        ss.j[b] = all;
+                        ss.m[b] = ~0ull;
+                        if (head >= 0)
+                            ss.m[head] = static_cast<unsigned long long>(b);
+                        else
+                            first_seg = b;
+                    }
+                    head = b;
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) {
+                        const unsigned long long has = __ballot(m[i] != 0);
+                        if (m[i]) {
+                            const long long at = b + 1 + tpos + __popcll(has & below);
+                            ss.j[at] = wlo + i0 + i * kWave;
+                            ss.m[at] = m[i];
+                        }
+                        tpos += __popcll(has);
+                    }
+                }
+            }
+            tiles += all;
+            nz += zall;
+            __syncthreads();   // the scan's buffer, s_base and s_min are reused
+        }
+        if constexpr (!FILL) {
+            if (tid == 0) {
+                ss.task[task.id] = TaskSize{fits && head >= 0 ? first_seg : -1ll, tiles, nz};
+                if (tiles > 0) {
+                    atomicAdd(reinterpret_cast<unsigned long long *>(row_tiles + row),
+                              static_cast<unsigned long long>(tiles));
+                    atomicAdd(reinterpret_cast<unsigned long long *>(row_nnz + row),
+                              static_cast<unsigned long long>(nz));
+                }
+            }
+        }
+    }
+}
+
+struct Product {
+    int col;
+    double val;
+};
+
+__global__ __launch_bounds__(kSlabThreads, 4) void numeric_slab_kernel(SlabOps o, COut c)
+{
+    __shared__ double s_acc[kNumVals];
+    __shared__ unsigned long long s_mask[kNumCols];   // of the window's C tiles, by column
+    __shared__ unsigned short s_at[kNumCols];         // their first values
+    __shared__ double s_a[kSlabThreads];
+    __shared__ Runs s;
+    __shared__ int s_fit[kSlabWaves], s_last[kSlabWaves], s_vals[kSlabWaves];
+    __shared__ int s_task[4];
+    __shared__ unsigned long long s_long;
+    const int tid = threadIdx.x, w = tid / kWave;
+    for (int i = tid; i < kNumVals; i += kSlabThreads)
+        s_acc[i] = 0.0;
+    for (int step = 0;; ++step) {
+        Task task;
+        if (!next_task(o, step, s_task, &s_long, &task))
+            break;
+        const int row = task.row;
+        int64_t t0 = c.tile_ptr[row];
+        int64_t nt = c.tile_ptr[row + 1] - t0;
+        if (task.parts > 1) {
+            // The part's C tiles.
+            const int *cols = c.col + t0;
+            const int n = static_cast<int>(nt);
+            const int from = task.part > 0 ? first_at(cols, 0, n, task.lo >> 3) : 0;
+            const int to = task.part + 1 < task.parts ? first_at(cols, from, n, task.hi >> 3) : n;
+            t0 += from;
+            nt = to - from;
+        }
+        const int s0 = o.a_row_off[row], s1 = o.a_row_off[row + 1];
+        const bool one = s1 - s0 <= kSlabThreads;
+        int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
+        int cur = 0, end = 0, r = 0;
+        double av = 0.0;
+        for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+            cur = end = 0;
+            if (c0 + tid < s1) {
+                slot_run(o, task, c0 + tid, &cur, &end);
+                r = o.a_r[c0 + tid];
+                av = o.a_vals[c0 + tid];
+                if (!one)
+                    cursors[c0 - s0 + tid] = make_int2(cur, end);
+            }
+        }
+        for (int64_t t_lo = 0; t_lo < nt;) {
+            // The window: as many tiles from t_lo on as the column map and
+            // the accumulator hold (at least one: a tile has at most 64
+            // values).  A thread looks at kNumTiles of the next kNumCols.
+            const int wlo = c.col[t0 + t_lo];
+            const int64_t v0 = c.tile_nnz[t0 + t_lo];
+            int fit = 0, last = 0, vals = 0;
+#pragma unroll
+            for (int i = 0; i < kNumTiles; ++i) {
+                const int64_t t = t_lo + i * kSlabThreads + tid;
+                if (t < nt) {
+                    const int j = c.col[t0 + t] - wlo;
+                    const uint64_t m = c.mask[t0 + t];
+                    const int64_t at = c.tile_nnz[t0 + t] - v0;
+                    const int64_t to = at + __popcll(m);
+                    if (j >= 0 && j < kNumCols && to <= kNumVals) {
+                        s_mask[j] = m;
+                        s_at[j] = static_cast<unsigned short>(at);
+                        ++fit;
+                        last = max(last, j);
+                        vals = max(vals, static_cast<int>(to));
+                    }
+                }
+            }
+            fit = wave_sum(fit);
+#pragma unroll
+            for (int d = kWave / 2; d > 0; d >>= 1) {
+                last = max(last, __shfl_xor(last, d, kWave));
+                vals = max(vals, __shfl_xor(vals, d, kWave));
+            }
+            if (lane_id() == 0) {
+                s_fit[w] = fit;
+                s_last[w] = last;
+                s_vals[w] = vals;
+            }
+            __syncthreads();
+            fit = last = vals = 0;
+#pragma unroll
+            for (int i = 0; i < kSlabWaves; ++i) {
+                fit += s_fit[i];
+                last = max(last, s_last[i]);
+                vals = max(vals, s_vals[i]);
+            }
+            const int64_t lim = (static_cast<int64_t>(wlo) + last + 1) * 8;
+            for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+                if (!one) {
+                    cur = end = 0;
+                    if (c0 + tid < s1) {
+                        const int2 run = cursors[c0 - s0 + tid];
+                        cur = run.x;
+                        end = run.y;
+                        r = o.a_r[c0 + tid];
+                        av = o.a_vals[c0 + tid];
+                    }
+                }
+                const int from = cur;
+                if (cur < end)
+                    cur = gallop(o.b_col, cur, end, lim);
+                if (!one && c0 + tid < s1)
+                    cursors[c0 - s0 + tid].x = cur;
+                for_products<Product>(
+                    s, cur - from, from, r, [&](int i) { s_a[i] = av; },
+                    [&](int e) { return Product{o.b_col[e], o.b_val[e]}; },
+                    [&](int i, const Product &x) {
+                        // Every product's tile lies in the window; the bounds
+                        // keep a damaged structure inside the LDS.
+                        const int j = (x.col >> 3) - wlo;
+                        if (j < 0 || j >= kNumCols)
+                            return;
+                        const int bit = s.r[i] * 8 + (x.col & 7);
+                        const int at = s_at[j] + __popcll(s_mask[j] & ((1ull << bit) - 1ull));
+                        if (at < kNumVals)
+                            atomicAdd(&s_acc[at], s_a[i] * x.val);
+                    });
+            }
+            for (int i = tid; i < vals; i += kSlabThreads) {
+                c.val[v0 + i] = s_acc[i];
+                s_acc[i] = 0.0;
+            }
+            t_lo += fit > 0 ? fit : nt;   // (a first tile always fits)
+            __syncthreads();   // the window's tables are rewritten
+        }
+    }
+}
+
+} // namespace
+
+static SlabOps slab_ops(const DevTiles &a, const SpgemmWork *w, const SlabTasks &tasks, int *queue,
+                        int static_rows)
+{
+    SlabOps o;
+    o.a_row_off = a.row_payload_off.as<int>();
+    o.a_k = w->slot_k.as<int>();
+    o.a_r = w->slot_r.as<uint8_t>();
+    o.a_vals = a.values.as<double>();
+    o.b_start = w->b_start.as<int>();
+    o.b_col = w->b_col.as<int>();
+    o.b_val = w->b_val.as<double>();
+    o.tasks = tasks;
+    o.queue = queue;
+    o.static_rows = static_rows;
+    o.cursors = w->slab_cursors.as<int2>();
+    o.cursor_stride = w->slab_cursor_stride;
+    return o;
+}
+
+// Workgroups of the slab passes: two fit a CU.
+static unsigned slab_blocks()
+{
+    return 2u * static_cast<unsigned>(ctx().num_cus > 0 ? ctx().num_cus : 256);
+}
+
+int64_t slab_target(unsigned long long pairs)
+{
+    // Sixteen tasks per workgroup on average, and at least the work that
+    // pays for a task's search of its cuts.
+    return static_cast<int64_t>(std::max<unsigned long long>(65536, pairs / (16ull * slab_blocks())));
+}
+
+// Cursors in memory for rows of more slots than a workgroup has threads.
+static int slab_cursors(SpgemmWork *w, int64_t longest)
+{
+    if (longest > kSlabThreads && longest > w->slab_cursor_stride) {
+        w->slab_cursor_stride = longest;
+        RTT_TRY(w->slab_cursors.ensure(static_cast<size_t>(slab_blocks()) *
+                                       static_cast<size_t>(longest) * sizeof(int2)));
+    }
+    return RTT_OK;
+}
+
+int slab_prepare(const DevTiles &a, DevTiles *b, BuildWork *bw, SpgemmWork *w)
+{
+    hipStream_t s = ctx().stream;
+    if (!w->slot_codes_ready) {
+        RTT_TRY(w->slot_k.ensure(static_cast<size_t>(a.payload > 0 ? a.payload : 1) * sizeof(int)));
+        RTT_TRY(w->slot_r.ensure(static_cast<size_t>(a.payload > 0 ? a.payload : 1)));
+        if (a.num_tiles > 0)
+            hipLaunchKernelGGL(slot_codes_kernel, dim3(blocks_for(a.num_tiles, 256)), dim3(256), 0,
+                               s, a.num_tiles, a.meta.as<int4>(), w->slot_k.as<int>(),
+                               w->slot_r.as<uint8_t>());
+        RTT_HIP(hipGetLastError());
+        w->slot_codes_ready = true;
+    }
+    // B = A^T at tile level has its column-ordered arrays only on request.
+    if (b->transpose_of)
+        RTT_TRY(materialize_tiles(b, bw));
+    const int R = b->tile_row_count;
+    const size_t n = static_cast<size_t>(b->payload > 0 ? b->payload : 1);
+    RTT_TRY(w->b_start.ensure((static_cast<size_t>(R) * 5 + 1) * sizeof(int)));
+    RTT_TRY(w->b_col.ensure(n * sizeof(int)));
+    RTT_TRY(w->b_val.ensure(n * sizeof(double)));
+    auto launch = [&](auto kernel, int per) {
+        hipLaunchKernelGGL(kernel, dim3(blocks_for(R, per)), dim3(256), 0, s, R,
+                           b->tile_row_ptr.as<int>(), b->tile_col_idx.as<int>(),
+                           b->masks.as<uint32_t>(), b->value_offsets.as<int>(),
+                           b->values.as<double>(), w->b_start.as<int>(), w->b_col.as<int>(),
+                           w->b_val.as<double>());
+    };
+    // A workgroup per tile row where rows average past 16 tiles (a hub row
+    // holds thousands), a wave otherwise.
+    if (R > 0 && b->num_tiles > 16 * static_cast<int64_t>(R))
+        launch(scalar_rows_kernel<256>, 1);
+    else if (R > 0)
+        launch(scalar_rows_kernel<kWave>, 256 / kWave);
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
+}
+
+static SlabStage slab_stage(const SpgemmWork *w, unsigned long long *cursor)
+{
+    SlabStage ss;
+    ss.task = w->slab_task_size.as<TaskSize>();
+    ss.cursor = cursor;
+    if (w->slab_stage_cap > 0) {
+        ss.j = w->slab_stage_j.as<int>();
+        ss.m = w->slab_stage_m.as<unsigned long long>();
+        ss.capacity = w->slab_stage_cap;
+    }
+    return ss;
+}
+
+int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
+                  int static_rows, unsigned long long *cursor, int64_t longest)
+{
+    RTT_TRY(slab_cursors(w, longest));
+    // Staging of the rows' tile lists: grown to what the previous calls
+    // needed, within a quarter of the free device memory; without it every
+    // row is recomputed by the fill pass.
+    if (w->slab_stage_need > w->slab_stage_cap) {
+        size_t free_b = 0, total_b = 0;
+        const uint64_t per = sizeof(int) + sizeof(unsigned long long);
+        uint64_t want = w->slab_stage_need + w->slab_stage_need / 16;
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
+            want = std::min<uint64_t>(want, free_b / 4 / per);
+        w->slab_stage_cap = 0;
+        if (want > 0 && w->slab_stage_j.ensure(want * sizeof(int)) == RTT_OK &&
+            w->slab_stage_m.ensure(want * sizeof(unsigned long long)) == RTT_OK)
+            w->slab_stage_cap = want;
+        clear_error();
+    }
+    RTT_TRY(w->slab_task_size.ensure(static_cast<size_t>(tasks.most) * sizeof(TaskSize)));
+    hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(slab_blocks()), dim3(kSlabThreads),
+                       0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows),
+                       w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(), slab_stage(w, cursor),
+                       COut{});
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
+}
+
+int slab_structure(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
+                   int static_rows, const COut &c)
+{
+    hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(slab_blocks()), dim3(kSlabThreads),
+                       0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows), nullptr,
+                       nullptr, slab_stage(w, nullptr), c);
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
+}
+
+int slab_numeric(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
+                 int static_rows, const COut &c, int64_t longest)
+{
+    RTT_TRY(slab_cursors(w, longest));
+    hipLaunchKernelGGL(numeric_slab_kernel, dim3(slab_blocks()), dim3(kSlabThreads), 0,
+                       ctx().stream, slab_ops(a, w, tasks, queue, static_rows), c);
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
+}
+
+} // namespace rtt

@@ -17,7 +17,7 @@
 //  * symbolic: the 8x8 masks of the row's C tiles are ORed into an LDS hash
 //    table, compacted, ranked by tile column and staged; after the size scan
 //    a light pass writes the final structure.  Rows whose tile set outgrows
-//    the table use a direct-mapped mask slab in HBM instead.
+//    the table go to the slab kernels (slab.hip).
 //  * numeric: the row's C layout (tile columns, masks, value offsets) and
 //    its A payload (column-major per tile) are loaded into LDS.  Each thread
 //    takes a pair, loads its 80-byte B record (packed meta + the first eight
@@ -34,8 +34,7 @@
 
 #include <hipcub/hipcub.hpp>
 
-#include "device.hpp"
-#include "internal.hpp"
+#include "core.hpp"
 
 namespace rtt {
 
@@ -117,6 +116,26 @@ constexpr uint32_t kDenseBit = 0x80000000u;
 // table; kLevelSlab: it outgrew that too.
 enum RowLevel : int { kLevelEmpty = 0, kLevelLds = 1, kLevelLarge = 2, kLevelSlab = 3 };
 
+// The numeric kernel that takes a row of the LDS level, by its sizes: the
+// smallest instance that holds it, the slab kernel when none does.
+enum RowClass : int { kRowTiny, kRowSmall, kRowMid, kRowLarge, kRowSlab, kRowClasses };
+
+// Counters the host reads back after the symbolic pass, and the state of the
+// kernels that fill them (zeroed with them).
+enum Counter : int {
+    kCtrPairs,       // (A tile, B tile) pairs
+    kCtrTiles,       // C tiles
+    kCtrNnz,         // nnz(C)
+    kCtrOutgrown,    // rows that outgrew the wave table
+    kCtrSymSlab,     // rows that outgrew the workgroup table too
+    kCtrSlabTiles,   // slab tiles the staging cursor handed out
+    kCtrLongest,     // most A payload slots in a slab row
+    kCtrRows,        // rows of each RowClass, kRowClasses of them
+    kCtrTicket = kCtrRows + kRowClasses,
+    kCtrDone,
+    kCounters
+};
+
 struct Operands {
     int a_tile_rows;
     const int *__restrict__ a_trp;
@@ -143,17 +162,6 @@ __device__ __forceinline__ bool tile_routed(float fill, int tiles, int payload)
 {
     return tiles > 0 && static_cast<float>(payload) >= fill * static_cast<float>(tiles);
 }
-
-struct COut {
-    const int64_t *__restrict__ tile_ptr;     // tilem + 1
-    const int64_t *__restrict__ row_nnz_off;  // tilem + 1
-    int *__restrict__ col;
-    uint64_t *__restrict__ mask;
-    int64_t *__restrict__ tile_nnz;
-    uint8_t *__restrict__ csr_ptr;
-    uint8_t *__restrict__ csr_col;
-    double *__restrict__ val;
-};
 
 struct Stage {
     int *__restrict__ j;
@@ -188,82 +196,6 @@ __device__ __forceinline__ int product_count(uint32_t a_bytes, uint32_t b_bytes)
     for (int k = 0; k < 4; ++k)
         n += __popc(byte_of(a_bytes, k)) * __popc(byte_of(b_bytes, k));
     return n;
-}
-
-// Byte r of the result is the number of set bits in bytes 0..r-1 of m (the
-// u8 row offsets of a C tile): per-byte popcounts, then an exclusive byte
-// prefix sum by multiplication (sums stay below 256, so no byte carries).
-__device__ __forceinline__ uint64_t packed_row_offsets(uint64_t m)
-{
-    uint64_t x = m - ((m >> 1) & 0x5555555555555555ull);
-    x = (x & 0x3333333333333333ull) + ((x >> 2) & 0x3333333333333333ull);
-    x = (x + (x >> 4)) & 0x0F0F0F0F0F0F0F0Full;
-    return (x * 0x0101010101010101ull) << 8;
-}
-
-__device__ __forceinline__ void write_tile_structure(const COut &c, int64_t t, int j,
-                                                     uint64_t m, int64_t off)
-{
-    c.col[t] = j;
-    c.mask[t] = m;
-    c.tile_nnz[t] = off;
-    reinterpret_cast<uint64_t *>(c.csr_ptr)[t] = packed_row_offsets(m);
-    int i = 0;
-    while (m) {
-        const int pos = __builtin_ctzll(m);
-        m &= m - 1;
-        c.csr_col[off + i++] = static_cast<uint8_t>(pos & 7);
-    }
-}
-
-// Exclusive scans of two values over a workgroup of NW waves with one
-// barrier; s2 (2 * NW ints) must not be reused without a barrier between.
-template <int NW = kWavesPerBlock>
-__device__ __forceinline__ void dual_exclusive_scan(int a, int b, int *s2, int *pa, int *pb,
-                                                    int *ta, int *tb)
-{
-    const int w = threadIdx.x / kWave;
-    const int ia = wave_inclusive_scan(a);
-    const int ib = wave_inclusive_scan(b);
-    if (lane_id() == kWave - 1) {
-        s2[w] = ia;
-        s2[NW + w] = ib;
-    }
-    __syncthreads();
-    int ba = 0, bb = 0, sa = 0, sb = 0;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-        const int x = s2[i], y = s2[NW + i];
-        ba += i < w ? x : 0;
-        bb += i < w ? y : 0;
-        sa += x;
-        sb += y;
-    }
-    *pa = ba + ia - a;
-    *pb = bb + ib - b;
-    *ta = sa;
-    *tb = sb;
-}
-
-// Exclusive scan over a workgroup of NW waves; *total receives the sum.
-template <int NW = kWavesPerBlock>
-__device__ __forceinline__ int block_exclusive_scan(int v, int *s_tmp, int *total)
-{
-    const int w = threadIdx.x / kWave;
-    const int incl = wave_inclusive_scan(v);
-    if (lane_id() == kWave - 1)
-        s_tmp[w] = incl;
-    __syncthreads();
-    int before = 0, all = 0;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-        const int t = s_tmp[i];
-        before += i < w ? t : 0;
-        all += t;
-    }
-    __syncthreads();
-    *total = all;
-    return before + incl - v;
 }
 
 template <typename T>
@@ -473,7 +405,7 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
 __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
     Operands g, int stage_limit, Stage st, const int *__restrict__ rows,
     int64_t *__restrict__ row_tiles, int64_t *__restrict__ row_nnz, int *__restrict__ row_level,
-    int *__restrict__ slab_rows, unsigned long long *__restrict__ n_slab)
+    int *__restrict__ slab_rows, unsigned long long *__restrict__ ctr)
 {
     __shared__ __align__(16) int s_key[kSymSlots];
     __shared__ unsigned long long s_msk[kSymSlots];
@@ -507,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
                 s_spread[k][tid] = rows_to_bytes(byte_of(ab, k));
         }
         int total = 0;
-        const int pre = block_exclusive_scan(nb, s_tmp, &total);
+        const int pre = block_exclusive_scan<kWavesPerBlock>(nb, s_tmp, &total);
         if (tid < n)
             s_pre[tid] = pre;
         for (int r0 = 0; r0 < total; r0 += kSeg) {
@@ -587,13 +519,15 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
         mine += rk[i] != kEmpty ? 1 : 0;
     }
     int nt = 0;
-    int pos = block_exclusive_scan(mine, s_tmp, &nt);
+    int pos = block_exclusive_scan<kWavesPerBlock>(mine, s_tmp, &nt);
     if (s_ovf || nt > stage_limit) {
         if (tid == 0) {
             row_level[row] = kLevelSlab;
             row_tiles[row] = 0;
             row_nnz[row] = 0;
-            slab_rows[atomicAdd(n_slab, 1ull)] = row;
+            slab_rows[atomicAdd(&ctr[kCtrSymSlab], 1ull)] = row;
+            atomicMax(&ctr[kCtrLongest],
+                      static_cast<unsigned long long>(g.a_row_off[row + 1] - g.a_row_off[row]));
         }
         return;
     }
@@ -759,20 +693,6 @@ __global__ __launch_bounds__(kThreads) void symbolic_write_kernel(
     }
 }
 
-// Work queue of the slab kernels: the workgroup's next position in the row
-// list, taken by one lane with a global atomic and shared through LDS.  The
-// head only grows, so every workgroup leaves once it passes the list's end.
-// The row bodies end with a barrier, so the slot is not rewritten while a
-// lane still reads it.
-__device__ __forceinline__ int next_row(int *queue)
-{
-    __shared__ int s_next;
-    if (threadIdx.x == 0)
-        s_next = atomicAdd(queue, 1);
-    __syncthreads();
-    return s_next;
-}
-
 // Cost of each listed row: the (A tile, B tile) pairs it visits.  One wave
 // per row.
 __global__ __launch_bounds__(kThreads) void row_pairs_kernel(const int *__restrict__ rows, int n,
@@ -790,277 +710,6 @@ __global__ __launch_bounds__(kThreads) void row_pairs_kernel(const int *__restri
     sum = wave_sum(sum);
     if (lane_id() == 0)
         cost[i] = static_cast<unsigned int>(sum < 0xffffffffull ? sum : 0xffffffffull);
-}
-
-// Rows whose tile set outgrows the LDS table: one workgroup per row, one
-// 64-bit mask per C tile column in an HBM slab, read back in column order.
-__device__ __forceinline__ unsigned long long load_coherent(const unsigned long long *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The slab kernels walk a row in windows: each A tile keeps a cursor into
-// every class run of its B row, each run sorted by column.
-constexpr int kSlabRuns = 5;       // class runs of a B row: heavy, light k = 0..3
-constexpr int kSlabWinTiles = 4096;  // A tiles up to which a slab row is walked in windows
-static_assert(kSlabRuns + 1 <= kClassSlots, "the runs' ends come from the class slots");
-constexpr int kSymWin = 2048;      // B tile columns a symbolic slab window covers
-
-// First index after a, within [a, end), whose B tile column is >= j, given
-// that a's column is below j (end when none): doubling steps from a, then a
-// binary search in the last step.
-__device__ __forceinline__ int gallop_col(const int4 *__restrict__ meta, int a, int end, int j)
-{
-    int step = 1;
-    while (a + step < end && meta[a + step].x < j) {
-        a += step;
-        step <<= 1;
-    }
-    int lo = a + 1, hi = min(a + step, end);
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (meta[mid].x < j)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
-// The count pass leaves each row's (column, mask) list, in column order, in
-// a grow-only staging buffer when it fits (row_off[row] = its first entry,
-// -1 otherwise); the fill pass then copies the list instead of repeating
-// the row's atomics.  cursor sums every row's tile count, fitted or not, so
-// that the caller learns the capacity the next call needs.
-struct SlabStage {
-    int *j = nullptr;
-    unsigned long long *m = nullptr;
-    int64_t *row_off = nullptr;
-    unsigned long long *cursor = nullptr;
-    unsigned long long capacity = 0;
-};
-
-template <bool FILL>
-__global__ __launch_bounds__(kThreads) void symbolic_slab_kernel(
-    Operands g, const int *__restrict__ rows, int nrows, int *__restrict__ queue,
-    int static_rows, unsigned long long *__restrict__ slabs, int64_t *__restrict__ row_tiles,
-    int64_t *__restrict__ row_nnz, SlabStage ss, COut c)
-{
-    __shared__ uint32_t s_ab[kThreads];
-    __shared__ int s_tmp[kWavesPerBlock];
-    __shared__ int s_lo, s_hi, s_min;
-    __shared__ long long s_base;
-    __shared__ unsigned long long s_wm[kSymWin];   // a window's masks
-    __shared__ int s_wpw[kSlabRuns * kThreads];    // per (tile, run): first B tile minus first pair
-    __shared__ int s_wpre[kSlabRuns * kThreads];   // per (tile, run): first pair
-    unsigned long long *slab = slabs + static_cast<int64_t>(blockIdx.x) * g.b_tile_cols;
-    const int tid = threadIdx.x;
-    for (int i = tid; i < kSymWin; i += kThreads)
-        s_wm[i] = 0;
-    for (int step = 0;; ++step) {
-        const int ri = static_rows ? static_cast<int>(blockIdx.x) + step * static_cast<int>(gridDim.x)
-                                   : next_row(queue);
-        if (ri >= nrows)
-            break;
-        const int row = rows[ri];
-        if constexpr (FILL) {
-            const int64_t base = ss.row_off ? ss.row_off[row] : -1;
-            if (base >= 0) {
-                // Staged: the structure in column order, value offsets by a scan.
-                const int64_t tb = c.tile_ptr[row];
-                const int nt = static_cast<int>(c.tile_ptr[row + 1] - tb);
-                int64_t zb = c.row_nnz_off[row];
-                for (int q0 = 0; q0 < nt; q0 += kThreads) {
-                    const int q = q0 + tid;
-                    unsigned long long m = 0;
-                    int j = 0;
-                    if (q < nt) {
-                        j = ss.j[base + q];
-                        m = ss.m[base + q];
-                    }
-                    int npc = 0;
-                    const int zpos = block_exclusive_scan(__popcll(m), s_tmp, &npc);
-                    if (q < nt)
-                        write_tile_structure(c, tb + q, j, m, zb + zpos);
-                    zb += npc;
-                }
-                __syncthreads();
-                continue;
-            }
-        }
-        const int a0 = g.a_trp[row], a1 = g.a_trp[row + 1];
-        if (tid == 0) {
-            s_lo = INT_MAX;
-            s_hi = -1;
-            s_min = INT_MAX;
-        }
-        __syncthreads();
-        // The column range the row's masks land in, from the pairs
-        // themselves (the tiles of a B row are not in column order).
-        int jlo = INT_MAX, jhi = -1;
-        // Each chunk's A tiles walk their B runs in windows of kSymWin
-        // columns, starting each window at the lowest column a cursor holds
-        // (so a chunk visits only windows it has pairs in).  A window's masks
-        // are ORed in LDS, then its nonzero masks into the HBM table at
-        // consecutive addresses.
-        for (int c0 = a0; c0 < a1; c0 += kThreads) {
-            const int n = min(kThreads, a1 - c0);
-            int cur[kSlabRuns], end[kSlabRuns];
-#pragma unroll
-            for (int r = 0; r < kSlabRuns; ++r)
-                cur[r] = end[r] = 0;
-            if (tid < n) {
-                const int4 am = g.a_meta[c0 + tid];
-                const uint32_t ab = static_cast<uint32_t>(am.z);
-                s_ab[tid] = ab;
-                const int *gp = g.b_groups + static_cast<int64_t>(kClassSlots) * am.x;
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r) {
-                    // Light run k meets only A tiles with entries in column k.
-                    if (r == 0 || byte_of(ab, r - 1) != 0) {
-                        cur[r] = gp[r];
-                        end[r] = gp[r + 1];
-                    }
-                }
-            }
-            for (;;) {
-                int mn = INT_MAX;
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r)
-                    if (cur[r] < end[r])
-                        mn = min(mn, g.b_meta[cur[r]].x);
-                if (mn != INT_MAX)
-                    atomicMin(&s_min, mn);
-                __syncthreads();
-                const int wlo = s_min;
-                if (wlo == INT_MAX)
-                    break;
-                const int whi = wlo + kSymWin;
-                int cnt[kSlabRuns], lo[kSlabRuns];
-                int mine = 0;
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r) {
-                    lo[r] = cur[r];
-                    cnt[r] = 0;
-                    if (cur[r] < end[r] && g.b_meta[cur[r]].x < whi) {
-                        const int h = gallop_col(g.b_meta, cur[r], end[r], whi);
-                        cnt[r] = h - cur[r];
-                        cur[r] = h;
-                    }
-                    mine += cnt[r];
-                }
-                int total = 0;
-                int pre = block_exclusive_scan(mine, s_tmp, &total);
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r) {
-                    s_wpre[kSlabRuns * tid + r] = pre;
-                    s_wpw[kSlabRuns * tid + r] = lo[r] - pre;
-                    pre += cnt[r];
-                }
-                if (tid == 0)
-                    s_min = INT_MAX;   // every thread read it before the scan's barriers
-                __syncthreads();
-                for (int p = tid; p < total; p += kThreads) {
-                    const int e = upper_index(s_wpre, kSlabRuns * n, p);
-                    const int4 bm = g.b_meta[s_wpw[e] + p];
-                    const uint64_t pm = bytes_product(s_ab[e / kSlabRuns], static_cast<uint32_t>(bm.z));
-                    if (pm && bm.x >= wlo && bm.x < whi)
-                        atomicOr(&s_wm[bm.x - wlo], static_cast<unsigned long long>(pm));
-                }
-                __syncthreads();
-                for (int i = tid; i < kSymWin; i += kThreads) {
-                    const unsigned long long m = s_wm[i];
-                    if (m) {
-                        s_wm[i] = 0;
-                        atomicOr(&slab[wlo + i], m);
-                        jlo = min(jlo, wlo + i);
-                        jhi = max(jhi, wlo + i);
-                    }
-                }
-                __syncthreads();
-            }
-            // Every thread has read the final (empty) window start before the
-            // next chunk lowers it again.
-            __syncthreads();
-        }
-        if (jhi >= 0) {
-            atomicMin(&s_lo, jlo);
-            atomicMax(&s_hi, jhi);
-        }
-        __threadfence();
-        __syncthreads();
-        const int lo = s_lo, hi = s_hi;
-        if constexpr (!FILL) {
-            // Sizes first, without consuming the masks.
-            int64_t tiles = 0, nz = 0;
-            for (int j0 = lo; j0 <= hi; j0 += kThreads) {
-                const int j = j0 + tid;
-                const unsigned long long m = j <= hi ? load_coherent(&slab[j]) : 0ull;
-                int ntile = 0, npc = 0;
-                block_exclusive_scan(m ? 1 : 0, s_tmp, &ntile);
-                block_exclusive_scan(__popcll(m), s_tmp, &npc);
-                tiles += ntile;
-                nz += npc;
-            }
-            if (tid == 0) {
-                long long b = -1;
-                if (ss.cursor && tiles > 0) {
-                    const unsigned long long at =
-                        atomicAdd(ss.cursor, static_cast<unsigned long long>(tiles));
-                    if (at + static_cast<unsigned long long>(tiles) <= ss.capacity)
-                        b = static_cast<long long>(at);
-                }
-                s_base = b;
-                row_tiles[row] = tiles;
-                row_nnz[row] = nz;
-                if (ss.row_off)
-                    ss.row_off[row] = b;
-            }
-            __syncthreads();
-            // Then the list, staged when it fits, and the slab cleared.
-            const long long base = s_base;
-            int64_t done = 0;
-            for (int j0 = lo; j0 <= hi; j0 += kThreads) {
-                const int j = j0 + tid;
-                unsigned long long m = 0;
-                if (j <= hi) {
-                    m = load_coherent(&slab[j]);
-                    if (m)
-                        slab[j] = 0;
-                }
-                int ntile = 0;
-                const int tpos = block_exclusive_scan(m ? 1 : 0, s_tmp, &ntile);
-                if (base >= 0 && m) {
-                    ss.j[base + done + tpos] = j;
-                    ss.m[base + done + tpos] = m;
-                }
-                done += ntile;
-            }
-        } else {
-            // Not staged: the masks again, written straight to C's structure.
-            int64_t tiles = 0, nz = 0;
-            const int64_t tb = c.tile_ptr[row];
-            const int64_t zb = c.row_nnz_off[row];
-            for (int j0 = lo; j0 <= hi; j0 += kThreads) {
-                const int j = j0 + tid;
-                unsigned long long m = 0;
-                if (j <= hi) {
-                    m = load_coherent(&slab[j]);
-                    if (m)
-                        slab[j] = 0;
-                }
-                int ntile = 0, npc = 0;
-                const int tpos = block_exclusive_scan(m ? 1 : 0, s_tmp, &ntile);
-                const int zpos = block_exclusive_scan(__popcll(m), s_tmp, &npc);
-                if (m)
-                    write_tile_structure(c, tb + tiles + tpos, j, m, zb + nz + zpos);
-                tiles += ntile;
-                nz += npc;
-            }
-        }
-        __threadfence();
-        __syncthreads();
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1510,330 +1159,6 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
         trace_mark(tl, true);
 }
 
-// ---------------------------------------------------------------------------
-// Numeric for rows beyond the LDS budgets, one workgroup per row at a time.
-// A direct-mapped HBM table, one int4 per B tile column {row, first value of
-// the C tile within the row, mask low word, mask high word}, gives a pair its
-// C tile in one load.  A's values are staged per chunk of A tiles in LDS
-// when they fit; B's come from the record planes.
-//
-// Each chunk of A tiles walks the row in windows of consecutive C tiles
-// that start within kSlabWinStep values of each other (at most kSlabWin
-// values).  A window's products accumulate in LDS.  Each A tile keeps a
-// cursor into every class run of its B row (each run is sorted by column)
-// and gallops it to the window's last column, about one load per run and
-// window.  A row of one chunk then stores each window to C with plain
-// coalesced stores (no clearing pass, no HBM atomics); a row of up to
-// kSlabWinTiles A tiles clears its C values first and each chunk adds its
-// windows' nonzero sums with FP64 atomics on consecutive addresses.  Longer
-// rows (hub rows, whose chunks would each walk every window) clear C and
-// add every product with an FP64 atomic in HBM.
-// ---------------------------------------------------------------------------
-constexpr int kSlabStage = 1024;   // A values a slab chunk stages in LDS
-constexpr int kSlabWin = 2048;     // C values a slab window accumulates in LDS
-constexpr int kSlabWinStep = kSlabWin - 64;   // tile starts per window; a tile holds <= 64
-
-// First tile in [lo, hi] of a row whose first value is at or after v (hi
-// when none); nnz holds the row's tile starts (hi + 1 entries from the row's
-// first tile, the last one the row's end).
-__device__ __forceinline__ int first_tile_from(const int64_t *__restrict__ nnz, int lo, int hi,
-                                               int64_t v)
-{
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (nnz[mid] < v)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
-// The products of one pair (A tile at, B record b with meta) into the C tile
-// whose values start at acc and whose mask is cm: into an LDS window (WIN)
-// or with FP64 atomics on C's values in HBM.
-template <bool WIN>
-__device__ __forceinline__ void slab_products(const int4 *__restrict__ recs, int64_t rec_n,
-                                              const double *__restrict__ b_vals_km, int64_t b,
-                                              int4 meta, int4 at, const double *abase,
-                                              uint64_t cm, double *acc)
-{
-    // Only the parts that hold the tile's values: most tiles of the rows that
-    // come here have one or two entries.
-    const int nbv = __popc(static_cast<uint32_t>(meta.z));
-    double rv[kRecVals];
-#pragma unroll
-    for (int i = 0; i < kRecVals / 2; ++i) {
-        double2 d = make_double2(0.0, 0.0);
-        if (2 * i < nbv)
-            d = reinterpret_cast<const double2 *>(recs + (i + 1) * rec_n)[b];
-        rv[2 * i] = d.x;
-        rv[2 * i + 1] = d.y;
-    }
-    const uint32_t ab = static_cast<uint32_t>(at.x);
-    const double *acol = abase + at.z;
-    const uint32_t apf = static_cast<uint32_t>(at.y);
-    const uint32_t boff = static_cast<uint32_t>(meta.w) & ~kDenseBit;
-    auto entry = [&](int pos, double vb) {
-        const int k = pos >> 3, cl = pos & 7;
-        const double *ap = acol + byte_of(apf, k);
-        uint32_t rr = byte_of(ab, k);
-        int i = 0;
-        while (rr) {
-            const int r = __builtin_ctz(rr);
-            rr &= rr - 1;
-            double *dst = &acc[__popcll(cm & ((1ull << (r * 8 + cl)) - 1ull))];
-            if constexpr (WIN)
-                atomicAdd(dst, ap[i++] * vb);
-            else
-                unsafeAtomicAdd(dst, ap[i++] * vb);
-        }
-    };
-    uint32_t mz = static_cast<uint32_t>(meta.z);
-#pragma unroll
-    for (int j = 0; j < kRecVals; ++j) {
-        if (mz) {
-            const int pos = __builtin_ctz(mz);
-            mz &= mz - 1;
-            entry(pos, rv[j]);
-        }
-    }
-    int j = kRecVals;
-    while (mz) {
-        const int pos = __builtin_ctz(mz);
-        mz &= mz - 1;
-        entry(pos, b_vals_km[boff + j]);
-        ++j;
-    }
-}
-
-// Per-chunk A tile info: {rows of column k (byte k), first value of column k
-// (byte k), first value relative to the chunk's, unused}.
-__device__ __forceinline__ int4 slab_a_tile(int4 am, int v0)
-{
-    const uint32_t ab = static_cast<uint32_t>(am.z);
-    const uint32_t p1 = __popc(byte_of(ab, 0));
-    const uint32_t p2 = p1 + __popc(byte_of(ab, 1));
-    const uint32_t p3 = p2 + __popc(byte_of(ab, 2));
-    return make_int4(static_cast<int>(ab), static_cast<int>((p1 << 8) | (p2 << 16) | (p3 << 24)),
-                     static_cast<int>(static_cast<uint32_t>(am.w) & ~kDenseBit) - v0, 0);
-}
-
-__global__ __launch_bounds__(kThreads) void numeric_slab_kernel(
-    Operands g, const int4 *__restrict__ recs, int64_t rec_n, const int *__restrict__ rows,
-    int nrows, int *__restrict__ queue, int static_rows, int4 *__restrict__ slabs, COut c)
-{
-    __shared__ double s_win[kSlabWin];
-    __shared__ double s_acol[kSlabStage + 8];
-    __shared__ int4 s_at[kThreads];
-    __shared__ int s_pw[kSlabRuns * kThreads];    // per (tile, run): first B tile minus first pair
-    __shared__ int s_pre[kSlabRuns * kThreads];   // per (tile, run): first pair
-    __shared__ int s_tmp[kWavesPerBlock];
-    int4 *slab = slabs + static_cast<int64_t>(blockIdx.x) * g.b_tile_cols;
-    const int tid = threadIdx.x;
-    for (int i = tid; i < kSlabWin; i += kThreads)
-        s_win[i] = 0.0;
-    for (int step = 0;; ++step) {
-        const int ri = static_rows ? static_cast<int>(blockIdx.x) + step * static_cast<int>(gridDim.x)
-                                   : next_row(queue);
-        if (ri >= nrows)
-            break;
-        const int row = rows[ri];
-        const int64_t t0 = c.tile_ptr[row];
-        const int nt = static_cast<int>(c.tile_ptr[row + 1] - t0);
-        const int64_t zb = c.row_nnz_off[row];
-        const int64_t nnz_row = c.row_nnz_off[row + 1] - zb;
-        const int a0 = g.a_trp[row], a1 = g.a_trp[row + 1];
-        // A row of one chunk stores its windows; a row of a few chunks clears
-        // C first and each chunk adds its windows' sums; a longer row, where
-        // chunks times windows would outweigh its pairs, adds every product.
-        const bool single = a1 - a0 <= kThreads;
-        const bool windowed = a1 - a0 <= kSlabWinTiles;
-        // Columns are checked against the table's extent, so that a damaged
-        // structure cannot send a store outside it.
-        for (int q = tid; q < nt; q += kThreads) {
-            const int j = c.col[t0 + q];
-            const uint64_t m = c.mask[t0 + q];
-            if (j >= 0 && j < g.b_tile_cols)
-                slab[j] = make_int4(row, static_cast<int>(c.tile_nnz[t0 + q] - zb),
-                                    static_cast<int>(static_cast<uint32_t>(m)),
-                                    static_cast<int>(static_cast<uint32_t>(m >> 32)));
-        }
-        if (!single)
-            for (int64_t i = tid; i < nnz_row; i += kThreads)
-                c.val[zb + i] = 0.0;
-        __threadfence();
-        __syncthreads();
-        double *cval = c.val + zb;
-        const int64_t *tnz = c.tile_nnz + t0;
-        for (int c0 = a0; windowed && c0 < a1; c0 += kThreads) {
-            // The chunk's A tiles, their staged values and their run cursors
-            // stay put for every window of the row.
-            const int n = min(kThreads, a1 - c0);
-            const int v0 = g.a_off[c0];
-            const int span = g.a_off[c0 + n] - v0;
-            const bool staged = span <= kSlabStage;
-            int cur[kSlabRuns], end[kSlabRuns];
-#pragma unroll
-            for (int r = 0; r < kSlabRuns; ++r)
-                cur[r] = end[r] = 0;
-            if (tid < n) {
-                const int4 am = g.a_meta[c0 + tid];
-                s_at[tid] = slab_a_tile(am, v0);
-                const uint32_t ab = static_cast<uint32_t>(am.z);
-                const int *gp = g.b_groups + static_cast<int64_t>(kClassSlots) * am.x;
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r) {
-                    // Light run k meets only A tiles with entries in column k.
-                    if (r == 0 || byte_of(ab, r - 1) != 0) {
-                        cur[r] = gp[r];
-                        end[r] = gp[r + 1];
-                    }
-                }
-            }
-            if (staged)
-                for (int i = tid; i < span; i += kThreads)
-                    s_acol[i] = g.a_vals_cm[v0 + i];
-            const double *abase = staged ? s_acol : g.a_vals_cm + v0;
-            // Every thread finds the same window bounds, so they need no exchange.
-            int t_lo = 0;
-            for (int64_t wend = kSlabWinStep; t_lo < nt; wend += kSlabWinStep) {
-                const int t_hi = first_tile_from(tnz, t_lo, nt, zb + wend);
-                if (t_hi == t_lo)
-                    continue;
-                const int vb = static_cast<int>(tnz[t_lo] - zb);
-                const int vs = static_cast<int>(tnz[t_hi] - zb) - vb;
-                const int jhi = c.col[t0 + t_hi - 1] + 1;
-                // B tiles before the window's first column that a cursor still
-                // covers are not C tiles of the row: they meet nothing.
-                int cnt[kSlabRuns], lo[kSlabRuns];
-                int mine = 0;
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r) {
-                    lo[r] = cur[r];
-                    cnt[r] = 0;
-                    if (cur[r] < end[r] && g.b_meta[cur[r]].x < jhi) {
-                        const int h = gallop_col(g.b_meta, cur[r], end[r], jhi);
-                        cnt[r] = h - cur[r];
-                        cur[r] = h;
-                    }
-                    mine += cnt[r];
-                }
-                int total = 0;
-                int pre = block_exclusive_scan(mine, s_tmp, &total);
-#pragma unroll
-                for (int r = 0; r < kSlabRuns; ++r) {
-                    s_pre[kSlabRuns * tid + r] = pre;
-                    s_pw[kSlabRuns * tid + r] = lo[r] - pre;
-                    pre += cnt[r];
-                }
-                __syncthreads();
-                // A window with no pairs in a longer row's chunk adds nothing.
-                if (total == 0 && !single) {
-                    t_lo = t_hi;
-                    continue;
-                }
-                for (int p = tid; p < total; p += kThreads) {
-                    const int e = upper_index(s_pre, kSlabRuns * n, p);
-                    const int4 at = s_at[e / kSlabRuns];
-                    const int64_t b = s_pw[e] + p;
-                    const int4 meta = recs[b];
-                    if (!product_count(static_cast<uint32_t>(at.x), static_cast<uint32_t>(meta.z)))
-                        continue;
-                    if (meta.x < 0 || meta.x >= g.b_tile_cols)
-                        continue;
-                    const int4 sl = slab[meta.x];
-                    if (sl.x != row || static_cast<unsigned>(sl.y - vb) >= static_cast<unsigned>(vs))
-                        continue;
-                    const uint64_t cm = (static_cast<uint64_t>(static_cast<uint32_t>(sl.w)) << 32) |
-                                        static_cast<uint32_t>(sl.z);
-                    slab_products<true>(recs, rec_n, g.b_vals_km, b, meta, at, abase, cm,
-                                        s_win + (sl.y - vb));
-                }
-                __syncthreads();
-                // The window's values, and the accumulator cleared for the next
-                // window by the thread that read it.  A single-chunk row
-                // stores every value (zeros included); a longer row adds the
-                // nonzero sums, consecutive addresses per wave.
-                for (int i = tid; i < vs; i += kThreads) {
-                    const double v = s_win[i];
-                    s_win[i] = 0.0;
-                    if (single)
-                        cval[vb + i] = v;
-                    else if (v != 0.0)
-                        unsafeAtomicAdd(&cval[vb + i], v);
-                }
-                __syncthreads();
-                t_lo = t_hi;
-            }
-        }
-        for (int c0 = a0; !windowed && c0 < a1; c0 += kThreads) {
-            const int n = min(kThreads, a1 - c0);
-            const int v0 = g.a_off[c0];
-            const int span = g.a_off[c0 + n] - v0;
-            const bool staged = span <= kSlabStage;
-            int nb = 0, bstart = 0;
-            if (tid < n) {
-                s_at[tid] = slab_a_tile(g.a_meta[c0 + tid], v0);
-                const int4 br = g.a_brange[c0 + tid];
-                nb = br.z;
-                bstart = br.x;
-            }
-            if (staged)
-                for (int i = tid; i < span; i += kThreads)
-                    s_acol[i] = g.a_vals_cm[v0 + i];
-            const double *abase = staged ? s_acol : g.a_vals_cm + v0;
-            int total = 0;
-            const int pre = block_exclusive_scan(nb, s_tmp, &total);
-            s_pw[tid] = bstart - pre;
-            s_pre[tid] = pre;
-            __syncthreads();
-            // A pair finds its A tile by a binary search over the chunk's
-            // first pairs: a tile whose B row is a hub column would make one
-            // thread fill most of a segment table.
-            for (int p = tid; p < total; p += kThreads) {
-                const int v = upper_index(s_pre, n, p);
-                const int4 at = s_at[v];
-                const int64_t b = s_pw[v] + p;
-                const int4 meta = recs[b];
-                if (!product_count(static_cast<uint32_t>(at.x), static_cast<uint32_t>(meta.z)))
-                    continue;
-                if (meta.x < 0 || meta.x >= g.b_tile_cols)
-                    continue;
-                const int4 sl = slab[meta.x];
-                if (sl.x != row)
-                    continue;
-                const uint64_t cm = (static_cast<uint64_t>(static_cast<uint32_t>(sl.w)) << 32) |
-                                    static_cast<uint32_t>(sl.z);
-                slab_products<false>(recs, rec_n, g.b_vals_km, b, meta, at, abase, cm,
-                                     cval + sl.y);
-            }
-            __syncthreads();
-        }
-        __threadfence();
-        __syncthreads();
-    }
-}
-
-// The numeric kernel that takes a row of the LDS level, by its sizes: the
-// smallest instance that holds it, the slab kernel when none does.
-enum RowClass : int { kRowTiny, kRowSmall, kRowMid, kRowLarge, kRowSlab, kRowClasses };
-
-// Counters the host reads back after the symbolic pass, and the state of the
-// kernels that fill them (zeroed with them).
-enum Counter : int {
-    kCtrPairs,       // (A tile, B tile) pairs
-    kCtrTiles,       // C tiles
-    kCtrNnz,         // nnz(C)
-    kCtrOutgrown,    // rows that outgrew the wave table
-    kCtrSymSlab,     // rows that outgrew the workgroup table too
-    kCtrSlabTiles,   // slab tiles the staging cursor handed out
-    kCtrRows,        // rows of each RowClass, kRowClasses of them
-    kCtrTicket = kCtrRows + kRowClasses,
-    kCtrDone,
-    kCounters
-};
-
 struct RowLists {
     int *__restrict__ rows[kRowClasses];
     int *__restrict__ outgrown;
@@ -1887,6 +1212,8 @@ __global__ __launch_bounds__(kThreads) void row_sizes_kernel(
                   : fits_row<MediumRow>(t, z, alen) ? kRowMid
                   : fits_row<LargeRow>(t, z, alen)  ? kRowLarge
                                                     : kRowSlab;
+            if (cls == kRowSlab)
+                atomicMax(&ctr[kCtrLongest], static_cast<unsigned long long>(alen));
         }
     }
     const unsigned long long ix = wave_inclusive_scan(nt), iy = wave_inclusive_scan(nz);
@@ -2063,51 +1390,61 @@ static int write_timeline(const char *path, const Timeline &tl, size_t slots, ui
     return RTT_OK;
 }
 
-// Copies a slab row list into w->rows_sorted, heaviest row (most pairs)
-// first, so that the work queue hands out the long rows before the short
-// ones.  Stream-ordered: the previous user of rows_sorted has been queued.
-static int order_rows_by_cost(const int *rows, int n, const Operands &g, SpgemmWork *w, hipStream_t s,
-                       const int **sorted)
+__global__ void slab_parts_kernel(int n, const unsigned int *__restrict__ cost, unsigned int target,
+                                  int *__restrict__ parts)
 {
-    RTT_TRY(w->row_cost.ensure(static_cast<size_t>(n) * sizeof(unsigned int)));
-    RTT_TRY(w->row_cost2.ensure(static_cast<size_t>(n) * sizeof(unsigned int)));
-    RTT_TRY(w->rows_sorted.ensure(static_cast<size_t>(n) * sizeof(int)));
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        parts[i] = 1 + static_cast<int>(min(cost[i] / target, static_cast<unsigned int>(kSlabParts - 1)));
+    else if (i == n)
+        parts[i] = 0;
+}
+
+// The tasks of a slab row list: its rows heaviest first (most pairs) with
+// `sorted`, so that the work queue hands out the long rows before the short
+// ones, and the tasks of every row.  Stream-ordered: the previous user of
+// the arrays has been queued.
+static int plan_slab_tasks(const int *rows, int n, bool sorted, unsigned long long pairs,
+                           const Operands &g, SpgemmWork *w, hipStream_t s, SlabTasks *out)
+{
+    const size_t bytes_n = (static_cast<size_t>(n) + 1) * sizeof(unsigned int);
+    RTT_TRY(w->row_cost.ensure(bytes_n));
+    RTT_TRY(w->row_cost2.ensure(bytes_n));
+    RTT_TRY(w->rows_sorted.ensure(bytes_n));
+    RTT_TRY(w->slab_base.ensure(bytes_n));
     unsigned int *cost = w->row_cost.as<unsigned int>();
     unsigned int *cost2 = w->row_cost2.as<unsigned int>();
-    int *out = w->rows_sorted.as<int>();
     hipLaunchKernelGGL(row_pairs_kernel, dim3(blocks_for(n, kWavesPerBlock)), dim3(kThreads), 0,
                        s, rows, n, g.a_trp, g.a_brange, cost);
     RTT_HIP(hipGetLastError());
     size_t bytes = 0;
-    RTT_HIP(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, bytes, cost, cost2, rows, out,
-                                                         n, 0, 32, s));
+    if (sorted) {
+        int *to = w->rows_sorted.as<int>();
+        RTT_HIP(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, bytes, cost, cost2, rows, to,
+                                                             n, 0, 32, s));
+        RTT_TRY(w->scan_tmp.ensure(bytes));
+        RTT_HIP(hipcub::DeviceRadixSort::SortPairsDescending(w->scan_tmp.ptr, bytes, cost, cost2,
+                                                             rows, to, n, 0, 32, s));
+        rows = to;
+        std::swap(cost, cost2);
+    }
+    const int64_t target = slab_target(pairs);
+    int *parts = reinterpret_cast<int *>(cost2), *base = w->slab_base.as<int>();
+    hipLaunchKernelGGL(slab_parts_kernel, dim3(blocks_for(n + 1, kThreads)), dim3(kThreads), 0, s,
+                       n, cost, static_cast<unsigned int>(std::min<int64_t>(target, UINT_MAX)),
+                       parts);
+    RTT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, parts, base, n + 1, s));
     RTT_TRY(w->scan_tmp.ensure(bytes));
-    RTT_HIP(hipcub::DeviceRadixSort::SortPairsDescending(w->scan_tmp.ptr, bytes, cost, cost2,
-                                                         rows, out, n, 0, 32, s));
-    *sorted = out;
+    RTT_HIP(hipcub::DeviceScan::ExclusiveSum(w->scan_tmp.ptr, bytes, parts, base, n + 1, s));
+    out->rows = rows;
+    out->base = base;
+    out->nrows = n;
+    out->most = n + static_cast<int64_t>(pairs / static_cast<unsigned long long>(target));
     return RTT_OK;
 }
 
-// Workgroups of a slab pass whose per-workgroup HBM table holds `cols`
-// entries of `entry` bytes: up to four per CU, fewer when the tables would
-// pass a quarter of the free device memory (plus what `table` already holds).
-// The passes take rows from a work queue (or round robin over the grid), so
-// any number of workgroups covers every row; one table that does not fit
-// fails the allocation with RTT_ERR_OOM.
-static int slab_grid(int rows, int num_cus, int64_t cols, size_t entry, const DevBuf &table)
-{
-    int blocks = std::max(1, std::min(rows, 4 * num_cus));
-    size_t free_b = 0, total_b = 0;
-    if (cols > 0 && hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
-        const uint64_t per = static_cast<uint64_t>(cols) * entry;
-        const uint64_t budget = free_b / 4 + table.bytes;
-        blocks = static_cast<int>(std::max<uint64_t>(1, std::min<uint64_t>(blocks, budget / per)));
-    }
-    return blocks;
-}
-
-int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Events *ev,
-                CoreTimes *times, int lb_mode, TileOpts *tile)
+int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, SpgemmWork *w,
+                Events *ev, CoreTimes *times, int lb_mode, const TileOpts *tile)
 {
     // tile: rows routed to the tile-pair kernel (all when fill is 0);
     // vector: rows left to the LDS-accumulator kernels.
@@ -2189,7 +1526,7 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     if (tail && b.transpose_of)
         tail = tail_possible(tile->longest_a, tile->longest_a, tile->threshold);
     if (count_columns)
-        RTT_TRY(longest_b_column(b, &tile->b_work->keys_in,
+        RTT_TRY(longest_b_column(b, &b_work->keys_in,
                                  w->host_counters.as<unsigned long long>() + kCounters));
     // One wave per row first; rows that outgrow its table go to the
     // workgroup table, and rows that outgrow that to the slab.
@@ -2201,7 +1538,6 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[1], s));
     int n_slab = 0;
-    COut none{};
     // Sizes of C from the per-row counts, the numeric routing lists and
     // every counter, in one launch and one wait.  Rows of the tile-pair
     // kernel are not listed.
@@ -2231,54 +1567,21 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
         hipLaunchKernelGGL(symbolic_count_kernel, dim3(n_large), dim3(kThreads), 0, s, g,
                            stage_limit, st, w->l3_rows.as<int>(), w->row_tiles.as<int64_t>(),
                            w->row_nnz.as<int64_t>(), w->row_level.as<int>(),
-                           w->sym_slab_rows.as<int>(), ctr + kCtrSymSlab);
+                           w->sym_slab_rows.as<int>(), ctr);
         RTT_HIP(hipGetLastError());
         RTT_HIP(hipEventRecord(ev->ev[1], s));
         RTT_TRY(finish_sizes(false));
         n_slab = static_cast<int>(hctr[kCtrSymSlab]);
     }
-    int slab_blocks = 0;
-    const int *slab_rows = nullptr;
     const int static_rows = lb_mode == RTT_LB_STATIC ? 1 : 0;
-    SlabStage ss;
+    const bool by_cost = lb_mode == RTT_LB_ADAPTIVE_TAIL;
+    SlabTasks tasks;
     if (n_slab > 0) {
-        // Staging of the slab rows' tile lists: grown to what the previous
-        // calls needed, within a quarter of the free device memory; without
-        // it every slab row is recomputed by the fill pass.
-        if (w->slab_stage_need > w->slab_stage_cap) {
-            size_t free_b = 0, total_b = 0;
-            const uint64_t per = sizeof(int) + sizeof(unsigned long long);
-            uint64_t want = w->slab_stage_need + w->slab_stage_need / 16;
-            if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
-                want = std::min<uint64_t>(want, free_b / 4 / per);
-            w->slab_stage_cap = 0;
-            if (want > 0 && w->slab_stage_j.ensure(want * sizeof(int)) == RTT_OK &&
-                w->slab_stage_m.ensure(want * sizeof(unsigned long long)) == RTT_OK)
-                w->slab_stage_cap = want;
-            clear_error();
-        }
-        RTT_TRY(w->slab_row_off.ensure(static_cast<size_t>(R) * sizeof(int64_t)));
-        ss.row_off = w->slab_row_off.as<int64_t>();
-        ss.cursor = ctr + kCtrSlabTiles;
-        if (w->slab_stage_cap > 0) {
-            ss.j = w->slab_stage_j.as<int>();
-            ss.m = w->slab_stage_m.as<unsigned long long>();
-            ss.capacity = w->slab_stage_cap;
-        }
-        slab_blocks = slab_grid(n_slab, num_cus, BC, sizeof(uint64_t), w->slab);
-        slab_rows = w->sym_slab_rows.as<int>();
-        if (lb_mode == RTT_LB_ADAPTIVE_TAIL)
-            RTT_TRY(order_rows_by_cost(slab_rows, n_slab, g, w, s, &slab_rows));
-        RTT_TRY(w->slab.ensure(static_cast<size_t>(slab_blocks) * BC * sizeof(uint64_t)));
-        hipLaunchKernelGGL(fill_u64_kernel,
-                           dim3(blocks_for(static_cast<int64_t>(slab_blocks) * BC, kThreads)),
-                           dim3(kThreads), 0, s, w->slab.as<unsigned long long>(),
-                           static_cast<int64_t>(slab_blocks) * BC);
-        hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(slab_blocks), dim3(kThreads), 0, s,
-                           g, slab_rows, n_slab, queue, static_rows,
-                           w->slab.as<unsigned long long>(), w->row_tiles.as<int64_t>(),
-                           w->row_nnz.as<int64_t>(), ss, none);
-        RTT_HIP(hipGetLastError());
+        RTT_TRY(slab_prepare(a, &b, b_work, w));
+        RTT_TRY(plan_slab_tasks(w->sym_slab_rows.as<int>(), n_slab, by_cost, hctr[kCtrPairs], g, w,
+                                s, &tasks));
+        RTT_TRY(slab_symbolic(a, w, tasks, queue, static_rows, ctr + kCtrSlabTiles,
+                              static_cast<int64_t>(hctr[kCtrLongest])));
         clear_sizes();
         RTT_TRY(finish_sizes(true));
     }
@@ -2333,9 +1636,7 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[3], s));
     if (n_slab > 0)
-        hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(slab_blocks), dim3(kThreads), 0, s,
-                           g, slab_rows, n_slab, queue + 1, static_rows,
-                           w->slab.as<unsigned long long>(), nullptr, nullptr, ss, co);
+        RTT_TRY(slab_structure(a, w, tasks, queue + 1, static_rows, co));
     if (!ended)
         hipLaunchKernelGGL(set_last_kernel, dim3(1), dim3(1), 0, s,
                            c->tile_nnz.as<int64_t>() + c->num_tiles,
@@ -2349,10 +1650,10 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     TileColumns columns;
     if (tail) {
         auto tc = Clock::now();
-        RTT_TRY(build_b_columns(tile->b, tile->b_work));
+        RTT_TRY(build_b_columns(&b, b_work));
         RTT_HIP(hipStreamSynchronize(s));
         times->b_columns_ms = ms_since(tc);
-        columns = b_columns(*tile->b);
+        columns = b_columns(b);
     }
     Timeline tl;
     size_t trace_slots = 0;
@@ -2411,20 +1712,12 @@ int spgemm_core(const DevTiles &a, const DevTiles &b, DevC *c, SpgemmWork *w, Ev
     rows_launch(numeric_row_kernel<MediumRow>, kRowMid, MediumRow::kThreads, false);
     rows_launch(numeric_row_kernel<LargeRow>, kRowLarge, LargeRow::kThreads, false);
     if (n_num_slab > 0) {
-        DevBuf &tab = w->slab;   // reused: the symbolic slab pass has been queued before
-        const int blocks = slab_grid(n_num_slab, num_cus, BC, sizeof(int4), tab);
-        const int64_t ents = static_cast<int64_t>(blocks) * BC;
-        RTT_TRY(tab.ensure(static_cast<size_t>(ents) * sizeof(int4)));
-        hipLaunchKernelGGL(fill_i32_kernel, dim3(blocks_for(4 * ents, kThreads)), dim3(kThreads), 0,
-                           s, tab.as<int>(), 4 * ents, -1);
-        // The symbolic fill pass above is queued before this sort reuses rows_sorted.
-        const int *num_rows = lists.rows[kRowSlab];
-        if (lb_mode == RTT_LB_ADAPTIVE_TAIL)
-            RTT_TRY(order_rows_by_cost(num_rows, n_num_slab, g, w, s, &num_rows));
-        hipLaunchKernelGGL(numeric_slab_kernel, dim3(blocks), dim3(kThreads), 0, s, g,
-                           b.records.as<int4>(), b.num_tiles, num_rows, n_num_slab, queue + 2,
-                           static_rows, tab.as<int4>(), co);
-        RTT_HIP(hipGetLastError());
+        if (n_slab == 0)
+            RTT_TRY(slab_prepare(a, &b, b_work, w));
+        // The structure pass above is queued before this plan reuses its arrays.
+        RTT_TRY(plan_slab_tasks(lists.rows[kRowSlab], n_num_slab, by_cost, pairs, g, w, s, &tasks));
+        RTT_TRY(slab_numeric(a, w, tasks, queue + 2, static_rows, co,
+                             static_cast<int64_t>(hctr[kCtrLongest])));
     }
     RTT_HIP(hipStreamSynchronize(s));
     if (any_tile && c->num_tiles > 0) {

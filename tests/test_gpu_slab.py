@@ -1,0 +1,113 @@
+"""Rows beyond the LDS tables at the edges of their passes: A rows around one
+and two chunks of 512 slots, C rows around a numeric window (4096 values, 2048
+tile columns) and a symbolic one (8192 tile columns), windows with more than
+16384 products, gaps of many windows between columns, dense A tiles (absent
+slots), empty B rows, and B = A^T.  The first call of a handle recomputes the
+structure, the later ones copy the staged lists: both against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_parity import as_tuple, check_c, csr_from
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_matrix(m, n, per, seed, cols=None):
+    rng = np.random.default_rng(seed)
+    pool = np.arange(n) if cols is None else cols
+    r = np.repeat(np.arange(m), per)
+    c = np.concatenate([np.sort(rng.choice(pool, p, replace=False)) for p in per])
+    return csr_from(m, n, r, c, rng.uniform(-1, 1, len(r)))
+
+
+def check(gpu, a, b, lb_mode="adaptive-tail", heavy=True):
+    pa = gpu.prepare_identity_a(a)
+    src = gpu.upload_csr(b)
+    ref = oracle.spgemm(as_tuple(a), as_tuple(b))
+    pb = None
+    for _ in range(2):
+        pb = gpu.rebuild_b_general(pa, src, pb)
+        tc, st = gpu.tilespgemm(pa, pb, gpu.schedule(numeric_path="vector", lb_mode=lb_mode))
+        check_c(gpu, tc, ref)
+        assert (st["heavy_rows"] > 0) == heavy
+
+
+@pytest.mark.parametrize("slots", [63, 64, 65, 128, 129, 257])
+@pytest.mark.parametrize("lb_mode", ["static", "dynamic", "adaptive-tail"])
+def test_chunks_of_slots(gpu, slots, lb_mode):
+    """8 * slots slots in one tile row: one, exactly one, and more chunks."""
+    a = rows_matrix(24, 900, np.r_[np.full(8, slots), np.full(8, 1), np.full(8, slots - 1)], slots)
+    b = gpu.gen_random(900, 40000, 25, 2)
+    check(gpu, a, b, lb_mode)
+
+
+@pytest.mark.parametrize("n", [8 * 2047, 8 * 2048, 8 * 2048 + 1, 8 * 8192, 8 * 8192 + 9, 8 * 30000])
+def test_windows(gpu, n):
+    a = rows_matrix(16, 400, np.full(16, 40), 7)
+    b = gpu.gen_random(400, n, min(60, n // 8), 8)
+    check(gpu, a, b)
+
+
+def test_full_tiles_fill_the_accumulator(gpu):
+    """Columns dense enough that a window ends by its values, not its columns."""
+    a = rows_matrix(16, 300, np.full(16, 60), 3)
+    b = gpu.gen_random(300, 12000, 900, 4)
+    check(gpu, a, b)
+
+
+def test_many_products_in_a_window(gpu):
+    a = rows_matrix(8, 700, np.full(8, 600), 5)
+    b = gpu.gen_random(700, 5000, 300, 6)
+    check(gpu, a, b)
+
+
+@pytest.mark.parametrize("lb_mode", ["static", "dynamic", "adaptive-tail"])
+def test_rows_cut_into_tasks(gpu, lb_mode):
+    """Rows of more than 65536 pairs, cut at columns of their longest B row,
+    beside rows of one task; B's columns skewed so that cuts coincide."""
+    rng = np.random.default_rng(21)
+    per_b = np.where(np.arange(900) % 10 == 0, 1500, 300)
+    pool = np.unique((30000 * rng.random(20000) ** 4).astype(np.int64))
+    b = rows_matrix(900, 30000, np.minimum(per_b, len(pool)), 22, pool)
+    a = rows_matrix(40, 900, np.where(np.arange(40) % 16 < 8, 700, 30), 23)
+    check(gpu, a, b, lb_mode)
+
+
+def test_gaps_and_empty_rows(gpu):
+    """B's columns in two clusters far apart; half of its rows empty."""
+    rng = np.random.default_rng(9)
+    pool = np.r_[np.arange(5000), np.arange(3_000_000, 3_005_000)]
+    per = np.where(np.arange(500) % 2 == 0, 0, 50)
+    b = rows_matrix(500, 3_100_000, per, 10, pool)
+    a = rows_matrix(24, 500, np.where(np.arange(24) % 3 == 0, 90, 3), 11)
+    check(gpu, a, b)
+
+
+@pytest.mark.parametrize("aat", [0, 1])
+def test_dense_a_tiles_and_transpose(gpu, aat):
+    """Dense A tiles (absent slots stored as zeros) on slab rows, squared and
+    times the transpose."""
+    rng = np.random.default_rng(12)
+    n = 7000
+    rows, cols = [], []
+    for i in range(n):
+        c = rng.choice(n, 3, replace=False)
+        if i < 16:
+            keep = rng.random(200) < 0.95
+            c = np.r_[c, np.arange(400, 600)[keep], rng.choice(n, 500, replace=False)]
+        c = np.unique(c)
+        rows.append(np.full(len(c), i))
+        cols.append(c)
+    rows, cols = np.concatenate(rows), np.concatenate(cols)
+    a = csr_from(n, n, rows, cols, rng.uniform(-1, 1, len(rows)))
+    pa = gpu.prepare_identity_a(a)
+    assert pa.tiles()["dense_tiles"] > 0
+    bt = gpu.csr_transpose(a) if aat else a
+    ref = oracle.spgemm(as_tuple(a), as_tuple(bt))
+    pb = None
+    for _ in range(2):
+        pb = gpu.rebuild_b(pa, aat, pb)
+        tc, st = gpu.tilespgemm(pa, pb, gpu.schedule(numeric_path="vector"))
+        check_c(gpu, tc, ref)
+    assert st["heavy_rows"] > 0
