@@ -8,7 +8,7 @@
 // (src/gpu_dmma_tiles.h:313-560).
 //
 // One launch counts, scans and fills.  A workgroup stages the columns of its
-// 256 rows in LDS, counts its tile rows' tiles, gets the totals of the
+// 512 rows in LDS, counts its tile rows' tiles, gets the totals of the
 // workgroups before it by a decoupled look-back, and fills its part of the
 // arrays.  The host does not know the totals beforehand: a workgroup whose
 // part lies past the arrays' capacity fills nothing, and the host, which
@@ -29,15 +29,25 @@ namespace rtt {
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 256;     // long rows and small kernels
+// The build kernel: 512 threads at 6 waves per SIMD.  256 took the AMG
+// batch's first build from 317 to 324 us (twice the workgroups to look back
+// over), 1024 to 470 us (its staging, walks and copy hardly overlap).
+constexpr int kBuild = 512;
+constexpr int kBuildWaves = kBuild / kWave;
 constexpr int kWaves = kThreads / kWave;
 
-// Columns a workgroup stages: the average of 256 rows and a tenth, at most
-// kStageMax (entries past the stage are walked in global memory).  Occupancy
-// is bound by this stage for full rows: 38 KB per workgroup for the block-FEM
-// operand leaves 4 workgroups per CU.
-constexpr int kStageMax = 12288;
+// Columns a workgroup stages: the average of its rows and a tenth, at most
+// kStageMax (entries past the stage are walked in global memory; 79 KB with
+// the skew, two workgroups per CU).  A stage cut to 64 KB, short of
+// block-FEM's rows, took its build from 0.53 to 0.8 ms.
+constexpr int kStageMax = 19200;
+constexpr int kLoads = 8;   // entries whose loads a thread issues together
 constexpr int kLongRow = 128;
+
+// LDS word of staged column x: lanes walk rows of like length, so equal
+// strides of a multiple of 32 words are skewed over the banks.
+__host__ __device__ constexpr int staged(int x) { return x + (x >> 5); }
 constexpr int kLongWin = 4096;   // tile columns a long row's window covers
 
 // Fields of a tile row's class counts: five classes of 12 bits.  Tile rows
@@ -160,26 +170,26 @@ __global__ void build_init_kernel(unsigned long long *p, int64_t n, unsigned lon
 // values: whole-line loads and stores that lie close together, against one
 // dependent load and store per entry and lane in the walk.  Duplicates
 // (adjacent equal columns in a sorted row) are summed in row order.
-// Bound by the walks (LDS reads and the dependent chain per tile), at 2.1
-// TB/s on block-FEM 500k: 0.66 ms, against 1.20 ms for separate count and
-// fill passes, their scans and a copy (AMG batch of 8, two builds: 0.67
-// against 1.1 ms).
+// Bound by latency, a workgroup at a time: block-FEM 500k 0.53 ms (2.6 TB/s),
+// 0.66 ms with the stage unskewed and one load per thread in flight, 1.20 ms
+// for separate count and fill passes, their scans and a copy (AMG batch of
+// 8, two builds: 0.65 against 1.1 ms).
 constexpr int kDup = -1, kOut = -2, kDone = -3;
 
 template <int TR, int TC, bool B>
-__global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
+__global__ __launch_bounds__(kBuild, 6) void tile_build_kernel(BuildArgs g)
 {
     static_assert(TR * TC == 32, "tiles hold 32 elements");
     static_assert(kWave % TR == 0, "a wave holds whole tile rows");
     extern __shared__ int s_stage[];
     __shared__ unsigned int s_block;
-    __shared__ unsigned long long s_x[kWaves + 1], s_y[kWaves + 1];
+    __shared__ unsigned long long s_x[kBuildWaves + 1], s_y[kBuildWaves + 1];
     const int tid = threadIdx.x;
     if (tid == 0)
         s_block = atomicAdd(&g.head->ticket, 1u);
     __syncthreads();
     const int64_t b = s_block;
-    const int64_t row0 = b * kThreads;
+    const int64_t row0 = b * kBuild;
     const int64_t row = row0 + tid;
     const int64_t tr = row / TR;
     const int r = static_cast<int>(row % TR);
@@ -188,10 +198,18 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
     int e0 = 0, ns = 0;
     if (!g.row_map && row0 < lim) {
         e0 = g.rp[row0];
-        ns = min(g.rp[min<int64_t>(row0 + kThreads, lim)] - e0, g.stage);
+        ns = min(g.rp[min<int64_t>(row0 + kBuild, lim)] - e0, g.stage);
     }
-    for (int x = tid; x < ns; x += kThreads)
-        s_stage[x] = g.ci[e0 + x];
+    for (int x0 = tid; x0 < ns; x0 += kLoads * kBuild) {
+        int v[kLoads];
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+            v[u] = x0 + u * kBuild < ns ? g.ci[e0 + x0 + u * kBuild] : 0;
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+            if (x0 + u * kBuild < ns)
+                s_stage[staged(x0 + u * kBuild)] = v[u];
+    }
     int p = 0, end = 0;
     if (row < lim) {
         const int src = g.row_map ? g.row_map[row] : static_cast<int>(row);
@@ -199,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
         end = g.rp[src + 1];
     }
     __syncthreads();
-    auto col = [&](int x) { return x - e0 < ns ? s_stage[x - e0] : g.ci[x]; };
+    auto col = [&](int x) { return x - e0 < ns ? s_stage[staged(x - e0)] : g.ci[x]; };
     // Long tile rows are counted and filled by their own kernels.
     const bool is_long = g.long_of && group_sum<TR>(end - p) > kLongRow * TR;
     if (g.long_of) {
@@ -207,7 +225,7 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
             const int l = __builtin_ctzll(m);
             const int lp = __shfl(p, l, kWave), le = __shfl(end, l, kWave);
             for (int x = lp - e0 + lane_id(); x < min(le - e0, ns); x += kWave)
-                s_stage[x] = kDone;
+                s_stage[staged(x)] = kDone;
         }
         if (is_long)
             end = p;
@@ -216,14 +234,18 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
     while (end > p && col(end - 1) >= g.active_cols) {
         --end;
         if (end - e0 < ns)
-            s_stage[end - e0] = kOut;
+            s_stage[staged(end - e0)] = kOut;
         else if (g.src_slot)
             g.src_slot[end] = -1;
     }
     // Next tile of the group from its lanes' positions x: its column, its
-    // mask, this lane's bits and the lane's entries [x, q) in it.
+    // mask, this lane's bits and the lane's entries [x, q) in it.  (Unsigned
+    // column arithmetic throughout: a shift and a mask each.)
+    constexpr unsigned kTC = TC;
+    auto bit_of = [&](unsigned c) { return 1u << (B ? (c % kTC) * TR + r : r * TC + c % kTC); };
     auto next_tile = [&](int x, int *head, uint32_t *bits, int *q, int (&cb)[TC]) {
-        const int h = group_min<TR>(x < end ? col(x) / TC : INT_MAX);
+        const int h = group_min<TR>(x < end ? static_cast<int>(static_cast<unsigned>(col(x)) / kTC)
+                                            : INT_MAX);
         *head = h;
         uint32_t v = 0;
         int y = x;
@@ -232,24 +254,21 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
         if (x + TC - e0 <= ns) {
 #pragma unroll
             for (int u = 0; u < TC; ++u)
-                cb[u] = x + u < end ? s_stage[x + u - e0] : INT_MIN;
+                cb[u] = x + u < end ? s_stage[staged(x + u - e0)] : INT_MIN;
             bool in = true;
 #pragma unroll
             for (int u = 0; u < TC; ++u) {
-                in = in && cb[u] >= 0 && cb[u] / TC == h;
-                if (in) {
-                    const int lc = cb[u] % TC;
-                    v |= 1u << (B ? lc * TR + r : r * TC + lc);
-                    ++y;
-                }
+                const unsigned c = static_cast<unsigned>(cb[u]);
+                in = in && c / kTC == static_cast<unsigned>(h);
+                v |= in ? bit_of(c) : 0u;
+                y += in ? 1 : 0;
             }
         }
         while (y < end) {
-            const int c = col(y);
-            if (c / TC != h)
+            const unsigned c = static_cast<unsigned>(col(y));
+            if (c / kTC != static_cast<unsigned>(h))
                 break;
-            const int lc = c % TC;
-            v |= 1u << (B ? lc * TR + r : r * TC + lc);
+            v |= bit_of(c);
             ++y;
         }
         *bits = v;
@@ -298,7 +317,7 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
     __syncthreads();
     unsigned long long all_x = 0, all_y = 0, bx = 0, by = 0;
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
+    for (int i = 0; i < kBuildWaves; ++i) {
         bx += i < w ? s_x[i] : 0ull;
         by += i < w ? s_y[i] : 0ull;
         all_x += s_x[i];
@@ -314,12 +333,12 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
                 publish(g.look, b, kUpTo, px + all_x, py + all_y);
         }
         if (lane_id() == 0) {
-            s_x[kWaves] = px;
-            s_y[kWaves] = py;
+            s_x[kBuildWaves] = px;
+            s_y[kBuildWaves] = py;
         }
     }
     __syncthreads();
-    const unsigned long long px = s_x[kWaves], py = s_y[kWaves];
+    const unsigned long long px = s_x[kBuildWaves], py = s_y[kBuildWaves];
     const long long end_tiles = static_cast<long long>((px + all_x) >> 31);
     const long long end_pay = static_cast<long long>(py + all_y);
     const bool fits = end_tiles <= g.cap_tiles && end_pay <= g.cap_payload;
@@ -327,7 +346,7 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
     const int lead = lane_id() & ~(TR - 1);
     const int t0 = __shfl(static_cast<int>((px + bx + ix - mine) >> 31), lead, kWave);
     const long long o0 = __shfl(static_cast<long long>(py + by + iy - my_pay), lead, kWave);
-    const bool last = (b + 1) * kThreads >= static_cast<int64_t>(g.R) * TR;
+    const bool last = (b + 1) * kBuild >= static_cast<int64_t>(g.R) * TR;
     unsigned long long at = 0;   // tiles of the classes below each class, kClassBits each
     if constexpr (B) {
 #pragma unroll
@@ -411,17 +430,17 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
                         g.values[o + phys] = 0.0;
                 }
             }
+            const uint32_t known = dense ? 0xFFFFFFFFu : mask;   // a dense tile's slots are its bits
             auto slot_of = [&](int c) {
-                const int lc = c % TC;
-                const int phys = B ? lc * TR + r : r * TC + lc;
-                return static_cast<int>(o) + payload_slot(mask, dense ? 32 : cnt, phys);
+                return static_cast<int>(o) +
+                       __popc(known & (bit_of(static_cast<unsigned>(c)) - 1u));
             };
             const int n = q - x;
             if (n <= TC && x + TC - e0 <= ns) {
 #pragma unroll
                 for (int u = 0; u < TC; ++u)
                     if (u < n)
-                        s_stage[x + u - e0] = u > 0 && cb[u] == cb[u - 1] ? kDup : slot_of(cb[u]);
+                        s_stage[staged(x + u - e0)] = u > 0 && cb[u] == cb[u - 1] ? kDup : slot_of(cb[u]);
             } else {
                 // Runs past the stage, and rows with more entries in the
                 // tile than columns (duplicates).
@@ -445,7 +464,7 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
                     }
                 }
                 for (y = x; y < q && y - e0 < ns; ++y)
-                    s_stage[y - e0] = kDone;
+                    s_stage[staged(y - e0)] = kDone;
             }
             ++t;
             o += dense ? 32 : cnt;
@@ -453,22 +472,35 @@ __global__ __launch_bounds__(kThreads) void tile_build_kernel(BuildArgs g)
         }
     }
     __syncthreads();
-    for (int x = tid; x < ns; x += kThreads) {
-        const int slot = s_stage[x];
-        if (slot >= 0) {
-            double s = g.val[e0 + x];
-            int y = x + 1;
-            for (; y < ns && s_stage[y] == kDup; ++y)
-                s += g.val[e0 + y];
-            g.values[slot] = s;
-            if (g.src_slot) {
-                for (int z = x; z < y; ++z)
-                    g.src_slot[e0 + z] = slot;
-                if (y - x > 1)
+    for (int x0 = tid; x0 < ns; x0 += kLoads * kBuild) {
+        int slot[kLoads];
+        bool dup[kLoads];
+        double v[kLoads];
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const int x = x0 + u * kBuild;
+            slot[u] = x < ns ? s_stage[staged(x)] : kDone;
+            dup[u] = x + 1 < ns && s_stage[staged(x + 1)] == kDup;
+            v[u] = slot[u] >= 0 ? g.val[e0 + x] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const int x = x0 + u * kBuild;
+            if (slot[u] >= 0) {
+                if (dup[u]) {
                     g.head->dups = 1u;
+                    for (int y = x + 1; y < ns && s_stage[staged(y)] == kDup; ++y) {
+                        v[u] += g.val[e0 + y];
+                        if (g.src_slot)
+                            g.src_slot[e0 + y] = slot[u];
+                    }
+                }
+                g.values[slot[u]] = v[u];
+                if (g.src_slot)
+                    g.src_slot[e0 + x] = slot[u];
+            } else if (slot[u] == kOut && g.src_slot) {
+                g.src_slot[e0 + x] = -1;
             }
-        } else if (slot == kOut && g.src_slot) {
-            g.src_slot[e0 + x] = -1;
         }
     }
 }
@@ -728,9 +760,9 @@ int stage_columns(const DevCsr &src, bool row_map)
 {
     if (row_map || src.rows <= 0)
         return 0;
-    const double per = 1.1 * kThreads * static_cast<double>(src.nnz) / src.rows;
+    const double per = 1.1 * kBuild * static_cast<double>(src.nnz) / src.rows;
     const int cap = per >= kStageMax ? kStageMax : (static_cast<int>(per) + 63) / 64 * 64;
-    return std::max(256, cap);
+    return std::max(kBuild, cap);
 }
 
 template <int TR, int TC, bool B>
@@ -741,7 +773,7 @@ int run_build(const DevCsr &src, const int *row_map, int active_rows, int active
     hipStream_t s = ctx().stream;
     const int R = out->tile_row_count;
     const int64_t rows = static_cast<int64_t>(R) * TR;
-    const int64_t blocks = std::max<int64_t>(1, (rows + kThreads - 1) / kThreads);
+    const int64_t blocks = std::max<int64_t>(1, (rows + kBuild - 1) / kBuild);
     const bool maybe_long = R > 0 && (src.max_row < 0 || src.max_row > kLongRow);
     static_assert(sizeof(BuildHead) % sizeof(unsigned long long) == 0, "head of whole words");
     constexpr int64_t kHeadWords = sizeof(BuildHead) / sizeof(unsigned long long);
@@ -768,7 +800,7 @@ int run_build(const DevCsr &src, const int *row_map, int active_rows, int active
     g.src_slot = src_slot;
     long long *totals = w->host_totals.as<long long>();
     g.totals = totals;
-    const size_t stage_bytes = static_cast<size_t>(g.stage) * sizeof(int);
+    const size_t stage_bytes = static_cast<size_t>(staged(g.stage)) * sizeof(int);
     const unsigned long_blocks = static_cast<unsigned>(8 * (ctx().num_cus > 0 ? ctx().num_cus : 256));
     if (maybe_long) {
         RTT_TRY(w->long_rows.ensure(static_cast<size_t>(R) * sizeof(int)));
@@ -803,7 +835,7 @@ int run_build(const DevCsr &src, const int *row_map, int active_rows, int active
                                dim3(kThreads), 0, s, g);
         }
         hipLaunchKernelGGL((tile_build_kernel<TR, TC, B>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(kThreads), stage_bytes, s, g);
+                           dim3(kBuild), stage_bytes, s, g);
         if (maybe_long)
             hipLaunchKernelGGL((long_rows_kernel<TR, TC, B, true>), dim3(long_blocks),
                                dim3(kThreads), 0, s, g);

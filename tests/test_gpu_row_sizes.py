@@ -1,5 +1,5 @@
 """C's sizes and the numeric routing at the edges of their pass: tile-row
-counts around its 256-row workgroups and the look-back's 64-workgroup step,
+counts around its 1024-row workgroups and the look-back's 64-workgroup step,
 rows that go through every symbolic pass in one call, handles that size C
 again after a smaller and a larger product, and thresholds that move rows
 between the kernels of one handle."""
@@ -20,7 +20,7 @@ def band(n, width, seed):
     return csr_from(n, n, keep // n, keep % n, rng.uniform(-1, 1, len(keep)))
 
 
-@pytest.mark.parametrize("tile_rows", [1, 255, 256, 257, 64 * 256, 64 * 256 + 1, 130 * 256 + 3])
+@pytest.mark.parametrize("tile_rows", [1, 255, 1023, 1024, 1025, 64 * 1024, 64 * 1024 + 1, 130 * 1024 + 3])
 def test_tile_row_counts(gpu, tile_rows):
     a = band(8 * tile_rows - 3, 3, tile_rows)
     pa = gpu.prepare_identity_a(a)

@@ -1,5 +1,5 @@
 """The CSR -> tile builder at its edges, bit for bit against the oracle's
-tiles: workgroup boundaries (64 B tile rows, 32 A tile rows), rows at and past
+tiles: workgroup boundaries (128 B tile rows, 64 A tile rows), rows at and past
 the limit of the merge (128 entries a scalar row on average over a tile row),
 long rows over several column windows (4096 tile columns), duplicates in both,
 rows past the column stage, and rebuilds of one handle from other operands."""
@@ -34,8 +34,9 @@ def check_b(rt, pa, pb, b, threshold=24):
 
 CASES = {
     # name: (rows, columns, entries per row, duplicates, column range)
-    "one workgroup": (256, 300, lambda i: 3, 0, None),
-    "one row past a workgroup": (257, 300, lambda i: 3 + i % 5, 0, None),
+    "half a workgroup": (256, 300, lambda i: 3, 0, None),
+    "one workgroup": (512, 300, lambda i: 3, 0, None),
+    "one row past a workgroup": (513, 300, lambda i: 3 + i % 5, 0, None),
     "at the limit": (40, 900, lambda i: 128, 0, None),
     "just past the limit": (40, 900, lambda i: 129 if i < 4 else 2, 0, None),
     "long and short mixed": (600, 4000, lambda i: 900 if i % 97 == 5 else i % 7, 0, None),
@@ -44,7 +45,8 @@ CASES = {
     "duplicates in short rows": (300, 200, lambda i: i % 12, 5, None),
     "duplicates in long rows": (36, 1500, lambda i: 400 if i < 8 else 4, 7, None),
     "duplicates filling tiles": (40, 64, lambda i: 8, 8, 8),
-    "past the stage": (512, 400, lambda i: 120 if i < 256 else 0, 0, None),
+    "past the stage": (1024, 400, lambda i: 120 if i < 512 else 0, 0, None),
+    "past the largest stage": (512, 400, lambda i: 126 if i < 300 else 3, 0, None),
     "empty rows": (520, 90, lambda i: 4 if 250 < i < 262 else 0, 0, None),
 }
 
