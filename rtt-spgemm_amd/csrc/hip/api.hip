@@ -29,6 +29,7 @@ struct rtt_prepared_a {
     rtt::SpgemmWork core;
     rtt::RowRouting routing;  // rows of the tile-pair kernel at the last threshold asked for
     rtt::Events events;
+    rtt::HostRing ring;       // pinned pieces of the host export
     rtt::DevC last_c;
     bool has_c = false;
     uint64_t id = 0;          // unique per preparation (never reused in a process)
@@ -125,14 +126,58 @@ int check_binding(const rtt_prepared_a *a, const rtt_dynamic_b *b, const char *w
     return RTT_OK;
 }
 
-int export_c(const rtt::DevC &c, rtt_smatrix *out)
+// Device arrays to host memory through a ring of pinned pieces: one piece
+// travels while the threads of host_copy spread another over the (freshly
+// allocated) destination.  A copy straight to pageable memory stages it by one
+// thread, which also takes every page fault: C of the 20k-node FEM product (82
+// MB) took 5 to 18 ms, now 4 to 5 (fresh pages are still to be zeroed).
+struct HostCopy {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+
+int staged_d2h(const HostCopy *items, int n, rtt::HostRing *ring)
+{
+    hipStream_t s = rtt::ctx().stream;
+    RTT_TRY(ring->create());
+    struct Piece {
+        void *dst;
+        size_t bytes;
+    } flight[rtt::HostRing::kPieces] = {};
+    size_t issued = 0, drained = 0;
+    auto drain = [&]() -> int {
+        const int slot = static_cast<int>(drained % rtt::HostRing::kPieces);
+        RTT_HIP(hipEventSynchronize(ring->ev[slot]));
+        rtt::host_copy(flight[slot].dst, ring->piece(slot), flight[slot].bytes);
+        ++drained;
+        return RTT_OK;
+    };
+    for (int i = 0; i < n; ++i) {
+        for (size_t at = 0; at < items[i].bytes; at += rtt::HostRing::kPieceBytes) {
+            if (issued - drained == rtt::HostRing::kPieces)
+                RTT_TRY(drain());
+            const int slot = static_cast<int>(issued % rtt::HostRing::kPieces);
+            const size_t bytes = std::min(rtt::HostRing::kPieceBytes, items[i].bytes - at);
+            RTT_HIP(hipMemcpyAsync(ring->piece(slot), static_cast<const char *>(items[i].src) + at,
+                                   bytes, hipMemcpyDeviceToHost, s));
+            RTT_HIP(hipEventRecord(ring->ev[slot], s));
+            flight[slot] = {static_cast<char *>(items[i].dst) + at, bytes};
+            ++issued;
+        }
+    }
+    while (drained < issued)
+        RTT_TRY(drain());
+    return RTT_OK;
+}
+
+int export_c(const rtt::DevC &c, rtt::HostRing *ring, rtt_smatrix *out)
 {
     if (c.num_tiles > INT_MAX || c.nnz > INT_MAX || c.tilem > INT_MAX)
         return fail(RTT_ERR_OVERFLOW,
                     "C has %lld tiles / %lld nonzeros: beyond the int32 SMatrix ABI "
                     "(use rtt_last_c_view for the 64-bit device result)",
                     (long long)c.num_tiles, (long long)c.nnz);
-    hipStream_t s = rtt::ctx().stream;
     const size_t T = static_cast<size_t>(c.num_tiles);
     const size_t Z = static_cast<size_t>(c.nnz);
     const size_t R = static_cast<size_t>(c.tilem);
@@ -144,42 +189,40 @@ int export_c(const rtt::DevC &c, rtt_smatrix *out)
     r.tilem = static_cast<int>(c.tilem);
     r.tilen = static_cast<int>(c.tilen);
     r.numtile = static_cast<int>(T);
-    r.tile_ptr = static_cast<int *>(std::malloc((R + 1) * sizeof(int)));
-    r.tile_columnidx = static_cast<int *>(std::malloc(std::max<size_t>(T, 1) * sizeof(int)));
-    r.tile_nnz = static_cast<int *>(std::malloc((T + 1) * sizeof(int)));
-    r.tile_csr_Ptr = static_cast<unsigned char *>(std::malloc(std::max<size_t>(T * 8, 1)));
-    r.tile_csr_Col = static_cast<unsigned char *>(std::malloc(std::max<size_t>(Z, 1)));
-    r.tile_csr_Value = static_cast<double *>(std::malloc(std::max<size_t>(Z, 1) * sizeof(double)));
-    std::vector<int64_t> tp(R + 1), tn(T + 1);
+    auto alloc = [](size_t bytes) { return rtt::host_alloc(std::max<size_t>(bytes, 1)); };
+    r.tile_ptr = static_cast<int *>(alloc((R + 1) * sizeof(int)));
+    r.tile_columnidx = static_cast<int *>(alloc(T * sizeof(int)));
+    r.tile_nnz = static_cast<int *>(alloc((T + 1) * sizeof(int)));
+    r.tile_csr_Ptr = static_cast<unsigned char *>(alloc(T * 8));
+    r.tile_csr_Col = static_cast<unsigned char *>(alloc(Z));
+    r.tile_csr_Value = static_cast<double *>(alloc(Z * sizeof(double)));
+    std::unique_ptr<int64_t, decltype(&std::free)> tp(
+        static_cast<int64_t *>(alloc((R + 1) * sizeof(int64_t))), &std::free);
+    std::unique_ptr<int64_t, decltype(&std::free)> tn(
+        static_cast<int64_t *>(alloc((T + 1) * sizeof(int64_t))), &std::free);
     if (!r.tile_ptr || !r.tile_columnidx || !r.tile_nnz || !r.tile_csr_Ptr || !r.tile_csr_Col ||
-        !r.tile_csr_Value) {
+        !r.tile_csr_Value || !tp || !tn) {
         rtt_destroy_smatrix(&r);
         return fail(RTT_ERR_OOM, "host allocation of the C export failed");
     }
-    auto copy = [&](void *dst, const void *src, size_t bytes) -> int {
-        if (bytes == 0)
-            return RTT_OK;
-        RTT_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-        return RTT_OK;
+    const HostCopy items[] = {
+        {tp.get(), c.tile_ptr.ptr, (R + 1) * sizeof(int64_t)},
+        {tn.get(), c.tile_nnz.ptr, (T + 1) * sizeof(int64_t)},
+        {r.tile_columnidx, c.tile_col.ptr, T * sizeof(int)},
+        {r.tile_csr_Ptr, c.tile_csr_ptr.ptr, T * 8},
+        {r.tile_csr_Col, c.tile_csr_col.ptr, Z},
+        {r.tile_csr_Value, c.tile_csr_val.ptr, Z * sizeof(double)},
     };
-    int rc = RTT_OK;
-    if ((rc = copy(tp.data(), c.tile_ptr.ptr, (R + 1) * sizeof(int64_t))) != RTT_OK ||
-        (rc = copy(tn.data(), c.tile_nnz.ptr, (T + 1) * sizeof(int64_t))) != RTT_OK ||
-        (rc = copy(r.tile_columnidx, c.tile_col.ptr, T * sizeof(int))) != RTT_OK ||
-        (rc = copy(r.tile_csr_Ptr, c.tile_csr_ptr.ptr, T * 8)) != RTT_OK ||
-        (rc = copy(r.tile_csr_Col, c.tile_csr_col.ptr, Z)) != RTT_OK ||
-        (rc = copy(r.tile_csr_Value, c.tile_csr_val.ptr, Z * sizeof(double))) != RTT_OK) {
+    const int rc = staged_d2h(items, 6, ring);
+    if (rc != RTT_OK) {
+        (void)hipStreamSynchronize(rtt::ctx().stream);   // pieces may still be in flight
         rtt_destroy_smatrix(&r);
         return rc;
     }
-    if (hipStreamSynchronize(s) != hipSuccess) {
-        rtt_destroy_smatrix(&r);
-        return fail(RTT_ERR_DEVICE, "C export synchronisation failed");
-    }
     for (size_t i = 0; i <= R; ++i)
-        r.tile_ptr[i] = static_cast<int>(tp[i]);
+        r.tile_ptr[i] = static_cast<int>(tp.get()[i]);
     for (size_t i = 0; i <= T; ++i)
-        r.tile_nnz[i] = static_cast<int>(tn[i]);
+        r.tile_nnz[i] = static_cast<int>(tn.get()[i]);
     rtt_destroy_smatrix(out);
     *out = r;
     return RTT_OK;
@@ -789,7 +832,7 @@ int rtt_tilespgemm(const rtt_prepared_a *a_const, const rtt_dynamic_b *b, rtt_sm
     stats->heavy_rows = times.heavy_rows;
     if (sc.materialize_output) {
         auto te = rtt::Clock::now();
-        RTT_TRY(export_c(a->last_c, output));
+        RTT_TRY(export_c(a->last_c, &a->ring, output));
         stats->output_copy_ms = rtt::ms_since(te);
         stats->output_materialized = 1;
     }

@@ -206,6 +206,19 @@ struct Events {
     ~Events();
 };
 
+// Pinned pieces that copies to pageable host memory travel through, with an
+// event each; created on first use, owned by one handle.
+struct HostRing {
+    static constexpr int kPieces = 4;
+    static constexpr size_t kPieceBytes = size_t(2) << 20;
+    PinnedBuf buf;
+    hipEvent_t ev[kPieces] = {};
+    bool ready = false;
+    int create();
+    char *piece(int i) const { return buf.as<char>() + static_cast<size_t>(i) * kPieceBytes; }
+    ~HostRing();
+};
+
 // Library-wide device context (one device per process).
 struct Context {
     int device = -1;

@@ -93,6 +93,25 @@ Events::~Events()
             (void)hipEventDestroy(e);
 }
 
+int HostRing::create()
+{
+    if (ready)
+        return RTT_OK;
+    RTT_TRY(buf.ensure(kPieces * kPieceBytes));
+    for (auto &e : ev)
+        if (!e)
+            RTT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    ready = true;
+    return RTT_OK;
+}
+
+HostRing::~HostRing()
+{
+    for (auto &e : ev)
+        if (e)
+            (void)hipEventDestroy(e);
+}
+
 int exclusive_scan_i64(const int64_t *in, int64_t *out, int64_t n, DevBuf *tmp,
                        hipStream_t s)
 {

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include <omp.h>
+#include <sys/mman.h>
 
 #include "../rtt_common.hpp"
 
@@ -34,6 +35,31 @@ void clear_error() { g_last_error.clear(); }
 
 const char *last_error_text() { return g_last_error.c_str(); }
 
+void *host_alloc(size_t bytes)
+{
+    constexpr size_t kHuge = size_t(2) << 20;
+    if (bytes < 2 * kHuge)
+        return std::malloc(bytes);
+    void *p = nullptr;
+    const size_t whole = (bytes + kHuge - 1) / kHuge * kHuge;
+    if (posix_memalign(&p, kHuge, whole) != 0)
+        return nullptr;
+    (void)madvise(p, whole, MADV_HUGEPAGE);
+    return p;
+}
+
+void host_copy(void *dst, const void *src, size_t bytes)
+{
+    constexpr size_t kPiece = size_t(256) << 10;
+    const long long pieces = static_cast<long long>((bytes + kPiece - 1) / kPiece);
+#pragma omp parallel for schedule(static) if (pieces > 3)
+    for (long long i = 0; i < pieces; ++i) {
+        const size_t at = static_cast<size_t>(i) * kPiece;
+        std::memcpy(static_cast<char *>(dst) + at, static_cast<const char *>(src) + at,
+                    std::min(kPiece, bytes - at));
+    }
+}
+
 } // namespace rtt
 
 using rtt::fail;
@@ -45,7 +71,7 @@ T *host_alloc(size_t count)
 {
     if (count == 0)
         count = 1;
-    return static_cast<T *>(std::malloc(count * sizeof(T)));
+    return static_cast<T *>(rtt::host_alloc(count * sizeof(T)));
 }
 
 // Allocates the CSR arrays of *out (zeroed struct first).
@@ -492,6 +518,21 @@ inline bool valid_col(int tile_col, unsigned char lc, int n, int *col)
     return true;
 }
 
+// Whether every column of the tile lies in the matrix, and every local
+// column in the tile: then no entry needs valid_col.
+inline bool tile_inside(int tile_col, int n)
+{
+    return tile_col >= 0 && (static_cast<long long>(tile_col) + 1) * kOutCols <= n;
+}
+
+inline bool plain_cols(const unsigned char *lc, int count)
+{
+    unsigned char all = 0;
+    for (int x = 0; x < count; ++x)
+        all |= lc[x];
+    return all < kOutCols;
+}
+
 void sort_rows(rtt_smatrix *m)
 {
 #pragma omp parallel for schedule(dynamic, 256)
@@ -543,10 +584,16 @@ int tile2csr_impl(rtt_smatrix *m, const int *row_new_to_old, int perm_size,
         for (int t = m->tile_ptr[tr]; t < m->tile_ptr[tr + 1]; ++t) {
             const int tnnz = m->tile_nnz[t + 1] - m->tile_nnz[t];
             const int base = m->tile_nnz[t];
+            const bool inside = tile_inside(m->tile_columnidx[t], m->n) &&
+                                plain_cols(m->tile_csr_Col + base, tnnz);
             for (int lr = 0; lr < rc; ++lr) {
                 int s, e, col;
                 row_bounds(m->tile_csr_Ptr, static_cast<size_t>(t) * kOutRows, lr, rc,
                            tnnz, &s, &e);
+                if (inside) {
+                    local[lr] += std::max(e - s, 0);
+                    continue;
+                }
                 for (int x = s; x < e; ++x)
                     if (valid_col(m->tile_columnidx[t], m->tile_csr_Col[base + x], m->n, &col))
                         ++local[lr];
@@ -573,9 +620,9 @@ int tile2csr_impl(rtt_smatrix *m, const int *row_new_to_old, int perm_size,
     }
     if (run > INT_MAX)
         return fail(RTT_ERR_OVERFLOW, "tile2csr: nnz(C) %lld exceeds int32", run);
-    int *rp = static_cast<int *>(std::malloc((static_cast<size_t>(m->m) + 1) * sizeof(int)));
-    int *ci = static_cast<int *>(std::malloc(std::max<size_t>(run, 1) * sizeof(int)));
-    double *vv = static_cast<double *>(std::malloc(std::max<size_t>(run, 1) * sizeof(double)));
+    int *rp = static_cast<int *>(rtt::host_alloc((static_cast<size_t>(m->m) + 1) * sizeof(int)));
+    int *ci = static_cast<int *>(rtt::host_alloc(std::max<size_t>(run, 1) * sizeof(int)));
+    double *vv = static_cast<double *>(rtt::host_alloc(std::max<size_t>(run, 1) * sizeof(double)));
     if (!rp || !ci || !vv) {
         std::free(rp);
         std::free(ci);
@@ -591,6 +638,8 @@ int tile2csr_impl(rtt_smatrix *m, const int *row_new_to_old, int perm_size,
         for (int t = m->tile_ptr[tr]; t < m->tile_ptr[tr + 1]; ++t) {
             const int tnnz = m->tile_nnz[t + 1] - m->tile_nnz[t];
             const int base = m->tile_nnz[t];
+            const bool inside = tile_inside(m->tile_columnidx[t], m->n) &&
+                                plain_cols(m->tile_csr_Col + base, tnnz);
             for (int lr = 0; lr < rc; ++lr) {
                 const int row = tr * kOutRows + lr;
                 if (restore && row >= perm_size)
@@ -599,6 +648,17 @@ int tile2csr_impl(rtt_smatrix *m, const int *row_new_to_old, int perm_size,
                 int s, e, col;
                 row_bounds(m->tile_csr_Ptr, static_cast<size_t>(t) * kOutRows, lr, rc,
                            tnnz, &s, &e);
+                if (inside) {
+                    int *pc = ci + rp[orow] + local[lr];
+                    double *pv = vv + rp[orow] + local[lr];
+                    const int c0 = m->tile_columnidx[t] * kOutCols;
+                    for (int x = s; x < e; ++x) {
+                        pc[x - s] = c0 + m->tile_csr_Col[base + x];
+                        pv[x - s] = m->tile_csr_Value[base + x];
+                    }
+                    local[lr] += std::max(e - s, 0);
+                    continue;
+                }
                 for (int x = s; x < e; ++x) {
                     if (!valid_col(m->tile_columnidx[t], m->tile_csr_Col[base + x], m->n, &col))
                         continue;

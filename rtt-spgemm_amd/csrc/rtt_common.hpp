@@ -3,6 +3,7 @@
 
 #include <chrono>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdint>
 
 #include "rtt_spgemm.h"
@@ -16,6 +17,15 @@ void clear_error();
 // Zeroes *out and mallocs its CSR arrays (m + 1 row pointers, nnz columns and
 // values); RTT_ERR_OVERFLOW beyond the int32 ABI, RTT_ERR_OOM on failure.
 int alloc_host_csr(int m, int n, int64_t nnz, rtt_smatrix *out);
+
+// Host memory to be released with free(), nullptr on failure.  Large blocks
+// are aligned to huge pages and advised to take them: a result of a few
+// hundred megabytes is then first touched by hundreds of faults instead of
+// tens of thousands.
+void *host_alloc(size_t bytes);
+// memcpy, by several threads when it is large (which also spreads the first
+// touch of fresh memory over them).
+void host_copy(void *dst, const void *src, size_t bytes);
 
 using Clock = std::chrono::steady_clock;
 inline double ms_since(Clock::time_point t0)

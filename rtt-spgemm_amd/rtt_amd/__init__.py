@@ -275,20 +275,35 @@ def _np_copy(ptr, count: int, dtype) -> np.ndarray:
     return np.array(np.ctypeslib.as_array(buf), dtype=dtype, copy=True)
 
 
-def _csr_from_smatrix(s: SMatrix) -> CsrMatrix:
-    out = CsrMatrix(s.m, s.n, _np_copy(s.rowpointer, s.m + 1, np.int32),
-                    _np_copy(s.columnindex, s.nnz, np.int32),
-                    _np_copy(s.value, s.nnz, np.float64), s.isSymmetric)
-    if s.m + 1 > 0 and out.rowptr.size == 0:
-        out.rowptr = np.zeros(s.m + 1, np.int32)
-    return out
+class _HostArrays:
+    """Owns the host arrays of an SMatrix the library allocated: numpy arrays
+    made with ``view`` keep it alive, and the last of them frees the arrays
+    (no copy of a result of hundreds of megabytes)."""
+
+    def __init__(self, s: SMatrix):
+        self._s = s
+
+    def view(self, ptr, count: int, dtype) -> np.ndarray:
+        if count <= 0 or not ptr:
+            return np.zeros(0, dtype=dtype)
+        ct = np.ctypeslib.as_ctypes_type(np.dtype(dtype))
+        buf = (ct * count).from_address(C.cast(ptr, C.c_void_p).value)
+        buf._owner = self   # the array's base holds buf
+        return np.frombuffer(buf, dtype=dtype)
+
+    def __del__(self):
+        if _lib is not None:
+            _lib.rtt_destroy_smatrix(C.byref(self._s))
 
 
 def _consume_csr(s: SMatrix) -> CsrMatrix:
-    try:
-        return _csr_from_smatrix(s)
-    finally:
-        load().rtt_destroy_smatrix(C.byref(s))
+    own = _HostArrays(s)
+    out = CsrMatrix(s.m, s.n, own.view(s.rowpointer, s.m + 1, np.int32),
+                    own.view(s.columnindex, s.nnz, np.int32),
+                    own.view(s.value, s.nnz, np.float64), s.isSymmetric)
+    if s.m + 1 > 0 and out.rowptr.size == 0:
+        out.rowptr = np.zeros(s.m + 1, np.int32)
+    return out
 
 
 # ---- host utilities ----------------------------------------------------------
@@ -428,14 +443,15 @@ class TileC:
         return s
 
 
-def _tilec_from_smatrix(s: SMatrix) -> TileC:
+def _consume_tilec(s: SMatrix) -> TileC:
+    own = _HostArrays(s)
     return TileC(s.m, s.n, s.tilem, s.tilen, s.numtile, s.nnz,
-                 _np_copy(s.tile_ptr, s.tilem + 1, np.int32),
-                 _np_copy(s.tile_columnidx, s.numtile, np.int32),
-                 _np_copy(s.tile_nnz, s.numtile + 1, np.int32),
-                 _np_copy(s.tile_csr_Ptr, 8 * s.numtile, np.uint8),
-                 _np_copy(s.tile_csr_Col, s.nnz, np.uint8),
-                 _np_copy(s.tile_csr_Value, s.nnz, np.float64))
+                 own.view(s.tile_ptr, s.tilem + 1, np.int32),
+                 own.view(s.tile_columnidx, s.numtile, np.int32),
+                 own.view(s.tile_nnz, s.numtile + 1, np.int32),
+                 own.view(s.tile_csr_Ptr, 8 * s.numtile, np.uint8),
+                 own.view(s.tile_csr_Col, s.nnz, np.uint8),
+                 own.view(s.tile_csr_Value, s.nnz, np.float64))
 
 
 def _download_tiles(view: DeviceTiles) -> dict:
@@ -761,13 +777,7 @@ def tilespgemm(a: PreparedA, b: DynamicB, sched: Schedule | None = None):
     _check(load().rtt_tilespgemm(a.handle, b.handle, C.byref(out), C.byref(st),
                                  C.byref(sched)), "tilespgemm")
     stats = {f: getattr(st, f) for f, _ in Stats._fields_}
-    tc = None
-    if sched.materialize_output:
-        try:
-            tc = _tilec_from_smatrix(out)
-        finally:
-            load().rtt_destroy_smatrix(C.byref(out))
-    return tc, stats
+    return (_consume_tilec(out) if sched.materialize_output else None), stats
 
 
 def batch_extract(a: PreparedA, row_offset: int, col_offset: int, m: int, n: int) -> TileC:
@@ -776,10 +786,7 @@ def batch_extract(a: PreparedA, row_offset: int, col_offset: int, m: int, n: int
     _check(load().rtt_batch_extract(a.handle, C.byref(C.c_int64(int(row_offset))),
                                     C.byref(C.c_int64(int(col_offset))), m, n, C.byref(out)),
            "batch_extract")
-    try:
-        return _tilec_from_smatrix(out)
-    finally:
-        load().rtt_destroy_smatrix(C.byref(out))
+    return _consume_tilec(out)
 
 
 def autotune(a: PreparedA, b: DynamicB, repeats: int = 2, sched: Schedule | None = None):
@@ -861,12 +868,7 @@ def last_c(a: PreparedA, with_values: bool = True) -> dict:
 def tile2csr(tc: TileC, canonical: bool = True) -> CsrMatrix:
     s = tc.as_smatrix()
     _check(load().rtt_tile2csr(C.byref(s), int(canonical)), "tile2csr")
-    try:
-        return CsrMatrix(s.m, s.n, _np_copy(s.rowpointer, s.m + 1, np.int32),
-                         _np_copy(s.columnindex, s.nnz, np.int32),
-                         _np_copy(s.value, s.nnz, np.float64))
-    finally:
-        _free_csr_part(s)
+    return _consume_csr_part(s)
 
 
 def tile2csr_restore_rows(tc: TileC, row_new_to_old, permutation_size: int,
@@ -875,20 +877,16 @@ def tile2csr_restore_rows(tc: TileC, row_new_to_old, permutation_size: int,
     perm = np.ascontiguousarray(row_new_to_old, dtype=np.int32)
     _check(load().rtt_tile2csr_restore_rows(C.byref(s), _ptr(perm), permutation_size,
                                             int(canonical)), "tile2csr_restore_rows")
-    try:
-        return CsrMatrix(s.m, s.n, _np_copy(s.rowpointer, s.m + 1, np.int32),
-                         _np_copy(s.columnindex, s.nnz, np.int32),
-                         _np_copy(s.value, s.nnz, np.float64))
-    finally:
-        _free_csr_part(s)
+    return _consume_csr_part(s)
 
 
-def _free_csr_part(s: SMatrix) -> None:
+def _consume_csr_part(s: SMatrix) -> CsrMatrix:
     # Only the CSR arrays belong to the library here; the tile arrays are
-    # numpy-owned, so free the CSR part through a separate struct.
+    # numpy's, so the CSR part goes to a struct of its own.
     t = SMatrix()
+    t.m, t.n, t.nnz = s.m, s.n, s.nnz
     t.rowpointer, t.columnindex, t.value = s.rowpointer, s.columnindex, s.value
-    load().rtt_destroy_smatrix(C.byref(t))
+    return _consume_csr(t)
 
 
 def abi_symbols(header: str = HEADER_PATH) -> list[str]:
