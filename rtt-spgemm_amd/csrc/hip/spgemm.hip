@@ -61,6 +61,8 @@ constexpr int kWSeg = 512;         // pairs per one-wave segment window
 constexpr int kWBatch = 6;         // pairs whose loads a lane of that kernel issues together
 
 constexpr int kColRegs = 3;         // values of an A column a numeric lane holds in registers
+constexpr int kOneVals = 3;         // B values a lane loads of the one row of a light pair
+constexpr int kSkew = 32;           // SpreadRow: accumulator slots between two unused ones
 constexpr int kExtVals = 3;         // B values past the record a numeric lane prefetches
 
 // The numeric instances: threads per workgroup (four pair runs of kChunk A
@@ -73,26 +75,45 @@ constexpr int kExtVals = 3;         // B values past the record a numeric lane p
 // on the rows between the two.
 struct TinyRow {
     static constexpr int kThreads = kWave, kChunk = kWave / 4, kSeg = 128;
-    static constexpr bool kLeavesTiny = false;
+    static constexpr bool kLeavesTiny = false, kSpread = false;
+    static constexpr int kWavesPerSimd = 7;
     static constexpr int kAcc = 128, kAStage = 64, kTiles = 16, kSlots = 32, kSlotBits = 5;
 };
 // SmallRow, launched over every row, leaves the rows within TinyRow's
 // budgets to that instance (launched over their list).
 struct SmallRow {
     static constexpr int kThreads = 256, kChunk = 64, kSeg = 1024;
-    static constexpr bool kLeavesTiny = true;
+    static constexpr bool kLeavesTiny = true, kSpread = false;
+    static constexpr int kWavesPerSimd = 7;
     static constexpr int kAcc = 1024, kAStage = 256, kTiles = 128, kSlots = 256, kSlotBits = 8;
 };
+// SmallRow for products whose C tiles hold kSpreadFill entries or fewer on
+// average: the lanes of a wave then add to the same few places of many C
+// tiles at once.  The accumulator has an unused slot after every kSkew, which
+// takes the tiles' like places to different LDS banks (the tiles of eight
+// equal C rows, stencils', otherwise lie a multiple of eight slots apart: an
+// add took 17 ns a wave and CU, with the slots 8), and a pair with a light
+// tile, of which such products have many, takes the one row it needs of B's
+// record instead of walking all of it.  The LDS pipe was busy 75 % of the
+// kernel's time and is now 58 %, vector instructions 70 %: 128^3 box stencil,
+// A*A^T (14 entries a C tile), 2.83 -> 2.29 ms; banded products (39 to 49)
+// take 0.59 ms with the extra index work against 0.57 without.
+struct SpreadRow : SmallRow {
+    static constexpr bool kSpread = true;
+};
+constexpr int kSpreadFill = 24;
 // MediumRow takes rows past SmallRow's accumulator with few C tiles and A
 // values (narrow bands squared) at a third of LargeRow's LDS.
 struct MediumRow {
     static constexpr int kThreads = 256, kChunk = 64, kSeg = 1024;
-    static constexpr bool kLeavesTiny = false;
+    static constexpr bool kLeavesTiny = false, kSpread = false;
+    static constexpr int kWavesPerSimd = 6;
     static constexpr int kAcc = 2048, kAStage = 256, kTiles = 64, kSlots = 128, kSlotBits = 7;
 };
 struct LargeRow {
     static constexpr int kThreads = 256, kChunk = 64, kSeg = 1024;
-    static constexpr bool kLeavesTiny = false;
+    static constexpr bool kLeavesTiny = false, kSpread = false;
+    static constexpr int kWavesPerSimd = 2;
     static constexpr int kAcc = 4096, kAStage = 2048, kTiles = 512, kSlots = 1024, kSlotBits = 10;
 };
 static_assert(LargeRow::kAcc <= 65536 && LargeRow::kTiles <= 32768, "packed tile slots");
@@ -189,13 +210,10 @@ __device__ __forceinline__ uint64_t bytes_product(uint32_t a_bytes, uint32_t b_b
     return out;
 }
 
-__device__ __forceinline__ int product_count(uint32_t a_bytes, uint32_t b_bytes)
+// Byte k is nonzero where byte k of v is (its bit 7 set).
+__device__ __forceinline__ uint32_t nonzero_tops(uint32_t v)
 {
-    int n = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        n += __popc(byte_of(a_bytes, k)) * __popc(byte_of(b_bytes, k));
-    return n;
+    return (((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v) & 0x80808080u;
 }
 
 template <typename T>
@@ -749,8 +767,8 @@ __device__ __forceinline__ bool is_run(uint32_t bits)
 }
 
 // Byte r: (slot of row r's first entry within the tile) - (its first
-// column) when the row's columns are contiguous, kNoRun when they are not,
-// 0 for an empty row (never addressed).
+// column) + kTileN, which is 1 to 64, when the row's columns are contiguous,
+// kNoRun when they are not, 0 for an empty row (never addressed).
 __device__ __forceinline__ uint64_t row_runs(uint64_t m)
 {
     uint64_t out = 0;
@@ -760,7 +778,7 @@ __device__ __forceinline__ uint64_t row_runs(uint64_t m)
         const uint32_t bits = static_cast<uint32_t>(m >> (8 * r)) & 0xFFu;
         uint32_t b = 0;
         if (bits)
-            b = is_run(bits) ? static_cast<uint32_t>(first - __builtin_ctz(bits)) & 0xFFu : kNoRun;
+            b = is_run(bits) ? static_cast<uint32_t>(first + kTileN - __builtin_ctz(bits)) : kNoRun;
         out |= static_cast<uint64_t>(b) << (8 * r);
         first += __popc(bits);
     }
@@ -769,7 +787,7 @@ __device__ __forceinline__ uint64_t row_runs(uint64_t m)
 
 __device__ __forceinline__ int run_base(uint64_t runs, int r)
 {
-    return static_cast<int8_t>((runs >> (8 * r)) & 0xFFu);
+    return static_cast<int>((runs >> (8 * r)) & 0xFFu) - kTileN;
 }
 
 // Byte k: rows of A column k as count | first row << 4, with bit 7 set when
@@ -786,6 +804,13 @@ __device__ __forceinline__ uint32_t a_column_runs(uint32_t ab)
         }
     }
     return out;
+}
+
+// Place of a C row's i-th value in the accumulator.
+template <class Cfg>
+__device__ __forceinline__ int acc_place(int i)
+{
+    return Cfg::kSpread ? i + i / kSkew : i;
 }
 
 // Sampled start/end times of the numeric kernel's waves (the timeline
@@ -817,13 +842,13 @@ __device__ __forceinline__ void trace_mark(const Timeline &tl, bool at_end)
 }
 
 template <class Cfg, bool TRACE = false>
-__global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
+__global__ __launch_bounds__(Cfg::kThreads, Cfg::kWavesPerSimd) void numeric_row_kernel(
     Operands g, const int4 *__restrict__ recs, int64_t rec_n, const int *__restrict__ rows,
     const int *__restrict__ row_level, Stage st, COut c, Timeline tl)
 {
     constexpr int kT = Cfg::kThreads, kCh = Cfg::kChunk, kSg = Cfg::kSeg, kNW = kT / kWave;
     static_assert(kT == 4 * kCh && kT % kWave == 0, "one thread per (pair run, chunk tile)");
-    __shared__ double s_acc[Cfg::kAcc];
+    __shared__ double s_acc[Cfg::kAcc + (Cfg::kSpread ? Cfg::kAcc / kSkew : 0)];
     __shared__ double s_acol[Cfg::kAStage + kColRegs];
     __shared__ unsigned long long s_cmask[Cfg::kTiles];   // C tile masks, bit r * 8 + cl
     __shared__ int s_cbase[Cfg::kTiles];   // first slot of each tile within the row's segment
@@ -887,7 +912,7 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
     }
     for (int i = tid; i < Cfg::kSlots; i += kT)
         s_slot[i] = make_int4(kEmpty, 0, 0, 0);
-    for (int i = tid; i < nnz_row; i += kT)
+    for (int i = tid; i < acc_place<Cfg>(static_cast<int>(nnz_row)); i += kT)
         s_acc[i] = 0.0;
     if (tid < a_len)
         s_acol[tid] = av0;
@@ -904,7 +929,10 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
         const uint32_t p1 = __popc(byte_of(ab, 0));
         const uint32_t p2 = p1 + __popc(byte_of(ab, 1));
         const uint32_t p3 = p2 + __popc(byte_of(ab, 2));
-        const uint32_t heavy = __popc(static_cast<uint32_t>(am.y)) >= kHeavyMin ? 1u : 0u;
+        const uint32_t heavy = __popc(static_cast<uint32_t>(am.y)) >= kHeavyMin ||
+                                       __popc(nonzero_tops(ab)) > 1
+                                   ? 1u
+                                   : 0u;
         s_at[tid] = make_int4(static_cast<int>(ab),
                               static_cast<int>(heavy | (p1 << 8) | (p2 << 16) | (p3 << 24)),
                               static_cast<int>(static_cast<uint32_t>(am.w) & ~kDenseBit) - a_base,
@@ -995,17 +1023,38 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
                     // first part.
                     static_assert(kHeavyMin - 1 <= 2, "light values fill one record part");
                     const bool light_b = v >= 2 * kCh;
+                    const bool one = Cfg::kSpread && v >= kCh;
 #pragma unroll
                     for (int i = 0; i < kRecVals / 2; ++i) {
                         double2 d = make_double2(0.0, 0.0);
-                        if (i < 1 || !light_b)
+                        if (one ? i < 1 && light_b : i < 1 || !light_b)
                             d = reinterpret_cast<const double2 *>(recs + (i + 1) * rec_n)[rb_idx];
                         rec.v[2 * i] = d.x;
                         rec.v[2 * i + 1] = d.y;
                     }
                     const uint32_t ab = static_cast<uint32_t>(at.x);
-                    if (!product_count(ab, static_cast<uint32_t>(rec.meta.z)))
+                    const uint32_t bb = static_cast<uint32_t>(rec.meta.z);
+                    const uint32_t boff = static_cast<uint32_t>(rec.meta.w) & ~kDenseBit;
+                    const uint32_t ks = nonzero_tops(ab) & nonzero_tops(bb);
+                    if (!ks)
                         continue;
+                    // One of the tiles is light: the pair is column k1 of A times
+                    // row k1 of B alone, whose values a light B tile has in its
+                    // first part.
+                    const int k1 = __builtin_ctz(ks) >> 3;
+                    const int j1 = __popc(bb & ((1u << (8 * k1)) - 1u));
+                    auto value = [&](int j) {
+                        return j < kRecVals ? reinterpret_cast<const double *>(
+                                                  recs + (1 + (j >> 1)) * rec_n + rb_idx)[j & 1]
+                                            : g.b_vals_km[boff + j];
+                    };
+                    if (one && !light_b) {
+                        const int n1 = __popc(byte_of(bb, k1));
+#pragma unroll
+                        for (int i = 0; i < kOneVals; ++i)
+                            if (i < n1)
+                                rec.v[i] = value(j1 + i);
+                    }
                     // C tile of the pair; every tile of the row is in the table and
                     // at least half of its slots are empty, so the probe ends.
                     uint32_t h = slot_of(rec.meta.x, Cfg::kSlotBits);
@@ -1022,17 +1071,33 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
                     const unsigned long long cruns =
                         (static_cast<unsigned long long>(static_cast<uint32_t>(sl.w)) << 32) |
                         static_cast<uint32_t>(sl.z);
-                    double *acc = s_acc + (sl.y & 0xFFFF);
+                    const int acc = sl.y & 0xFFFF;   // first slot of the tile
                     const uint32_t apf = static_cast<uint32_t>(at.y) & ~0xFFu;
                     const uint32_t aruns = static_cast<uint32_t>(at.w);
                     const double *acol = s_acol + at.z;
-                    const uint32_t boff = static_cast<uint32_t>(rec.meta.w) & ~kDenseBit;
                     // B entries in k-major order: the record's values, then the
                     // payload's.  The first kExtVals payload values are loaded once
                     // kExtVals record values have been used, into the registers
                     // those held, and arrive while the rest of the record is walked.
                     auto walk = [&](auto &&entry) {
-                        uint32_t mz = static_cast<uint32_t>(rec.meta.z);
+                        uint32_t mz = bb;
+                        if (one) {
+                            mz &= 0xFFu << (8 * k1);
+#pragma unroll
+                            for (int j = 0; j < kOneVals; ++j) {
+                                if (mz) {
+                                    const int pos = __builtin_ctz(mz);
+                                    mz &= mz - 1;
+                                    entry(pos, rec.v[j]);
+                                }
+                            }
+                            for (int j = j1 + kOneVals; mz; ++j) {
+                                const int pos = __builtin_ctz(mz);
+                                mz &= mz - 1;
+                                entry(pos, value(j));
+                            }
+                            return;
+                        }
                         const int nbv = __popc(mz);
                         double ext[kExtVals > 0 ? kExtVals : 1];
 #pragma unroll
@@ -1065,7 +1130,10 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
                             ++j;
                         }
                     };
-                    if (((cruns & 0x8080808080808080ull) | (aruns & 0x80808080u)) == 0) {
+                    // The wave takes one way together: with lanes on both it
+                    // would run both (banded batch: 0.60 and 0.46 ms against
+                    // 0.57 and 0.42 in the two instances it uses).
+                    if (__all(((cruns & 0x8080808080808080ull) | (aruns & 0x80808080u)) == 0)) {
                         // All runs, and no A column longer than kColRegs: at each
                         // new k the lane takes the values and the row bases of the
                         // rows r0, r0 + 1, ... of A column k into registers.
@@ -1088,12 +1156,12 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
                                 for (int i = 0; i < kColRegs; ++i)
                                     av[i] = ap[i];
                             }
-                            double *pc = acc + cl;
+                            const int pc = acc + cl;
                             const int na = static_cast<int>(kd & 15u);
 #pragma unroll
                             for (int i = 0; i < kColRegs; ++i)
                                 if (i < na)
-                                    atomicAdd(pc + run_base(rb, i), av[i] * vb);
+                                    atomicAdd(s_acc + acc_place<Cfg>(pc + run_base(rb, i)), av[i] * vb);
                         });
                     } else {
                         // Slots from popcounts of the tile mask.
@@ -1106,8 +1174,9 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
                             while (rr) {
                                 const int r = __builtin_ctz(rr);
                                 rr &= rr - 1;
-                                atomicAdd(&acc[__popcll(cm & ((1ull << (r * 8 + cl)) - 1ull))],
-                                          ap[i++] * vb);
+                                const int slot =
+                                    acc + __popcll(cm & ((1ull << (r * 8 + cl)) - 1ull));
+                                atomicAdd(s_acc + acc_place<Cfg>(slot), ap[i++] * vb);
                             }
                         });
                     }
@@ -1136,7 +1205,7 @@ __global__ __launch_bounds__(Cfg::kThreads) void numeric_row_kernel(
     }
     __syncthreads();
     for (int64_t i = tid; i < nnz_row; i += kT)
-        c.val[zb + i] = s_acc[i];
+        c.val[zb + i] = s_acc[acc_place<Cfg>(static_cast<int>(i))];
     // Words [0, nw) of the row's column bytes from the aligned word at zb -
     // shift; the first and last may hold bytes of the neighbouring rows and
     // are written byte by byte.
@@ -1703,13 +1772,19 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     // its own (a list entry is one more dependent load per row).  Launched
     // over every row whatever its class, as the traced form still is, the
     // workgroups that leave at once took 0.3 of the AMG batch's 3.0 ms.
-    if (trace_slots && any_vector)
-        hipLaunchKernelGGL((numeric_row_kernel<SmallRow, true>), dim3(R), dim3(kThreads), 0, s, g,
-                           b.records.as<int4>(), b.num_tiles, nullptr, w->row_level.as<int>(), st,
-                           co, tl);
+    auto small_launch = [&](auto cfg) {
+        using Cfg = decltype(cfg);
+        if (trace_slots && any_vector)
+            hipLaunchKernelGGL((numeric_row_kernel<Cfg, true>), dim3(R), dim3(kThreads), 0, s, g,
+                               b.records.as<int4>(), b.num_tiles, nullptr, w->row_level.as<int>(),
+                               st, co, tl);
+        else
+            rows_launch(numeric_row_kernel<Cfg>, kRowSmall, Cfg::kThreads, n_rows[kRowSmall] == R);
+    };
+    if (c->nnz <= kSpreadFill * c->num_tiles)
+        small_launch(SpreadRow{});
     else
-        rows_launch(numeric_row_kernel<SmallRow>, kRowSmall, SmallRow::kThreads,
-                    n_rows[kRowSmall] == R);
+        small_launch(SmallRow{});
     RTT_HIP(hipGetLastError());
     if (!any_tile)
         RTT_HIP(hipEventRecord(ev->ev[5], s));
