@@ -55,11 +55,12 @@ __device__ __forceinline__ uint32_t stride4_bits(uint32_t mask, int k)
 // Bit r of `rows` -> byte r of the result is 0xFF.
 __device__ __forceinline__ uint64_t rows_to_bytes(uint32_t rows)
 {
-    uint64_t s = rows;
-    s = (s | (s << 28)) & 0x0000000F0000000Full;
-    s = (s | (s << 14)) & 0x0003000300030003ull;
-    s = (s | (s << 7)) & 0x0101010101010101ull;
-    return s * 0xFFull;
+    auto nibble = [](uint32_t x) {
+        x = (x | (x << 14)) & 0x00030003u;
+        x = (x | (x << 7)) & 0x01010101u;
+        return (x << 8) - x;
+    };
+    return (static_cast<uint64_t>(nibble(rows >> 4)) << 32) | nibble(rows & 15u);
 }
 
 // Structural product of an 8x4 A tile mask (bit r*4+k) and a 4x8 B tile
@@ -99,6 +100,22 @@ __device__ __forceinline__ T wave_inclusive_scan(T v)
     }
     return v;
 }
+
+// The same for ints by data-parallel moves: shifts within the rows of 16
+// lanes, then each row's last lane into the rows after it.  Six adds, where
+// the form above takes six trips through the LDS.
+__device__ __forceinline__ int wave_inclusive_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15, rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31, rows 2 and 3
+    return v;
+}
+
+__device__ __forceinline__ int last_lane(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
 
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)

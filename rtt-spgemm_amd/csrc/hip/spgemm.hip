@@ -198,22 +198,38 @@ __device__ __forceinline__ uint32_t slot_of(int j, int bits)
 
 __device__ __forceinline__ uint32_t byte_of(uint32_t v, int k) { return (v >> (8 * k)) & 0xFFu; }
 
-// Structural product from the per-k row/column byte sets of the A tile
-// (rows present in column k) and the B tile (columns present in row k).
-__device__ __forceinline__ uint64_t bytes_product(uint32_t a_bytes, uint32_t b_bytes)
-{
-    uint64_t out = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        out |= rows_to_bytes(byte_of(a_bytes, k)) &
-               (static_cast<uint64_t>(byte_of(b_bytes, k)) * 0x0101010101010101ull);
-    return out;
-}
-
 // Byte k is nonzero where byte k of v is (its bit 7 set).
 __device__ __forceinline__ uint32_t nonzero_tops(uint32_t v)
 {
     return (((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v) & 0x80808080u;
+}
+
+// An A tile spread for products with many B tiles: word k of lo (hi) is 0xFF
+// in byte r where row r (row 4 + r) has an entry in column k.
+__device__ __forceinline__ void spread_tile(uint32_t ab, uint4 *lo, uint4 *hi)
+{
+    uint64_t s[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        s[k] = rows_to_bytes(byte_of(ab, k));
+    *lo = make_uint4(static_cast<uint32_t>(s[0]), static_cast<uint32_t>(s[1]),
+                     static_cast<uint32_t>(s[2]), static_cast<uint32_t>(s[3]));
+    *hi = make_uint4(static_cast<uint32_t>(s[0] >> 32), static_cast<uint32_t>(s[1] >> 32),
+                     static_cast<uint32_t>(s[2] >> 32), static_cast<uint32_t>(s[3] >> 32));
+}
+
+// Structural product of a spread A tile and the per-k column bytes of a B
+// tile: byte k of b_bytes to every byte of a word, then a bitwise select each.
+__device__ __forceinline__ uint64_t spread_product(const uint4 &lo, const uint4 &hi,
+                                                   uint32_t b_bytes)
+{
+    const uint32_t b0 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x00000000u);
+    const uint32_t b1 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x01010101u);
+    const uint32_t b2 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x02020202u);
+    const uint32_t b3 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x03030303u);
+    const uint32_t l = (lo.x & b0) | (lo.y & b1) | (lo.z & b2) | (lo.w & b3);
+    const uint32_t h = (hi.x & b0) | (hi.y & b1) | (hi.z & b2) | (hi.w & b3);
+    return (static_cast<uint64_t>(h) << 32) | l;
 }
 
 template <typename T>
@@ -246,15 +262,14 @@ __device__ __forceinline__ void fill_segments(unsigned char *s_seg, int pre, int
 // workgroup kernel below, with a kWSlots table, so that a CU holds four times
 // as many rows and their load latencies overlap.  Pairs come in two runs per
 // chunk of kWChunk A tiles, the heavy and then the light tiles of the B
-// rows; lane t owns both runs of tile t.  A pair's mask sums only the k where
-// both A's column and B's row are nonempty.  A row that outgrows the table is marked
-// kLevelLarge for the workgroup kernel.
+// rows; lane t owns both runs of tile t.  A row that outgrows the table is
+// marked kLevelLarge for the workgroup kernel.
+// Vector instructions bound it (88 % of its cycles on the 128^3 stencil), so
+// they were cut: a pair's mask without a loop over its k or a multiply,
+// scans by data-parallel moves, two entries ranked at a time: 0.73 -> 0.61 ms
+// there, 0.42 -> 0.33 on the AMG batch, 0.28 -> 0.21 on the 500k-node FEM
+// square.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v)
-{
-    const uint32_t nz = (((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v) & 0x80808080u;
-    return ((nz >> 7) | (nz >> 14) | (nz >> 21) | (nz >> 28)) & 0xFu;
-}
 
 __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
     Operands g, Stage st, int64_t *__restrict__ row_tiles, int64_t *__restrict__ row_nnz,
@@ -262,8 +277,7 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
 {
     __shared__ __align__(16) int s_key[kWSlots];
     __shared__ unsigned long long s_msk[kWSlots];
-    __shared__ unsigned long long s_spread[4][kWChunk];
-    __shared__ int s_acls[kWChunk];   // nonempty columns (bits 0-3)
+    __shared__ uint4 s_lo[kWChunk], s_hi[kWChunk];   // spread_tile of the chunk's tiles
     __shared__ int s_pw[2 * kWChunk]; // per (run, tile): first B tile minus first pair
     __shared__ unsigned char s_seg[kWSeg];
     static_assert(2 * kWChunk <= 256, "segment entries are bytes");
@@ -283,11 +297,7 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
             const int4 am = g.a_meta[c0 + lane];
             const int4 br = g.a_brange[c0 + lane];
             const int2 bl = g.a_blight[c0 + lane];
-            const uint32_t ab = static_cast<uint32_t>(am.z);
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                s_spread[k][lane] = rows_to_bytes(byte_of(ab, k));
-            s_acls[lane] = static_cast<int>(nonzero_bytes(ab));
+            spread_tile(static_cast<uint32_t>(am.z), &s_lo[lane], &s_hi[lane]);
             nh = br.y;
             bh = br.x;
             nl = bl.y;
@@ -295,8 +305,8 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
         }
         // Pair offsets: the heavy runs of all tiles, then the light runs.
         const int ih = wave_inclusive_scan(nh), il = wave_inclusive_scan(nl);
-        const int heavy_total = __shfl(ih, kWave - 1, kWave);
-        const int total = heavy_total + __shfl(il, kWave - 1, kWave);
+        const int heavy_total = last_lane(ih);
+        const int total = heavy_total + last_lane(il);
         const int ph = ih - nh, pl = heavy_total + il - nl;
         s_pw[lane] = bh - ph;
         s_pw[kWChunk + lane] = bls - pl;
@@ -326,15 +336,8 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
                 for (int u = 0; u < kWBatch; ++u) {
                     if (ai[u] < 0)
                         continue;
-                    const uint32_t bb = static_cast<uint32_t>(bm[u].z);
-                    uint32_t kk = static_cast<uint32_t>(s_acls[ai[u]]) & nonzero_bytes(bb);
-                    uint64_t pm = 0;
-                    while (kk) {
-                        const int k = __builtin_ctz(kk);
-                        kk &= kk - 1;
-                        const uint32_t b4 = byte_of(bb, k) * 0x01010101u;
-                        pm |= s_spread[k][ai[u]] & ((static_cast<uint64_t>(b4) << 32) | b4);
-                    }
+                    const uint64_t pm = spread_product(s_lo[ai[u]], s_hi[ai[u]],
+                                                       static_cast<uint32_t>(bm[u].z));
                     if (!pm)
                         continue;
                     const int j = bm[u].x;
@@ -374,7 +377,7 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
         mine += rk[i] != kEmpty ? 1 : 0;
     }
     const int incl = wave_inclusive_scan(mine);
-    const int nt = __shfl(incl, kWave - 1, kWave);
+    const int nt = last_lane(incl);
     if (ovf || nt > kWStage) {
         if (lane == 0)
             row_level[row] = kLevelLarge;
@@ -382,7 +385,7 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
     }
     __syncthreads();
     int pos = incl - mine;
-    long long nz = 0;
+    int nz = 0;
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
         if (rk[i] != kEmpty) {
@@ -391,25 +394,42 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
             nz += __popcll(rm[i]);
             ++pos;
         }
+    static_assert(kWStage + 4 <= kWSlots, "padding of the key list");
+    if (lane < 4)
+        s_key[nt + lane] = INT_MAX;   // to whole groups of four
     __syncthreads();
-    // Rank by counting: entry t goes to the number of smaller columns.
+    // Rank by counting: entry t goes to the number of smaller columns.  Two
+    // entries a lane share the reads of the list.
     const int64_t sb = static_cast<int64_t>(row) * st.stride;
     const int4 *k4 = reinterpret_cast<const int4 *>(s_key);
-    const int full = nt & ~3;
-    for (int t = lane; t < nt; t += kWave) {
-        const int mj = s_key[t];
-        int rank = 0;
-        for (int f = 0; f < full / 4; ++f) {
-            const int4 kk = k4[f];
-            rank += (kk.x < mj ? 1 : 0) + (kk.y < mj ? 1 : 0) + (kk.z < mj ? 1 : 0) +
-                    (kk.w < mj ? 1 : 0);
-        }
-        for (int f = full; f < nt; ++f)
-            rank += s_key[f] < mj ? 1 : 0;
+    auto below = [](const int4 &kk, int mj) {
+        return (kk.x < mj ? 1 : 0) + (kk.y < mj ? 1 : 0) + (kk.z < mj ? 1 : 0) +
+               (kk.w < mj ? 1 : 0);
+    };
+    auto place = [&](int t, int mj, int rank) {
         st.j[sb + rank] = mj;
         st.m[sb + rank] = s_msk[t];
+    };
+    for (int t = lane, left = nt; left > 0; t += 2 * kWave, left -= 2 * kWave) {
+        const int t1 = t + kWave;
+        const int j0 = t < nt ? s_key[t] : INT_MIN, j1 = t1 < nt ? s_key[t1] : INT_MIN;
+        int r0 = 0, r1 = 0;
+        if (left <= kWave) {
+            for (int f = 0; f < (nt + 3) / 4; ++f)
+                r0 += below(k4[f], j0);
+        } else {
+            for (int f = 0; f < (nt + 3) / 4; ++f) {
+                const int4 kk = k4[f];
+                r0 += below(kk, j0);
+                r1 += below(kk, j1);
+            }
+        }
+        if (t < nt)
+            place(t, j0, r0);
+        if (t1 < nt)
+            place(t1, j1, r1);
     }
-    nz = wave_sum(nz);
+    nz = last_lane(wave_inclusive_scan(nz));
     if (lane == 0) {
         row_level[row] = nt > 0 ? kLevelLds : kLevelEmpty;
         row_tiles[row] = nt;
@@ -427,7 +447,7 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
 {
     __shared__ __align__(16) int s_key[kSymSlots];
     __shared__ unsigned long long s_msk[kSymSlots];
-    __shared__ unsigned long long s_spread[4][kChunk];
+    __shared__ uint4 s_lo[kChunk], s_hi[kChunk];   // spread_tile of the chunk's tiles
     __shared__ int s_b0[kChunk];
     __shared__ int s_pre[kChunk];
     __shared__ unsigned char s_seg[kSeg];
@@ -452,9 +472,7 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
             const int4 br = g.a_brange[c0 + tid];
             nb = br.z;
             s_b0[tid] = br.x;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                s_spread[k][tid] = rows_to_bytes(byte_of(ab, k));
+            spread_tile(ab, &s_lo[tid], &s_hi[tid]);
         }
         int total = 0;
         const int pre = block_exclusive_scan<kWavesPerBlock>(nb, s_tmp, &total);
@@ -484,12 +502,8 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
                 for (int u = 0; u < kSymBatch; ++u) {
                     if (ai[u] < 0)
                         continue;
-                    const uint32_t bb = static_cast<uint32_t>(bm[u].z);
-                    uint64_t pm = 0;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        pm |= s_spread[k][ai[u]] &
-                              (static_cast<uint64_t>(byte_of(bb, k)) * 0x0101010101010101ull);
+                    const uint64_t pm = spread_product(s_lo[ai[u]], s_hi[ai[u]],
+                                                       static_cast<uint32_t>(bm[u].z));
                     if (!pm)
                         continue;
                     const int j = bm[u].x;
@@ -701,7 +715,7 @@ __global__ __launch_bounds__(kThreads) void symbolic_write_kernel(
                 }
             }
         }
-        carry += __shfl(incl, kWave - 1, kWave);
+        carry += last_lane(incl);
     }
     if (staged) {
         wave_sync();

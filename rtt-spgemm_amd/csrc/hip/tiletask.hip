@@ -695,7 +695,7 @@ __device__ __forceinline__ unsigned long long tile_row(const TileTask &g,
                 nb = br.z;
             }
             const int incl = wave_inclusive_scan(nb);
-            const int total = __shfl(incl, kWave - 1, kWave);
+            const int total = last_lane(incl);
             s.start[lane] = incl - nb;
             s.b0[lane] = b0 - (incl - nb);
             s.word[lane] = 0ull;
@@ -740,7 +740,7 @@ __device__ __forceinline__ unsigned long long tile_row(const TileTask &g,
             const unsigned long long word = whole ? s.word[lane] : 0ull;
             const int cnt = __popcll(word);
             const int pi = wave_inclusive_scan(cnt);
-            const int pairs = __shfl(pi, kWave - 1, kWave);
+            const int pairs = last_lane(pi);
             s.word[lane] = word;
             s.base[lane] = pi - cnt;
             wave_sync();
