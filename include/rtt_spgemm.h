@@ -362,7 +362,7 @@ enum rtt_numeric_path {
  * relative to the largest exponent of its tile row over a batch of at most
  * eight pairs of one C tile, into eight exact 8-bit slices (B entries
  * likewise per tile column); all 64 slice products of a pair run on
- * v_mfma_f32_16x16x32_bf16 with exact FP32 sums (eight instructions per
+ * v_mfma_f32_16x16x32_bf16 with exact FP32 sums (four instructions per
  * pair), and the slice sums are recombined and accumulated in FP64 on the
  * GPU.  Each entry keeps 64 bits below its row (column) maximum, so
  * |c - c*| <= 2^-62 sum_k (max_row|a| |b_kj| + |a_ik| max_col|b|) plus FP64
@@ -415,7 +415,7 @@ typedef struct rtt_stats {       /* DmmaSpGemmStats subset */
                                           when a C tile can reach the tail queue) */
     unsigned long long mfma_pairs;     /* TILE: tile pairs multiplied: one FP64 MFMA
                                           (4 blocks x 4x4x4, 512 flops) each, or for
-                                          SPLIT_BF16 eight BF16 16x16x32 MFMAs */
+                                          SPLIT_BF16 four BF16 16x16x32 MFMAs */
     int precision;                     /* enum rtt_precision that ran */
     int tail_reason;                   /* TILE, adaptive-tail: tail gate decision --
                                           1 split, 4 no heavy tile, 5 record capacity

@@ -188,7 +188,6 @@ struct Fp64Product {
     struct Acc {
         double v = 0.0;
     };
-    static constexpr unsigned long long kMfmaPerPair = 1;
     // Waves per SIMD the tile kernel is compiled for: its waves wait 64 % of
     // their time for memory and its vector units are busy 53 %, and 4 waves
     // (at most 128 VGPRs) ran it 20 % faster than the 3 the compiler picks
@@ -331,11 +330,19 @@ struct Fp64Product {
 //   P_d[r][c] = sum_{k, e+f=d} qa_e[r][k] qb_f[k][c]
 // have at most 8 x 4 terms of at most 255^2 per pair, so eight pairs' sums
 // stay below 2^24 and the FP32 accumulation of v_mfma_f32_16x16x32_bf16 is
-// exact.  The reduction dimension of one instruction is 32 = (k, slice e):
-// lane group k holds the eight slices of a(r, k); B supplies, for output
-// column c + 8h, the slices qb_{d-e} with d = 2t + h, so instruction t gives
-// P_{2t} and P_{2t+1} side by side (rows 8..15 of the 16x16 output are
-// unused).  Each batch is then recombined in FP64 on the GPU,
+// exact.  The reduction dimension of one instruction is 32 = (k, slot x):
+// lane group k holds eight slots of a(r, k), and B has in slot x of output
+// column c + 8h the slice qb_{D-x} (zero outside 0..7), D = 3 + 2t + h.  Row r
+// of the A operand has qa_x in slot x, which gives P_D; row r + 8 has
+// qa_{x-4} for t = 0, 1, which gives P_{D-4}, and qa_{x+4} for t = 2, 3, which
+// gives P_{D+4} (the slices those shifts push out meet no slice of B).  So
+// four instructions give every P_d, -1..14, once, P_{-1} = 0.  With the
+// slices unshifted and rows 8..15 empty it took eight, with twice the
+// registers (two waves per SIMD) and FP64 work for the sums, four outputs in
+// a quarter of the lanes instead of one in each, and fractions by 64-bit
+// shifts: 772 vector instructions a C tile of 3.2 pairs.  Block-FEM 50k, 2.15e6
+// pairs: 1.31 -> 0.70 ms.
+// Each batch is recombined in FP64 on the GPU,
 //   C[r][c] += 2^(E_r + E_c) sum_d P_d 2^(-8(d+2)),
 // and batches and C tiles accumulate in FP64.  The only approximation is the
 // truncation of every operand 64 bits below its row (column) maximum, a
@@ -354,88 +361,92 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitBatch = 8;   // pairs whose slice sums stay exact in FP32
 
-// Biased exponent of |x| for alignment (subnormals count as 1, zero as 0).
-__device__ __forceinline__ int align_exp(double x)
-{
-    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
-    const int ex = static_cast<int>((b >> 52) & 0x7FF);
-    return ex ? ex : ((b << 1) ? 1 : 0);
-}
-
-// 64-bit fixed-point fraction of |x| / 2^(emax - 1022) (emax >= align_exp(x),
-// emax >= 1): floor(|x| 2^(64 - (emax - 1022))).
-__device__ __forceinline__ unsigned long long fixed_fraction(double x, int emax)
-{
-    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
-    int ex = static_cast<int>((b >> 52) & 0x7FF);
-    unsigned long long m = b & ((1ull << 52) - 1ull);
-    if (ex)
-        m |= 1ull << 52;
-    else
-        ex = 1;
-    const int sh = ex - emax + 11;   // |x| = m 2^(ex - 1075)
-    if (sh >= 0)
-        return m << sh;
-    return sh > -64 ? (m >> -sh) : 0ull;
-}
-
-// BF16 bits of the integer byte (0..255) of v at byte position `byte`.
-__device__ __forceinline__ uint32_t byte_bf16(uint32_t v, int byte)
-{
-    return __float_as_uint(static_cast<float>((v >> (8 * byte)) & 0xFFu)) >> 16;
-}
-
 // A batch whose A row (B column) exponents span more than this many binades
 // is multiplied on the FP64 matrix cores instead: its smallest entries would
 // keep fewer than 64 - 1 - kSpreadBits = 43 bits of the slices.
 constexpr int kSpreadBits = 20;
 
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// Biased exponent of x in the low half (subnormals count as 1), and 0x7FF
+// minus it in the high half, zeros for a zero: the larger of each gives both
+// extremes.
+__device__ __forceinline__ u16x2 extremes(double x)
+{
+    const uint32_t hi = static_cast<uint32_t>(__double2hiint(x));
+    const int e = max(static_cast<int>((hi >> 20) & 0x7FFu), 1);
+    const uint32_t w = x != 0.0 ? static_cast<uint32_t>((0x7FF << 16) - __mul24(e, 0xFFFF)) : 0u;
+    return __builtin_bit_cast(u16x2, w);
+}
+
+// 64-bit fixed-point fraction of |x| / 2^(emax - 1022), floor(|x| 2^(64 -
+// (emax - 1022))), high word in y.  emax is at least x's exponent and, unless
+// x is zero, at most kSpreadBits above it.
+__device__ __forceinline__ uint2 fixed_fraction(double x, int emax)
+{
+    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
+    const uint32_t hi = static_cast<uint32_t>(b >> 32), lo = static_cast<uint32_t>(b);
+    const uint32_t ex = (hi >> 20) & 0x7FFu;
+    const uint32_t mh = (hi & 0xFFFFFu) | (min(ex, 1u) << 20);   // |x| = {mh, lo} 2^(ex - 1075)
+    const uint32_t d = static_cast<uint32_t>(emax) - max(ex, 1u);
+    const uint32_t h1 = __builtin_amdgcn_alignbit(mh, lo, 32 - 11);
+    return make_uint2(__builtin_amdgcn_alignbit(h1, lo << 11, d), h1 >> (d & 31u));
+}
+
+// Slices (bytes) i of x and j of y, the first in the low half.
+__device__ __forceinline__ uint32_t slices(uint32_t x, int i, uint32_t y, int j)
+{
+    const uint32_t fx = __float_as_uint(static_cast<float>((x >> (8 * i)) & 0xFFu));
+    const uint32_t fy = __float_as_uint(static_cast<float>((y >> (8 * j)) & 0xFFu));
+    return __builtin_amdgcn_perm(fy, fx, 0x07060302u);
+}
+
+
 struct SplitProduct {
     struct Lane {
-        int a_phys;      // A tile bit this lane supplies (rows 0..7 only)
-        bool a_live;     // lane's A row < 8
+        int a_phys;      // A tile bit this lane supplies
+        bool high;       // its A operand row is 8..15: shifted slices
         int b_phys;      // B tile bit
-        int h;           // output column half: d = 2t + h
-        int out_row0;    // first of the four C rows this lane's outputs cover
-        int out_col;     // C column of this lane's outputs
-        bool out_live;   // lane holds C outputs (rows 0..7, h = 0) after the halves combine
+        int h;           // output column half: D = 3 + 2t + h
+        uint32_t b_low, b_mid, b_top;   // byte selectors: B's slices, one byte up for h = 1
+        int c_bit;       // C tile bit of this lane's output
+        int d0;          // d of its sums at t = 0, 1 (2 apart); d2: at t = 2, 3
+        int d2;
         LaneRoles f64;   // roles in the FP64 fallback (v_mfma_f64_4x4x4f64)
-        int f64_lane[4]; // lane whose FP64 entry is this lane's output v
+        int f64_lane;    // lane whose FP64 entry is this lane's output
         __device__ Lane(int lane) : f64(lane)
         {
             const int i = lane & 15, k = lane >> 4;
-            a_live = i < 8;
+            high = i >= 8;
             a_phys = (i & 7) * 4 + k;
             b_phys = (lane & 7) * 4 + k;
             h = (lane >> 3) & 1;
-            out_row0 = 4 * (lane >> 4);
-            out_col = lane & 7;
-            out_live = lane < 32 && h == 0;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = (out_row0 + v) & 7, c = out_col;
-                const int b = ((r >> 2) << 1) | (c >> 2);
-                f64_lane[v] = (c & 3) + 4 * b + 16 * (r & 3);
-            }
+            b_low = h ? 0x0201000Cu : 0x03020100u;
+            b_mid = h ? 0x06050403u : 0x07060504u;
+            b_top = h ? 0x0C0C0C07u : 0x0C0C0C0Cu;
+            // Outputs before the lanes' sums are shared out: rows 4 (k & 1) +
+            // 0..3, those of the A operand's rows 8..15 for k >= 2.
+            d0 = (k < 2 ? 3 : -1) + h;
+            d2 = (k < 2 ? 7 : 11) + h;
+            const int r = 4 * (k & 1) + (k & 2) + h, c = lane & 7;
+            c_bit = r * 8 + c;
+            f64_lane = (c & 3) + 4 * (((r >> 2) << 1) | (c >> 2)) + 16 * (r & 3);
         }
     };
     struct Acc {
-        double v[4] = {0.0, 0.0, 0.0, 0.0};
+        double v = 0.0;
         double f64 = 0.0;   // FP64-fallback partial, v_mfma_f64_4x4x4f64 layout
     };
-    static constexpr unsigned long long kMfmaPerPair = 8;
-    // No register cap: held to 4 waves per SIMD this product spills about 240
-    // VGPRs to scratch, and that build gave wrong values; unconstrained it
-    // needs about 207 VGPRs (2 waves) and spills nothing.
-    static constexpr int kOccupancy = 1;
+    // 144 VGPRs, three waves per SIMD; held to four it spills 30 of them for 5 %.
+    // Loading the next batch's B entries before the current one is worked on
+    // was no faster: vector instructions take 80 % of its cycles.
+    static constexpr int kOccupancy = 3;
 
-    // Lane's four outputs with the FP64-fallback partials added (every lane
-    // takes part in the shuffles).
-    __device__ static void finish(const Lane &ln, const Acc &acc, double out[4])
+    // Lane's output with the FP64-fallback partial added (every lane takes part
+    // in the shuffle).
+    __device__ static double finish(const Lane &ln, const Acc &acc)
     {
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            out[v] = acc.v[v] + __shfl(acc.f64, ln.f64_lane[v], kWave);
+        return acc.v + __shfl(acc.f64, ln.f64_lane, kWave);
     }
 
     __device__ static void store(const TileTask &g, const Lane &ln, int c_local,
@@ -443,34 +454,55 @@ struct SplitProduct {
     {
         const unsigned long long m = read_lane64(cm, c_local);
         const long long off = static_cast<long long>(read_lane64(static_cast<unsigned long long>(co), c_local));
-        double out[4];
-        finish(ln, acc, out);
-        if (!ln.out_live)
-            return;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int bit = (ln.out_row0 + v) * 8 + ln.out_col;
-            if ((m >> bit) & 1ull)
-                g.c_val[off + __popcll(m & ((1ull << bit) - 1ull))] = out[v];
-        }
+        const double out = finish(ln, acc);
+        if ((m >> ln.c_bit) & 1ull)
+            g.c_val[off + __popcll(m & ((1ull << ln.c_bit) - 1ull))] = out;
     }
 
     __device__ static void dump(const Lane &ln, const Acc &acc, double *slot64)
     {
-        double out[4];
-        finish(ln, acc, out);
-        if (!ln.out_live)
-            return;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            slot64[(ln.out_row0 + v) * 8 + ln.out_col] = out[v];
+        slot64[ln.c_bit] = finish(ln, acc);
     }
 
-    // Smallest biased exponent of the nonzero entries (0x7FF when none).
-    __device__ static int min_exp(double x)
+    // The larger of each half over the four k of a row (column): lanes x, x +
+    // 16, x + 32, x + 48.
+    __device__ static u16x2 over_k(u16x2 v)
     {
-        const int e = align_exp(x);
-        return e ? e : 0x7FF;
+        const uint32_t w = __builtin_bit_cast(uint32_t, v);
+        const auto r = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+        const u16x2 m = __builtin_elementwise_max(__builtin_bit_cast(u16x2, static_cast<uint32_t>(r[0])),
+                                                  __builtin_bit_cast(u16x2, static_cast<uint32_t>(r[1])));
+        const uint32_t x = __builtin_bit_cast(uint32_t, m);
+        const auto q = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return __builtin_elementwise_max(__builtin_bit_cast(u16x2, static_cast<uint32_t>(q[0])),
+                                         __builtin_bit_cast(u16x2, static_cast<uint32_t>(q[1])));
+    }
+
+    __device__ static bool wide_spread(u16x2 e)
+    {
+        return e.y != 0 && e.x - (0x7FF - e.y) > kSpreadBits;
+    }
+
+    // Lanes below 32: a + a of lane + 32; the others: b + b of lane - 32.
+    __device__ static double halves_sum(double a, double b)
+    {
+        const unsigned long long ua = static_cast<unsigned long long>(__double_as_longlong(a)),
+                                 ub = static_cast<unsigned long long>(__double_as_longlong(b));
+        const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(ua),
+                                                         static_cast<uint32_t>(ub), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(
+            static_cast<uint32_t>(ua >> 32), static_cast<uint32_t>(ub >> 32), false, false);
+        auto word = [](uint32_t h, uint32_t l) {
+            return __longlong_as_double(
+                static_cast<long long>((static_cast<unsigned long long>(h) << 32) | l));
+        };
+        return word(hi[0], lo[0]) + word(hi[1], lo[1]);
+    }
+
+    // 2^(-8 (d + 2))
+    __device__ static double slice_weight(int d)
+    {
+        return __longlong_as_double(static_cast<long long>(1023 - 8 * (d + 2)) << 52);
     }
 
     __device__ static double entry(const double *vals, int mask, int off, int phys, uint32_t zero)
@@ -484,35 +516,25 @@ struct SplitProduct {
                                  uint32_t a_zero, const int4 *pm, int p0, int n, Acc &acc)
     {
         double av[kSplitBatch], bv[kSplitBatch];
-        int ea = 0, eb = 0, ea_lo = 0x7FF, eb_lo = 0x7FF;
 #pragma unroll
         for (int i = 0; i < kSplitBatch; ++i) {
-            av[i] = 0.0;
-            bv[i] = 0.0;
-            if (i < n) {
-                const int4 m = pm[p0 + i];
-                if (ln.a_live)
-                    av[i] = entry(a_vals, m.x, m.y, ln.a_phys, a_zero);
-                bv[i] = entry(g.b_vals, m.z, m.w, ln.b_phys, g.b_zero);
-            }
-            ea = max(ea, align_exp(av[i]));
-            eb = max(eb, align_exp(bv[i]));
-            ea_lo = min(ea_lo, min_exp(av[i]));
-            eb_lo = min(eb_lo, min_exp(bv[i]));
+            if (i >= n)
+                break;
+            const int4 m = pm[p0 + i];
+            av[i] = entry(a_vals, m.x, m.y, ln.a_phys, a_zero);
+            bv[i] = entry(g.b_vals, m.z, m.w, ln.b_phys, g.b_zero);
         }
-        // Row (column) maxima and minima over the four k of the tile: lanes
-        // x, x+16, x+32, x+48 hold one row (column).
-        ea = max(ea, __shfl_xor(ea, 16, kWave));
-        ea = max(ea, __shfl_xor(ea, 32, kWave));
-        eb = max(eb, __shfl_xor(eb, 16, kWave));
-        eb = max(eb, __shfl_xor(eb, 32, kWave));
-        ea_lo = min(ea_lo, __shfl_xor(ea_lo, 16, kWave));
-        ea_lo = min(ea_lo, __shfl_xor(ea_lo, 32, kWave));
-        eb_lo = min(eb_lo, __shfl_xor(eb_lo, 16, kWave));
-        eb_lo = min(eb_lo, __shfl_xor(eb_lo, 32, kWave));
-        const bool wide = (ea_lo != 0x7FF && ea - ea_lo > kSpreadBits) ||
-                          (eb_lo != 0x7FF && eb - eb_lo > kSpreadBits);
-        if (__ballot(wide)) {
+        u16x2 xa = {0, 0}, xb = {0, 0};
+#pragma unroll
+        for (int i = 0; i < kSplitBatch; ++i) {
+            if (i >= n)
+                break;
+            xa = __builtin_elementwise_max(xa, extremes(av[i]));
+            xb = __builtin_elementwise_max(xb, extremes(bv[i]));
+        }
+        xa = over_k(xa);
+        xb = over_k(xb);
+        if (__ballot(wide_spread(xa) || wide_spread(xb))) {
             // Too wide a spread for the slices: these pairs on the FP64 cores.
 #pragma unroll
             for (int i = 0; i < kSplitBatch; ++i) {
@@ -525,95 +547,70 @@ struct SplitProduct {
             }
             return;
         }
-        ea = max(ea, 1);
-        eb = max(eb, 1);
-        f32x4 acc_t[8];
+        const int ea = max(static_cast<int>(xa.x), 1), eb = max(static_cast<int>(xb.x), 1);
+        f32x4 acc_t[4];
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < 4; ++t)
             acc_t[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < kSplitBatch; ++i) {
             if (i >= n)
                 break;
-            // A slices in element order e = 0..7 (most significant first).
-            const unsigned long long fa = fixed_fraction(av[i], ea);
-            const uint32_t ahi = static_cast<uint32_t>(fa >> 32), alo = static_cast<uint32_t>(fa);
+            // A's slices, most significant first, two a word.
+            const uint2 fa = fixed_fraction(av[i], ea);
             const uint32_t asg = av[i] < 0.0 ? 0x80008000u : 0u;
-            u32x4 aw;
-            aw[0] = (byte_bf16(ahi, 3) | (byte_bf16(ahi, 2) << 16)) | asg;
-            aw[1] = (byte_bf16(ahi, 1) | (byte_bf16(ahi, 0) << 16)) | asg;
-            aw[2] = (byte_bf16(alo, 3) | (byte_bf16(alo, 2) << 16)) | asg;
-            aw[3] = (byte_bf16(alo, 1) | (byte_bf16(alo, 0) << 16)) | asg;
-            // B slices q0..q7 laid out so that instruction t reads
-            // qb_{2t+h-e} for element e from words 8-t..11-t.
-            const unsigned long long fb = fixed_fraction(bv[i], eb);
-            const uint32_t bhi = static_cast<uint32_t>(fb >> 32), blo = static_cast<uint32_t>(fb);
+            const uint32_t a0 = slices(fa.y, 3, fa.y, 2) | asg, a1 = slices(fa.y, 1, fa.y, 0) | asg,
+                           a2 = slices(fa.x, 3, fa.x, 2) | asg, a3 = slices(fa.x, 1, fa.x, 0) | asg;
+            const u32x4 up = ln.high ? u32x4{0u, 0u, a0, a1} : u32x4{a0, a1, a2, a3};
+            const u32x4 down = ln.high ? u32x4{a2, a3, 0u, 0u} : u32x4{a0, a1, a2, a3};
+            // B's slices, least significant first (one slot later for h = 1),
+            // two a word: instruction t reads four words from word 3 - t.
+            const uint2 fb = fixed_fraction(bv[i], eb);
+            const uint32_t blo = __builtin_amdgcn_perm(fb.y, fb.x, ln.b_low);
+            const uint32_t bhi = __builtin_amdgcn_perm(fb.y, fb.x, ln.b_mid);
+            const uint32_t last = __builtin_amdgcn_perm(fb.y, fb.x, ln.b_top);
             const uint32_t bsg = bv[i] < 0.0 ? 0x80008000u : 0u;
-            const uint32_t q0 = byte_bf16(bhi, 3), q1 = byte_bf16(bhi, 2), q2 = byte_bf16(bhi, 1),
-                           q3 = byte_bf16(bhi, 0), q4 = byte_bf16(blo, 3), q5 = byte_bf16(blo, 2),
-                           q6 = byte_bf16(blo, 1), q7 = byte_bf16(blo, 0);
-            uint32_t wv[12];
+            const uint32_t w[7] = {0u,
+                                   slices(blo, 0, blo, 1) | bsg,
+                                   slices(blo, 2, blo, 3) | bsg,
+                                   slices(bhi, 0, bhi, 1) | bsg,
+                                   slices(bhi, 2, bhi, 3) | bsg,
+                                   (__float_as_uint(static_cast<float>(last & 0xFFu)) >> 16) | bsg,
+                                   0u};
 #pragma unroll
-            for (int x = 0; x < 12; ++x)
-                wv[x] = 0u;
-            if (ln.h == 0) {
-                wv[4] = (q7 << 16) | bsg;
-                wv[5] = (q6 | (q5 << 16)) | bsg;
-                wv[6] = (q4 | (q3 << 16)) | bsg;
-                wv[7] = (q2 | (q1 << 16)) | bsg;
-                wv[8] = q0 | bsg;
-            } else {
-                wv[5] = (q7 | (q6 << 16)) | bsg;
-                wv[6] = (q5 | (q4 << 16)) | bsg;
-                wv[7] = (q3 | (q2 << 16)) | bsg;
-                wv[8] = (q1 | (q0 << 16)) | bsg;
-            }
-            const bf16x8 aop = __builtin_bit_cast(bf16x8, aw);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                u32x4 bw;
-                bw[0] = wv[8 - t];
-                bw[1] = wv[9 - t];
-                bw[2] = wv[10 - t];
-                bw[3] = wv[11 - t];
+            for (int t = 0; t < 4; ++t) {
+                const u32x4 bw = {w[3 - t], w[4 - t], w[5 - t], w[6 - t]};
                 acc_t[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    aop, __builtin_bit_cast(bf16x8, bw), acc_t[t], 0, 0, 0);
+                    __builtin_bit_cast(bf16x8, t < 2 ? up : down), __builtin_bit_cast(bf16x8, bw),
+                    acc_t[t], 0, 0, 0);
             }
         }
-        // Recombination in FP64: lane's outputs are rows out_row0 + v, column
-        // (lane & 15) -> C column lane & 7 at d = 2t + h.
-        const int lane = lane_id();
-        const int ecol = __shfl(eb, lane & 7, kWave) - 1022;
+        // Recombination in FP64.  A lane has, for four rows, the P_d of d0, d0
+        // + 2, d2 and d2 + 2 of one column; the others' lie in the lanes 8 and
+        // 32 away, so each lane ends with one of the four rows.
+        const double w0 = slice_weight(ln.d0), w1 = slice_weight(ln.d0 + 2),
+                     w2 = slice_weight(ln.d2), w3 = slice_weight(ln.d2 + 2);
+        double sum[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int erow = __shfl(ea, (ln.out_row0 + v) & 7, kWave) - 1022;
-            double sum = 0.0;
-            double w = ln.h ? 0x1p-24 : 0x1p-16;   // 2^(-8(d+2)) at t = 0
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                sum += static_cast<double>(acc_t[t][v]) * w;
-                w *= 0x1p-16;
-            }
-            sum = ldexp(sum, erow + ecol);
-            sum += __shfl_xor(sum, 8, kWave);   // the d = 2t + 1 half
-            acc.v[v] += sum;
-        }
+        for (int v = 0; v < 4; ++v)
+            sum[v] = fma(static_cast<double>(acc_t[0][v]), w0,
+                         fma(static_cast<double>(acc_t[1][v]), w1,
+                             fma(static_cast<double>(acc_t[2][v]), w2,
+                                 static_cast<double>(acc_t[3][v]) * w3)));
+        const double s0 = halves_sum(sum[0], sum[2]), s1 = halves_sum(sum[1], sum[3]);
+        const double out = (ln.h ? s1 : s0) + from_lane_xor8(ln.h ? s0 : s1);
+        const int erow = __shfl(ea, ln.c_bit >> 3, kWave);
+        acc.v += ldexp(out, erow + eb - 2 * 1022);
     }
 
-    // Lane's four outputs of a C tile as store() left them.
+    // Lane's output of a C tile as store() left it.
     __device__ static void load(const TileTask &g, const Lane &ln, int c_local,
                                 unsigned long long cm, long long co, Acc &acc)
     {
         const unsigned long long m = read_lane64(cm, c_local);
         const long long off = static_cast<long long>(read_lane64(static_cast<unsigned long long>(co), c_local));
-        if (!ln.out_live)
-            return;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int bit = (ln.out_row0 + v) * 8 + ln.out_col;
-            if ((m >> bit) & 1ull)
-                acc.v[v] = g.c_val[off + __popcll(m & ((1ull << bit) - 1ull))];
-        }
+        if ((m >> ln.c_bit) & 1ull)
+            acc.v = g.c_val[off + __popcll(m & ((1ull << ln.c_bit) - 1ull))];
     }
 
     static __device__ __forceinline__ void run(const TileTask &g, const Lane &ln, const double *a_vals,
