@@ -25,7 +25,7 @@
 // 64-bit word.  The words give every pair its place: C tiles in order, within
 // one the number of lower bits (its smaller K).  The pairs are written there
 // into an LDS list and run by P::run, which keeps a batch of operand loads in
-// flight behind the products and stores each C tile when its pairs end.
+// flight behind the products and puts each C tile out when its pairs end.
 // Every B tile enumerated belongs to a pair (or to no C tile at all), and B
 // needs no column structure; the search of A's keys for every entry of every
 // B column that this replaces, with the radix sort that made the columns,
@@ -46,11 +46,12 @@ namespace {
 
 constexpr int kTThreads = 128;
 constexpr int kTWaves = kTThreads / kWave;
-constexpr int kAVals = 512;     // A payload values of a row staged in LDS
-constexpr int kPairCap = 192;   // pairs a wave buffers before running them: 9.3 KB of LDS per
-                                // wave lets the 16 waves run that the registers allow
+constexpr int kAVals = 384;     // A payload values of a row staged in LDS
+constexpr int kPairCap = 128;   // pairs a wave buffers before running them
 constexpr int kBatch = 8;       // pairs whose operand loads are issued together
-constexpr int kEnumRounds = 4;  // rounds of 64 B tiles whose metas are loaded together (and
+constexpr int kOutVals = 128;   // C values a wave stages before it stores them
+static_assert(kOutVals >= 64, "a C tile fits the stage");
+constexpr int kEnumRounds = 2;  // rounds of 64 B tiles whose metas are loaded together (and
                                 // kept, when they are all there is)
 constexpr int kXcdChunk = 4;    // workgroups of consecutive units dealt to an XCD at a time
 constexpr int kPairShards = 256;   // counters of the pairs multiplied, a 128-byte line each (one
@@ -59,7 +60,7 @@ constexpr int kMaxParts = 4;    // most units a tile row is cut into
 constexpr int kPairWords = kPairCap / 64;
 constexpr int kPad = 2 * kBatch;   // pairs of zeros past a list: the batch that its last pairs
                                    // share, and the batch loaded ahead of that one
-static_assert(kPairCap % 64 == 0 && kPairWords == 3, "words of the end bits");
+static_assert(kPairCap % 64 == 0 && kPairWords == 2, "words of the end bits");
 static_assert(kPairCap >= kWave, "a C tile has at most 64 pairs per group of A tiles");
 
 struct TileTask {
@@ -188,28 +189,54 @@ struct Fp64Product {
     struct Acc {
         double v = 0.0;
     };
-    // Waves per SIMD the tile kernel is compiled for: its waves wait 64 % of
-    // their time for memory and its vector units are busy 53 %, and 4 waves
-    // (at most 128 VGPRs) ran it 20 % faster than the 3 the compiler picks
-    // unconstrained.  Block-FEM 500k: 2.18 ms for 2.16e7 pairs (5.1 TFLOP/s
-    // on the matrix cores), 2.95 ms with the column search, 2.51 ms before
-    // the list took dense masks and zero slots (31 vector instructions a
-    // pair, 46 before).
-    static constexpr int kOccupancy = 4;
+    // Waves per SIMD the tile kernel is compiled for (94 VGPRs) and its LDS is
+    // cut to: its waves wait for loads more than half of their time.  Block-FEM
+    // 500k, 2.16e7 pairs: 1.69 ms (6.5 TFLOP/s on the matrix cores); 1.80 at
+    // four waves with 512 A values staged and four enumeration rounds kept,
+    // 1.90 with twice the output stage, 1.89 at six waves, batches of four and
+    // spills; 2.17 before the output was staged, 2.95 with the search of B's
+    // columns.  B tiles loaded whole and spread by lane permutes, a third of
+    // the cache accesses, were slower (2.01 against 1.90).
+    static constexpr int kOccupancy = 5;
 
-    __device__ static void store(const TileTask &g, const Lane &ln, int c_local,
-                                 unsigned long long cm, long long co, const Acc &acc)
+    // C values on their way out: `count` values from `base` on wait in `vals`.
+    // The C tiles of a row lie one behind the other, so they leave together,
+    // in whole lines.  Stored tile by tile, every batch waited for the stores
+    // of the one before: loads and stores come back in one order, and a wait
+    // for operands cannot tell how many stores are behind them (8000 cycles a
+    // batch of eight pairs): block-FEM 500k 2.17 -> 1.80 ms.
+    struct Out {
+        double *vals;
+        long long base;
+        int count;
+    };
+    static __device__ __forceinline__ void flush(const TileTask &g, Out &out)
+    {
+        wave_sync();
+        for (int i = lane_id(); i < out.count; i += kWave)
+            g.c_val[out.base + i] = out.vals[i];
+        wave_sync();
+        out.count = 0;
+    }
+
+    static __device__ __forceinline__ void put(const TileTask &g, const Lane &ln, int c_local,
+                                               unsigned long long cm, long long co, const Acc &acc,
+                                               Out &out)
     {
         const unsigned long long m = read_lane64(cm, c_local);
         const long long off = static_cast<long long>(read_lane64(static_cast<unsigned long long>(co), c_local));
+        const int n = __popcll(m);
+        if (off != out.base + out.count || out.count + n > kOutVals) {
+            flush(g, out);
+            out.base = off;
+        }
         const int bit = ln.roles.c_bit;
-        if (m == ~0ull)   // a full tile, the same in every lane
-            g.c_val[off + bit] = acc.v;
-        else if ((m >> bit) & 1ull)
-            g.c_val[off + __popcll(m & ((1ull << bit) - 1ull))] = acc.v;
+        if ((m >> bit) & 1ull)
+            out.vals[out.count + __popcll(m & ((1ull << bit) - 1ull))] = acc.v;
+        out.count += n;
     }
 
-    // Lane's entry of a C tile as store() left it.
+    // Lane's entry of a C tile stored earlier.
     __device__ static double load(const TileTask &g, const Lane &ln, int c_local,
                                   unsigned long long cm, long long co)
     {
@@ -278,7 +305,7 @@ struct Fp64Product {
         }
     }
 
-    // Runs a list of whole C tiles in order, storing each after its last pair.
+    // Runs a list of whole C tiles in order, putting each out after its last pair.
     // cnt: pairs of the lane's C tile; ends: bit p set when a tile ends with
     // pair p (all of them in scalar registers, off the vector units); live:
     // the listed tiles.  A C tile in `started` has its sum over earlier A
@@ -287,9 +314,10 @@ struct Fp64Product {
                                uint32_t a_zero, const int4 *pm, int n, int,
                                const unsigned long long (&ends)[kPairWords],
                                unsigned long long live, unsigned long long started,
-                               unsigned long long cm, long long co)
+                               unsigned long long cm, long long co, double *out_vals)
     {
         Acc acc;
+        Out out = {out_vals, 0, 0};
         auto begin = [&]() {
             const int t = __builtin_ctzll(live);
             acc.v = (started >> t) & 1ull ? load(g, ln, t, cm, co) : 0.0;
@@ -299,15 +327,16 @@ struct Fp64Product {
         unsigned long long word = 0;
         products(g, ln, a_vals, a_zero, pm, n, acc, [&](int p0, int i) {
             if (i == 0)
-                word = (p0 < 64 ? ends[0] : (p0 < 128 ? ends[1] : ends[2])) >> (p0 & 63);
+                word = (p0 < 64 ? ends[0] : ends[1]) >> (p0 & 63);
             if ((word >> i) & 1ull) {
-                store(g, ln, __builtin_ctzll(live), cm, co, acc);
+                put(g, ln, __builtin_ctzll(live), cm, co, acc, out);
                 live &= live - 1;
                 acc.v = 0.0;
                 if (started && live)
                     begin();
             }
         });
+        flush(g, out);
     }
 
     // Adds listed pairs [0, n) to acc.
@@ -616,7 +645,8 @@ struct SplitProduct {
     static __device__ __forceinline__ void run(const TileTask &g, const Lane &ln, const double *a_vals,
                                uint32_t a_zero, const int4 *pm, int, int cnt,
                                const unsigned long long (&)[kPairWords], unsigned long long live,
-                               unsigned long long started, unsigned long long cm, long long co)
+                               unsigned long long started, unsigned long long cm, long long co,
+                               double *)
     {
         for (int p = 0; live; live &= live - 1) {
             const int t = __builtin_ctzll(live);
@@ -643,6 +673,7 @@ struct SplitProduct {
 struct WaveStage {
     double av[kAVals + 2];            // A row's payload, when it fits; then 0.0
     int4 pm[kPairCap + kPad];         // {A mask, A offset, B mask, B offset}
+    double out[kOutVals];             // C values on their way out
     unsigned long long word[kWave];   // per C tile: its A tiles
     unsigned long long ends[kPairWords + 1];   // bit p: a C tile ends with pair p
     int2 am[kWave];                   // per A tile: {mask, offset}
@@ -776,12 +807,16 @@ __device__ __forceinline__ unsigned long long tile_row(const TileTask &g,
 #pragma unroll
                 for (int i = 0; i < kPairWords; ++i)
                     ends[i] = read_lane64(s.ends[i], 0);
-                P::run(g, ln, a_vals, a_zero, s.pm, hi - lo, cnt, ends, live, started, cm, co);
+                P::run(g, ln, a_vals, a_zero, s.pm, hi - lo, cnt, ends, live, started, cm, co, s.out);
                 lo = hi;
                 wave_sync();
             }
             done += static_cast<unsigned long long>(pairs);
             started |= __ballot(cnt > 0);
+            if (ag + kWave < na) {
+                // Other lanes than those that stored them may load the sums.
+                __threadfence_block();
+            }
             wave_sync();
         }
         wave_sync();

@@ -36,6 +36,7 @@ CASES = {
     "many pairs": ([60] * 5, 260, 40, 320),
     "one row": ([17], 80, 9, 100),
     "sparse tiles": ([30, 70, 3, 11, 50], 320, 12, 700),
+    "whole tiles at the A stage's edge": ([11, 12, 13, 2, 4], 60, 8, 90),
 }
 
 
@@ -43,7 +44,7 @@ CASES = {
 @pytest.mark.parametrize("name", list(CASES))
 def test_lists(gpu, name, precision):
     per_row, k, per_b, n = CASES[name]
-    fill = 0.4 if name == "sparse tiles" else 0.97
+    fill = 0.4 if name == "sparse tiles" else 1.0 if name.startswith("whole") else 0.97
     m = 8 * len(per_row) - 2
     a = blocks(m, k, per_row, 3, fill)
     b = gpu.gen_random(k, n, per_b, 5)
