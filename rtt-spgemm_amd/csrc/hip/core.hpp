@@ -29,19 +29,27 @@ __device__ __forceinline__ uint64_t packed_row_offsets(uint64_t m)
     return (x * 0x0101010101010101ull) << 8;
 }
 
+// C tile t's structure; put takes its entries' local columns in order.
+template <class Put>
 __device__ __forceinline__ void write_tile_structure(const COut &c, int64_t t, int j,
-                                                     uint64_t m, int64_t off)
+                                                     uint64_t m, int64_t off, Put &&put)
 {
     c.col[t] = j;
     c.mask[t] = m;
     c.tile_nnz[t] = off;
     reinterpret_cast<uint64_t *>(c.csr_ptr)[t] = packed_row_offsets(m);
-    int i = 0;
     while (m) {
         const int pos = __builtin_ctzll(m);
         m &= m - 1;
-        c.csr_col[off + i++] = static_cast<uint8_t>(pos & 7);
+        put(static_cast<uint8_t>(pos & 7));
     }
+}
+
+__device__ __forceinline__ void write_tile_structure(const COut &c, int64_t t, int j,
+                                                     uint64_t m, int64_t off)
+{
+    uint8_t *bytes = c.csr_col + off;
+    write_tile_structure(c, t, j, m, off, [&](uint8_t col) { *bytes++ = col; });
 }
 
 // Exclusive scans of two values over a workgroup of NW waves with one

@@ -10,7 +10,7 @@
 // columns ascending, from its tiles (rebuilt by every call that has such
 // rows).  A workgroup owns one tile row of C, or a part of it, at a time.  A thread owns one
 // slot of the row's A payload, with a cursor into the B row it selects, for
-// chunks of kSlabThreads slots.
+// chunks of as many slots as the workgroup has threads.
 //
 // The row is walked in windows of C columns.  In a window, every thread
 // gallops its cursor to the window's end; the products are numbered by a
@@ -19,15 +19,21 @@
 // Consecutive lanes so take consecutive entries of a B row.
 //  * symbolic: the window's C tile masks are ORed in LDS, then counted and
 //    appended to the staged lists, or written to C's structure.
-//  * numeric: the window's C tiles (masks and first values) lie in LDS
-//    directly mapped by column, and their values accumulate in LDS in C's
-//    order, to be stored once, whatever the number of A entries.
+//  * numeric: the window's C tiles (masks and first values) lie in LDS, found
+//    by a bit per tile column and a count of those before each word, and their
+//    values accumulate in LDS in C's order, to be stored once, whatever the
+//    number of A entries.
 //
 // On R-MAT 2^18 (2.9e9 products, a pair of tiles carries 1.3) the count takes
-// 8.0 ms and the numeric pass 23.8 ms, at about 4 TB/s of L2 fetches: short
-// pieces of B rows, of which the L2s reuse little.  Tile by tile, with a binary
-// search over 1280 runs and a 16-byte table entry from HBM per pair, they took
-// 35 and 108 ms, waiting on dependent loads.
+// 7.7 ms and the numeric pass 16.9 ms, waiting for short pieces of B rows, of
+// which the L2s reuse little: the wider the window, the longer the pieces.
+// With tables directly mapped by column, 2048 tile columns and 4096 values a
+// window, and two workgroups of 512 threads on a CU it took 23.8 ms (twice the
+// L2 reads); mapped tables of 4096 columns for one workgroup of 1024 took 19.6.
+// Searching a cursor's next stop by eight probes at a time was slower (18.8).
+// Tile by tile, with a binary search over 1280 runs and a 16-byte table entry
+// from HBM per pair, the two passes took 35 and 108 ms, waiting on dependent
+// loads.
 #include <algorithm>
 #include <climits>
 
@@ -37,17 +43,23 @@ namespace rtt {
 
 namespace {
 
-constexpr int kSlabThreads = 512;
-constexpr int kSlabWaves = kSlabThreads / kWave;
+constexpr int kSymThreads = 512;               // symbolic pass: two workgroups fit a CU
+constexpr int kNumThreads = 1024;              // numeric pass: one, with all of its LDS
 constexpr int kSubProducts = 16384;            // products numbered by the bit words at once
 constexpr int kSubWords = kSubProducts / 64;
 constexpr int kSymWin = 8192;                  // C tile columns of a symbolic window
-constexpr int kNumCols = 2048;                 // C tile columns of a numeric window
-constexpr int kNumVals = 4096;                 // C values of a numeric window
-constexpr int kNumTiles = kNumCols / kSlabThreads;   // C tiles a thread looks at per window
+constexpr int kFillBytes = 8192;               // column bytes of C staged at a time
+constexpr int kNumSpan = 32768;                // C tile columns a numeric window may span,
+constexpr int kNumTiles = 3072;                // C tiles it may hold,
+constexpr int kNumVals = 13312;                // and C values
+constexpr int kNumWords = kNumSpan / 64;
+constexpr int kLookTiles = kNumTiles / kNumThreads;   // C tiles a thread looks at per window
 constexpr int kUnroll = 4;                     // products a thread loads together
 static_assert(kSubWords <= 4 * kWave, "one wave ranks the bit words");
-static_assert(kNumVals <= 65536 - 64, "16-bit value positions");
+static_assert(kNumVals <= 65536 - 64 && kNumTiles <= 65536, "16-bit value and tile positions");
+static_assert(kNumTiles % kNumThreads == 0 && kNumWords % kWave == 0 &&
+                  kNumWords / kWave * kWave <= kNumThreads,
+              "shares of a window's tables");
 
 // Column (-1: an absent slot of a dense tile) and row of every slot of A's
 // payload; a thread per tile.
@@ -184,6 +196,7 @@ struct Task {
 // are quantiles of the longest B row it selects: hub columns hold most of a
 // power-law row's products, and equal stretches of columns would leave most
 // of them in the first part.
+template <int T>
 __device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_task,
                                           unsigned long long *s_long, Task *t)
 {
@@ -216,7 +229,7 @@ __device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_tas
         // {entries, slot from the end}: the longest, the first of equals.
         unsigned long long best = 0;
         const int s0 = o.a_row_off[t->row], s1 = o.a_row_off[t->row + 1];
-        for (int x = s0 + static_cast<int>(threadIdx.x); x < s1; x += kSlabThreads) {
+        for (int x = s0 + static_cast<int>(threadIdx.x); x < s1; x += T) {
             const int k = o.a_k[x];
             if (k < 0)
                 continue;
@@ -305,25 +318,26 @@ __device__ __forceinline__ void lds_min(int *at, int v)
 
 // A window's runs in LDS: run i (one per thread with products) covers the
 // products from s_pre on, entry = pw + product.
+template <int T>
 struct Runs {
-    int pw[kSlabThreads];
-    uint8_t r[kSlabThreads];
+    int pw[T];
+    uint8_t r[T];
     unsigned long long bits[kSubWords];   // bit p: a run begins with product p
     int rank[kSubWords];                  // runs that begin before the word
-    int scan[2 * kSlabWaves];
+    int scan[2 * (T / kWave)];
 };
 
 // The products of the workgroup's threads, cnt each from entry `first` of B
 // on.  stage(i) stores the thread's operands as those of run i; load(e)
 // fetches what product needs of B's entry e, use(i, x) consumes it.  Every
 // thread calls it; it ends with a barrier.
-template <class X, class StageF, class LoadF, class UseF>
-__device__ __forceinline__ void for_products(Runs &s, int cnt, int first, int r, StageF &&stage,
+template <class X, int T, class StageF, class LoadF, class UseF>
+__device__ __forceinline__ void for_products(Runs<T> &s, int cnt, int first, int r, StageF &&stage,
                                              LoadF &&load, UseF &&use)
 {
     const int tid = threadIdx.x;
     int pre, run, total, nrun;
-    dual_exclusive_scan<kSlabWaves>(cnt, cnt > 0 ? 1 : 0, s.scan, &pre, &run, &total, &nrun);
+    dual_exclusive_scan<T / kWave>(cnt, cnt > 0 ? 1 : 0, s.scan, &pre, &run, &total, &nrun);
     if (cnt > 0) {
         s.pw[run] = first - pre;
         s.r[run] = static_cast<uint8_t>(r);
@@ -354,12 +368,12 @@ __device__ __forceinline__ void for_products(Runs &s, int cnt, int first, int r,
         }
         __syncthreads();
         const int n = min(total - q0, kSubProducts);
-        for (int p0 = tid; p0 < n; p0 += kUnroll * kSlabThreads) {
+        for (int p0 = tid; p0 < n; p0 += kUnroll * T) {
             X x[kUnroll];
             int id[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
-                const int p = p0 + u * kSlabThreads;
+                const int p = p0 + u * T;
                 id[u] = -1;
                 if (p < n) {
                     // The run that begins last at or before p.
@@ -397,24 +411,25 @@ struct SlabStage {
 };
 
 template <bool FILL>
-__global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps o,
+__global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o,
                                                                      int64_t *__restrict__ row_tiles,
                                                                      int64_t *__restrict__ row_nnz,
                                                                      SlabStage ss, COut c)
 {
     __shared__ unsigned long long s_wm[kSymWin];
-    __shared__ Runs s;
+    __shared__ Runs<kSymThreads> s;
     __shared__ int s_min[2];
     __shared__ long long s_base;
     __shared__ int s_task[4];
     __shared__ unsigned long long s_long;
+    __shared__ __align__(4) unsigned char s_bytes[FILL ? kFillBytes + 4 : 4];
     const int tid = threadIdx.x;
-    constexpr int kPer = kSymWin / kSlabThreads;
-    for (int i = tid; i < kSymWin; i += kSlabThreads)
+    constexpr int kPer = kSymWin / kSymThreads;
+    for (int i = tid; i < kSymWin; i += kSymThreads)
         s_wm[i] = 0ull;
     for (int step = 0;; ++step) {
         Task task;
-        if (!next_task(o, step, s_task, &s_long, &task))
+        if (!next_task<kSymThreads>(o, step, s_task, &s_long, &task))
             break;
         const int row = task.row;
         int64_t tb = 0, zb = 0;
@@ -429,7 +444,7 @@ __global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps 
             if (seg >= 0) {
                 while (seg >= 0) {
                     const int n = ss.j[seg];
-                    for (int q0 = 0; q0 < n; q0 += kSlabThreads) {
+                    for (int q0 = 0; q0 < n; q0 += kSymThreads) {
                         const int q = q0 + tid;
                         unsigned long long m = 0;
                         int j = 0;
@@ -438,9 +453,34 @@ __global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps 
                             m = ss.m[seg + 1 + q];
                         }
                         int npc = 0;
-                        const int zpos = block_exclusive_scan<kSlabWaves>(__popcll(m), s.scan, &npc);
-                        if (q < n)
-                            write_tile_structure(c, tb + q, j, m, zb + zpos);
+                        const int zpos = block_exclusive_scan<kSymThreads / kWave>(__popcll(m), s.scan, &npc);
+                        // The tiles' column bytes lie one behind the other:
+                        // through LDS they go out a word at a time.  A lane
+                        // writing its own tile's to memory byte by byte took
+                        // 4.7 ms on R-MAT 2^18; now 4.1.
+                        const bool stage = npc <= kFillBytes;
+                        const int shift = static_cast<int>(zb & 3);
+                        if (q < n) {
+                            int at = shift + zpos;
+                            if (stage)
+                                write_tile_structure(c, tb + q, j, m, zb + zpos,
+                                                     [&](uint8_t col) { s_bytes[at++] = col; });
+                            else
+                                write_tile_structure(c, tb + q, j, m, zb + zpos);
+                        }
+                        if (stage) {
+                            __syncthreads();
+                            unsigned char *to = c.csr_col + (zb - shift);
+                            for (int i = tid; i < (shift + npc + 3) >> 2; i += kSymThreads) {
+                                const uint32_t v = reinterpret_cast<const uint32_t *>(s_bytes)[i];
+                                if (4 * i >= shift && 4 * i + 4 <= shift + npc) {
+                                    reinterpret_cast<uint32_t *>(to)[i] = v;
+                                    continue;
+                                }
+                                for (int x = max(4 * i, shift); x < min(4 * i + 4, shift + npc); ++x)
+                                    to[x] = s_bytes[x];
+                            }
+                        }
                         zb += npc;
                     }
                     tb += n;
@@ -450,13 +490,13 @@ __global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps 
             }
         }
         const int s0 = o.a_row_off[row], s1 = o.a_row_off[row + 1];
-        const bool one = s1 - s0 <= kSlabThreads;   // one chunk: cursors in registers
+        const bool one = s1 - s0 <= kSymThreads;   // one chunk: cursors in registers
         int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
         int cur = 0, end = 0;
         if (tid == 0)
             s_min[0] = INT_MAX;
         __syncthreads();
-        for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+        for (int c0 = s0; c0 < s1; c0 += kSymThreads) {
             cur = end = 0;
             if (c0 + tid < s1)
                 slot_run(o, task, c0 + tid, &cur, &end);
@@ -479,7 +519,7 @@ __global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps 
             __syncthreads();
             const int wlo = first >> 3;
             const int64_t lim = (static_cast<int64_t>(wlo) + kSymWin) * 8;
-            for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+            for (int c0 = s0; c0 < s1; c0 += kSymThreads) {
                 int r = 0;
                 if (!one) {
                     cur = end = 0;
@@ -521,13 +561,13 @@ __global__ __launch_bounds__(kSlabThreads, 4) void symbolic_slab_kernel(SlabOps 
             npc = wave_sum(npc);
             if (lane_id() == 0) {
                 s.scan[tid / kWave] = nt;
-                s.scan[kSlabWaves + tid / kWave] = npc;
+                s.scan[kSymThreads / kWave + tid / kWave] = npc;
             }
             __syncthreads();
             int tpos = 0, zpos = 0, all = 0, zall = 0;
 #pragma unroll
-            for (int i = 0; i < kSlabWaves; ++i) {
-                const int x = s.scan[i], y = s.scan[kSlabWaves + i];
+            for (int i = 0; i < kSymThreads / kWave; ++i) {
+                const int x = s.scan[i], y = s.scan[kSymThreads / kWave + i];
                 tpos += i < tid / kWave ? x : 0;
                 zpos += i < tid / kWave ? y : 0;
                 all += x;
@@ -605,22 +645,26 @@ struct Product {
     double val;
 };
 
-__global__ __launch_bounds__(kSlabThreads, 4) void numeric_slab_kernel(SlabOps o, COut c)
+__global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o, COut c)
 {
     __shared__ double s_acc[kNumVals];
-    __shared__ unsigned long long s_mask[kNumCols];   // of the window's C tiles, by column
-    __shared__ unsigned short s_at[kNumCols];         // their first values
-    __shared__ double s_a[kSlabThreads];
-    __shared__ Runs s;
-    __shared__ int s_fit[kSlabWaves], s_last[kSlabWaves], s_vals[kSlabWaves];
+    __shared__ unsigned long long s_mask[kNumTiles];  // of the window's C tiles
+    __shared__ unsigned short s_at[kNumTiles];        // their first values
+    // Bit j: a C tile lies j tile columns into the window; tiles before a word.
+    __shared__ unsigned long long s_col[kNumWords];
+    __shared__ unsigned short s_rank[kNumWords];
+    __shared__ double s_a[kNumThreads];
+    __shared__ Runs<kNumThreads> s;
+    constexpr int kNumWaves = kNumThreads / kWave;
+    __shared__ int s_fit[kNumWaves], s_last[kNumWaves], s_vals[kNumWaves];
     __shared__ int s_task[4];
     __shared__ unsigned long long s_long;
     const int tid = threadIdx.x, w = tid / kWave;
-    for (int i = tid; i < kNumVals; i += kSlabThreads)
+    for (int i = tid; i < kNumVals; i += kNumThreads)
         s_acc[i] = 0.0;
     for (int step = 0;; ++step) {
         Task task;
-        if (!next_task(o, step, s_task, &s_long, &task))
+        if (!next_task<kNumThreads>(o, step, s_task, &s_long, &task))
             break;
         const int row = task.row;
         int64_t t0 = c.tile_ptr[row];
@@ -635,11 +679,11 @@ __global__ __launch_bounds__(kSlabThreads, 4) void numeric_slab_kernel(SlabOps o
             nt = to - from;
         }
         const int s0 = o.a_row_off[row], s1 = o.a_row_off[row + 1];
-        const bool one = s1 - s0 <= kSlabThreads;
+        const bool one = s1 - s0 <= kNumThreads;
         int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
         int cur = 0, end = 0, r = 0;
         double av = 0.0;
-        for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+        for (int c0 = s0; c0 < s1; c0 += kNumThreads) {
             cur = end = 0;
             if (c0 + tid < s1) {
                 slot_run(o, task, c0 + tid, &cur, &end);
@@ -650,23 +694,28 @@ __global__ __launch_bounds__(kSlabThreads, 4) void numeric_slab_kernel(SlabOps o
             }
         }
         for (int64_t t_lo = 0; t_lo < nt;) {
-            // The window: as many tiles from t_lo on as the column map and
-            // the accumulator hold (at least one: a tile has at most 64
-            // values).  A thread looks at kNumTiles of the next kNumCols.
+            // The window: as many tiles from t_lo on as the tables and the
+            // accumulator hold (at least one: a tile has at most 64 values).
+            // A thread looks at kLookTiles of the next kNumTiles.
+            for (int i = tid; i < kNumWords; i += kNumThreads)
+                s_col[i] = 0ull;
+            __syncthreads();
             const int wlo = c.col[t0 + t_lo];
             const int64_t v0 = c.tile_nnz[t0 + t_lo];
             int fit = 0, last = 0, vals = 0;
 #pragma unroll
-            for (int i = 0; i < kNumTiles; ++i) {
-                const int64_t t = t_lo + i * kSlabThreads + tid;
+            for (int i = 0; i < kLookTiles; ++i) {
+                const int x = i * kNumThreads + tid;
+                const int64_t t = t_lo + x;
                 if (t < nt) {
                     const int j = c.col[t0 + t] - wlo;
                     const uint64_t m = c.mask[t0 + t];
                     const int64_t at = c.tile_nnz[t0 + t] - v0;
                     const int64_t to = at + __popcll(m);
-                    if (j >= 0 && j < kNumCols && to <= kNumVals) {
-                        s_mask[j] = m;
-                        s_at[j] = static_cast<unsigned short>(at);
+                    if (j >= 0 && j < kNumSpan && to <= kNumVals) {
+                        s_mask[x] = m;
+                        s_at[x] = static_cast<unsigned short>(at);
+                        atomicOr(&s_col[j >> 6], 1ull << (j & 63));
                         ++fit;
                         last = max(last, j);
                         vals = max(vals, static_cast<int>(to));
@@ -685,15 +734,30 @@ __global__ __launch_bounds__(kSlabThreads, 4) void numeric_slab_kernel(SlabOps o
                 s_vals[w] = vals;
             }
             __syncthreads();
+            if (tid < kWave) {
+                constexpr int kPer = kNumWords / kWave;
+                int n[kPer], sum = 0;
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    n[i] = __popcll(s_col[tid * kPer + i]);
+                    sum += n[i];
+                }
+                int at = wave_inclusive_scan(sum) - sum;
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    s_rank[tid * kPer + i] = static_cast<unsigned short>(at);
+                    at += n[i];
+                }
+            }
             fit = last = vals = 0;
 #pragma unroll
-            for (int i = 0; i < kSlabWaves; ++i) {
+            for (int i = 0; i < kNumWaves; ++i) {
                 fit += s_fit[i];
                 last = max(last, s_last[i]);
                 vals = max(vals, s_vals[i]);
             }
             const int64_t lim = (static_cast<int64_t>(wlo) + last + 1) * 8;
-            for (int c0 = s0; c0 < s1; c0 += kSlabThreads) {
+            for (int c0 = s0; c0 < s1; c0 += kNumThreads) {
                 if (!one) {
                     cur = end = 0;
                     if (c0 + tid < s1) {
@@ -716,15 +780,19 @@ __global__ __launch_bounds__(kSlabThreads, 4) void numeric_slab_kernel(SlabOps o
                         // Every product's tile lies in the window; the bounds
                         // keep a damaged structure inside the LDS.
                         const int j = (x.col >> 3) - wlo;
-                        if (j < 0 || j >= kNumCols)
+                        if (j < 0 || j >= kNumSpan)
+                            return;
+                        const int t = s_rank[j >> 6] +
+                                      __popcll(s_col[j >> 6] & ((1ull << (j & 63)) - 1ull));
+                        if (t >= kNumTiles)
                             return;
                         const int bit = s.r[i] * 8 + (x.col & 7);
-                        const int at = s_at[j] + __popcll(s_mask[j] & ((1ull << bit) - 1ull));
+                        const int at = s_at[t] + __popcll(s_mask[t] & ((1ull << bit) - 1ull));
                         if (at < kNumVals)
                             atomicAdd(&s_acc[at], s_a[i] * x.val);
                     });
             }
-            for (int i = tid; i < vals; i += kSlabThreads) {
+            for (int i = tid; i < vals; i += kNumThreads) {
                 c.val[v0 + i] = s_acc[i];
                 s_acc[i] = 0.0;
             }
@@ -755,7 +823,7 @@ static SlabOps slab_ops(const DevTiles &a, const SpgemmWork *w, const SlabTasks 
     return o;
 }
 
-// Workgroups of the slab passes: two fit a CU.
+// Workgroups of the symbolic passes; the numeric pass has half as many.
 static unsigned slab_blocks()
 {
     return 2u * static_cast<unsigned>(ctx().num_cus > 0 ? ctx().num_cus : 256);
@@ -763,15 +831,15 @@ static unsigned slab_blocks()
 
 int64_t slab_target(unsigned long long pairs)
 {
-    // Sixteen tasks per workgroup on average, and at least the work that
+    // Sixteen tasks per workgroup of the symbolic passes on average, and at least the work that
     // pays for a task's search of its cuts.
     return static_cast<int64_t>(std::max<unsigned long long>(65536, pairs / (16ull * slab_blocks())));
 }
 
-// Cursors in memory for rows of more slots than a workgroup has threads.
+// Cursors in memory for rows of more slots than a workgroup may have threads.
 static int slab_cursors(SpgemmWork *w, int64_t longest)
 {
-    if (longest > kSlabThreads && longest > w->slab_cursor_stride) {
+    if (longest > kSymThreads && longest > w->slab_cursor_stride) {
         w->slab_cursor_stride = longest;
         RTT_TRY(w->slab_cursors.ensure(static_cast<size_t>(slab_blocks()) *
                                        static_cast<size_t>(longest) * sizeof(int2)));
@@ -850,7 +918,7 @@ int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int 
         clear_error();
     }
     RTT_TRY(w->slab_task_size.ensure(static_cast<size_t>(tasks.most) * sizeof(TaskSize)));
-    hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(slab_blocks()), dim3(kSlabThreads),
+    hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(slab_blocks()), dim3(kSymThreads),
                        0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows),
                        w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(), slab_stage(w, cursor),
                        COut{});
@@ -861,7 +929,7 @@ int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int 
 int slab_structure(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
                    int static_rows, const COut &c)
 {
-    hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(slab_blocks()), dim3(kSlabThreads),
+    hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(slab_blocks()), dim3(kSymThreads),
                        0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows), nullptr,
                        nullptr, slab_stage(w, nullptr), c);
     RTT_HIP(hipGetLastError());
@@ -872,7 +940,7 @@ int slab_numeric(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *
                  int static_rows, const COut &c, int64_t longest)
 {
     RTT_TRY(slab_cursors(w, longest));
-    hipLaunchKernelGGL(numeric_slab_kernel, dim3(slab_blocks()), dim3(kSlabThreads), 0,
+    hipLaunchKernelGGL(numeric_slab_kernel, dim3(slab_blocks() / 2), dim3(kNumThreads), 0,
                        ctx().stream, slab_ops(a, w, tasks, queue, static_rows), c);
     RTT_HIP(hipGetLastError());
     return RTT_OK;

@@ -1,7 +1,8 @@
 """Rows beyond the LDS tables at the edges of their passes: A rows around one
-and two chunks of 512 slots, C rows around a numeric window (4096 values, 2048
-tile columns) and a symbolic one (8192 tile columns), windows with more than
-16384 products, gaps of many windows between columns, dense A tiles (absent
+and two chunks of 512 slots (1024 in the numeric pass), C rows around a numeric
+window (13312 values, 3072 tiles, 32768 tile columns) and a symbolic one (8192
+tile columns), more column bytes than are staged at a time (8192), windows with
+more than 16384 products, gaps of many windows between columns, dense A tiles (absent
 slots), empty B rows, and B = A^T.  The first call of a handle recomputes the
 structure, the later ones copy the staged lists: both against the oracle."""
 import numpy as np
@@ -42,10 +43,26 @@ def test_chunks_of_slots(gpu, slots, lb_mode):
     check(gpu, a, b, lb_mode)
 
 
-@pytest.mark.parametrize("n", [8 * 2047, 8 * 2048, 8 * 2048 + 1, 8 * 8192, 8 * 8192 + 9, 8 * 30000])
+@pytest.mark.parametrize("n", [8 * 2047, 8 * 2048, 8 * 2048 + 1, 8 * 8192, 8 * 8192 + 9, 8 * 30000,
+                               8 * 32768, 8 * 32768 + 3, 8 * 70000])
 def test_windows(gpu, n):
     a = rows_matrix(16, 400, np.full(16, 40), 7)
     b = gpu.gen_random(400, n, min(60, n // 8), 8)
+    check(gpu, a, b)
+
+
+@pytest.mark.parametrize("tiles", [3071, 3072, 3073, 6145])
+@pytest.mark.parametrize("vals", [1, 4, 5])
+def test_tiles_of_a_window(gpu, tiles, vals):
+    """One tile row of C with `tiles` tiles of `vals` values, from B rows that
+    share them out."""
+    a = rows_matrix(8, 16, np.r_[16, np.zeros(7, int)], 1)
+    cells = np.arange(tiles * vals)
+    cols = cells // vals * 8 + cells % vals
+    r = cells % 16
+    order = np.lexsort((cols, r))
+    rng = np.random.default_rng(tiles + vals)
+    b = csr_from(16, 8 * tiles, r[order], cols[order], rng.uniform(-1, 1, len(cols)))
     check(gpu, a, b)
 
 
