@@ -191,6 +191,34 @@ struct Stage {
 };
 
 
+// The look-back words and the counters from `first` on to be zeroed before a
+// sizes pass; with a pair total, also that counter to be set and the queue
+// heads to be zeroed.  The symbolic pass before it does so on the side: a
+// launch of its own took 1.3 us of the smallest product's 122.
+struct SizesInit {
+    unsigned long long *ctr;
+    int first;
+    unsigned long long *look;
+    int64_t words;
+    const unsigned long long *pair_total;
+    int *queue;
+    int n_queue;
+};
+
+__device__ __forceinline__ void sizes_init(const SizesInit &z)
+{
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+         i < max<int64_t>(z.words, kCounters); i += stride) {
+        if (i < z.words)
+            z.look[i] = 0ull;
+        if (i < kCounters && i >= z.first)
+            z.ctr[i] = i == kCtrPairs && z.pair_total ? *z.pair_total : 0ull;
+        if (z.pair_total && i < z.n_queue)
+            z.queue[i] = 0;
+    }
+}
+
 __device__ __forceinline__ uint32_t slot_of(int j, int bits)
 {
     return hash_tile_col(j) >> (32 - bits);
@@ -273,8 +301,9 @@ __device__ __forceinline__ void fill_segments(unsigned char *s_seg, int pre, int
 
 __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
     Operands g, Stage st, int64_t *__restrict__ row_tiles, int64_t *__restrict__ row_nnz,
-    int *__restrict__ row_level)
+    int *__restrict__ row_level, SizesInit init)
 {
+    sizes_init(init);
     __shared__ __align__(16) int s_key[kWSlots];
     __shared__ unsigned long long s_msk[kWSlots];
     __shared__ uint4 s_lo[kWChunk], s_hi[kWChunk];   // spread_tile of the chunk's tiles
@@ -443,8 +472,9 @@ __global__ __launch_bounds__(kWave) void symbolic_wave_kernel(
 __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
     Operands g, int stage_limit, Stage st, const int *__restrict__ rows,
     int64_t *__restrict__ row_tiles, int64_t *__restrict__ row_nnz, int *__restrict__ row_level,
-    int *__restrict__ slab_rows, unsigned long long *__restrict__ ctr)
+    int *__restrict__ slab_rows, unsigned long long *__restrict__ ctr, SizesInit init)
 {
+    sizes_init(init);   // (the counters below `first` are in use here)
     __shared__ __align__(16) int s_key[kSymSlots];
     __shared__ unsigned long long s_msk[kSymSlots];
     __shared__ uint4 s_lo[kChunk], s_hi[kChunk];   // spread_tile of the chunk's tiles
@@ -1382,19 +1412,9 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
     }
 }
 
-// Zeroes the look-back words and the counters from `first` on; with a pair
-// total, also sets that counter and the queue heads.
-__global__ void sizes_init_kernel(unsigned long long *ctr, int first, unsigned long long *look,
-                                  int64_t words, const unsigned long long *pair_total, int *queue,
-                                  int n_queue)
+__global__ void sizes_init_kernel(SizesInit z)
 {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < words)
-        look[i] = 0ull;
-    if (i < kCounters && i >= first)
-        ctr[i] = i == kCtrPairs && pair_total ? *pair_total : 0ull;
-    if (pair_total && i < n_queue)
-        queue[i] = 0;
+    sizes_init(z);
 }
 
 __global__ void fill_i32_kernel(int *p, int64_t n, int v)
@@ -1601,10 +1621,8 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     RTT_TRY(w->queue.ensure(4 * sizeof(int)));
     int *queue = w->queue.as<int>();
     // The pair total was summed by the B update's pair-extent pass.
-    hipLaunchKernelGGL(sizes_init_kernel,
-                       dim3(blocks_for(std::max<int64_t>(words, kCounters), kThreads)),
-                       dim3(kThreads), 0, s, ctr, 0, look, words,
-                       b.pair_total.as<unsigned long long>(), queue, 4);
+    const SizesInit start{ctr, 0, look, words, b.pair_total.as<unsigned long long>(), queue, 4};
+    const SizesInit again{ctr, static_cast<int>(kCtrRows), look, words, nullptr, nullptr, 0};
     // The tail queue needs B's tile columns only if some C tile can clear its
     // threshold: told from B's tile rows where that is enough, else from its
     // longest tile column (for B = A^T at tile level A's longest tile row),
@@ -1622,7 +1640,9 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     if (R > 0)
         hipLaunchKernelGGL(symbolic_wave_kernel, dim3(R), dim3(kWave), 0, s, g, st,
                            w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(),
-                           w->row_level.as<int>());
+                           w->row_level.as<int>(), start);
+    else
+        hipLaunchKernelGGL(sizes_init_kernel, dim3(1), dim3(kThreads), 0, s, start);
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[1], s));
     int n_slab = 0;
@@ -1641,21 +1661,15 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
         RTT_HIP(hipStreamSynchronize(s));
         return RTT_OK;
     };
-    auto clear_sizes = [&]() {
-        hipLaunchKernelGGL(sizes_init_kernel, dim3(blocks_for(words, kThreads)), dim3(kThreads), 0,
-                           s, ctr, static_cast<int>(kCtrRows), look, words, nullptr, nullptr, 0);
-    };
-    static_assert(kCounters <= kThreads, "one workgroup clears the counters");
     // Sized at once, as if every row fit the wave table: one wait when none
     // outgrew it (the usual case), redone when some did.
     RTT_TRY(finish_sizes(false));
     const int n_large = static_cast<int>(hctr[kCtrOutgrown]);
     if (n_large > 0) {
-        clear_sizes();
         hipLaunchKernelGGL(symbolic_count_kernel, dim3(n_large), dim3(kThreads), 0, s, g,
                            stage_limit, st, w->l3_rows.as<int>(), w->row_tiles.as<int64_t>(),
                            w->row_nnz.as<int64_t>(), w->row_level.as<int>(),
-                           w->sym_slab_rows.as<int>(), ctr);
+                           w->sym_slab_rows.as<int>(), ctr, again);
         RTT_HIP(hipGetLastError());
         RTT_HIP(hipEventRecord(ev->ev[1], s));
         RTT_TRY(finish_sizes(false));
@@ -1670,7 +1684,8 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
                                 s, &tasks));
         RTT_TRY(slab_symbolic(a, w, tasks, queue, static_rows, ctr + kCtrSlabTiles,
                               static_cast<int64_t>(hctr[kCtrLongest])));
-        clear_sizes();
+        hipLaunchKernelGGL(sizes_init_kernel, dim3(blocks_for(words, kThreads)), dim3(kThreads), 0,
+                               s, again);
         RTT_TRY(finish_sizes(true));
     }
     w->slab_stage_need = std::max<uint64_t>(w->slab_stage_need, hctr[kCtrSlabTiles]);
