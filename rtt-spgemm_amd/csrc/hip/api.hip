@@ -140,7 +140,16 @@ struct HostCopy {
 int staged_d2h(const HostCopy *items, int n, rtt::HostRing *ring)
 {
     hipStream_t s = rtt::ctx().stream;
-    RTT_TRY(ring->create());
+    if (ring->create() != RTT_OK) {
+        // No pinned memory to be had: straight to the destinations.
+        rtt::clear_error();
+        for (int i = 0; i < n; ++i)
+            if (items[i].bytes)
+                RTT_HIP(hipMemcpyAsync(items[i].dst, items[i].src, items[i].bytes,
+                                       hipMemcpyDeviceToHost, s));
+        RTT_HIP(hipStreamSynchronize(s));
+        return RTT_OK;
+    }
     struct Piece {
         void *dst;
         size_t bytes;
