@@ -284,7 +284,7 @@ def split_form(args):
                      "numeric_kernel_ms": round(st["numeric_kernel_ms"], 4),
                      "numeric_path": {v: k for k, v in rt.NUMERIC_PATHS.items()}[st["numeric_path"]],
                      "mfma": {"instruction": "v_mfma_f64_4x4x4f64" if prec == "fp64"
-                              else "v_mfma_f32_16x16x32_bf16 (8 per pair)",
+                              else "v_mfma_f32_16x16x32_bf16 (4 per pair)",
                               "pairs": st["mfma_pairs"]}}
     # (|A||A|)_ij with the FP64 kernels: the forward-error scale of every entry.
     absa = rt.CsrMatrix(a.m, a.n, a.rowptr, a.col, np.abs(a.val))
@@ -411,7 +411,7 @@ def c1_line(rt, steps=20, warmup=5, repeats=5):
 
 # Kernel names in the rocprofv3 counter summaries, per breakdown key.
 PROFILE_KERNELS = {
-    "numeric": "numeric_row_kernel<SmallRow",
+    "numeric": "numeric_row_kernel<SpreadRow",
     "numeric_tile": "tile_numeric_kernel<Fp64Product>",
     "symbolic_count": "symbolic_wave_kernel",
     "symbolic_fill": "symbolic_write_kernel",

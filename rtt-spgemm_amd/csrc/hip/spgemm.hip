@@ -24,8 +24,8 @@
 //    values in k-major order), walks B's entries row by row with A's column
 //    in registers, and adds each scalar product into an LDS FP64 accumulator
 //    laid out exactly like the row's output segment, which is finally
-//    streamed to HBM.  Rows that exceed the LDS budgets fall back to a
-//    workgroup path with FP64 atomics in HBM.
+//    streamed to HBM.  Rows that exceed the LDS budgets go to the slab
+//    kernels (slab.hip).
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -95,7 +95,7 @@ struct SmallRow {
 // add took 17 ns a wave and CU, with the slots 8), and a pair with a light
 // tile, of which such products have many, takes the one row it needs of B's
 // record instead of walking all of it.  The LDS pipe was busy 75 % of the
-// kernel's time and is now 58 %, vector instructions 70 %: 128^3 box stencil,
+// kernel's time and is now 55 %, vector instructions 74 %: 128^3 box stencil,
 // A*A^T (14 entries a C tile), 2.83 -> 2.29 ms; banded products (39 to 49)
 // take 0.59 ms with the extra index work against 0.57 without.
 struct SpreadRow : SmallRow {
