@@ -325,7 +325,7 @@ def cpu_baseline(a, aat, nnz_cub, budget_s=2.5, repeats=5):
     """Times the oracle's row SPA (structure + values in reference order) on a
     contiguous block of rows sized to about budget_s seconds, `repeats`
     times; reports the median.  Threads: OMP_NUM_THREADS when set (the host's
-    CPU share on a GPU box), else every core."""
+    CPU share on a shared machine), else every core."""
     import oracle
     threads = int(os.environ.get("OMP_NUM_THREADS", "0")) or (os.cpu_count() or 1)
     os.environ["OMP_NUM_THREADS"] = str(threads)
