@@ -177,53 +177,67 @@ __global__ void row_ptr_from_sorted_kernel(const int *__restrict__ keys, int64_t
         ptr[k] = static_cast<int>(i);
 }
 
+// Position of the n-th set bit of m (n below its count).
+__device__ __forceinline__ int nth_bit(uint32_t m, int n)
+{
+    int pos = 0;
+#pragma unroll
+    for (int w = 16; w >= 1; w >>= 1) {
+        const int c = __popc((m >> pos) & ((1u << w) - 1u));
+        if (n >= c) {
+            n -= c;
+            pos += w;
+        }
+    }
+    return pos;
+}
+
 // Value planes (1 .. kRecParts-1) of B's records and the k-major copy of what
-// they do not hold, from the payload: one tile per thread.  A record holds
-// its tile's first kRecVals values in k-major order (row k's entries
-// contiguous, columns ascending); the values past them go to the same places
-// of the k-major copy, whose first kRecVals slots per tile nothing reads.
-// All of the record's values are loaded before the first plane is written;
-// consecutive threads write consecutive entries of every plane.  The planes
-// past a tile's values are never read.  Against a re-pack of every value
-// into the copy followed by a pass from the copy to the planes: one read of
-// the payload instead of two, and no copy at all for tiles of up to kRecVals
-// entries (AMG batch of 8: 0.58 ms for the two passes before).
+// they do not hold, from the payload.  A record holds its tile's first
+// kRecVals values in k-major order (row k's entries contiguous, columns
+// ascending); the values past them go to the same places of the k-major copy,
+// whose first kRecVals slots per tile nothing reads.  The planes past a
+// tile's values are never read.
+// Four lanes per tile, lane q the values 2q, 2q + 1 of every eight: a wave
+// reads its 16 tiles' values a line at a time and writes 256 contiguous bytes
+// of every plane.  (One lane per tile where tiles hold two values or fewer on
+// average, which the first lane has anyway: four took 1.4 us more on the random
+// rectangular product's 880000.)  With a tile per thread every load met 64 lines, and they
+// were gone from the L1 before a tile's next value was asked for: banded batch
+// 257 -> 168 us, AMG batch 233 -> 222 us (its tiles hold few values).
+template <int L>
 __global__ void record_values_kernel(int64_t n, const double *__restrict__ vals,
                                      int4 *__restrict__ planes, double *__restrict__ kmajor)
 {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n)
-        return;
-    const int4 m = planes[t];
-    const uint32_t mask = static_cast<uint32_t>(m.y);
-    const bool dense = m.w < 0;
-    const uint32_t off = static_cast<uint32_t>(m.w) & 0x7FFFFFFFu;
-    const int nv = __popc(mask);
-    uint32_t mz = static_cast<uint32_t>(m.z);   // bit k * 8 + c
-    // Next entry's value: bit c * 4 + k of the payload's order.
-    auto next = [&]() {
-        const int pos = __builtin_ctz(mz);
-        mz &= mz - 1;
-        const int phys = (pos & 7) * 4 + (pos >> 3);
-        return vals[off + (dense ? phys : __popc(mask & ((1u << phys) - 1u)))];
-    };
-    double v[kRecVals];
-#pragma unroll
-    for (int j = 0; j < kRecVals; ++j)
-        v[j] = mz ? next() : 0.0;
-#pragma unroll
-    for (int part = 1; part < kRecParts; ++part)
-        if (2 * (part - 1) < nv)
-            planes[part * n + t] = *reinterpret_cast<const int4 *>(
-                &reinterpret_cast<const double2 *>(v)[part - 1]);
-    for (int j = kRecVals; mz; j += kRecVals) {
-#pragma unroll
-        for (int u = 0; u < kRecVals; ++u)
-            v[u] = mz ? next() : 0.0;
-#pragma unroll
-        for (int u = 0; u < kRecVals; ++u)
-            if (j + u < nv)
-                kmajor[off + j + u] = v[u];
+    const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x / L;
+    const int q = static_cast<int>(gid % L);
+    for (int64_t t = gid / L; t < n; t += step) {
+        const int4 m = planes[t];
+        const uint32_t mask = static_cast<uint32_t>(m.y);
+        const bool dense = m.w < 0;
+        const uint32_t off = static_cast<uint32_t>(m.w) & 0x7FFFFFFFu;
+        const int nv = __popc(mask);
+        const uint32_t mz = static_cast<uint32_t>(m.z);   // bit k * 8 + c
+        // Value of the entry at bit pos: bit c * 4 + k of the payload's order.
+        auto at = [&](int pos) {
+            const int phys = (pos & 7) * 4 + (pos >> 3);
+            return vals[off + (dense ? phys : __popc(mask & ((1u << phys) - 1u)))];
+        };
+        for (int j = 2 * q; j < nv; j += 2 * L) {
+            const int p0 = nth_bit(mz, j);
+            const uint32_t rest = p0 < 31 ? mz >> (p0 + 1) : 0u;
+            double2 v;
+            v.x = at(p0);
+            v.y = j + 1 < nv ? at(p0 + 1 + __builtin_ctz(rest | 0x80000000u)) : 0.0;
+            if (j < kRecVals) {
+                planes[(1 + j / 2) * n + t] = *reinterpret_cast<const int4 *>(&v);
+            } else {
+                kmajor[off + j] = v.x;
+                if (j + 1 < nv)
+                    kmajor[off + j + 1] = v.y;
+            }
+        }
     }
 }
 
@@ -653,10 +667,15 @@ static int write_record_values(DevTiles *b)
 {
     RTT_TRY(b->values_cm.ensure(static_cast<size_t>(b->payload > 0 ? b->payload : 1) *
                                 sizeof(double)));
-    if (b->num_tiles > 0)
-        hipLaunchKernelGGL(record_values_kernel, dim3(blocks_for(b->num_tiles, kThreads)),
+    auto launch = [&](auto kernel, int lanes) {
+        hipLaunchKernelGGL(kernel, dim3(std::min(blocks_for(b->num_tiles * lanes, kThreads), 1u << 22)),
                            dim3(kThreads), 0, ctx().stream, b->num_tiles, b->values.as<double>(),
                            b->records.as<int4>(), b->values_cm.as<double>());
+    };
+    if (b->num_tiles > 0 && b->payload <= 2 * b->num_tiles)
+        launch(record_values_kernel<1>, 1);
+    else if (b->num_tiles > 0)
+        launch(record_values_kernel<4>, 4);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
