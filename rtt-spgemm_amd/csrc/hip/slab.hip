@@ -840,9 +840,11 @@ int64_t slab_target(unsigned long long pairs)
 static int slab_cursors(SpgemmWork *w, int64_t longest)
 {
     if (longest > kSymThreads && longest > w->slab_cursor_stride) {
-        w->slab_cursor_stride = longest;
+        // ensure() gives the old buffer up first: no stride until it has the new one.
+        w->slab_cursor_stride = 0;
         RTT_TRY(w->slab_cursors.ensure(static_cast<size_t>(slab_blocks()) *
                                        static_cast<size_t>(longest) * sizeof(int2)));
+        w->slab_cursor_stride = longest;
     }
     return RTT_OK;
 }
