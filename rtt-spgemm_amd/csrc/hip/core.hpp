@@ -116,6 +116,9 @@ struct SlabTasks {
 };
 constexpr int kSlabParts = 256;   // most tasks of a row
 int64_t slab_target(unsigned long long pairs);
+// Workgroups of a slab pass whose longest row has `longest` slots, with `held`
+// bytes of cursors there and `free_bytes` of device memory free.
+unsigned slab_cursor_blocks(int64_t longest, size_t held, size_t free_bytes);
 // Counts the listed rows' tiles and entries into w->row_tiles / row_nnz and
 // stages their tile lists; *cursor sums what the staging needs.  longest:
 // most slots of A's payload in one of the rows.

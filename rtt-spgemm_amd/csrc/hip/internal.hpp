@@ -176,7 +176,8 @@ struct SpgemmWork {
     // row (every call that has such rows) and the cursors of long rows.
     DevBuf slot_k, slot_r, b_start, b_col, b_val, slab_cursors;
     bool slot_codes_ready = false;
-    int64_t slab_cursor_stride = 0;
+    int64_t slab_cursor_stride = 0;         // of the last slab pass: slots per workgroup
+    unsigned slab_cursor_blocks = 0;        // and the workgroups that have cursors
     // Slab rows' (column, mask) lists between the symbolic passes: entries
     // allocated, and the most the previous calls needed (grown at the next
     // call's start, never while a fill pass may still read the buffer).

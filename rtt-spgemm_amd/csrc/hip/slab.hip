@@ -836,16 +836,41 @@ int64_t slab_target(unsigned long long pairs)
     return static_cast<int64_t>(std::max<unsigned long long>(65536, pairs / (16ull * slab_blocks())));
 }
 
-// Cursors in memory for rows of more slots than a workgroup may have threads.
+// A workgroup's cursors take 8 bytes a slot of the longest row: 128 MB for a
+// hub of 16 million entries, 67 GB for all workgroups.  Fewer workgroups then
+// take the tasks, as many as a quarter of the free memory (and what is held)
+// has room for, rather than none for want of memory.
+unsigned slab_cursor_blocks(int64_t longest, size_t held, size_t free_bytes)
+{
+    const uint64_t per = static_cast<uint64_t>(longest) * sizeof(int2);
+    return static_cast<unsigned>(
+        std::max<uint64_t>(1, std::min<uint64_t>(slab_blocks(), (free_bytes / 4 + held) / per)));
+}
+
+// Cursors in memory for rows of more slots than a workgroup may have threads,
+// and the workgroups they serve.
 static int slab_cursors(SpgemmWork *w, int64_t longest)
 {
-    if (longest > kSymThreads && longest > w->slab_cursor_stride) {
-        // ensure() gives the old buffer up first: no stride until it has the new one.
-        w->slab_cursor_stride = 0;
-        RTT_TRY(w->slab_cursors.ensure(static_cast<size_t>(slab_blocks()) *
-                                       static_cast<size_t>(longest) * sizeof(int2)));
-        w->slab_cursor_stride = longest;
+    constexpr size_t kUnasked = size_t(1) << 30;   // taken without a look at the free memory
+    const DevBuf &buf = w->slab_cursors;
+    w->slab_cursor_stride = 0;   // (no buffer behind it, should its allocation fail)
+    w->slab_cursor_blocks = slab_blocks();
+    if (longest <= kSymThreads)
+        return RTT_OK;
+    const size_t per = static_cast<size_t>(longest) * sizeof(int2);
+    if (buf.bytes < slab_blocks() * per) {
+        unsigned blocks = slab_blocks();
+        const bool large = blocks * per > kUnasked;
+        size_t free_b = 0, total_b = 0;
+        if (large && hipMemGetInfo(&free_b, &total_b) == hipSuccess)
+            blocks = slab_cursor_blocks(longest, buf.bytes, free_b);
+        // A large buffer is kept while it serves half of what there is room for.
+        if (!large || buf.bytes / per < (blocks + 1) / 2)
+            RTT_TRY(w->slab_cursors.ensure(blocks * per));
+        w->slab_cursor_blocks =
+            static_cast<unsigned>(std::min<uint64_t>(slab_blocks(), buf.bytes / per));
     }
+    w->slab_cursor_stride = longest;
     return RTT_OK;
 }
 
@@ -920,7 +945,7 @@ int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int 
         clear_error();
     }
     RTT_TRY(w->slab_task_size.ensure(static_cast<size_t>(tasks.most) * sizeof(TaskSize)));
-    hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(slab_blocks()), dim3(kSymThreads),
+    hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(w->slab_cursor_blocks), dim3(kSymThreads),
                        0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows),
                        w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(), slab_stage(w, cursor),
                        COut{});
@@ -931,7 +956,7 @@ int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int 
 int slab_structure(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
                    int static_rows, const COut &c)
 {
-    hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(slab_blocks()), dim3(kSymThreads),
+    hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(w->slab_cursor_blocks), dim3(kSymThreads),
                        0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows), nullptr,
                        nullptr, slab_stage(w, nullptr), c);
     RTT_HIP(hipGetLastError());
@@ -942,7 +967,7 @@ int slab_numeric(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *
                  int static_rows, const COut &c, int64_t longest)
 {
     RTT_TRY(slab_cursors(w, longest));
-    hipLaunchKernelGGL(numeric_slab_kernel, dim3(slab_blocks() / 2), dim3(kNumThreads), 0,
+    hipLaunchKernelGGL(numeric_slab_kernel, dim3(std::max(1u, w->slab_cursor_blocks / 2)), dim3(kNumThreads), 0,
                        ctx().stream, slab_ops(a, w, tasks, queue, static_rows), c);
     RTT_HIP(hipGetLastError());
     return RTT_OK;

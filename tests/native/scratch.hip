@@ -30,10 +30,27 @@ void cursors_after_a_failed_allocation()
            "the cursor stride fits the buffer held");
 }
 
+// A hub row's cursors for every workgroup may not fit: fewer workgroups then.
+void cursors_of_long_rows()
+{
+    const size_t gib = size_t(1) << 30;
+    const unsigned all = rtt::slab_cursor_blocks(1024, 0, 288 * gib);
+    expect(all >= 256, "short rows: every workgroup");
+    for (int64_t longest : {int64_t(1) << 20, int64_t(1) << 24, int64_t(1) << 27, int64_t(1) << 30})
+        for (size_t free_bytes : {size_t(0), gib, 20 * gib, 288 * gib}) {
+            const unsigned n = rtt::slab_cursor_blocks(longest, 0, free_bytes);
+            expect(n >= 1 && n <= all, "a workgroup at least, the full grid at most");
+            expect(n == 1 || n * static_cast<size_t>(longest) * sizeof(int2) <= free_bytes / 4,
+                   "cursors within a quarter of the free memory");
+        }
+    expect(rtt::slab_cursor_blocks(int64_t(1) << 24, 16 * gib, gib) > 100, "held memory counts");
+}
+
 } // namespace
 
 int main()
 {
     cursors_after_a_failed_allocation();
+    cursors_of_long_rows();
     return failures ? 1 : 0;
 }
