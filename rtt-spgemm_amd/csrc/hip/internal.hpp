@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <climits>
 #include <cstdint>
 #include <vector>
 
@@ -68,6 +70,15 @@ struct DevBuf {
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
 };
+
+// Entries of `size` bytes that a buffer of `bytes` holds beside `spare` more.
+// Positions of tiles and payload slots are ints, so a buffer with room for
+// more (allocations are rounded up) counts as one for INT_MAX: a tile build
+// beyond that then writes nothing, and is refused.
+inline int64_t entries_held(size_t bytes, size_t size, int64_t spare)
+{
+    return std::min<int64_t>(static_cast<int64_t>(bytes / size) - spare, INT_MAX);
+}
 
 // Grow-only pinned host buffer (hipHostMalloc) for small readbacks.
 struct PinnedBuf {

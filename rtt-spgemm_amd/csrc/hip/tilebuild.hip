@@ -813,13 +813,12 @@ int run_build(const DevCsr &src, const int *row_map, int active_rows, int active
     for (int attempt = 0;; ++attempt) {
         DevBuf &meta = B ? out->records : out->meta;   // B: plane 0 of the records
         const size_t meta_size = B ? sizeof(BRecord) : sizeof(int4);
-        g.cap_tiles = static_cast<long long>(
-            std::min({out->tile_col_idx.bytes / sizeof(int), out->masks.bytes / sizeof(uint32_t),
-                      meta.bytes / meta_size}));
-        g.cap_tiles = std::min<long long>(
-            g.cap_tiles, static_cast<long long>(out->value_offsets.bytes / sizeof(int)) - 1);
+        g.cap_tiles = std::min({entries_held(out->tile_col_idx.bytes, sizeof(int), 0),
+                                entries_held(out->masks.bytes, sizeof(uint32_t), 0),
+                                entries_held(meta.bytes, meta_size, 0),
+                                entries_held(out->value_offsets.bytes, sizeof(int), 1)});
         // One slot more than the payload: a zero (see DevTiles::values).
-        g.cap_payload = static_cast<long long>(out->values.bytes / sizeof(double)) - 1;
+        g.cap_payload = entries_held(out->values.bytes, sizeof(double), 1);
         g.tile_col_idx = out->tile_col_idx.as<int>();
         g.masks = out->masks.as<uint32_t>();
         g.value_offsets = out->value_offsets.as<int>();

@@ -46,11 +46,24 @@ void cursors_of_long_rows()
     expect(rtt::slab_cursor_blocks(int64_t(1) << 24, 16 * gib, gib) > 100, "held memory counts");
 }
 
+// Positions are ints: a buffer with room for more entries than INT_MAX does
+// not count as such (the tile build would write at negative positions).
+void entries_of_large_buffers()
+{
+    const size_t most = INT_MAX;
+    expect(rtt::entries_held(0, 8, 1) == -1, "nothing held");
+    expect(rtt::entries_held(256, 8, 1) == 31, "a small buffer");
+    expect(rtt::entries_held((most + 1) * 8, 8, 1) == INT_MAX, "INT_MAX slots and the zero");
+    for (size_t bytes : {(most + 2) * 8, (most + 1) * 9, size_t(1) << 36})
+        expect(rtt::entries_held(bytes, 8, 1) == INT_MAX, "larger buffers");
+}
+
 } // namespace
 
 int main()
 {
     cursors_after_a_failed_allocation();
     cursors_of_long_rows();
+    entries_of_large_buffers();
     return failures ? 1 : 0;
 }
