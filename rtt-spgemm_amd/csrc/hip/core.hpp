@@ -103,9 +103,12 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *s_tmp, int *tota
 }
 
 // ---- rows beyond the LDS tables (slab.hip) ------------------------------------
-// A's slot codes (once per prepared A) and B's entries by scalar row (every
-// call that has such rows).
-int slab_prepare(const DevTiles &a, DevTiles *b, BuildWork *bw, SpgemmWork *w);
+// A's slot codes and B's entries by scalar row for a call with such rows, `n`
+// tile rows listed in `rows` and n_more in `more` (device): of all of A and B, or
+// where the rows are few of these and the B rows they select (one host wait).
+// longest: most slots of A's payload in one of them.
+int slab_prepare(const DevTiles &a, const DevTiles &b, BuildWork *bw, SpgemmWork *w,
+                 const int *rows, int n, const int *more, int n_more, int64_t longest);
 // Slab rows in the order they are taken, tasks base[i] .. base[i + 1] of row
 // i: as many as its pairs hold slab_target.  most: at least all of them.
 struct SlabTasks {

@@ -183,10 +183,14 @@ struct SpgemmWork {
     DevBuf row_cost, row_cost2, rows_sorted;   // slab rows, heaviest first
     DevBuf slab_base;                       // their tasks
     DevBuf trace_start, trace_end, trace_cu;   // numeric timeline samples
-    // Slab rows: A's slot codes (once per prepared A), B's entries by scalar
-    // row (every call that has such rows) and the cursors of long rows.
+    // Slab rows: A's slot codes (of all of A, once; or of a call's rows), B's
+    // entries by scalar row (every call that has such rows) and the cursors of
+    // long rows.
     DevBuf slot_k, slot_r, b_start, b_col, b_val, slab_cursors;
-    bool slot_codes_ready = false;
+    bool slot_codes_ready = false;          // slot_k and slot_r hold all of A's
+    DevBuf row_slot_k, row_slot_r, code_off;
+    DevBuf slab_pick;                       // B rows that a few slab rows select
+    PinnedBuf host_pick;
     int64_t slab_cursor_stride = 0;         // of the last slab pass: slots per workgroup
     unsigned slab_cursor_blocks = 0;        // and the workgroups that have cursors
     // Slab rows' (column, mask) lists between the symbolic passes: entries

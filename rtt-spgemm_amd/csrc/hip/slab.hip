@@ -6,11 +6,13 @@
 // of R-MAT 2^18 held one workgroup for 88 ms).
 //
 // Operands: every slot of A's payload gets its column and its row within the
-// tile (built once per prepared A); B's entries are laid out by scalar row,
-// columns ascending, from its tiles (rebuilt by every call that has such
-// rows).  A workgroup owns one tile row of C, or a part of it, at a time.  A thread owns one
-// slot of the row's A payload, with a cursor into the B row it selects, for
-// chunks of as many slots as the workgroup has threads.
+// tile, and B's entries are laid out by scalar row, columns ascending, from its
+// tiles.  Where a product has many such rows this is done for all of A (once
+// per prepared A) and all of B; where it has few, for the rows themselves and
+// the rows of B they select (slab_prepare).  A workgroup owns one tile row of C, or a
+// part of it, at a time.  A thread owns one slot of the row's A payload, with a
+// cursor into the B row it selects, for chunks of as many slots as the workgroup
+// has threads.
 //
 // The row is walked in windows of C columns.  In a window, every thread
 // gallops its cursor to the window's end; the products are numbered by a
@@ -61,44 +63,206 @@ static_assert(kNumTiles % kNumThreads == 0 && kNumWords % kWave == 0 &&
                   kNumWords / kWave * kWave <= kNumThreads,
               "shares of a window's tables");
 
-// Column (-1: an absent slot of a dense tile) and row of every slot of A's
-// payload; a thread per tile.
-__global__ void slot_codes_kernel(int64_t n, const int4 *__restrict__ meta, int *__restrict__ k,
-                                  uint8_t *__restrict__ r)
+// Column (-1: an absent slot of a dense tile) and row of every slot of the A
+// tile with meta m, from slot `at` of the codes on.
+__device__ __forceinline__ void write_slot_codes(const int4 &m, int64_t at, int *__restrict__ k,
+                                                 uint8_t *__restrict__ r)
 {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n)
-        return;
-    const int4 m = meta[t];
     const uint32_t mask = static_cast<uint32_t>(m.y);
-    const uint32_t off = static_cast<uint32_t>(m.w) & 0x7FFFFFFFu;
     const bool dense = m.w < 0;
     for (int phys = 0, j = 0; phys < 32; ++phys) {
         const bool has = (mask >> phys) & 1u;
         if (!has && !dense)
             continue;
-        k[off + j] = has ? 4 * m.x + (phys & 3) : -1;
-        r[off + j] = static_cast<uint8_t>(phys >> 2);
+        k[at + j] = has ? 4 * m.x + (phys & 3) : -1;
+        r[at + j] = static_cast<uint8_t>(phys >> 2);
         ++j;
     }
 }
 
-// B's entries by scalar row: tile row K's entries lie in its stretch of the
-// payload, row 4K first, columns ascending; row 4K + k is start[5K + k] ..
-// start[5K + k + 1].  T threads per tile row (a wave, or a workgroup).
-template <int T>
-__global__ __launch_bounds__(256) void scalar_rows_kernel(
-    int R, const int *__restrict__ trp, const int *__restrict__ tcol,
-    const uint32_t *__restrict__ masks, const int *__restrict__ offs,
-    const double *__restrict__ vals, int *__restrict__ start, int *__restrict__ col,
-    double *__restrict__ val)
+// For every slot of A's payload; a thread per tile.
+__global__ void slot_codes_kernel(int64_t n, const int4 *__restrict__ meta, int *__restrict__ k,
+                                  uint8_t *__restrict__ r)
 {
-    constexpr int kRows = 256 / T;   // tile rows per workgroup
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t < n)
+        write_slot_codes(meta[t], meta[t].w & 0x7FFFFFFF, k, r);
+}
+
+// ---- the rows of a few slab rows ------------------------------------------------
+// The B tile rows that the listed rows select, and those rows' entries.
+struct Picked {
+    unsigned long long rows, entries;
+};
+
+// Listed rows of two lists; workgroups x, y take every gridDim.y-th 256 A tiles
+// of row x: the slot codes of its A payload, `stride` slots from the row before
+// it, and a flag for every B tile row it selects.
+__global__ __launch_bounds__(256) void pick_rows_kernel(
+    const int *__restrict__ rows, int n, const int *__restrict__ more, int64_t stride,
+    const int *__restrict__ a_trp, const int4 *__restrict__ a_meta,
+    const int *__restrict__ a_row_off, int *__restrict__ flag, int *__restrict__ code_off,
+    int *__restrict__ k, uint8_t *__restrict__ r)
+{
+    const int i = blockIdx.x;
+    const int row = i < n ? rows[i] : more[i - n];
+    if (code_off && blockIdx.y == 0 && threadIdx.x == 0)
+        code_off[row] = static_cast<int>(i * stride);
+    const int64_t shift = i * stride - a_row_off[row];
+    const int t1 = a_trp[row + 1];
+    for (int t = a_trp[row] + static_cast<int>(blockIdx.y * 256 + threadIdx.x); t < t1;
+         t += static_cast<int>(gridDim.y) * 256) {
+        const int4 m = a_meta[t];
+        flag[m.x] = 1;
+        if (k)
+            write_slot_codes(m, shift + (m.w & 0x7FFFFFFF), k, r);
+    }
+}
+
+// B's tile rows (the listed ones, or without a list all R) and where their
+// entries go.
+struct BRows {
+    int R;
+    const int *__restrict__ list;              // null: all rows
+    const unsigned long long *__restrict__ n;  // rows listed
+    const int *__restrict__ trp;
+    const int *__restrict__ groups;            // start of each (row, class) run
+    const int4 *__restrict__ meta;             // rows in class order
+    const int *__restrict__ order;             // per row, its tiles by column; null: the arrays are
+    const int *__restrict__ tcol;
+    const uint32_t *__restrict__ masks;
+    const int *__restrict__ offs;
+    const double *__restrict__ vals;
+    int *__restrict__ start;                   // see scalar_rows_kernel
+    int *__restrict__ col;
+    double *__restrict__ val;
+};
+
+// The tile row of threads [i T, i T + T), -1 past the last.
+template <int T>
+__device__ __forceinline__ int b_row(const BRows &g)
+{
+    const int i = static_cast<int>(blockIdx.x) * (256 / T) + static_cast<int>(threadIdx.x) / T;
+    if (!g.list)
+        return i < g.R ? i : -1;
+    return i < static_cast<int>(*g.n) ? g.list[i] : -1;
+}
+
+// Exclusive sum of n over the workgroup's 256 threads and the workgroups that
+// have added to *total (one atomic a workgroup: on one address they take 7 ns
+// each, one a row took 0.45 ms of 65000 rows).
+__device__ __forceinline__ int64_t grid_place(int n, unsigned long long *total)
+{
+    __shared__ int s_tmp[256 / kWave];
+    __shared__ unsigned long long s_base;
+    int all = 0;
+    const int before = block_exclusive_scan<256 / kWave>(n, s_tmp, &all);
+    if (threadIdx.x == 0)
+        s_base = all ? atomicAdd(total, static_cast<unsigned long long>(all)) : 0ull;
+    __syncthreads();
+    return static_cast<int64_t>(s_base) + before;
+}
+
+// The flagged rows' list; a thread per row of B.
+__global__ __launch_bounds__(256) void list_rows_kernel(int R, const int *__restrict__ flag,
+                                                        Picked *picked, int *__restrict__ list)
+{
+    const int K = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+    const int has = K < R && flag[K] ? 1 : 0;
+    const int64_t at = grid_place(has, &picked->rows);
+    if (has)
+        list[at] = K;
+}
+
+// Entries of every row, for place_rows_kernel.
+template <int T>
+__global__ __launch_bounds__(256) void count_rows_kernel(BRows g)
+{
+    const int K = b_row<T>(g);
+    if (K < 0)
+        return;   // a whole wave or workgroup
+    __shared__ int s_sum[256 / kWave];
+    int n = 0;
+    for (int t = g.trp[K] + static_cast<int>(threadIdx.x) % T; t < g.trp[K + 1]; t += T)
+        n += __popc(static_cast<uint32_t>(g.meta[t].y));
+    n = wave_sum(n);
+    if constexpr (T > kWave) {
+        if (lane_id() == 0)
+            s_sum[threadIdx.x / kWave] = n;
+        __syncthreads();
+        n = 0;
+        for (int w = 0; w < T / kWave; ++w)
+            n += s_sum[w];
+    }
+    if (threadIdx.x % T == 0)
+        g.start[5 * static_cast<int64_t>(K) + 4] = n;
+}
+
+// The place of every row's entries; a thread per row.  Rows built from a CSR
+// get the slots of their payload.
+__global__ __launch_bounds__(256) void place_rows_kernel(BRows g, Picked *picked)
+{
+    const int K = b_row<1>(g);
+    int n = 0;
+    if (K >= 0)
+        n = g.order ? g.start[5 * static_cast<int64_t>(K) + 4]
+                    : g.offs[g.trp[K + 1]] - g.offs[g.trp[K]];
+    const int64_t at = grid_place(n, &picked->entries);
+    if (K >= 0)
+        g.start[5 * static_cast<int64_t>(K)] = static_cast<int>(at);
+}
+
+// A row's tiles by column, from its class runs, each of which has ascending
+// columns: a tile's place is its own run's before it and, of the other runs,
+// those with smaller columns.
+template <int T>
+__global__ __launch_bounds__(256) void order_tiles_kernel(BRows g, int *__restrict__ order)
+{
+    const int K = b_row<T>(g);
+    if (K < 0)
+        return;
+    const int *gp = g.groups + static_cast<int64_t>(kClassSlots) * K;
+    constexpr int kRuns = 5;   // heavy, light k = 0..3
+    int at[kRuns + 1];
+#pragma unroll
+    for (int c = 0; c <= kRuns; ++c)
+        at[c] = gp[c];
+    for (int t = at[0] + static_cast<int>(threadIdx.x) % T; t < at[kRuns]; t += T) {
+        const int j = g.meta[t].x;
+        int rank = 0;
+#pragma unroll
+        for (int c = 0; c < kRuns; ++c) {
+            if (t >= at[c] && t < at[c + 1]) {
+                rank += t - at[c];
+                continue;
+            }
+            int lo = at[c], hi = at[c + 1];
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (g.meta[mid].x < j)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            rank += lo - at[c];
+        }
+        order[at[0] + rank] = t;
+    }
+}
+
+// B's entries by scalar row: the entries of tile row K lie together, row 4K
+// first, columns ascending; row 4K + k is start[5K + k] .. start[5K + k + 1].
+// They begin at start[5K] where the rows were placed (PLACED), else at the
+// row's place in the payload.  T threads per tile row (a wave, or a workgroup).
+template <int T, bool PLACED>
+__global__ __launch_bounds__(256) void scalar_rows_kernel(BRows g)
+{
     __shared__ unsigned long long s_sum[256 / kWave];
     const int lt = threadIdx.x % T;
-    const int K = blockIdx.x * kRows + threadIdx.x / T;
-    const bool live = K < R;
-    const int t0 = live ? trp[K] : 0, t1 = live ? trp[K + 1] : 0;
+    const int K = b_row<T>(g);
+    if (K < 0)
+        return;   // a whole wave or workgroup
+    const int t0 = g.trp[K], t1 = g.trp[K + 1];
     // Entries per k in 16-bit fields (at most 8 per tile and k).
     auto count = [&](uint32_t m) {
         unsigned long long c = 0;
@@ -106,6 +270,9 @@ __global__ __launch_bounds__(256) void scalar_rows_kernel(
         for (int k = 0; k < 4; ++k)
             c |= static_cast<unsigned long long>(__popc(m & (0x11111111u << k))) << (16 * k);
         return c;
+    };
+    auto mask_of = [&](int t) {
+        return g.order ? static_cast<uint32_t>(g.meta[g.order[t]].y) : g.masks[t];
     };
     // Sum over the row's threads of c, and before[]: the threads below.
     auto scan = [&](unsigned long long c, unsigned long long *before) {
@@ -129,41 +296,51 @@ __global__ __launch_bounds__(256) void scalar_rows_kernel(
     int total[4] = {0, 0, 0, 0};
     for (int t = t0; t < t1; t += T) {
         unsigned long long before;
-        const unsigned long long all =
-            scan(t + lt < t1 ? count(masks[t + lt]) : 0ull, &before);
+        const unsigned long long all = scan(t + lt < t1 ? count(mask_of(t + lt)) : 0ull, &before);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             total[k] += static_cast<int>(all >> (16 * k) & 0xFFFFull);
     }
-    if (!live)
-        return;   // a whole wave or workgroup
     int at[4];
-    int run = offs[t0];
+    int run = PLACED ? g.start[5 * static_cast<int64_t>(K)] : g.offs[t0];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         at[k] = run;
         run += total[k];
     }
-    if (lt < 5)
-        start[5 * static_cast<int64_t>(K) + lt] =
-            lt == 0 ? at[0] : (lt == 1 ? at[1] : (lt == 2 ? at[2] : (lt == 3 ? at[3] : run)));
+    if (lt > 0 && lt < 5)
+        g.start[5 * static_cast<int64_t>(K) + lt] =
+            lt == 1 ? at[1] : (lt == 2 ? at[2] : (lt == 3 ? at[3] : run));
+    if (!PLACED && lt == 0)
+        g.start[5 * static_cast<int64_t>(K)] = at[0];
     for (int t = t0; t < t1; t += T) {
-        const uint32_t m = t + lt < t1 ? masks[t + lt] : 0u;
+        uint32_t m = 0;
+        int off = 0, c0 = 0;
+        bool dense = false;
+        if (t + lt < t1) {
+            if (g.order) {
+                const int4 e = g.meta[g.order[t + lt]];
+                m = static_cast<uint32_t>(e.y);
+                off = e.w & 0x7FFFFFFF;
+                dense = e.w < 0;
+                c0 = 8 * e.x;
+            } else {
+                m = g.masks[t + lt];
+                off = g.offs[t + lt];
+                dense = g.offs[t + lt + 1] - off == 32;
+                c0 = 8 * g.tcol[t + lt];
+            }
+        }
         unsigned long long before;
         const unsigned long long all = scan(count(m), &before);
-        if (m) {
-            const int off = offs[t + lt];
-            const bool dense = offs[t + lt + 1] - off == 32;
-            const int c0 = 8 * tcol[t + lt];
-            int j = 0;
-            for (uint32_t x = m; x; x &= x - 1, ++j) {
-                const int phys = __builtin_ctz(x), k = phys & 3;
-                const int below = __popc(m & (0x11111111u << k) & ((1u << phys) - 1u));
-                const int base = k == 0 ? at[0] : (k == 1 ? at[1] : (k == 2 ? at[2] : at[3]));
-                const int p = base + static_cast<int>(before >> (16 * k) & 0xFFFFull) + below;
-                col[p] = c0 + (phys >> 2);
-                val[p] = vals[off + (dense ? phys : j)];
-            }
+        int j = 0;
+        for (uint32_t x = m; x; x &= x - 1, ++j) {
+            const int phys = __builtin_ctz(x), k = phys & 3;
+            const int below = __popc(m & (0x11111111u << k) & ((1u << phys) - 1u));
+            const int base = k == 0 ? at[0] : (k == 1 ? at[1] : (k == 2 ? at[2] : at[3]));
+            const int p = base + static_cast<int>(before >> (16 * k) & 0xFFFFull) + below;
+            g.col[p] = c0 + (phys >> 2);
+            g.val[p] = g.vals[off + (dense ? phys : j)];
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k)
@@ -171,10 +348,19 @@ __global__ __launch_bounds__(256) void scalar_rows_kernel(
     }
 }
 
+__global__ void zero_ints_kernel(int *__restrict__ p, int64_t n)
+{
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n)
+        p[i] = 0;
+}
+
 struct SlabOps {
     const int *__restrict__ a_row_off;   // A payload offset of each tile row
-    const int *__restrict__ a_k;         // per slot: column, -1 absent
-    const uint8_t *__restrict__ a_r;     // per slot: row within the tile
+    const int *__restrict__ a_code_off;  // first slot code of each listed row; null: as
+                                         // the payload's
+    const int *__restrict__ a_k;         // per slot code: column, -1 absent
+    const uint8_t *__restrict__ a_r;     // per slot code: row within the tile
     const double *__restrict__ a_vals;
     const int *__restrict__ b_start;     // scalar_rows_kernel's layout
     const int *__restrict__ b_col;
@@ -184,6 +370,10 @@ struct SlabOps {
     int static_rows;
     int2 *__restrict__ cursors;          // per workgroup: a run per slot of a long row
     int64_t cursor_stride;
+    __device__ int code_off(int row) const
+    {
+        return a_code_off ? a_code_off[row] : a_row_off[row];
+    }
 };
 
 // A workgroup's task: part `part` of `parts` of a tile row, cut by columns.
@@ -228,7 +418,8 @@ __device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_tas
     if (t->parts > 1) {
         // {entries, slot from the end}: the longest, the first of equals.
         unsigned long long best = 0;
-        const int s0 = o.a_row_off[t->row], s1 = o.a_row_off[t->row + 1];
+        const int s0 = o.code_off(t->row);
+        const int s1 = s0 + o.a_row_off[t->row + 1] - o.a_row_off[t->row];
         for (int x = s0 + static_cast<int>(threadIdx.x); x < s1; x += T) {
             const int k = o.a_k[x];
             if (k < 0)
@@ -273,7 +464,7 @@ __device__ __forceinline__ int first_at(const int *__restrict__ col, int lo, int
     return lo;
 }
 
-// Entries [*lo, *hi) of the B row that slot s of A selects, within the task.
+// Entries [*lo, *hi) of the B row that slot code s of A selects, within the task.
 __device__ __forceinline__ void slot_run(const SlabOps &o, const Task &t, int s, int *lo, int *hi)
 {
     const int k = o.a_k[s];
@@ -489,7 +680,8 @@ __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o
                 continue;
             }
         }
-        const int s0 = o.a_row_off[row], s1 = o.a_row_off[row + 1];
+        const int s0 = o.code_off(row);
+        const int s1 = s0 + o.a_row_off[row + 1] - o.a_row_off[row];
         const bool one = s1 - s0 <= kSymThreads;   // one chunk: cursors in registers
         int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
         int cur = 0, end = 0;
@@ -678,7 +870,9 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
             t0 += from;
             nt = to - from;
         }
-        const int s0 = o.a_row_off[row], s1 = o.a_row_off[row + 1];
+        const int s0 = o.code_off(row);
+        const int s1 = s0 + o.a_row_off[row + 1] - o.a_row_off[row];
+        const double *a_vals = o.a_vals + (static_cast<int64_t>(o.a_row_off[row]) - s0);
         const bool one = s1 - s0 <= kNumThreads;
         int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
         int cur = 0, end = 0, r = 0;
@@ -688,7 +882,7 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
             if (c0 + tid < s1) {
                 slot_run(o, task, c0 + tid, &cur, &end);
                 r = o.a_r[c0 + tid];
-                av = o.a_vals[c0 + tid];
+                av = a_vals[c0 + tid];
                 if (!one)
                     cursors[c0 - s0 + tid] = make_int2(cur, end);
             }
@@ -765,7 +959,7 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
                         cur = run.x;
                         end = run.y;
                         r = o.a_r[c0 + tid];
-                        av = o.a_vals[c0 + tid];
+                        av = a_vals[c0 + tid];
                     }
                 }
                 const int from = cur;
@@ -809,8 +1003,15 @@ static SlabOps slab_ops(const DevTiles &a, const SpgemmWork *w, const SlabTasks 
 {
     SlabOps o;
     o.a_row_off = a.row_payload_off.as<int>();
-    o.a_k = w->slot_k.as<int>();
-    o.a_r = w->slot_r.as<uint8_t>();
+    if (w->slot_codes_ready) {
+        o.a_code_off = nullptr;
+        o.a_k = w->slot_k.as<int>();
+        o.a_r = w->slot_r.as<uint8_t>();
+    } else {
+        o.a_code_off = w->code_off.as<int>();
+        o.a_k = w->row_slot_k.as<int>();
+        o.a_r = w->row_slot_r.as<uint8_t>();
+    }
     o.a_vals = a.values.as<double>();
     o.b_start = w->b_start.as<int>();
     o.b_col = w->b_col.as<int>();
@@ -874,40 +1075,118 @@ static int slab_cursors(SpgemmWork *w, int64_t longest)
     return RTT_OK;
 }
 
-int slab_prepare(const DevTiles &a, DevTiles *b, BuildWork *bw, SpgemmWork *w)
+int slab_prepare(const DevTiles &a, const DevTiles &b, BuildWork *bw, SpgemmWork *w,
+                 const int *rows, int n, const int *more, int n_more, int64_t longest)
 {
     hipStream_t s = ctx().stream;
-    if (!w->slot_codes_ready) {
-        RTT_TRY(w->slot_k.ensure(static_cast<size_t>(a.payload > 0 ? a.payload : 1) * sizeof(int)));
-        RTT_TRY(w->slot_r.ensure(static_cast<size_t>(a.payload > 0 ? a.payload : 1)));
-        if (a.num_tiles > 0)
-            hipLaunchKernelGGL(slot_codes_kernel, dim3(blocks_for(a.num_tiles, 256)), dim3(256), 0,
-                               s, a.num_tiles, a.meta.as<int4>(), w->slot_k.as<int>(),
-                               w->slot_r.as<uint8_t>());
+    const int R = b.tile_row_count;
+    const int listed = n + n_more;
+    if (R == 0 || listed == 0)
+        return RTT_OK;
+    // Few rows are served by their own slots and the rows of B they select, for
+    // a host wait; many select most of B.  64^3 box stencil (6.9e6 entries, 32768
+    // tile rows) with 64, 512, 2048 and 4096 wide rows, A*A: 1.12, 1.32, 1.88
+    // and 2.33 ms with all of B, 1.01, 1.25, 1.86 and 2.35 ms with the rows
+    // selected; A*A^T: 1.07, 1.45, 2.01, 2.55 and 0.85, 1.33, 2.02, 2.60.  One
+    // row of 60 entries more in the 128^3 stencil, A*A^T: 6.78 -> 3.75 ms (3.52
+    // without it).  By slots, a hub of 10000, 100000 and 300000 entries in a
+    // 1000^2 Laplacian: 2.81, 7.94, 15.3 and 2.70, 7.79, 15.4 ms.
+    const bool few = static_cast<int64_t>(listed) * 16 < a.tile_row_count &&
+                     listed * longest * 16 < a.payload;
+    const bool transposed = b.transpose_of != nullptr;
+    const size_t rows_b = static_cast<size_t>(R), rows_a = static_cast<size_t>(a.tile_row_count);
+    RTT_TRY(w->b_start.ensure((rows_b * 5 + 1) * sizeof(int)));
+    BRows g{};
+    g.R = R;
+    g.trp = b.tile_row_ptr.as<int>();
+    g.groups = b.row_groups.as<int>();
+    g.meta = b.records.as<int4>();
+    g.tcol = b.tile_col_idx.as<int>();
+    g.masks = b.masks.as<uint32_t>();
+    g.offs = b.value_offsets.as<int>();
+    g.vals = b.payload_values();
+    g.start = w->b_start.as<int>();
+    if (transposed) {
+        // B = A^T at tile level has its rows in class order alone.
+        RTT_TRY(bw->keys_in.ensure(static_cast<size_t>(std::max<int64_t>(1, b.num_tiles)) *
+                                   sizeof(int)));
+        g.order = bw->keys_in.as<int>();
+    }
+    // A workgroup per tile row where rows average past 16 tiles (a hub row
+    // holds thousands), a wave otherwise.
+    const bool wide = b.num_tiles > 16 * static_cast<int64_t>(R);
+    auto over_rows = [&](auto wave_kernel, auto block_kernel, int64_t count, auto... args) {
+        if (wide)
+            hipLaunchKernelGGL(block_kernel, dim3(static_cast<unsigned>(count)), dim3(256), 0, s, g,
+                               args...);
+        else
+            hipLaunchKernelGGL(wave_kernel, dim3(blocks_for(count, 256 / kWave)), dim3(256), 0, s, g,
+                               args...);
+    };
+    int64_t count = R;             // B rows laid out (to be looked at, while it isn't known)
+    int64_t entries = b.payload;   // at most
+    Picked *picked = nullptr;
+    if (few || transposed) {
+        constexpr size_t kHeadInts = sizeof(Picked) / sizeof(int);
+        RTT_TRY(w->slab_pick.ensure((kHeadInts + 2 * rows_b) * sizeof(int)));
+        picked = w->slab_pick.as<Picked>();
+        int *flag = w->slab_pick.as<int>() + kHeadInts, *list = flag + R;
+        const int64_t clear = static_cast<int64_t>(kHeadInts) + (few ? R : 0);
+        hipLaunchKernelGGL(zero_ints_kernel, dim3(blocks_for(clear, 256)), dim3(256), 0, s,
+                           w->slab_pick.as<int>(), clear);
+        if (few) {
+            const size_t slots = static_cast<size_t>(listed * longest);
+            const bool codes = !w->slot_codes_ready;
+            if (codes) {
+                RTT_TRY(w->code_off.ensure(rows_a * sizeof(int)));
+                RTT_TRY(w->row_slot_k.ensure(slots * sizeof(int)));
+                RTT_TRY(w->row_slot_r.ensure(slots));
+            }
+            hipLaunchKernelGGL(pick_rows_kernel, dim3(static_cast<unsigned>(listed), 4), dim3(256),
+                               0, s, rows, n, more, longest, a.tile_row_ptr.as<int>(),
+                               a.meta.as<int4>(), a.row_payload_off.as<int>(), flag,
+                               codes ? w->code_off.as<int>() : nullptr,
+                               codes ? w->row_slot_k.as<int>() : nullptr,
+                               codes ? w->row_slot_r.as<uint8_t>() : nullptr);
+            hipLaunchKernelGGL(list_rows_kernel, dim3(blocks_for(R, 256)), dim3(256), 0, s, R, flag,
+                               picked, list);
+            g.list = list;
+            g.n = &picked->rows;
+            count = std::min<int64_t>(R, listed * longest);
+        }
+        if (transposed)
+            over_rows(count_rows_kernel<kWave>, count_rows_kernel<256>, count);
+        hipLaunchKernelGGL(place_rows_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, s, g,
+                           picked);
+        RTT_HIP(hipGetLastError());
+    }
+    if (few) {
+        RTT_TRY(w->host_pick.ensure(sizeof(Picked)));
+        RTT_HIP(hipMemcpyAsync(w->host_pick.ptr, picked, sizeof(Picked), hipMemcpyDeviceToHost, s));
+        RTT_HIP(hipStreamSynchronize(s));
+        count = static_cast<int64_t>(w->host_pick.as<Picked>()->rows);
+        entries = static_cast<int64_t>(w->host_pick.as<Picked>()->entries);
+    } else if (!w->slot_codes_ready) {
+        RTT_TRY(w->slot_k.ensure(static_cast<size_t>(std::max<int64_t>(1, a.payload)) * sizeof(int)));
+        RTT_TRY(w->slot_r.ensure(static_cast<size_t>(std::max<int64_t>(1, a.payload))));
+        hipLaunchKernelGGL(slot_codes_kernel, dim3(blocks_for(a.num_tiles, 256)), dim3(256), 0, s,
+                           a.num_tiles, a.meta.as<int4>(), w->slot_k.as<int>(),
+                           w->slot_r.as<uint8_t>());
         RTT_HIP(hipGetLastError());
         w->slot_codes_ready = true;
     }
-    // B = A^T at tile level has its column-ordered arrays only on request.
-    if (b->transpose_of)
-        RTT_TRY(materialize_tiles(b, bw));
-    const int R = b->tile_row_count;
-    const size_t n = static_cast<size_t>(b->payload > 0 ? b->payload : 1);
-    RTT_TRY(w->b_start.ensure((static_cast<size_t>(R) * 5 + 1) * sizeof(int)));
-    RTT_TRY(w->b_col.ensure(n * sizeof(int)));
-    RTT_TRY(w->b_val.ensure(n * sizeof(double)));
-    auto launch = [&](auto kernel, int per) {
-        hipLaunchKernelGGL(kernel, dim3(blocks_for(R, per)), dim3(256), 0, s, R,
-                           b->tile_row_ptr.as<int>(), b->tile_col_idx.as<int>(),
-                           b->masks.as<uint32_t>(), b->value_offsets.as<int>(),
-                           b->values.as<double>(), w->b_start.as<int>(), w->b_col.as<int>(),
-                           w->b_val.as<double>());
-    };
-    // A workgroup per tile row where rows average past 16 tiles (a hub row
-    // holds thousands), a wave otherwise.
-    if (R > 0 && b->num_tiles > 16 * static_cast<int64_t>(R))
-        launch(scalar_rows_kernel<256>, 1);
-    else if (R > 0)
-        launch(scalar_rows_kernel<kWave>, 256 / kWave);
+    RTT_TRY(w->b_col.ensure(static_cast<size_t>(std::max<int64_t>(1, entries)) * sizeof(int)));
+    RTT_TRY(w->b_val.ensure(static_cast<size_t>(std::max<int64_t>(1, entries)) * sizeof(double)));
+    g.col = w->b_col.as<int>();
+    g.val = w->b_val.as<double>();
+    if (count == 0)
+        return RTT_OK;
+    if (transposed)
+        over_rows(order_tiles_kernel<kWave>, order_tiles_kernel<256>, count, bw->keys_in.as<int>());
+    if (picked)
+        over_rows(scalar_rows_kernel<kWave, true>, scalar_rows_kernel<256, true>, count);
+    else
+        over_rows(scalar_rows_kernel<kWave, false>, scalar_rows_kernel<256, false>, count);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }

@@ -1678,8 +1678,12 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     const int static_rows = lb_mode == RTT_LB_STATIC ? 1 : 0;
     const bool by_cost = lb_mode == RTT_LB_ADAPTIVE_TAIL;
     SlabTasks tasks;
+    // Rows for the slab kernels: those that outgrew both tables, and those whose
+    // C outgrows the numeric kernels'.
+    RTT_TRY(slab_prepare(a, b, b_work, w, w->sym_slab_rows.as<int>(), n_slab, lists.rows[kRowSlab],
+                         static_cast<int>(hctr[kCtrRows + kRowSlab]),
+                         static_cast<int64_t>(hctr[kCtrLongest])));
     if (n_slab > 0) {
-        RTT_TRY(slab_prepare(a, &b, b_work, w));
         RTT_TRY(plan_slab_tasks(w->sym_slab_rows.as<int>(), n_slab, by_cost, hctr[kCtrPairs], g, w,
                                 s, &tasks));
         RTT_TRY(slab_symbolic(a, w, tasks, queue, static_rows, ctr + kCtrSlabTiles,
@@ -1821,8 +1825,6 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     rows_launch(numeric_row_kernel<MediumRow>, kRowMid, MediumRow::kThreads, false);
     rows_launch(numeric_row_kernel<LargeRow>, kRowLarge, LargeRow::kThreads, false);
     if (n_num_slab > 0) {
-        if (n_slab == 0)
-            RTT_TRY(slab_prepare(a, &b, b_work, w));
         // The structure pass above is queued before this plan reuses its arrays.
         RTT_TRY(plan_slab_tasks(lists.rows[kRowSlab], n_num_slab, by_cost, pairs, g, w, s, &tasks));
         RTT_TRY(slab_numeric(a, w, tasks, queue + 2, static_rows, co,
