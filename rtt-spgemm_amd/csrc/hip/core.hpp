@@ -18,6 +18,42 @@ struct COut {
     double *__restrict__ val;
 };
 
+__device__ __forceinline__ uint32_t byte_of(uint32_t v, int k) { return (v >> (8 * k)) & 0xFFu; }
+
+// Byte k is nonzero where byte k of v is (its bit 7 set).
+__device__ __forceinline__ uint32_t nonzero_tops(uint32_t v)
+{
+    return (((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v) & 0x80808080u;
+}
+
+// An A tile spread for products with many B tiles: word k of lo (hi) is 0xFF
+// in byte r where row r (row 4 + r) has an entry in column k.
+__device__ __forceinline__ void spread_tile(uint32_t ab, uint4 *lo, uint4 *hi)
+{
+    uint64_t s[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        s[k] = rows_to_bytes(byte_of(ab, k));
+    *lo = make_uint4(static_cast<uint32_t>(s[0]), static_cast<uint32_t>(s[1]),
+                     static_cast<uint32_t>(s[2]), static_cast<uint32_t>(s[3]));
+    *hi = make_uint4(static_cast<uint32_t>(s[0] >> 32), static_cast<uint32_t>(s[1] >> 32),
+                     static_cast<uint32_t>(s[2] >> 32), static_cast<uint32_t>(s[3] >> 32));
+}
+
+// Structural product of a spread A tile and the per-k column bytes of a B
+// tile: byte k of b_bytes to every byte of a word, then a bitwise select each.
+__device__ __forceinline__ uint64_t spread_product(const uint4 &lo, const uint4 &hi,
+                                                   uint32_t b_bytes)
+{
+    const uint32_t b0 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x00000000u);
+    const uint32_t b1 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x01010101u);
+    const uint32_t b2 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x02020202u);
+    const uint32_t b3 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x03030303u);
+    const uint32_t l = (lo.x & b0) | (lo.y & b1) | (lo.z & b2) | (lo.w & b3);
+    const uint32_t h = (hi.x & b0) | (hi.y & b1) | (hi.z & b2) | (hi.w & b3);
+    return (static_cast<uint64_t>(h) << 32) | l;
+}
+
 // Byte r of the result is the number of set bits in bytes 0..r-1 of m (the
 // u8 row offsets of a C tile): per-byte popcounts, then an exclusive byte
 // prefix sum by multiplication (sums stay below 256, so no byte carries).
@@ -122,14 +158,21 @@ int64_t slab_target(unsigned long long pairs);
 // Workgroups of a slab pass whose longest row has `longest` slots, with `held`
 // bytes of cursors there and `free_bytes` of device memory free.
 unsigned slab_cursor_blocks(int64_t longest, size_t held, size_t free_bytes);
+// Rows listed: most slots of A's payload and most tiles of A in one of them, and
+// those of all.
+struct SlabSizes {
+    int64_t longest = 0, most_tiles = 0, slots = 0, tiles = 0;
+};
+// Whether the symbolic passes of such rows go by tiles: they then need no
+// slab_prepare.
+bool slab_by_tiles(const DevTiles &b, const SlabSizes &rows);
 // Counts the listed rows' tiles and entries into w->row_tiles / row_nnz and
-// stages their tile lists; *cursor sums what the staging needs.  longest:
-// most slots of A's payload in one of the rows.
-int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
-                  int static_rows, unsigned long long *cursor, int64_t longest);
+// stages their tile lists; *cursor sums what the staging needs.
+int slab_symbolic(const DevTiles &a, const DevTiles &b, SpgemmWork *w, const SlabTasks &tasks,
+                  int *queue, int static_rows, unsigned long long *cursor, const SlabSizes &rows);
 // Writes the structure of the rows slab_symbolic counted.
-int slab_structure(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
-                   int static_rows, const COut &c);
+int slab_structure(const DevTiles &a, const DevTiles &b, SpgemmWork *w, const SlabTasks &tasks,
+                   int *queue, int static_rows, const COut &c);
 // Values of the listed rows, whose structure is written.
 int slab_numeric(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
                  int static_rows, const COut &c, int64_t longest);

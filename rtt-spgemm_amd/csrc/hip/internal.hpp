@@ -188,10 +188,11 @@ struct SpgemmWork {
     // long rows.
     DevBuf slot_k, slot_r, b_start, b_col, b_val, slab_cursors;
     bool slot_codes_ready = false;          // slot_k and slot_r hold all of A's
-    DevBuf row_slot_k, row_slot_r, code_off;
+    DevBuf row_slot_k, row_slot_r, row_slot_v, code_off;
     DevBuf slab_pick;                       // B rows that a few slab rows select
     PinnedBuf host_pick;
     int64_t slab_cursor_stride = 0;         // of the last slab pass: slots per workgroup
+    bool slab_by_tiles = false;             // its symbolic passes go by tiles
     unsigned slab_cursor_blocks = 0;        // and the workgroups that have cursors
     // Slab rows' (column, mask) lists between the symbolic passes: entries
     // allocated, and the most the previous calls needed (grown at the next

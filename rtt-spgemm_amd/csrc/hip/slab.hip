@@ -20,7 +20,8 @@
 // product p of the window finds its thread with one word and one count.
 // Consecutive lanes so take consecutive entries of a B row.
 //  * symbolic: the window's C tile masks are ORed in LDS, then counted and
-//    appended to the staged lists, or written to C's structure.
+//    appended to the staged lists, or written to C's structure.  Operands whose
+//    tiles are well filled go tile by tile here (slab_by_tiles).
 //  * numeric: the window's C tiles (masks and first values) lie in LDS, found
 //    by a bit per tile column and a count of those before each word, and their
 //    values accumulate in LDS in C's order, to be stored once, whatever the
@@ -49,13 +50,16 @@ constexpr int kSymThreads = 512;               // symbolic pass: two workgroups 
 constexpr int kNumThreads = 1024;              // numeric pass: one, with all of its LDS
 constexpr int kSubProducts = 16384;            // products numbered by the bit words at once
 constexpr int kSubWords = kSubProducts / 64;
-constexpr int kSymWin = 8192;                  // C tile columns of a symbolic window
+constexpr int kSymWin = 8192;                  // C tile columns of a symbolic window,
+constexpr int kTileWin = 4096;                 // of one by tiles
+constexpr double kTileProducts = 2.0;          // products a pair of tiles from which it does
 constexpr int kFillBytes = 8192;               // column bytes of C staged at a time
 constexpr int kNumSpan = 32768;                // C tile columns a numeric window may span,
 constexpr int kNumTiles = 3072;                // C tiles it may hold,
 constexpr int kNumVals = 13312;                // and C values
 constexpr int kNumWords = kNumSpan / 64;
 constexpr int kLookTiles = kNumTiles / kNumThreads;   // C tiles a thread looks at per window
+constexpr int kRuns = 5;                       // classes of a row of B: heavy, light k = 0..3
 constexpr int kUnroll = 4;                     // products a thread loads together
 static_assert(kSubWords <= 4 * kWave, "one wave ranks the bit words");
 static_assert(kNumVals <= 65536 - 64 && kNumTiles <= 65536, "16-bit value and tile positions");
@@ -96,13 +100,14 @@ struct Picked {
 };
 
 // Listed rows of two lists; workgroups x, y take every gridDim.y-th 256 A tiles
-// of row x: the slot codes of its A payload, `stride` slots from the row before
-// it, and a flag for every B tile row it selects.
+// of row x: the slot codes and values of its A payload, `stride` slots from the
+// row before it, and a flag for every B tile row it selects.
 __global__ __launch_bounds__(256) void pick_rows_kernel(
     const int *__restrict__ rows, int n, const int *__restrict__ more, int64_t stride,
     const int *__restrict__ a_trp, const int4 *__restrict__ a_meta,
-    const int *__restrict__ a_row_off, int *__restrict__ flag, int *__restrict__ code_off,
-    int *__restrict__ k, uint8_t *__restrict__ r)
+    const int *__restrict__ a_row_off, const double *__restrict__ a_vals, int *__restrict__ flag,
+    int *__restrict__ code_off, int *__restrict__ k, uint8_t *__restrict__ r,
+    double *__restrict__ v)
 {
     const int i = blockIdx.x;
     const int row = i < n ? rows[i] : more[i - n];
@@ -114,8 +119,13 @@ __global__ __launch_bounds__(256) void pick_rows_kernel(
          t += static_cast<int>(gridDim.y) * 256) {
         const int4 m = a_meta[t];
         flag[m.x] = 1;
-        if (k)
-            write_slot_codes(m, shift + (m.w & 0x7FFFFFFF), k, r);
+        if (k) {
+            const int off = m.w & 0x7FFFFFFF;
+            write_slot_codes(m, shift + off, k, r);
+            const int slots = m.w < 0 ? 32 : __popc(static_cast<uint32_t>(m.y));
+            for (int j = 0; j < slots; ++j)
+                v[shift + off + j] = a_vals[off + j];
+        }
     }
 }
 
@@ -222,7 +232,6 @@ __global__ __launch_bounds__(256) void order_tiles_kernel(BRows g, int *__restri
     if (K < 0)
         return;
     const int *gp = g.groups + static_cast<int64_t>(kClassSlots) * K;
-    constexpr int kRuns = 5;   // heavy, light k = 0..3
     int at[kRuns + 1];
 #pragma unroll
     for (int c = 0; c <= kRuns; ++c)
@@ -356,12 +365,15 @@ __global__ void zero_ints_kernel(int *__restrict__ p, int64_t n)
 }
 
 struct SlabOps {
+    const int *__restrict__ a_trp;       // A's and B's tiles, for the pass by tiles
+    const int4 *__restrict__ a_meta;
+    const int4 *__restrict__ b_meta;
+    const int *__restrict__ b_groups;
     const int *__restrict__ a_row_off;   // A payload offset of each tile row
-    const int *__restrict__ a_code_off;  // first slot code of each listed row; null: as
-                                         // the payload's
+    const int *__restrict__ a_code_off;  // first slot code of each tile row
     const int *__restrict__ a_k;         // per slot code: column, -1 absent
     const uint8_t *__restrict__ a_r;     // per slot code: row within the tile
-    const double *__restrict__ a_vals;
+    const double *__restrict__ a_vals;   // per slot code
     const int *__restrict__ b_start;     // scalar_rows_kernel's layout
     const int *__restrict__ b_col;
     const double *__restrict__ b_val;
@@ -370,9 +382,58 @@ struct SlabOps {
     int static_rows;
     int2 *__restrict__ cursors;          // per workgroup: a run per slot of a long row
     int64_t cursor_stride;
-    __device__ int code_off(int row) const
+};
+
+// What a thread takes of a tile row, [first, first + count) of them, and the run
+// of B it selects, by ascending column: a slot of A's payload with a scalar row
+// of B (BY_TILES false), or a tile of A with one class of the tiles of its row of
+// B.  at(e) is the column of B's entry (tile) e.
+template <bool BY_TILES>
+struct Slots;
+
+template <>
+struct Slots<false> {
+    static constexpr int kToTile = 3;   // at(e) >> kToTile: its tile column
+    __device__ static int first(const SlabOps &o, int row) { return o.a_code_off[row]; }
+    __device__ static int count(const SlabOps &o, int row)
     {
-        return a_code_off ? a_code_off[row] : a_row_off[row];
+        return o.a_row_off[row + 1] - o.a_row_off[row];
+    }
+    __device__ static int at(const SlabOps &o, int64_t e) { return o.b_col[e]; }
+    __device__ static void run(const SlabOps &o, int, int x, int *lo, int *hi)
+    {
+        const int k = o.a_k[x];
+        *lo = *hi = 0;
+        if (k >= 0) {
+            const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
+            *lo = p[0];
+            *hi = p[1];
+        }
+    }
+};
+
+template <>
+struct Slots<true> {
+    static constexpr int kToTile = 0;
+    __device__ static int first(const SlabOps &, int) { return 0; }
+    __device__ static int count(const SlabOps &o, int row)
+    {
+        return kRuns * (o.a_trp[row + 1] - o.a_trp[row]);
+    }
+    __device__ static int at(const SlabOps &o, int64_t e) { return o.b_meta[e].x; }
+    __device__ static int4 tile(const SlabOps &o, int row, int x)
+    {
+        return o.a_meta[o.a_trp[row] + x / kRuns];
+    }
+    __device__ static void run(const SlabOps &o, int row, int x, int *lo, int *hi)
+    {
+        const int4 m = tile(o, row, x);
+        const int c = x % kRuns;
+        const int *p = o.b_groups + static_cast<int64_t>(kClassSlots) * m.x + c;
+        *lo = *hi = p[0];
+        // A light tile of row k meets the tiles with entries in column k alone.
+        if (c == 0 || byte_of(static_cast<uint32_t>(m.z), c - 1))
+            *hi = p[1];
     }
 };
 
@@ -386,7 +447,7 @@ struct Task {
 // are quantiles of the longest B row it selects: hub columns hold most of a
 // power-law row's products, and equal stretches of columns would leave most
 // of them in the first part.
-template <int T>
+template <int T, class S>
 __device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_task,
                                           unsigned long long *s_long, Task *t)
 {
@@ -407,26 +468,26 @@ __device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_tas
         *s_long = 0ull;
     }
     __syncthreads();
-    t->id = s_task[0];
-    t->row = s_task[1];
+    // The same in every lane: scalar registers.
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    t->id = uniform(s_task[0]);
+    t->row = uniform(s_task[1]);
     if (t->row < 0)
         return false;
-    t->part = s_task[2];
-    t->parts = s_task[3];
+    t->part = uniform(s_task[2]);
+    t->parts = uniform(s_task[3]);
     t->lo = 0;
     t->hi = INT64_MAX;
     if (t->parts > 1) {
         // {entries, slot from the end}: the longest, the first of equals.
         unsigned long long best = 0;
-        const int s0 = o.code_off(t->row);
-        const int s1 = s0 + o.a_row_off[t->row + 1] - o.a_row_off[t->row];
+        const int s0 = S::first(o, t->row), s1 = s0 + S::count(o, t->row);
         for (int x = s0 + static_cast<int>(threadIdx.x); x < s1; x += T) {
-            const int k = o.a_k[x];
-            if (k < 0)
-                continue;
-            const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
-            best = max(best, (static_cast<unsigned long long>(p[1] - p[0]) << 32) |
-                                 static_cast<uint32_t>(s1 - x));
+            int lo, hi;
+            S::run(o, t->row, x, &lo, &hi);
+            if (lo < hi)
+                best = max(best, (static_cast<unsigned long long>(hi - lo) << 32) |
+                                     static_cast<uint32_t>(s1 - x));
         }
 #pragma unroll
         for (int d = kWave / 2; d > 0; d >>= 1)
@@ -434,29 +495,30 @@ __device__ __forceinline__ bool next_task(const SlabOps &o, int step, int *s_tas
         if (lane_id() == 0)
             atomicMax(s_long, best);
         __syncthreads();
-        const int x = s1 - static_cast<int>(*s_long & 0xFFFFFFFFull);
         if (*s_long != 0) {
-            const int k = o.a_k[x];
-            const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
-            const int64_t len = p[1] - p[0];
+            int lo, hi;
+            S::run(o, t->row, s1 - static_cast<int>(*s_long & 0xFFFFFFFFull), &lo, &hi);
+            const int64_t len = hi - lo;
             auto cut = [&](int q) {
-                return static_cast<int64_t>(o.b_col[p[0] + len * q / t->parts]) & ~int64_t(7);
+                return static_cast<int64_t>(S::at(o, lo + static_cast<int>(len * q / t->parts)) >>
+                                            S::kToTile) * 8;
             };
-            if (len > 0 && t->part > 0)
+            if (t->part > 0)
                 t->lo = cut(t->part);
-            if (len > 0 && t->part + 1 < t->parts)
+            if (t->part + 1 < t->parts)
                 t->hi = cut(t->part + 1);
         }
     }
     return true;
 }
 
-// First entry of [lo, hi) whose column is >= lim.
-__device__ __forceinline__ int first_at(const int *__restrict__ col, int lo, int hi, int64_t lim)
+// First entry of [lo, hi) with at(entry) >= lim.
+template <class At>
+__device__ __forceinline__ int first_at(At &&at, int lo, int hi, int64_t lim)
 {
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (col[mid] < lim)
+        if (at(mid) < lim)
             lo = mid + 1;
         else
             hi = mid;
@@ -464,37 +526,30 @@ __device__ __forceinline__ int first_at(const int *__restrict__ col, int lo, int
     return lo;
 }
 
-// Entries [*lo, *hi) of the B row that slot code s of A selects, within the task.
-__device__ __forceinline__ void slot_run(const SlabOps &o, const Task &t, int s, int *lo, int *hi)
+// Entries [*lo, *hi) of the B row that slot x of A selects, within the task.
+template <class S>
+__device__ __forceinline__ void slot_run(const SlabOps &o, const Task &t, int x, int *lo, int *hi)
 {
-    const int k = o.a_k[s];
-    *lo = *hi = 0;
-    if (k >= 0) {
-        const int *p = o.b_start + 5 * static_cast<int64_t>(k >> 2) + (k & 3);
-        *lo = t.part > 0 ? first_at(o.b_col, p[0], p[1], t.lo) : p[0];
-        *hi = t.part + 1 < t.parts ? first_at(o.b_col, *lo, p[1], t.hi) : p[1];
-    }
+    S::run(o, t.row, x, lo, hi);
+    auto at = [&](int64_t e) { return S::at(o, e); };
+    if (t.part > 0)
+        *lo = first_at(at, *lo, *hi, t.lo >> (3 - S::kToTile));
+    if (t.part + 1 < t.parts)
+        *hi = first_at(at, *lo, *hi, t.hi >> (3 - S::kToTile));
 }
 
-// First entry at or after a, below end, whose column is >= lim: doubling
+// First entry at or after a, below end, with at(entry) >= lim: doubling
 // steps, then a binary search in the last one.
-__device__ __forceinline__ int gallop(const int *__restrict__ col, int a, int end, int64_t lim)
+template <class At>
+__device__ __forceinline__ int gallop(At &&at, int a, int end, int64_t lim)
 {
     int lo = a;
     int64_t step = 1;
-    while (lo + step <= end && col[lo + step - 1] < lim) {
+    while (lo + step <= end && at(lo + step - 1) < lim) {
         lo += static_cast<int>(step);
         step <<= 1;
     }
-    int hi = static_cast<int>(min<int64_t>(lo + step - 1, end));
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (col[mid] < lim)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
+    return first_at(at, lo, static_cast<int>(min<int64_t>(lo + step - 1, end)), lim);
 }
 
 // *at = min(*at, v) over the workgroup's threads (one LDS atomic per wave).
@@ -601,13 +656,16 @@ struct SlabStage {
     unsigned long long capacity = 0;
 };
 
-template <bool FILL>
+template <bool FILL, bool BY_TILES>
 __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o,
                                                                      int64_t *__restrict__ row_tiles,
                                                                      int64_t *__restrict__ row_nnz,
                                                                      SlabStage ss, COut c)
 {
-    __shared__ unsigned long long s_wm[kSymWin];
+    using S = Slots<BY_TILES>;
+    constexpr int kWin = BY_TILES ? kTileWin : kSymWin;
+    __shared__ unsigned long long s_wm[kWin];
+    __shared__ uint4 s_tile[2 * (BY_TILES ? kSymThreads : 1)];   // spread_tile of every run's A tile
     __shared__ Runs<kSymThreads> s;
     __shared__ int s_min[2];
     __shared__ long long s_base;
@@ -615,12 +673,12 @@ __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o
     __shared__ unsigned long long s_long;
     __shared__ __align__(4) unsigned char s_bytes[FILL ? kFillBytes + 4 : 4];
     const int tid = threadIdx.x;
-    constexpr int kPer = kSymWin / kSymThreads;
-    for (int i = tid; i < kSymWin; i += kSymThreads)
+    constexpr int kPer = kWin / kSymThreads;
+    for (int i = tid; i < kWin; i += kSymThreads)
         s_wm[i] = 0ull;
     for (int step = 0;; ++step) {
         Task task;
-        if (!next_task<kSymThreads>(o, step, s_task, &s_long, &task))
+        if (!next_task<kSymThreads, S>(o, step, s_task, &s_long, &task))
             break;
         const int row = task.row;
         int64_t tb = 0, zb = 0;
@@ -680,8 +738,7 @@ __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o
                 continue;
             }
         }
-        const int s0 = o.code_off(row);
-        const int s1 = s0 + o.a_row_off[row + 1] - o.a_row_off[row];
+        const int s0 = S::first(o, row), s1 = s0 + S::count(o, row);
         const bool one = s1 - s0 <= kSymThreads;   // one chunk: cursors in registers
         int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
         int cur = 0, end = 0;
@@ -691,8 +748,8 @@ __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o
         for (int c0 = s0; c0 < s1; c0 += kSymThreads) {
             cur = end = 0;
             if (c0 + tid < s1)
-                slot_run(o, task, c0 + tid, &cur, &end);
-            lds_min(&s_min[0], cur < end ? o.b_col[cur] : INT_MAX);
+                slot_run<S>(o, task, c0 + tid, &cur, &end);
+            lds_min(&s_min[0], cur < end ? S::at(o, cur) : INT_MAX);
             if (!one && c0 + tid < s1)
                 cursors[c0 - s0 + tid] = make_int2(cur, end);
         }
@@ -709,8 +766,8 @@ __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o
             if (tid == 0)
                 s_min[w ^ 1] = INT_MAX;
             __syncthreads();
-            const int wlo = first >> 3;
-            const int64_t lim = (static_cast<int64_t>(wlo) + kSymWin) * 8;
+            const int wlo = first >> S::kToTile;
+            const int64_t lim = (static_cast<int64_t>(wlo) + kWin) << S::kToTile;
             for (int c0 = s0; c0 < s1; c0 += kSymThreads) {
                 int r = 0;
                 if (!one) {
@@ -721,22 +778,43 @@ __global__ __launch_bounds__(kSymThreads, 4) void symbolic_slab_kernel(SlabOps o
                         end = run.y;
                     }
                 }
-                if (c0 + tid < s1)
-                    r = o.a_r[c0 + tid];
+                if constexpr (!BY_TILES) {
+                    if (c0 + tid < s1)
+                        r = o.a_r[c0 + tid];
+                }
                 const int from = cur;
                 if (cur < end)
-                    cur = gallop(o.b_col, cur, end, lim);
-                lds_min(&s_min[w ^ 1], cur < end ? o.b_col[cur] : INT_MAX);
+                    cur = gallop([&](int64_t e) { return S::at(o, e); }, cur, end, lim);
+                lds_min(&s_min[w ^ 1], cur < end ? S::at(o, cur) : INT_MAX);
                 if (!one && c0 + tid < s1)
                     cursors[c0 - s0 + tid].x = cur;
-                for_products<int>(
-                    s, cur - from, from, r, [](int) {}, [&](int e) { return o.b_col[e]; },
-                    [&](int i, int col) {
-                        const int t = (col >> 3) - wlo;
-                        const int rr = s.r[i];
-                        atomicOr(reinterpret_cast<unsigned int *>(&s_wm[t]) + (rr >> 2),
-                                 1u << ((rr & 3) * 8 + (col & 7)));
-                    });
+                if constexpr (BY_TILES) {
+                    uint4 lo{}, hi{};
+                    if (from < cur)
+                        spread_tile(static_cast<uint32_t>(S::tile(o, row, c0 + tid).z), &lo, &hi);
+                    for_products<int4>(
+                        s, cur - from, from, 0,
+                        [&](int i) {
+                            s_tile[i] = lo;
+                            s_tile[kSymThreads + i] = hi;
+                        },
+                        [&](int e) { return o.b_meta[e]; },
+                        [&](int i, const int4 &m) {
+                            const uint64_t pm = spread_product(s_tile[i], s_tile[kSymThreads + i],
+                                                               static_cast<uint32_t>(m.z));
+                            if (pm)
+                                atomicOr(&s_wm[m.x - wlo], static_cast<unsigned long long>(pm));
+                        });
+                } else {
+                    for_products<int>(
+                        s, cur - from, from, r, [](int) {}, [&](int e) { return o.b_col[e]; },
+                        [&](int i, int col) {
+                            const int t = (col >> 3) - wlo;
+                            const int rr = s.r[i];
+                            atomicOr(reinterpret_cast<unsigned int *>(&s_wm[t]) + (rr >> 2),
+                                     1u << ((rr & 3) * 8 + (col & 7)));
+                        });
+                }
             }
             // A wave's stretch of the window's masks, 64 at a time, counted
             // and cleared.
@@ -856,23 +934,22 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
         s_acc[i] = 0.0;
     for (int step = 0;; ++step) {
         Task task;
-        if (!next_task<kNumThreads>(o, step, s_task, &s_long, &task))
+        if (!next_task<kNumThreads, Slots<false>>(o, step, s_task, &s_long, &task))
             break;
         const int row = task.row;
         int64_t t0 = c.tile_ptr[row];
         int64_t nt = c.tile_ptr[row + 1] - t0;
         if (task.parts > 1) {
             // The part's C tiles.
-            const int *cols = c.col + t0;
+            auto cols = [at = c.col + t0](int t) { return at[t]; };
             const int n = static_cast<int>(nt);
             const int from = task.part > 0 ? first_at(cols, 0, n, task.lo >> 3) : 0;
             const int to = task.part + 1 < task.parts ? first_at(cols, from, n, task.hi >> 3) : n;
             t0 += from;
             nt = to - from;
         }
-        const int s0 = o.code_off(row);
+        const int s0 = o.a_code_off[row];
         const int s1 = s0 + o.a_row_off[row + 1] - o.a_row_off[row];
-        const double *a_vals = o.a_vals + (static_cast<int64_t>(o.a_row_off[row]) - s0);
         const bool one = s1 - s0 <= kNumThreads;
         int2 *cursors = o.cursors + static_cast<int64_t>(blockIdx.x) * o.cursor_stride;
         int cur = 0, end = 0, r = 0;
@@ -880,9 +957,9 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
         for (int c0 = s0; c0 < s1; c0 += kNumThreads) {
             cur = end = 0;
             if (c0 + tid < s1) {
-                slot_run(o, task, c0 + tid, &cur, &end);
+                slot_run<Slots<false>>(o, task, c0 + tid, &cur, &end);
                 r = o.a_r[c0 + tid];
-                av = a_vals[c0 + tid];
+                av = o.a_vals[c0 + tid];
                 if (!one)
                     cursors[c0 - s0 + tid] = make_int2(cur, end);
             }
@@ -959,12 +1036,12 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
                         cur = run.x;
                         end = run.y;
                         r = o.a_r[c0 + tid];
-                        av = a_vals[c0 + tid];
+                        av = o.a_vals[c0 + tid];
                     }
                 }
                 const int from = cur;
                 if (cur < end)
-                    cur = gallop(o.b_col, cur, end, lim);
+                    cur = gallop([&](int64_t e) { return o.b_col[e]; }, cur, end, lim);
                 if (!one && c0 + tid < s1)
                     cursors[c0 - s0 + tid].x = cur;
                 for_products<Product>(
@@ -998,13 +1075,19 @@ __global__ __launch_bounds__(kNumThreads, 4) void numeric_slab_kernel(SlabOps o,
 
 } // namespace
 
-static SlabOps slab_ops(const DevTiles &a, const SpgemmWork *w, const SlabTasks &tasks, int *queue,
+static SlabOps slab_ops(const DevTiles &a, const DevTiles *b, const SpgemmWork *w, const SlabTasks &tasks, int *queue,
                         int static_rows)
 {
-    SlabOps o;
+    SlabOps o{};
+    if (b) {
+        o.a_trp = a.tile_row_ptr.as<int>();
+        o.a_meta = a.meta.as<int4>();
+        o.b_meta = b->records.as<int4>();
+        o.b_groups = b->row_groups.as<int>();
+    }
     o.a_row_off = a.row_payload_off.as<int>();
     if (w->slot_codes_ready) {
-        o.a_code_off = nullptr;
+        o.a_code_off = o.a_row_off;
         o.a_k = w->slot_k.as<int>();
         o.a_r = w->slot_r.as<uint8_t>();
     } else {
@@ -1012,7 +1095,7 @@ static SlabOps slab_ops(const DevTiles &a, const SpgemmWork *w, const SlabTasks 
         o.a_k = w->row_slot_k.as<int>();
         o.a_r = w->row_slot_r.as<uint8_t>();
     }
-    o.a_vals = a.values.as<double>();
+    o.a_vals = w->slot_codes_ready ? a.values.as<double>() : w->row_slot_v.as<double>();
     o.b_start = w->b_start.as<int>();
     o.b_col = w->b_col.as<int>();
     o.b_val = w->b_val.as<double>();
@@ -1141,13 +1224,15 @@ int slab_prepare(const DevTiles &a, const DevTiles &b, BuildWork *bw, SpgemmWork
                 RTT_TRY(w->code_off.ensure(rows_a * sizeof(int)));
                 RTT_TRY(w->row_slot_k.ensure(slots * sizeof(int)));
                 RTT_TRY(w->row_slot_r.ensure(slots));
+                RTT_TRY(w->row_slot_v.ensure(slots * sizeof(double)));
             }
             hipLaunchKernelGGL(pick_rows_kernel, dim3(static_cast<unsigned>(listed), 4), dim3(256),
                                0, s, rows, n, more, longest, a.tile_row_ptr.as<int>(),
-                               a.meta.as<int4>(), a.row_payload_off.as<int>(), flag,
+                               a.meta.as<int4>(), a.row_payload_off.as<int>(), a.values.as<double>(), flag,
                                codes ? w->code_off.as<int>() : nullptr,
                                codes ? w->row_slot_k.as<int>() : nullptr,
-                               codes ? w->row_slot_r.as<uint8_t>() : nullptr);
+                               codes ? w->row_slot_r.as<uint8_t>() : nullptr,
+                               codes ? w->row_slot_v.as<double>() : nullptr);
             hipLaunchKernelGGL(list_rows_kernel, dim3(blocks_for(R, 256)), dim3(256), 0, s, R, flag,
                                picked, list);
             g.list = list;
@@ -1204,10 +1289,28 @@ static SlabStage slab_stage(const SpgemmWork *w, unsigned long long *cursor)
     return ss;
 }
 
-int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
-                  int static_rows, unsigned long long *cursor, int64_t longest)
+// Whether the symbolic passes go by tiles: where an A tile of the rows and a B
+// tile carry several products on average (spread evenly, a quarter of the
+// product of their entries), one select of their masks does for all of them,
+// and where it has no more runs to start than entries (kRuns a tile: a hub of
+// 1.7 entries a tile in a 1000^2 Laplacian took 10.5 ms by tiles, 3.4 by entries).  All but the
+// numeric pass of 16384 rows of 100 random full 8x8 blocks a tile row, 256
+// products a pair: 18.6 ms by entries, 2.3 by tiles (their first call 60 and 28
+// ms, 44 with the passes before these); 40 such blocks at 8 % (1.9): 0.55 and
+// 0.52 ms; R-MAT 2^18 (0.5): 16.2 and 19.6; a band of 8000 at 2 % (0.5): 9.3
+// and 11.7.
+bool slab_by_tiles(const DevTiles &b, const SlabSizes &rows)
 {
-    RTT_TRY(slab_cursors(w, longest));
+    const double fa = static_cast<double>(rows.slots) / static_cast<double>(rows.tiles);
+    const double fb = static_cast<double>(b.payload) / static_cast<double>(b.num_tiles);
+    return fa * fb / 4.0 >= kTileProducts && fa >= kRuns && rows.most_tiles <= INT_MAX / kRuns;
+}
+
+int slab_symbolic(const DevTiles &a, const DevTiles &b, SpgemmWork *w, const SlabTasks &tasks,
+                  int *queue, int static_rows, unsigned long long *cursor, const SlabSizes &rows)
+{
+    w->slab_by_tiles = slab_by_tiles(b, rows);
+    RTT_TRY(slab_cursors(w, w->slab_by_tiles ? kRuns * rows.most_tiles : rows.longest));
     // Staging of the rows' tile lists: grown to what the previous calls
     // needed, within a quarter of the free device memory; without it every
     // row is recomputed by the fill pass.
@@ -1224,20 +1327,31 @@ int slab_symbolic(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int 
         clear_error();
     }
     RTT_TRY(w->slab_task_size.ensure(static_cast<size_t>(tasks.most) * sizeof(TaskSize)));
-    hipLaunchKernelGGL((symbolic_slab_kernel<false>), dim3(w->slab_cursor_blocks), dim3(kSymThreads),
-                       0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows),
-                       w->row_tiles.as<int64_t>(), w->row_nnz.as<int64_t>(), slab_stage(w, cursor),
-                       COut{});
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(w->slab_cursor_blocks), dim3(kSymThreads), 0, ctx().stream,
+                           slab_ops(a, &b, w, tasks, queue, static_rows), w->row_tiles.as<int64_t>(),
+                           w->row_nnz.as<int64_t>(), slab_stage(w, cursor), COut{});
+    };
+    if (w->slab_by_tiles)
+        launch(symbolic_slab_kernel<false, true>);
+    else
+        launch(symbolic_slab_kernel<false, false>);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
 
-int slab_structure(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *queue,
-                   int static_rows, const COut &c)
+int slab_structure(const DevTiles &a, const DevTiles &b, SpgemmWork *w, const SlabTasks &tasks,
+                   int *queue, int static_rows, const COut &c)
 {
-    hipLaunchKernelGGL((symbolic_slab_kernel<true>), dim3(w->slab_cursor_blocks), dim3(kSymThreads),
-                       0, ctx().stream, slab_ops(a, w, tasks, queue, static_rows), nullptr,
-                       nullptr, slab_stage(w, nullptr), c);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(w->slab_cursor_blocks), dim3(kSymThreads), 0, ctx().stream,
+                           slab_ops(a, &b, w, tasks, queue, static_rows), nullptr, nullptr,
+                           slab_stage(w, nullptr), c);
+    };
+    if (w->slab_by_tiles)
+        launch(symbolic_slab_kernel<true, true>);
+    else
+        launch(symbolic_slab_kernel<true, false>);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }
@@ -1247,7 +1361,7 @@ int slab_numeric(const DevTiles &a, SpgemmWork *w, const SlabTasks &tasks, int *
 {
     RTT_TRY(slab_cursors(w, longest));
     hipLaunchKernelGGL(numeric_slab_kernel, dim3(std::max(1u, w->slab_cursor_blocks / 2)), dim3(kNumThreads), 0,
-                       ctx().stream, slab_ops(a, w, tasks, queue, static_rows), c);
+                       ctx().stream, slab_ops(a, nullptr, w, tasks, queue, static_rows), c);
     RTT_HIP(hipGetLastError());
     return RTT_OK;
 }

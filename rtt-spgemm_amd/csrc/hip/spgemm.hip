@@ -151,6 +151,8 @@ enum Counter : int {
     kCtrSymSlab,     // rows that outgrew the workgroup table too
     kCtrSlabTiles,   // slab tiles the staging cursor handed out
     kCtrLongest,     // most A payload slots in a slab row
+    kCtrMostTiles,   // most A tiles in one
+    kCtrSymSizes,    // A tiles (upper half) and payload slots of the symbolic pass's
     kCtrRows,        // rows of each RowClass, kRowClasses of them
     kCtrTicket = kCtrRows + kRowClasses,
     kCtrDone,
@@ -222,42 +224,6 @@ __device__ __forceinline__ void sizes_init(const SizesInit &z)
 __device__ __forceinline__ uint32_t slot_of(int j, int bits)
 {
     return hash_tile_col(j) >> (32 - bits);
-}
-
-__device__ __forceinline__ uint32_t byte_of(uint32_t v, int k) { return (v >> (8 * k)) & 0xFFu; }
-
-// Byte k is nonzero where byte k of v is (its bit 7 set).
-__device__ __forceinline__ uint32_t nonzero_tops(uint32_t v)
-{
-    return (((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v) & 0x80808080u;
-}
-
-// An A tile spread for products with many B tiles: word k of lo (hi) is 0xFF
-// in byte r where row r (row 4 + r) has an entry in column k.
-__device__ __forceinline__ void spread_tile(uint32_t ab, uint4 *lo, uint4 *hi)
-{
-    uint64_t s[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        s[k] = rows_to_bytes(byte_of(ab, k));
-    *lo = make_uint4(static_cast<uint32_t>(s[0]), static_cast<uint32_t>(s[1]),
-                     static_cast<uint32_t>(s[2]), static_cast<uint32_t>(s[3]));
-    *hi = make_uint4(static_cast<uint32_t>(s[0] >> 32), static_cast<uint32_t>(s[1] >> 32),
-                     static_cast<uint32_t>(s[2] >> 32), static_cast<uint32_t>(s[3] >> 32));
-}
-
-// Structural product of a spread A tile and the per-k column bytes of a B
-// tile: byte k of b_bytes to every byte of a word, then a bitwise select each.
-__device__ __forceinline__ uint64_t spread_product(const uint4 &lo, const uint4 &hi,
-                                                   uint32_t b_bytes)
-{
-    const uint32_t b0 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x00000000u);
-    const uint32_t b1 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x01010101u);
-    const uint32_t b2 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x02020202u);
-    const uint32_t b3 = __builtin_amdgcn_perm(b_bytes, b_bytes, 0x03030303u);
-    const uint32_t l = (lo.x & b0) | (lo.y & b1) | (lo.z & b2) | (lo.w & b3);
-    const uint32_t h = (hi.x & b0) | (hi.y & b1) | (hi.z & b2) | (hi.w & b3);
-    return (static_cast<uint64_t>(h) << 32) | l;
 }
 
 template <typename T>
@@ -588,8 +554,6 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
             row_tiles[row] = 0;
             row_nnz[row] = 0;
             slab_rows[atomicAdd(&ctr[kCtrSymSlab], 1ull)] = row;
-            atomicMax(&ctr[kCtrLongest],
-                      static_cast<unsigned long long>(g.a_row_off[row + 1] - g.a_row_off[row]));
         }
         return;
     }
@@ -1311,6 +1275,8 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
     const int64_t i = b * kSizeThreads + tid;
     unsigned long long nt = 0, nz = 0;
     int cls = -1;   // list the row goes to, kRowClasses for an outgrown row
+    bool slab = false, sym_slab = false;
+    int slots_of = 0, tiles_of = 0;
     if (i < n) {
         const int lv = level[i];
         const bool sized = lv == kLevelLds || (lv == kLevelSlab && slab_done);
@@ -1330,9 +1296,33 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
                   : fits_row<MediumRow>(t, z, alen) ? kRowMid
                   : fits_row<LargeRow>(t, z, alen)  ? kRowLarge
                                                     : kRowSlab;
-            if (cls == kRowSlab)
-                atomicMax(&ctr[kCtrLongest], static_cast<unsigned long long>(alen));
         }
+        slab = (lv == kLevelSlab && !slab_done) || cls == kRowSlab;
+        sym_slab = lv == kLevelSlab && !slab_done;
+        if (slab)
+            slots_of = static_cast<int>(alen), tiles_of = a_tiles;
+    }
+    // Sizes of the slab rows, an atomic each for a wave that has some: one for
+    // every row took 20 us of a pass over 2000 of them.
+    if (__any(slab)) {
+        unsigned long long sum =
+            sym_slab ? (static_cast<unsigned long long>(tiles_of) << 32) |
+                           static_cast<unsigned int>(slots_of)
+                     : 0ull;
+        sum = wave_sum(sum);
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            slots_of = max(slots_of, __shfl_xor(slots_of, o, kWave));
+            tiles_of = max(tiles_of, __shfl_xor(tiles_of, o, kWave));
+        }
+        if (lane_id() == 0) {
+            atomicMax(&ctr[kCtrLongest], static_cast<unsigned long long>(slots_of));
+            atomicMax(&ctr[kCtrMostTiles], static_cast<unsigned long long>(tiles_of));
+            if (sum)
+                atomicAdd(&ctr[kCtrSymSizes], sum);
+        }
+        // There before the workgroup counts as done, whichever wave this is.
+        __threadfence();
     }
     const unsigned long long ix = wave_inclusive_scan(nt), iy = wave_inclusive_scan(nz);
     if (lane_id() == kWave - 1) {
@@ -1402,12 +1392,15 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
         __hip_atomic_store(&ctr[kCtrTiles], px + all_x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&ctr[kCtrNnz], py + all_y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (tid == 0) {
-        __threadfence();
-        if (atomicAdd(&ctr[kCtrDone], 1ull) + 1 == gridDim.x) {
+    if (w == 0) {
+        int last = 0;
+        if (tid == 0) {
             __threadfence();
-            for (int c = 0; c < kCtrTicket; ++c)
-                host[c] = __hip_atomic_load(&ctr[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = atomicAdd(&ctr[kCtrDone], 1ull) + 1 == gridDim.x ? 1 : 0;
+        }
+        if (__shfl(last, 0, kWave) && tid < kCtrTicket) {
+            __threadfence();
+            host[tid] = __hip_atomic_load(&ctr[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -1678,16 +1671,21 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     const int static_rows = lb_mode == RTT_LB_STATIC ? 1 : 0;
     const bool by_cost = lb_mode == RTT_LB_ADAPTIVE_TAIL;
     SlabTasks tasks;
-    // Rows for the slab kernels: those that outgrew both tables, and those whose
-    // C outgrows the numeric kernels'.
-    RTT_TRY(slab_prepare(a, b, b_work, w, w->sym_slab_rows.as<int>(), n_slab, lists.rows[kRowSlab],
-                         static_cast<int>(hctr[kCtrRows + kRowSlab]),
-                         static_cast<int64_t>(hctr[kCtrLongest])));
+    // Entry by entry, the symbolic passes need the rows' operands, and those of
+    // the rows whose C outgrows the numeric kernels' come with them.
+    const SlabSizes sym_rows{static_cast<int64_t>(hctr[kCtrLongest]),
+                             static_cast<int64_t>(hctr[kCtrMostTiles]),
+                             static_cast<int64_t>(hctr[kCtrSymSizes] & 0xFFFFFFFFull),
+                             static_cast<int64_t>(hctr[kCtrSymSizes] >> 32)};
+    const bool entries_first = n_slab > 0 && !slab_by_tiles(b, sym_rows);
+    if (entries_first)
+        RTT_TRY(slab_prepare(a, b, b_work, w, w->sym_slab_rows.as<int>(), n_slab,
+                             lists.rows[kRowSlab], static_cast<int>(hctr[kCtrRows + kRowSlab]),
+                             static_cast<int64_t>(hctr[kCtrLongest])));
     if (n_slab > 0) {
         RTT_TRY(plan_slab_tasks(w->sym_slab_rows.as<int>(), n_slab, by_cost, hctr[kCtrPairs], g, w,
                                 s, &tasks));
-        RTT_TRY(slab_symbolic(a, w, tasks, queue, static_rows, ctr + kCtrSlabTiles,
-                              static_cast<int64_t>(hctr[kCtrLongest])));
+        RTT_TRY(slab_symbolic(a, b, w, tasks, queue, static_rows, ctr + kCtrSlabTiles, sym_rows));
         hipLaunchKernelGGL(sizes_init_kernel, dim3(blocks_for(words, kThreads)), dim3(kThreads), 0,
                                s, again);
         RTT_TRY(finish_sizes(true));
@@ -1698,6 +1696,9 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     for (int k = 0; k < kRowClasses; ++k)
         n_rows[k] = static_cast<int>(hctr[kCtrRows + k]);
     const int n_num_slab = n_rows[kRowSlab];
+    if (n_num_slab > 0 && !entries_first)
+        RTT_TRY(slab_prepare(a, b, b_work, w, lists.rows[kRowSlab], n_num_slab, nullptr, 0,
+                             static_cast<int64_t>(hctr[kCtrLongest])));
     const int64_t total_tiles = static_cast<int64_t>(hctr[kCtrTiles]);
     const int64_t total_nnz = static_cast<int64_t>(hctr[kCtrNnz]);
     const double sym_count_ms = ms_since(t_sym);
@@ -1743,7 +1744,7 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     RTT_HIP(hipGetLastError());
     RTT_HIP(hipEventRecord(ev->ev[3], s));
     if (n_slab > 0)
-        RTT_TRY(slab_structure(a, w, tasks, queue + 1, static_rows, co));
+        RTT_TRY(slab_structure(a, b, w, tasks, queue + 1, static_rows, co));
     if (!ended)
         hipLaunchKernelGGL(set_last_kernel, dim3(1), dim3(1), 0, s,
                            c->tile_nnz.as<int64_t>() + c->num_tiles,

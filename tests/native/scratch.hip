@@ -24,7 +24,8 @@ void cursors_after_a_failed_allocation()
     rtt::SpgemmWork w;
     rtt::DevTiles a;
     const int64_t longest = int64_t(1) << 40;
-    const int rc = rtt::slab_symbolic(a, &w, rtt::SlabTasks{}, nullptr, 0, nullptr, longest);
+    const int rc = rtt::slab_symbolic(a, a, &w, rtt::SlabTasks{}, nullptr, 0, nullptr,
+                                      rtt::SlabSizes{longest, 1, 1, 1});
     expect(rc == RTT_ERR_OOM, "cursors of 2^40 slots are refused");
     expect(w.slab_cursor_stride <= static_cast<int64_t>(w.slab_cursors.bytes / sizeof(int2)),
            "the cursor stride fits the buffer held");
