@@ -441,10 +441,10 @@ int rtt_tilespgemm(const rtt_prepared_a *a, const rtt_dynamic_b *b,
  * (by rtt_tilespgemm with B = b, every row on the TILE path, b not rebuilt
  * since; a values-only rtt_update_b_values in between is what it is for)
  * into c_values, nnz(C) doubles of device memory the caller owns, in C's
- * value order, with `precision` (enum rtt_precision).  Allocates nothing and
- * needs no scratch.  Heavy tiles run whole (no tail split).  Queues one kernel
- * on the library stream and returns;
- * rtt_sync() waits for it. */
+ * value order, with `precision` (enum rtt_precision).  Allocates nothing (the
+ * list of C's wide tile rows that it reads was made with C).  Heavy tiles run
+ * whole (no tail split).  Queues one kernel, or two when C has wide rows, on
+ * the library stream and returns; rtt_sync() waits for them. */
 int rtt_tile_values_noalloc(const rtt_prepared_a *a, const rtt_dynamic_b *b, int precision,
                             double *c_values);
 

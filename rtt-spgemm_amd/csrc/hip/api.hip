@@ -1031,7 +1031,7 @@ int rtt_tile_values_noalloc(const rtt_prepared_a *a, const rtt_dynamic_b *b, int
         return fail(RTT_ERR_INVALID,
                     "rtt_tile_values_noalloc: needs C's structure from an rtt_tilespgemm on this "
                     "(A, B) whose rows all took the TILE path, with B not rebuilt since");
-    return rtt::tile_values_noalloc(a->tiles, b->tiles, a->last_c, precision, c_values,
+    return rtt::tile_values_noalloc(a->tiles, b->tiles, a->last_c, a->core, precision, c_values,
                                     rtt::ctx().stream);
 }
 

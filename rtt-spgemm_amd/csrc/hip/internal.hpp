@@ -199,6 +199,10 @@ struct SpgemmWork {
     // call's start, never while a fill pass may still read the buffer).
     DevBuf slab_stage_j, slab_stage_m, slab_task_size;
     uint64_t slab_stage_cap = 0, slab_stage_need = 0;
+    // Tile-pair path: units of the rows of many C tiles (a count, padded to an
+    // int4, then {row, part, parts, -} each), and the most there can be.
+    DevBuf wide_units;
+    int64_t wide_units_most = 0;
     DevBuf tile_pairs;                      // u64: pairs the tile-pair kernel multiplied, sharded
     PinnedBuf host_tile_stats;              // u64: pairs, tail reason, records, chunks
     // Tail queue of the tile-pair path: records, state, chunk prefix, heavy
@@ -319,11 +323,18 @@ bool tail_possible(int a_tiles, int64_t b_tiles, float threshold);
 struct TileOpts;
 int tile_numeric(const DevTiles &a, const DevTiles &b, const DevC &c, const TileOpts &opt,
                  const TileColumns *tail_columns, SpgemmWork *w, hipStream_t s);
-// C's values for C's existing structure, every row on the tile-pair kernel,
-// written to c_values.  One kernel: no scratch, no allocation, no host
-// synchronisation; no tail split.
-int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, int precision,
-                        double *c_values, hipStream_t s);
+// C's values for C's existing structure, every row on the tile-pair kernels
+// (the wide rows by the units that the call before it planned), written to
+// c_values.  Kernels alone: no allocation, no host synchronisation; no tail
+// split.
+int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, const SpgemmWork &w,
+                        int precision, double *c_values, hipStream_t s);
+// Cuts the tile-pair rows of more than kWideTiles C tiles, wide_rows of them with
+// wide_tiles C tiles, into the units of their own kernel (w->wide_units); C's
+// tile_ptr is written.  For tile_numeric and tile_values_noalloc.
+constexpr int kWideTiles = 64;
+int plan_wide_rows(const DevTiles &a, const DevC &c, float fill, int64_t wide_rows,
+                   int64_t wide_tiles, SpgemmWork *w, hipStream_t s);
 // The admitted records (slot order): tile, merge scans and matches, chunks.
 int tail_records(SpgemmWork *w, int max_records, long long *task, int *scans, int *matches,
                  int *chunks, int *count);

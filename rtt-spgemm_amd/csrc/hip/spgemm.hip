@@ -154,10 +154,14 @@ enum Counter : int {
     kCtrMostTiles,   // most A tiles in one
     kCtrSymSizes,    // A tiles (upper half) and payload slots of the symbolic pass's
     kCtrRows,        // rows of each RowClass, kRowClasses of them
-    kCtrTicket = kCtrRows + kRowClasses,
+    kCtrWide = kCtrRows + kRowClasses,   // tile-pair rows of many C tiles: the rows (upper 28
+                                         // bits) and their C tiles
+    kCtrTicket,
     kCtrDone,
     kCounters
 };
+
+constexpr int kWideRowShift = 36;
 
 struct Operands {
     int a_tile_rows;
@@ -1277,6 +1281,7 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
     int cls = -1;   // list the row goes to, kRowClasses for an outgrown row
     bool slab = false, sym_slab = false;
     int slots_of = 0, tiles_of = 0;
+    unsigned long long wide = 0;
     if (i < n) {
         const int lv = level[i];
         const bool sized = lv == kLevelLds || (lv == kLevelSlab && slab_done);
@@ -1297,6 +1302,8 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
                   : fits_row<LargeRow>(t, z, alen)  ? kRowLarge
                                                     : kRowSlab;
         }
+        if (sized && nt > kWideTiles && tile_routed(tile_fill, a_tiles, static_cast<int>(alen)))
+            wide = (1ull << kWideRowShift) + nt;
         slab = (lv == kLevelSlab && !slab_done) || cls == kRowSlab;
         sym_slab = lv == kLevelSlab && !slab_done;
         if (slab)
@@ -1323,6 +1330,12 @@ __global__ __launch_bounds__(kSizeThreads) void row_sizes_kernel(
         }
         // There before the workgroup counts as done, whichever wave this is.
         __threadfence();
+    }
+    if (__any(wide != 0)) {
+        wide = wave_sum(wide);
+        if (lane_id() == 0)
+            atomicAdd(&ctr[kCtrWide], wide);
+        __threadfence();   // (likewise)
     }
     const unsigned long long ix = wave_inclusive_scan(nt), iy = wave_inclusive_scan(nz);
     if (lane_id() == kWave - 1) {
@@ -1792,6 +1805,9 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     }
     RTT_HIP(hipEventRecord(ev->ev[4], s));
     if (any_tile) {
+        const unsigned long long wide = hctr[kCtrWide];
+        RTT_TRY(plan_wide_rows(a, *c, tile->fill, static_cast<int64_t>(wide >> kWideRowShift),
+                               static_cast<int64_t>(wide & ((1ull << kWideRowShift) - 1ull)), w, s));
         RTT_TRY(tile_numeric(a, b, *c, *tile, tail ? &columns : nullptr, w, s));
         RTT_HIP(hipEventRecord(ev->ev[5], s));
     }

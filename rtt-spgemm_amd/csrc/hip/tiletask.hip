@@ -37,8 +37,7 @@
 #include <cmath>
 #include <vector>
 
-#include "device.hpp"
-#include "internal.hpp"
+#include "core.hpp"
 
 namespace rtt {
 
@@ -56,6 +55,7 @@ constexpr int kEnumRounds = 2;  // rounds of 64 B tiles whose metas are loaded t
 constexpr int kXcdChunk = 4;    // workgroups of consecutive units dealt to an XCD at a time
 constexpr int kPairShards = 256;   // counters of the pairs multiplied, a 128-byte line each (one
 constexpr int kShardStride = 16;   // counter would take an atomic from every wave)
+constexpr int kWideLeast = 32, kWideMost = 512;   // C tiles of a wide row's unit
 constexpr int kMaxParts = 4;    // most units a tile row is cut into
 constexpr int kPairWords = kPairCap / 64;
 constexpr int kPad = 2 * kBatch;   // pairs of zeros past a list: the batch that its last pairs
@@ -70,6 +70,7 @@ struct TileTask {
     const double *__restrict__ a_vals;   // A payload, each tile row-major
     const int4 *__restrict__ a_brange;   // per A tile: {first B tile of row K, -, tiles}
     const int4 *__restrict__ b_meta;     // B tiles row by row: {J, mask, bytes, offset | dense}
+    const int *__restrict__ b_groups;    // start of each (row, class) run of B
     const double *__restrict__ b_vals;   // B payload, each tile column-major
     uint32_t a_zero, b_zero;             // slots past the payloads that hold 0.0
     const int *__restrict__ b_cptr;      // tail only: B tile column pointer
@@ -198,6 +199,7 @@ struct Fp64Product {
     // columns.  B tiles loaded whole and spread by lane permutes, a third of
     // the cache accesses, were slower (2.01 against 1.90).
     static constexpr int kOccupancy = 5;
+    static constexpr int kWideOccupancy = 4;
 
     // C values on their way out: `count` values from `base` on wait in `vals`.
     // The C tiles of a row lie one behind the other, so they leave together,
@@ -470,6 +472,7 @@ struct SplitProduct {
     // Loading the next batch's B entries before the current one is worked on
     // was no faster: vector instructions take 80 % of its cycles.
     static constexpr int kOccupancy = 3;
+    static constexpr int kWideOccupancy = 3;
 
     // Lane's output with the FP64-fallback partial added (every lane takes part
     // in the shuffle).
@@ -839,6 +842,8 @@ void tile_numeric_kernel(TileTask g)
     if (row >= g.rows)
         return;
     const int64_t r0 = g.c_ptr[row], nt = g.c_ptr[row + 1] - r0;
+    if (nt > kWideTiles)
+        return;   // tile_wide_kernel's
     const int64_t c0 = r0 + nt * part / g.parts, c1 = r0 + nt * (part + 1) / g.parts;
     const int a0 = g.a_trp[row];
     const int na = g.a_trp[row + 1] - a0;
@@ -863,6 +868,272 @@ void tile_numeric_kernel(TileTask g)
     }
     if (lane == 0 && done && g.mfma_pairs)
         atomicAdd(&g.mfma_pairs[blockIdx.x % kPairShards * kShardStride], done);
+}
+
+// ---------------------------------------------------------------------------
+// Rows of more than kWideTiles C tiles.  tile_row above enumerates all of the
+// row's B tiles again for every 64 C tiles and every kPairCap pairs of those:
+// for rows of hundreds of C tiles that is most of its time.  Here a lane keeps,
+// for its A tile, where it is in each class run of its B row (whose columns
+// ascend), and takes only the tiles between the first and last column of the
+// next few C tiles, as many of those as make one list: every pair is met once.
+// The A tiles go 64 at a time around that, so a C tile's sum waits in C between
+// them; a tile sums the same pairs in the same order as in tile_row.
+// A unit is a stretch of a row's C tiles, of a length that fills the chip.
+// R-MAT 2^17 (edge factor 8) on this path: 5434 -> 62 ms; dense 4096^2: 537 -> 19;
+// 200-wide band of 100000 rows (up to 63 C tiles a row and more): 12.3 -> 8.1.
+// Rows of few C tiles stay with tile_row, which starts sooner: with no limit the
+// 200k-node FEM square took 1.48 ms against 1.22, dense 256^2 0.42 against 0.35;
+// with one of 256 the band 12.4 and dense 2048^2 65 ms against 3.2.
+// ---------------------------------------------------------------------------
+constexpr int kRuns = 5;   // classes of a row of B: heavy, light k = 0..3
+constexpr int kWideList = 2 * kWave;   // B tiles taken at a time
+static_assert(kWideList <= kPairCap, "their pairs are one list");
+
+struct WideStage {
+    int4 pm[kPairCap + kPad];         // as in WaveStage
+    double out[kOutVals];
+    unsigned long long word[kWave];
+    unsigned long long ends[kPairWords + 1];
+    int2 am[kWave];
+    int start[kWave];                 // per A tile: its first B tile in the enumeration
+    int lo[kRuns][kWave];             // per A tile: first B tile taken of each run,
+    int cum[kRuns - 1][kWave];        // and the tiles taken of the runs up to each
+    int cj[kWave];
+    int base[kWave];
+};
+
+// First tile of [lo, hi), columns ascending, in column j or beyond: doubling
+// steps, then a binary search in the last one.
+__device__ __forceinline__ int tile_at(const int4 *__restrict__ meta, int lo, int hi, int j)
+{
+    int64_t step = 1;
+    while (lo + step <= hi && meta[lo + step - 1].x < j) {
+        lo += static_cast<int>(step);
+        step <<= 1;
+    }
+    int end = static_cast<int>(min<int64_t>(lo + step - 1, hi));
+    while (lo < end) {
+        const int mid = (lo + end) >> 1;
+        if (meta[mid].x < j)
+            lo = mid + 1;
+        else
+            end = mid;
+    }
+    return lo;
+}
+
+template <class P>
+__global__ __launch_bounds__(kTThreads) __attribute__((amdgpu_waves_per_eu(P::kWideOccupancy)))
+void tile_wide_kernel(TileTask g, const int4 *__restrict__ units,
+                      const unsigned long long *__restrict__ n_units)
+{
+    __shared__ WideStage s_wave[kTWaves];
+    const int w = threadIdx.x / kWave;
+    const int lane = lane_id();
+    WideStage &s = s_wave[w];
+    const int64_t u =
+        static_cast<int64_t>(xcd_chunk_row<kXcdChunk>(static_cast<int>(blockIdx.x),
+                                                      static_cast<int>(gridDim.x))) * kTWaves + w;
+    if (u >= static_cast<int64_t>(*n_units))
+        return;
+    const int4 unit = units[u];
+    const int row = __builtin_amdgcn_readfirstlane(unit.x),
+              part = __builtin_amdgcn_readfirstlane(unit.y),
+              parts = __builtin_amdgcn_readfirstlane(unit.z);
+    const int64_t r0 = g.c_ptr[row], nt = g.c_ptr[row + 1] - r0;
+    const int64_t c0 = r0 + nt * part / parts, c1 = r0 + nt * (part + 1) / parts;
+    const int a0 = g.a_trp[row];
+    const int na = g.a_trp[row + 1] - a0;
+    const bool heavy_on = g.heavy && g.tail->enabled;
+    const typename P::Lane ln(lane);
+    // Sums of C tiles that wait for later A tiles.
+    if (na > kWave) {
+        for (int64_t i = g.c_off[c0] + lane; i < g.c_off[c1]; i += kWave)
+            g.c_val[i] = 0.0;
+        __threadfence_block();
+    }
+    unsigned long long done = 0;
+    for (int ag = 0; ag < na; ag += kWave) {
+        const int n = min(kWave, na - ag);
+        // The lane's A tile: where it is in the runs of its B row, the column
+        // there, and the runs' ends.
+        int cur[kRuns], end[kRuns], head[kRuns];
+#pragma unroll
+        for (int c = 0; c < kRuns; ++c) {
+            cur[c] = end[c] = 0;
+            head[c] = INT_MAX;
+        }
+        if (lane < n) {
+            const int4 m = g.a_meta[a0 + ag + lane];
+            s.am[lane] = make_int2(static_cast<int>(list_mask(m.y, m.w)),
+                                   static_cast<int>(static_cast<uint32_t>(m.w) & ~kDense));
+            const int *gp = g.b_groups + static_cast<int64_t>(kClassSlots) * m.x;
+#pragma unroll
+            for (int c = 0; c < kRuns; ++c) {
+                cur[c] = gp[c];
+                end[c] = gp[c + 1];
+                head[c] = cur[c] < end[c] ? g.b_meta[cur[c]].x : INT_MAX;
+            }
+        }
+        int width = kWave;
+        for (int64_t cc = c0; cc < c1;) {
+            width = static_cast<int>(min<int64_t>(width, c1 - cc));
+            unsigned long long cm = 0;
+            long long co = 0;
+            int cj = INT_MAX;
+            bool whole = false;   // not a heavy tile (the chunk kernels compute those)
+            if (lane < width) {
+                const int64_t t = cc + lane;
+                cj = g.c_col[t];
+                cm = g.c_mask[t];
+                co = g.c_off[t];
+                whole = !(heavy_on && ((g.heavy[t >> 5] >> (t & 31)) & 1u));
+            }
+            const int first = read_lane(cj, 0);
+            int to[kRuns], nb = 0;
+#pragma unroll
+            for (int c = 0; c < kRuns; ++c) {
+                if (head[c] < first) {
+                    cur[c] = tile_at(g.b_meta, cur[c], end[c], first);
+                    head[c] = cur[c] < end[c] ? g.b_meta[cur[c]].x : INT_MAX;
+                }
+                to[c] = end[c];
+            }
+            int incl = 0, total = 0;
+            for (;;) {
+                const int last = read_lane(cj, width - 1);
+                nb = 0;
+#pragma unroll
+                for (int c = 0; c < kRuns; ++c) {
+                    to[c] = head[c] <= last ? tile_at(g.b_meta, cur[c] + 1, to[c], last + 1) : cur[c];
+                    nb += to[c] - cur[c];
+                }
+                incl = wave_inclusive_scan(nb);
+                total = last_lane(incl);
+                // (One C tile meets at most one B tile per A tile.)
+                if (total <= kWideList || width == 1)
+                    break;
+                width >>= 1;
+            }
+            const bool in = lane < width;
+            const int step = width;
+            if (total > 0) {
+                s.cj[lane] = in ? cj : INT_MAX;
+                s.start[lane] = incl - nb;
+                s.word[lane] = 0ull;
+                int sum = 0;
+#pragma unroll
+                for (int c = 0; c < kRuns; ++c) {
+                    s.lo[c][lane] = cur[c] - sum;
+                    sum += to[c] - cur[c];
+                    if (c < kRuns - 1)
+                        s.cum[c][lane] = sum;
+                }
+                if (lane < kPairWords)
+                    s.ends[lane] = 0ull;
+                wave_sync();
+                int key[2], bm[2], bo[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int p = i * kWave + lane;
+                    key[i] = -1;
+                    if (p < total) {
+                        const int k = upper_index(s.start, n, p);
+                        const int q = p - s.start[k];
+                        int c = 0;
+#pragma unroll
+                        for (int x = 0; x < kRuns - 1; ++x)
+                            c += q >= s.cum[x][k] ? 1 : 0;
+                        const int4 m = g.b_meta[s.lo[c][k] + q];
+                        int at = 0;   // the C tiles with smaller columns
+#pragma unroll
+                        for (int d = kWave / 2; d > 0; d >>= 1)
+                            at += s.cj[at + d - 1] < m.x ? d : 0;
+                        if (s.cj[at] == m.x) {
+                            key[i] = k | (at << 8);
+                            bm[i] = static_cast<int>(list_mask(m.y, m.w));
+                            bo[i] = static_cast<int>(static_cast<uint32_t>(m.w) & ~kDense);
+                            atomicOr(&s.word[at], 1ull << k);
+                        }
+                    }
+                }
+                wave_sync();
+                const unsigned long long word = whole && in ? s.word[lane] : 0ull;
+                const int cnt = __popcll(word);
+                const int pi = wave_inclusive_scan(cnt);
+                const int pairs = last_lane(pi);
+                s.word[lane] = word;
+                s.base[lane] = pi - cnt;
+                if (lane < kPad)
+                    s.pm[pairs + lane] = make_int4(0, 0, 0, 0);
+                if (cnt > 0)
+                    atomicOr(&s.ends[(pi - 1) >> 6], 1ull << ((pi - 1) & 63));
+                wave_sync();
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (key[i] < 0)
+                        continue;
+                    const int c = key[i] >> 8, k = key[i] & 63;
+                    const unsigned long long wd = s.word[c];
+                    if ((wd >> k) & 1ull) {
+                        const int2 m = s.am[k];
+                        s.pm[s.base[c] + __popcll(wd & ((1ull << k) - 1ull))] =
+                            make_int4(m.x, m.y, bm[i], bo[i]);
+                    }
+                }
+                wave_sync();
+                if (pairs > 0) {
+                    unsigned long long ends[kPairWords];
+#pragma unroll
+                    for (int i = 0; i < kPairWords; ++i)
+                        ends[i] = read_lane64(s.ends[i], 0);
+                    P::run(g, ln, g.a_vals, g.a_zero, s.pm, pairs, cnt, ends, __ballot(cnt > 0),
+                           ag > 0 ? ~0ull : 0ull, cm, co, s.out);
+                    done += static_cast<unsigned long long>(pairs);
+                }
+                wave_sync();
+            }
+#pragma unroll
+            for (int c = 0; c < kRuns; ++c)
+                if (to[c] > cur[c]) {
+                    cur[c] = to[c];
+                    head[c] = cur[c] < end[c] ? g.b_meta[cur[c]].x : INT_MAX;
+                }
+            cc += step;
+            if (total <= kWideList / 3)
+                width = min(2 * width, kWave);
+        }
+        if (ag + kWave < na)
+            __threadfence_block();   // other lanes than those that stored them may load the sums
+    }
+    if (lane == 0 && done && g.mfma_pairs)
+        atomicAdd(&g.mfma_pairs[blockIdx.x % kPairShards * kShardStride], done);
+}
+
+// The units of the wide rows: parts of about `target` C tiles.
+__global__ __launch_bounds__(256) void wide_units_kernel(
+    int rows, const int64_t *__restrict__ c_ptr, const int *__restrict__ a_trp,
+    const int *__restrict__ a_row_off, float fill, int target, unsigned long long *n_units,
+    int4 *__restrict__ units)
+{
+    __shared__ int s_tmp[256 / kWave];
+    __shared__ unsigned long long s_base;
+    const int row = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+    int parts = 0;
+    if (row < rows) {
+        const int64_t nt = c_ptr[row + 1] - c_ptr[row];
+        if (nt > kWideTiles && static_cast<float>(a_row_off[row + 1] - a_row_off[row]) >=
+                                   fill * static_cast<float>(a_trp[row + 1] - a_trp[row]))
+            parts = static_cast<int>((nt + target - 1) / target);
+    }
+    int all = 0;
+    const int before = block_exclusive_scan<256 / kWave>(parts, s_tmp, &all);
+    if (threadIdx.x == 0)
+        s_base = all ? atomicAdd(n_units, static_cast<unsigned long long>(all)) : 0ull;
+    __syncthreads();
+    for (int i = 0; i < parts; ++i)
+        units[s_base + before + i] = make_int4(row, i, parts, 0);
 }
 
 // Chunks of a task whose merge takes `scans` steps with `matches` matched
@@ -1217,6 +1488,7 @@ TileTask make_task(const DevTiles &a, const DevTiles &b, const DevC &c, float fi
     g.a_vals = a.values.as<double>();
     g.a_brange = b.a_brange.as<int4>();
     g.b_meta = b.records.as<int4>();
+    g.b_groups = b.row_groups.as<int>();
     g.b_vals = b.payload_values();
     g.a_zero = static_cast<uint32_t>(a.payload);
     g.b_zero = static_cast<uint32_t>(b.payload);   // of B = A^T: A's, whose payload it is
@@ -1235,7 +1507,57 @@ TileTask make_task(const DevTiles &a, const DevTiles &b, const DevC &c, float fi
     return g;
 }
 
+// The rows of the tile-pair kernel, then the wide ones by their units.
+int launch_tiles(const TileTask &g, int precision, unsigned blocks, const SpgemmWork &w,
+                 hipStream_t s)
+{
+    if (precision == 0)
+        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(blocks), dim3(kTThreads), 0, s, g);
+    else
+        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(blocks), dim3(kTThreads), 0, s,
+                           g);
+    if (w.wide_units_most > 0) {
+        const dim3 grid(blocks_for(w.wide_units_most, kTWaves));
+        const unsigned long long *n = w.wide_units.as<unsigned long long>();
+        const int4 *units = w.wide_units.as<int4>() + 1;
+        if (precision == 0)
+            hipLaunchKernelGGL(tile_wide_kernel<Fp64Product>, grid, dim3(kTThreads), 0, s, g, units,
+                               n);
+        else
+            hipLaunchKernelGGL(tile_wide_kernel<SplitProduct>, grid, dim3(kTThreads), 0, s, g,
+                               units, n);
+    }
+    RTT_HIP(hipGetLastError());
+    return RTT_OK;
+}
+
 } // namespace
+
+int plan_wide_rows(const DevTiles &a, const DevC &c, float fill, int64_t wide_rows,
+                   int64_t wide_tiles, SpgemmWork *w, hipStream_t s)
+{
+    w->wide_units_most = 0;
+    if (wide_rows == 0)
+        return RTT_OK;
+    const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    // Twice the waves the chip holds, and no unit so short that finding its
+    // place in every B row shows.
+    const int64_t target = std::min<int64_t>(
+        kWideMost, std::max<int64_t>(kWideLeast, wide_tiles / (2 * cus * 16)));
+    const int64_t most = wide_tiles / target + wide_rows;
+    // One int4 in front: the count.
+    RTT_TRY(w->wide_units.ensure((static_cast<size_t>(most) + 1) * sizeof(int4)));
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(4), 0, s, w->wide_units.as<uint32_t>(),
+                       int64_t(4));
+    const int rows = static_cast<int>(c.tilem);
+    hipLaunchKernelGGL(wide_units_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0, s, rows,
+                       c.tile_ptr.as<int64_t>(), a.tile_row_ptr.as<int>(),
+                       a.row_payload_off.as<int>(), fill, static_cast<int>(target),
+                       w->wide_units.as<unsigned long long>(), w->wide_units.as<int4>() + 1);
+    RTT_HIP(hipGetLastError());
+    w->wide_units_most = most;
+    return RTT_OK;
+}
 
 TileColumns b_columns(const DevTiles &b)
 {
@@ -1395,13 +1717,7 @@ int tile_numeric(const DevTiles &a, const DevTiles &b, const DevC &c, const Tile
         g.heavy = t.heavy;
         g.tail = t.state;
     }
-    if (precision == 0)
-        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(blocks),
-                           dim3(kTThreads), 0, s, g);
-    else
-        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(blocks),
-                           dim3(kTThreads), 0, s, g);
-    RTT_HIP(hipGetLastError());
+    RTT_TRY(launch_tiles(g, precision, blocks, *w, s));
     if (tail_columns) {
         if (precision == 0)
             hipLaunchKernelGGL(tail_chunk_kernel<Fp64Product>, dim3(cus * 4), dim3(kTThreads), 0,
@@ -1419,8 +1735,8 @@ int tile_numeric(const DevTiles &a, const DevTiles &b, const DevC &c, const Tile
     return RTT_OK;
 }
 
-int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, int precision,
-                        double *c_values, hipStream_t s)
+int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, const SpgemmWork &w,
+                        int precision, double *c_values, hipStream_t s)
 {
     if (c.tilem > INT_MAX)
         return fail(RTT_ERR_INVALID, "C has %lld tile rows: beyond the kernel's range",
@@ -1431,14 +1747,7 @@ int tile_values_noalloc(const DevTiles &a, const DevTiles &b, const DevC &c, int
         return RTT_OK;
     unsigned blocks = 0;
     const TileTask g = make_task(a, b, c, 0.f, c_values, nullptr, &blocks);
-    if (precision == 0)
-        hipLaunchKernelGGL(tile_numeric_kernel<Fp64Product>, dim3(blocks),
-                           dim3(kTThreads), 0, s, g);
-    else
-        hipLaunchKernelGGL(tile_numeric_kernel<SplitProduct>, dim3(blocks),
-                           dim3(kTThreads), 0, s, g);
-    RTT_HIP(hipGetLastError());
-    return RTT_OK;
+    return launch_tiles(g, precision, blocks, w, s);
 }
 
 bool tail_possible(int a_tiles, int64_t b_tiles, float threshold)
