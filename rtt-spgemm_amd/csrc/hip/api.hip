@@ -29,7 +29,6 @@ struct rtt_prepared_a {
     rtt::SpgemmWork core;
     rtt::RowRouting routing;  // rows of the tile-pair kernel at the last threshold asked for
     rtt::Events events;
-    rtt::HostRing ring;       // pinned pieces of the host export
     rtt::DevC last_c;
     bool has_c = false;
     uint64_t id = 0;          // unique per preparation (never reused in a process)
@@ -102,10 +101,25 @@ uint64_t register_a()
     return id;
 }
 
+// Pinned pieces of the host exports, one ring for every handle: an export
+// drains it before it returns, and holds the mutex until then.  Given back with
+// the last prepared A (not by a static destructor, which could follow the
+// runtime's own).
+std::mutex g_ring_mu;
+rtt::HostRing *g_ring = nullptr;
+
 void unregister_a(uint64_t id)
 {
-    std::lock_guard<std::mutex> lock(g_live_mu);
-    g_live_a.erase(id);
+    bool none = false;
+    {
+        std::lock_guard<std::mutex> lock(g_live_mu);
+        none = g_live_a.erase(id) && g_live_a.empty();
+    }
+    if (none) {
+        std::lock_guard<std::mutex> lock(g_ring_mu);
+        delete g_ring;
+        g_ring = nullptr;
+    }
 }
 
 bool a_alive(uint64_t id)
@@ -130,26 +144,47 @@ int check_binding(const rtt_prepared_a *a, const rtt_dynamic_b *b, const char *w
 // travels while the threads of host_copy spread another over the (freshly
 // allocated) destination.  A copy straight to pageable memory stages it by one
 // thread, which also takes every page fault: C of the 20k-node FEM product (82
-// MB) took 5 to 18 ms, now 4 to 5 (fresh pages are still to be zeroed).
+// MB) took 5 to 18 ms, now 4 to 5 (fresh pages are still to be zeroed); of 7 KB
+// 0.080 and 0.049 ms.  A ring of a quarter of C a piece was slower (140 KB: 0.073
+// against 0.060 ms), straight copies of small results too (0.075).
 struct HostCopy {
     void *dst;
     const void *src;
     size_t bytes;
 };
 
-int staged_d2h(const HostCopy *items, int n, rtt::HostRing *ring)
+int straight_d2h(const HostCopy *items, int n)
 {
     hipStream_t s = rtt::ctx().stream;
-    if (ring->create() != RTT_OK) {
-        // No pinned memory to be had: straight to the destinations.
-        rtt::clear_error();
-        for (int i = 0; i < n; ++i)
-            if (items[i].bytes)
-                RTT_HIP(hipMemcpyAsync(items[i].dst, items[i].src, items[i].bytes,
-                                       hipMemcpyDeviceToHost, s));
-        RTT_HIP(hipStreamSynchronize(s));
-        return RTT_OK;
+    for (int i = 0; i < n; ++i)
+        if (items[i].bytes)
+            RTT_HIP(hipMemcpyAsync(items[i].dst, items[i].src, items[i].bytes,
+                                   hipMemcpyDeviceToHost, s));
+    RTT_HIP(hipStreamSynchronize(s));
+    return RTT_OK;
+}
+
+int staged_d2h(const HostCopy *items, int n)
+{
+    hipStream_t s = rtt::ctx().stream;
+    std::lock_guard<std::mutex> lock(g_ring_mu);
+    if (!g_ring)
+        g_ring = new (std::nothrow) rtt::HostRing();
+    rtt::HostRing *ring = g_ring;
+    if (!ring || ring->create() != RTT_OK) {
+        rtt::clear_error();   // no pinned memory to be had
+        return straight_d2h(items, n);
     }
+    // Nothing may travel into the ring once the mutex is let go.
+    struct Drain {
+        hipStream_t s;
+        bool done = false;
+        ~Drain()
+        {
+            if (!done)
+                (void)hipStreamSynchronize(s);
+        }
+    } guard{s};
     struct Piece {
         void *dst;
         size_t bytes;
@@ -177,10 +212,11 @@ int staged_d2h(const HostCopy *items, int n, rtt::HostRing *ring)
     }
     while (drained < issued)
         RTT_TRY(drain());
+    guard.done = true;
     return RTT_OK;
 }
 
-int export_c(const rtt::DevC &c, rtt::HostRing *ring, rtt_smatrix *out)
+int export_c(const rtt::DevC &c, rtt_smatrix *out)
 {
     if (c.num_tiles > INT_MAX || c.nnz > INT_MAX || c.tilem > INT_MAX)
         return fail(RTT_ERR_OVERFLOW,
@@ -222,9 +258,9 @@ int export_c(const rtt::DevC &c, rtt::HostRing *ring, rtt_smatrix *out)
         {r.tile_csr_Col, c.tile_csr_col.ptr, Z},
         {r.tile_csr_Value, c.tile_csr_val.ptr, Z * sizeof(double)},
     };
-    const int rc = staged_d2h(items, 6, ring);
+    const int rc = staged_d2h(items, 6);
     if (rc != RTT_OK) {
-        (void)hipStreamSynchronize(rtt::ctx().stream);   // pieces may still be in flight
+        (void)hipStreamSynchronize(rtt::ctx().stream);   // copies may still be in flight
         rtt_destroy_smatrix(&r);
         return rc;
     }
@@ -841,7 +877,7 @@ int rtt_tilespgemm(const rtt_prepared_a *a_const, const rtt_dynamic_b *b, rtt_sm
     stats->heavy_rows = times.heavy_rows;
     if (sc.materialize_output) {
         auto te = rtt::Clock::now();
-        RTT_TRY(export_c(a->last_c, &a->ring, output));
+        RTT_TRY(export_c(a->last_c, output));
         stats->output_copy_ms = rtt::ms_since(te);
         stats->output_materialized = 1;
     }

@@ -228,7 +228,7 @@ struct Events {
 };
 
 // Pinned pieces that copies to pageable host memory travel through, with an
-// event each; created on first use, owned by one handle.
+// event each; created on first use.
 struct HostRing {
     static constexpr int kPieces = 4;
     static constexpr size_t kPieceBytes = size_t(2) << 20;
