@@ -409,18 +409,20 @@ def c1_line(rt, steps=20, warmup=5, repeats=5):
                         "sample": f"whole product, median of {repeats} runs (row SPA, oracle)"}}
 
 
-# Kernel names in the rocprofv3 counter summaries, per breakdown key.
+# Kernel names in the rocprofv3 counter summaries, per breakdown key: the rows of
+# a product go to as many of a key's kernels as it needs.
 PROFILE_KERNELS = {
-    "numeric": "numeric_row_kernel<SpreadRow",
-    "numeric_tile": "tile_numeric_kernel<Fp64Product>",
-    "symbolic_count": "symbolic_wave_kernel",
-    "symbolic_fill": "symbolic_write_kernel",
+    "numeric": ("numeric_row_kernel<", "numeric_slab_kernel"),
+    "numeric_tile": ("tile_numeric_kernel<Fp64Product>", "tile_wide_kernel<Fp64Product>"),
+    "symbolic_count": ("symbolic_wave_kernel",),
+    "symbolic_fill": ("symbolic_write_kernel",),
 }
 
 
 def profile_traffic(workload, kernel):
-    """HBM bytes per launch of `kernel` from the committed rocprofv3 counter
-    summary of this workload: FETCH_SIZE and WRITE_SIZE (KiB per dispatch,
+    """HBM bytes of a call's `kernel` launches (one of each of its kernels that
+    the summary has) from the committed rocprofv3 counter summary of this
+    workload: FETCH_SIZE and WRITE_SIZE (KiB per dispatch,
     from the table whose first counter columns they are), each scaled by what
     the counter reads for a device copy of known size.  None when no summary
     covers the kernel."""
@@ -434,20 +436,20 @@ def profile_traffic(workload, kernel):
     if not m:
         return None, None
     sf, sw = float(m.group(1)), float(m.group(2))
-    name = PROFILE_KERNELS.get(kernel)
-    in_table = False
+    names = PROFILE_KERNELS.get(kernel, ())
+    in_table, total = False, None
     for line in text.splitlines():
         cells = [c.strip(" `") for c in line.strip().strip("|").split("|")]
         if len(cells) >= 3 and cells[0] == "kernel":
             in_table = cells[1].startswith("FETCH_SIZE") and cells[2].startswith("WRITE_SIZE")
             continue
-        if in_table and len(cells) >= 3 and name and cells[0].startswith(name):
+        if in_table and len(cells) >= 3 and cells[0].startswith(names):
             try:
                 fetch_kib, write_kib = float(cells[1]), float(cells[2])
             except ValueError:
                 continue
-            return fetch_kib * 1024 * sf + write_kib * 1024 * sw, os.path.relpath(path, ROOT)
-    return None, None
+            total = (total or 0.0) + fetch_kib * 1024 * sf + write_kib * 1024 * sw
+    return (None, None) if total is None else (total, os.path.relpath(path, ROOT))
 
 
 # The precision and batching forms the metric compares with plain FP64, each

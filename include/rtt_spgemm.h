@@ -400,7 +400,7 @@ typedef struct rtt_stats {       /* DmmaSpGemmStats subset */
     /* device-event durations of the main kernels, last call */
     double symbolic_count_kernel_ms;
     double symbolic_fill_kernel_ms;
-    double numeric_kernel_ms;
+    double numeric_kernel_ms;    /* every numeric kernel the rows took */
     unsigned long long pair_count;     /* (A tile, B tile) products visited */
     unsigned long long output_tiles;   /* 8x8 C tiles */
     unsigned long long output_nnz;     /* nnz(C) */

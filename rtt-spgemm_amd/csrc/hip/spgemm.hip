@@ -1809,7 +1809,6 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
         RTT_TRY(plan_wide_rows(a, *c, tile->fill, static_cast<int64_t>(wide >> kWideRowShift),
                                static_cast<int64_t>(wide & ((1ull << kWideRowShift) - 1ull)), w, s));
         RTT_TRY(tile_numeric(a, b, *c, *tile, tail ? &columns : nullptr, w, s));
-        RTT_HIP(hipEventRecord(ev->ev[5], s));
     }
     auto rows_launch = [&](auto kernel, int cls, int threads, bool every) {
         if (n_rows[cls] > 0)
@@ -1836,8 +1835,6 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     else
         small_launch(SmallRow{});
     RTT_HIP(hipGetLastError());
-    if (!any_tile)
-        RTT_HIP(hipEventRecord(ev->ev[5], s));
     rows_launch(numeric_row_kernel<TinyRow>, kRowTiny, TinyRow::kThreads, false);
     rows_launch(numeric_row_kernel<MediumRow>, kRowMid, MediumRow::kThreads, false);
     rows_launch(numeric_row_kernel<LargeRow>, kRowLarge, LargeRow::kThreads, false);
@@ -1847,6 +1844,7 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
         RTT_TRY(slab_numeric(a, w, tasks, queue + 2, static_rows, co,
                              static_cast<int64_t>(hctr[kCtrLongest])));
     }
+    RTT_HIP(hipEventRecord(ev->ev[5], s));   // behind the numeric kernels of every class
     RTT_HIP(hipStreamSynchronize(s));
     if (any_tile && c->num_tiles > 0) {
         // Written by the last of the tile-pair path's kernels.
