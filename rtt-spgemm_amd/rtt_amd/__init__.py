@@ -275,20 +275,36 @@ def _np_copy(ptr, count: int, dtype) -> np.ndarray:
     return np.array(np.ctypeslib.as_array(buf), dtype=dtype, copy=True)
 
 
+class _HostArray:
+    """Owns one host array the library allocated: the numpy array made of it
+    keeps it alive and frees it (no copy of a result of hundreds of megabytes).
+    Such an array does not own its data to numpy: ndarray.resize refuses it."""
+
+    def __init__(self, address: int):
+        self._s = SMatrix()
+        self._s.columnindex = C.cast(C.c_void_p(address), C.POINTER(C.c_int))
+
+    def __del__(self):
+        if _lib is not None:
+            _lib.rtt_destroy_smatrix(C.byref(self._s))   # frees what the struct holds
+
+
 class _HostArrays:
-    """Owns the host arrays of an SMatrix the library allocated: numpy arrays
-    made with ``view`` keep it alive, and the last of them frees the arrays
-    (no copy of a result of hundreds of megabytes)."""
+    """Hands out the host arrays of an SMatrix the library allocated, each as a
+    numpy array of its own lifetime; what was not taken is freed with this."""
 
     def __init__(self, s: SMatrix):
         self._s = s
 
-    def view(self, ptr, count: int, dtype) -> np.ndarray:
+    def take(self, field: str, count: int, dtype) -> np.ndarray:
+        ptr = getattr(self._s, field)
         if count <= 0 or not ptr:
             return np.zeros(0, dtype=dtype)
+        address = C.cast(ptr, C.c_void_p).value
         ct = np.ctypeslib.as_ctypes_type(np.dtype(dtype))
-        buf = (ct * count).from_address(C.cast(ptr, C.c_void_p).value)
-        buf._owner = self   # the array's base holds buf
+        buf = (ct * count).from_address(address)
+        buf._owner = _HostArray(address)   # the array's base holds buf
+        setattr(self._s, field, type(ptr)())
         return np.frombuffer(buf, dtype=dtype)
 
     def __del__(self):
@@ -298,9 +314,9 @@ class _HostArrays:
 
 def _consume_csr(s: SMatrix) -> CsrMatrix:
     own = _HostArrays(s)
-    out = CsrMatrix(s.m, s.n, own.view(s.rowpointer, s.m + 1, np.int32),
-                    own.view(s.columnindex, s.nnz, np.int32),
-                    own.view(s.value, s.nnz, np.float64), s.isSymmetric)
+    out = CsrMatrix(s.m, s.n, own.take("rowpointer", s.m + 1, np.int32),
+                    own.take("columnindex", s.nnz, np.int32),
+                    own.take("value", s.nnz, np.float64), s.isSymmetric)
     if s.m + 1 > 0 and out.rowptr.size == 0:
         out.rowptr = np.zeros(s.m + 1, np.int32)
     return out
@@ -446,12 +462,12 @@ class TileC:
 def _consume_tilec(s: SMatrix) -> TileC:
     own = _HostArrays(s)
     return TileC(s.m, s.n, s.tilem, s.tilen, s.numtile, s.nnz,
-                 own.view(s.tile_ptr, s.tilem + 1, np.int32),
-                 own.view(s.tile_columnidx, s.numtile, np.int32),
-                 own.view(s.tile_nnz, s.numtile + 1, np.int32),
-                 own.view(s.tile_csr_Ptr, 8 * s.numtile, np.uint8),
-                 own.view(s.tile_csr_Col, s.nnz, np.uint8),
-                 own.view(s.tile_csr_Value, s.nnz, np.float64))
+                 own.take("tile_ptr", s.tilem + 1, np.int32),
+                 own.take("tile_columnidx", s.numtile, np.int32),
+                 own.take("tile_nnz", s.numtile + 1, np.int32),
+                 own.take("tile_csr_Ptr", 8 * s.numtile, np.uint8),
+                 own.take("tile_csr_Col", s.nnz, np.uint8),
+                 own.take("tile_csr_Value", s.nnz, np.float64))
 
 
 def _download_tiles(view: DeviceTiles) -> dict:
