@@ -96,12 +96,16 @@ struct SmallRow {
 // tile, of which such products have many, takes the one row it needs of B's
 // record instead of walking all of it.  The LDS pipe was busy 75 % of the
 // kernel's time and is now 55 %, vector instructions 74 %: 128^3 box stencil,
-// A*A^T (14 entries a C tile), 2.83 -> 2.29 ms; banded products (39 to 49)
-// take 0.59 ms with the extra index work against 0.57 without.
+// A*A^T (14 entries a C tile), 2.83 -> 2.29 ms.  With more to a C tile the extra
+// index work costs more than the conflicts: bands of 400000 rows with 21, 23,
+// 26, 30 and 38 entries a C tile take 0.46, 0.48, 0.50, 0.53 and 0.75 ms a step
+// with it, 0.43, 0.46, 0.49, 0.51 and 0.73 without.  (It is the rows' likeness
+// that counts, which the fill only hints at: block FEM on this path, 31 entries,
+// takes 1.31 ms with it and 1.44 without.)
 struct SpreadRow : SmallRow {
     static constexpr bool kSpread = true;
 };
-constexpr int kSpreadFill = 24;
+constexpr int kSpreadFill = 18;
 // MediumRow takes rows past SmallRow's accumulator with few C tiles and A
 // values (narrow bands squared) at a third of LargeRow's LDS.
 struct MediumRow {
