@@ -63,20 +63,6 @@ __device__ __forceinline__ uint64_t rows_to_bytes(uint32_t rows)
     return (static_cast<uint64_t>(nibble(rows >> 4)) << 32) | nibble(rows & 15u);
 }
 
-// Structural product of an 8x4 A tile mask (bit r*4+k) and a 4x8 B tile
-// mask (bit c*4+k): the 8x8 C tile mask (bit r*8+c).
-__device__ __forceinline__ uint64_t tile_bool_product(uint32_t am, uint32_t bm)
-{
-    uint64_t out = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t rows = stride4_bits(am, k);
-        const uint32_t cols = stride4_bits(bm, k);
-        out |= rows_to_bytes(rows) & (static_cast<uint64_t>(cols) * 0x0101010101010101ull);
-    }
-    return out;
-}
-
 // Payload slot of physical position `phys` of a hybrid tile.
 __device__ __forceinline__ int payload_slot(uint32_t mask, int span, int phys)
 {

@@ -79,8 +79,9 @@ struct TinyRow {
     static constexpr int kWavesPerSimd = 7;
     static constexpr int kAcc = 128, kAStage = 64, kTiles = 16, kSlots = 32, kSlotBits = 5;
 };
-// SmallRow, launched over every row, leaves the rows within TinyRow's
-// budgets to that instance (launched over their list).
+// SmallRow leaves the rows within TinyRow's budgets to that instance.  (Its
+// launch goes over its own rows' list, or over every row where all are its own
+// and in the traced form.)
 struct SmallRow {
     static constexpr int kThreads = 256, kChunk = 64, kSeg = 1024;
     static constexpr bool kLeavesTiny = true, kSpread = false;
@@ -168,21 +169,14 @@ enum Counter : int {
 constexpr int kWideRowShift = 36;
 
 struct Operands {
-    int a_tile_rows;
     const int *__restrict__ a_trp;
     const int4 *__restrict__ a_meta;
     const int4 *__restrict__ a_brange;   // per A tile: first B tile, heavy, count
     const int2 *__restrict__ a_blight;   // per A tile: the light B tiles it can meet
-    const int *__restrict__ a_off;
-    const double *__restrict__ a_vals;
     const double *__restrict__ a_vals_cm;   // A payload, each tile column-major
     const int *__restrict__ a_row_off;      // A payload offset of each tile row
     const double *__restrict__ b_vals_km;   // B payload, each tile k-major
-    const int *__restrict__ b_trp;
     const int4 *__restrict__ b_meta;        // B records' plane 0
-    const int *__restrict__ b_groups;       // per B row: start of each class run (kClassSlots)
-    const double *__restrict__ b_vals;
-    int b_tile_cols;
     float tile_fill;   // rows whose A tiles hold this many values on average go to the
                        // tile-pair kernel (+inf: none)
 };
@@ -459,7 +453,7 @@ __global__ __launch_bounds__(kThreads) void symbolic_count_kernel(
     __shared__ long long s_tmp64[kWavesPerBlock];
     __shared__ int s_ovf;
 
-    const int row = rows ? rows[blockIdx.x] : static_cast<int>(blockIdx.x);
+    const int row = rows[blockIdx.x];
     const int tid = threadIdx.x;
     for (int i = tid; i < kSymSlots; i += kThreads) {
         s_key[i] = kEmpty;
@@ -1579,21 +1573,14 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     c->cols = b.cols;
 
     Operands g;
-    g.a_tile_rows = R;
     g.a_trp = a.tile_row_ptr.as<int>();
     g.a_meta = a.meta.as<int4>();
     g.a_brange = b.a_brange.as<int4>();
     g.a_blight = b.a_blight.as<int2>();
-    g.a_off = a.value_offsets.as<int>();
-    g.a_vals = a.values.as<double>();
     g.a_vals_cm = a.values_cm.as<double>();
     g.a_row_off = a.row_payload_off.as<int>();
     g.b_vals_km = b.payload_kmajor();
-    g.b_trp = b.tile_row_ptr.as<int>();
     g.b_meta = b.records.as<int4>();   // part 0 of every record is the tile's meta
-    g.b_groups = b.row_groups.as<int>();
-    g.b_vals = b.payload_values();
-    g.b_tile_cols = BC;
     g.tile_fill = tile ? tile->fill : INFINITY;
 
     const int num_cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
@@ -1628,10 +1615,10 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     RTT_TRY(w->c_row_nnz_off.ensure((R + 1) * sizeof(int64_t)));
     Stage st{w->stage_j.as<int>(), w->stage_m.as<unsigned long long>(), stage_limit};
     // Queue heads: [0] symbolic slab count, [1] symbolic slab fill, [2] numeric slab.
-    RTT_TRY(w->queue.ensure(4 * sizeof(int)));
+    RTT_TRY(w->queue.ensure(3 * sizeof(int)));
     int *queue = w->queue.as<int>();
     // The pair total was summed by the B update's pair-extent pass.
-    const SizesInit start{ctr, 0, look, words, b.pair_total.as<unsigned long long>(), queue, 4};
+    const SizesInit start{ctr, 0, look, words, b.pair_total.as<unsigned long long>(), queue, 3};
     const SizesInit again{ctr, static_cast<int>(kCtrRows), look, words, nullptr, nullptr, 0};
     // The tail queue needs B's tile columns only if some C tile can clear its
     // threshold: told from B's tile rows where that is enough, else from its
@@ -1748,8 +1735,8 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     RTT_HIP(hipEventRecord(ev->ev[2], s));
     // The numeric LDS kernels write the structure of their own rows from the
     // staged lists; this pass writes it for the staged rows they cannot hold
-    // (the numeric fallback list, whose slab rows it skips).  The tile-pair
-    // path needs the whole structure first: every staged row.
+    // (the numeric fallback list, whose slab rows it skips), and for the rows of
+    // the tile-pair kernels, which need their structure first.
     if (any_tile && R > 0 && c->num_tiles > 0)
         hipLaunchKernelGGL(symbolic_write_kernel, dim3(blocks_for(R, kWavesPerBlock)),
                            dim3(kThreads), 0, s, nullptr, R, st, w->row_level.as<int>(), co,
