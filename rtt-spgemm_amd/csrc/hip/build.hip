@@ -201,8 +201,9 @@ __device__ __forceinline__ int nth_bit(uint32_t m, int n)
 // Four lanes per tile, lane q the values 2q, 2q + 1 of every eight: a wave
 // reads its 16 tiles' values a line at a time and writes 256 contiguous bytes
 // of every plane.  (One lane per tile where tiles hold two values or fewer on
-// average, which the first lane has anyway: four took 1.4 us more on the random
-// rectangular product's 880000.)  With a tile per thread every load met 64 lines, and they
+// average, which the first lane has anyway: four took 1 % more of a step there,
+// scattered columns with 2, 6 and 16 entries a row; above, no difference was seen
+// at two to four values, and the batches below gained.)  With a tile per thread every load met 64 lines, and they
 // were gone from the L1 before a tile's next value was asked for: banded batch
 // 257 -> 168 us, AMG batch 233 -> 222 us (its tiles hold few values).
 template <int L>

@@ -1196,7 +1196,9 @@ int slab_prepare(const DevTiles &a, const DevTiles &b, BuildWork *bw, SpgemmWork
         g.order = bw->keys_in.as<int>();
     }
     // A workgroup per tile row where rows average past 16 tiles (a hub row
-    // holds thousands), a wave otherwise.
+    // holds thousands), a wave otherwise: R-MAT 2^13, 2^16 and 2^18 took 19, 69 and
+    // 370 us in workgroups, 37, 154 and 745 in waves; a 64^3 box stencil with 4096
+    // wide rows 185 and 99, a band of 40 entries a row 16 and 13.
     const bool wide = b.num_tiles > 16 * static_cast<int64_t>(R);
     auto over_rows = [&](auto wave_kernel, auto block_kernel, int64_t count, auto... args) {
         if (wide)

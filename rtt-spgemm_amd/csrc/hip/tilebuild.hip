@@ -18,7 +18,11 @@
 // Tile rows with more than kLongRow entries per scalar row on average would
 // hold one lane each for thousands of steps; a workgroup each counts and
 // fills those, parallel over entries (the hub rows of R-MAT 2^18 held the
-// rebuild to 37 ms; now 1.8 ms).
+// rebuild to 37 ms; now 1.8 ms).  That takes longer than a lane each where most
+// rows are like that, and less where few are: a step of block FEM with 124
+// entries a row (240000 rows) takes 6.2 ms with the limit at 128, 6.5 at 96, and
+// 84 entries 3.0 and 3.4; 40 rows of 400 entries in a 500^2 Laplacian 1.37 and
+// 0.65 ms, a band of 150 entries in 4000 rows 0.49 and 0.37.
 #include <algorithm>
 #include <climits>
 

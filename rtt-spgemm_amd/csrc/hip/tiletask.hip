@@ -190,8 +190,9 @@ struct Fp64Product {
     struct Acc {
         double v = 0.0;
     };
-    // Waves per SIMD the tile kernel is compiled for (94 VGPRs) and its LDS is
-    // cut to: its waves wait for loads more than half of their time.  Block-FEM
+    // Waves per SIMD the tile kernel is compiled for (94 VGPRs); its LDS, 17 KB a
+    // workgroup of two waves, lets nine workgroups on a CU, 4.5 waves per SIMD.
+    // The waves wait for loads more than half of their time.  Block-FEM
     // 500k, 2.16e7 pairs: 1.69 ms (6.5 TFLOP/s on the matrix cores); 1.80 at
     // four waves with 512 A values staged and four enumeration rounds kept,
     // 1.90 with twice the output stage, 1.89 at six waves, batches of four and
