@@ -723,6 +723,9 @@ int rtt_dynamic_b_view(const rtt_dynamic_b *b_const, rtt_device_tiles *view)
     // pointer + packed per-tile records); the remaining DmmaDeviceTiles
     // arrays and the tile CSC are completed here, on first request.
     rtt_dynamic_b *b = const_cast<rtt_dynamic_b *>(b_const);
+    if (b->a_id == 0)   // its arrays may be those of no one build
+        return fail(RTT_ERR_INVALID, "rtt_dynamic_b_view: B has not been built (its last "
+                                     "rebuild failed)");
     if (b->tiles.transpose_of && !a_alive(b->a_id))
         return fail(RTT_ERR_INVALID,
                     "rtt_dynamic_b_view: the A this B = A^T was built from has been destroyed");
