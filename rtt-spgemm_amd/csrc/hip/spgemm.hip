@@ -1567,6 +1567,7 @@ int spgemm_core(const DevTiles &a, DevTiles &b, BuildWork *b_work, DevC *c, Spge
     hipStream_t s = ctx().stream;
     const int R = a.tile_row_count;
     const int BC = b.tile_col_count;
+    w->tail_ran = false;   // until the tail queue admits for this call
     c->tilem = R;
     c->tilen = BC;
     c->rows = a.rows;
