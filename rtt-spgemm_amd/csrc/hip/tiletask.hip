@@ -882,7 +882,7 @@ void tile_numeric_kernel(TileTask g)
 // them; a tile sums the same pairs in the same order as in tile_row.
 // A unit is a stretch of a row's C tiles, of a length that fills the chip.
 // R-MAT 2^17 (edge factor 8) on this path: 5434 -> 62 ms; dense 4096^2: 537 -> 19;
-// 200-wide band of 100000 rows (up to 63 C tiles a row and more): 12.3 -> 8.1.
+// band of 200 either side, 100000 rows (101 C tiles a row): 12.3 -> 8.1.
 // Rows of few C tiles stay with tile_row, which starts sooner: with no limit the
 // 200k-node FEM square took 1.48 ms against 1.22, dense 256^2 0.42 against 0.35;
 // with one of 256 the band 12.4 and dense 2048^2 65 ms against 3.2.
